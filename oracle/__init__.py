@@ -67,12 +67,13 @@ _SIGS = {
 
 
 def build(force=False):
-    """Compile liboracle.so (and oracle/_ref when the reference tree exists)."""
+    """Compile liboracle.so (and oracle/_ref when the reference sources exist)."""
     cmd = ["make", "-s", "-C", HERE]
     if force:
         cmd.append("-B")
     subprocess.run(cmd + ["all"], check=True)
-    if os.path.isdir(os.environ.get("GQF_REFERENCE", "/root/reference")):
+    ref = os.environ.get("GQF_REFERENCE", "/root/reference")
+    if os.path.isfile(os.path.join(ref, "standardQuotientFilter", "CPU_version", "quotientFilter.cpp")):
         subprocess.run(cmd + ["ref"], check=True)
 
 
