@@ -1,0 +1,200 @@
+// gqf_local.hpp -- localized updates: the parts that the SQF's and the RSQF's
+// in-place inserts and deletes of small sorted batches share.
+//
+// A table is cut into windows of LW_SLOTS slots, one wave64 each.  A batch
+// key changes only the slots from its quotient to the end of the cluster
+// there (insert: up to the empty slot it takes; delete: up to the next slot
+// that holds nothing or an entry at its own quotient).  Keys whose ranges
+// meet form a region; a region is updated by one lane, key after key, and
+// regions never share a slot, so they run in parallel.  Three steps:
+//   1. k_*_plan   per window, from the table as it was: what the keys of the
+//                 window need (below), and the window's scan state;
+//   2. lw_scan    the states' exclusive scan over the windows;
+//   3. k_*_apply  per window with keys: the window's slots in LDS, a lane per
+//                 region that starts in the window, the changed 64-slot
+//                 blocks written back.
+// Which keys start a region ("heads"):
+//   insert  with E_k the empty slots before key k's quotient, key k takes the
+//           empty slot of rank J_k = max(E_k, J_{k-1} + 1) at the latest (a
+//           key that is already stored takes none); it starts a region iff
+//           J_{k-1} < E_k.  Over a window with n keys and e empty slots, the
+//           keys that overflow into the next window are x -> max(0, x + n - e,
+//           max_k(E_k - k) + n - e) of those that overflow into it: the
+//           state (a, b) of x -> max(x + a, b).
+//   delete  key k starts a region iff a boundary (a slot that is empty or
+//           whose entry is at its own quotient) lies after key k-1's quotient
+//           and at or before its own; the state is the last boundary.
+// A region that passes its window's end is followed into the table directly
+// by its lane; the next window's wave leaves those slots, and the keys there,
+// alone.  The 64-slot block where a window's first region starts may hold the
+// end of an earlier window's region: it too is updated in the table, slot by
+// slot, and never written back as a whole.
+//   Work is per key and per keyed window; a window without keys is read only
+// when its predecessor has some (it must absorb what overflows).  Batches
+// that do not fit this form raise ctr[CTR_MISC] before anything is written
+// and the call takes its general path: more than LW_KEYS keys in a window,
+// a whole aligned group
+// of 64 keys without a head, fewer than LW_SPILL empty slots in a
+// window (clusters longer than a window), an overflow above LW_SPILL.
+#pragma once
+
+#include "gqf_rebuild.hpp"
+
+namespace gqf {
+
+constexpr uint32_t LW_SLOTS = 4096;  // slots per window: 64 lanes x one 64-slot block
+constexpr uint32_t LW_KEYS = 512;    // keys per window
+constexpr int32_t LW_SPILL = 64;     // keys that may overflow into a window
+constexpr uint32_t LW_MAX_WINDOWS = RBS_PER * 64;  // one state per window: the scan's limit
+
+// Automatic choice: batches of up to 1/32 of the slots, 1/80 where the
+// windows do not fill the chip twice over and the time is that of the
+// longest regions.  SQF inserts, ms per call, localized / rebuild:
+//   q=26 r=5  fill 0.45  2^20 keys 0.134 / 0.286   2^21 0.212 / 0.342   2^22 0.315 / 0.376
+//             fill 0.75  2^20 keys 0.152 / 0.347   2^21 0.267 / 0.401   2^22 0.476 / 0.438
+//             fill 0.8   2^10 keys 0.057 / 0.317   2^21 0.312 / 0.414   2^22 0.612 / 0.457
+//   q=22 r=5  fill 0.75  2^13 keys 0.061 / 0.098   2^16 0.087 / 0.097   2^18 0.179 / 0.103
+//   q=19 r=13 fill 0.8   2^10 keys 0.049 / 0.073   2^13 0.089 / 0.086   2^16 0.118 / 0.091
+static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8192ull * LW_SLOTS) ? 32 : 80) <= slots; }
+
+static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }
+
+// Scan state of a window: overflow map x -> max(x + a, b) (insert), and 1 +
+// the last boundary slot (delete; 0: none).
+struct LW {
+  int32_t a, b;
+  uint32_t lb;
+};
+__host__ __device__ __forceinline__ LW lw_combine(LW x, LW y) {
+  const int32_t b = x.b + y.a;
+  return LW{x.a + y.a, b > y.b ? b : y.b, x.lb > y.lb ? x.lb : y.lb};
+}
+__device__ __forceinline__ LW lw_none() { return LW{0, 0, 0u}; }
+__device__ __forceinline__ uint4 lw_pack(LW x) { return make_uint4((uint32_t)x.a, (uint32_t)x.b, x.lb, 0u); }
+__device__ __forceinline__ LW lw_unpack(uint4 w) { return LW{(int32_t)w.x, (int32_t)w.y, w.z}; }
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ LW lw_dpp(LW x) {
+  return LW{(int32_t)dpp_u32<CTRL, ROW_MASK>(0u, (uint32_t)x.a), (int32_t)dpp_u32<CTRL, ROW_MASK>(0u, (uint32_t)x.b),
+            dpp_u32<CTRL, ROW_MASK>(0u, x.lb)};
+}
+__device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
+  LW inc = x;
+  inc = lw_combine(lw_dpp<DPP_ROW_SHR | 1>(inc), inc);
+  inc = lw_combine(lw_dpp<DPP_ROW_SHR | 2>(inc), inc);
+  inc = lw_combine(lw_dpp<DPP_ROW_SHR | 4>(inc), inc);
+  inc = lw_combine(lw_dpp<DPP_ROW_SHR | 8>(inc), inc);
+  inc = lw_combine(lw_dpp<DPP_ROW_BCAST15, 0xA>(inc), inc);
+  inc = lw_combine(lw_dpp<DPP_ROW_BCAST31, 0xC>(inc), inc);
+  *total = LW{(int32_t)wave_read((uint32_t)inc.a, 63), (int32_t)wave_read((uint32_t)inc.b, 63), wave_read(inc.lb, 63)};
+  return lw_dpp<DPP_WAVE_SHR1>(inc);
+}
+// Inclusive maximum over the lanes of a wave.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
+  auto mx = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 1>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 2>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 4>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 8>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_BCAST15, 0xA>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_BCAST31, 0xC>(0u, x));
+  return x;
+}
+
+// Exclusive scan of the window states in two launches (as rb_scan): pre[w] =
+// {keys that overflow into window w, 1 + the last boundary before it}.  More
+// than LW_SPILL of the former, or any past the last window, raise the flag.
+[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_reduce(const uint4* __restrict__ st, uint32_t W,
+                                                                            uint4* __restrict__ part) {
+  __shared__ uint4 s_wave[16];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
+  LW t;
+  (void)lw_wave_excl(i < W ? lw_unpack(st[i]) : lw_none(), &t);
+  if (lane == 0) s_wave[wid] = lw_pack(t);
+  __syncthreads();
+  if (wid == 0) {
+    LW tot;
+    (void)lw_wave_excl(lane < 16 ? lw_unpack(s_wave[lane]) : lw_none(), &tot);
+    if (lane == 0) part[blockIdx.x] = lw_pack(tot);
+  }
+}
+
+[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W,
+                                                                          const uint4* __restrict__ part,
+                                                                          uint2* __restrict__ pre,
+                                                                          uint32_t* __restrict__ ctr) {
+  __shared__ uint4 s_wave[17];  // wave aggregates, then their prefixes; [16] = carry
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
+  const LW x = i < W ? lw_unpack(st[i]) : lw_none();
+  if (wid == 0) {
+    LW carry;
+    (void)lw_wave_excl(lane < blockIdx.x ? lw_unpack(part[lane]) : lw_none(), &carry);
+    if (lane == 0) s_wave[16] = lw_pack(carry);
+  }
+  LW wt;
+  const LW ex = lw_wave_excl(x, &wt);
+  if (lane == 0) s_wave[wid] = lw_pack(wt);
+  __syncthreads();
+  if (wid == 0) {
+    const LW carry = lw_unpack(s_wave[16]);
+    LW tot;
+    const LW xe = lw_wave_excl(lane < 16 ? lw_unpack(s_wave[lane]) : lw_none(), &tot);
+    if (lane < 16) s_wave[lane] = lw_pack(lw_combine(carry, xe));
+  }
+  __syncthreads();
+  if (i >= W) return;
+  const LW p = lw_combine(lw_unpack(s_wave[wid]), ex);
+  const int32_t o = p.a > p.b ? p.a : p.b;  // the map of the windows before, at 0
+  pre[i] = make_uint2(o > 0 ? (uint32_t)o : 0u, p.lb);
+  bool bad = o > LW_SPILL;
+  if (i + 1 == W) {
+    const LW all = lw_combine(p, x);
+    bad = bad || (all.a > all.b ? all.a : all.b) > 0;
+  }
+  if (bad) ctr[CTR_MISC] = 1u;
+}
+
+static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
+static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre, uint32_t* ctr) {
+  const uint32_t P = (W + RBS_PER - 1) / RBS_PER;
+  uint4* part = ar.take<uint4>(P ? P : 1);
+  if (ar.used > ar.cap) {
+    set_error("internal: window scan workspace overflow");
+    return GQF_ERR_INVALID;
+  }
+  GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part);
+  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, ctr);
+  return GQF_OK;
+}
+
+// Each window's range of the sorted batch: bstart[x] = first fingerprint with
+// quotient >= LW_SLOTS x (x = 0 .. W), 8 lanes per window (group8_search).
+// Also resets the counters.
+constexpr uint32_t WB_LANES = 8;
+template <typename K>
+__global__ __launch_bounds__(256) void k_wm_bounds(const K* __restrict__ B, uint32_t n, uint32_t r, uint32_t W,
+                                                   uint32_t* __restrict__ bstart, uint32_t* __restrict__ ctr) {
+  if (blockIdx.x == 0 && threadIdx.x >= CTR_OP && threadIdx.x < CTR_TOTAL) ctr[threadIdx.x] = 0u;
+  const uint32_t gt = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t x = gt / WB_LANES;
+  // every lane stays for the ballots; groups past W search an empty range
+  const uint64_t key = ((uint64_t)x * LW_SLOTS) << r;
+  const uint32_t b = group8_search(0u, x <= W ? n : 0u, [&](uint32_t m) { return (uint64_t)B[m] < key; });
+  if (gt % WB_LANES == 0 && x <= W) bstart[x] = b;
+}
+
+// Heads among the 64 keys [k0, k0 + 64) of a window, one per lane, from
+// v = E_k - k (valid lanes only) and the running maximum M of the keys before
+// (initially the overflow into the window): bit of the calling lane.
+__device__ __forceinline__ bool lw_insert_head(int32_t v, bool valid, int32_t& M) {
+  // maxima over values shifted to unsigned, 0 the identity
+  const uint32_t u = valid ? (uint32_t)v ^ 0x80000000u : 0u;
+  const uint32_t inc = wave_incl_max(u);
+  const uint32_t ex = dpp_u32<DPP_WAVE_SHR1>(0u, inc);
+  const uint32_t m0 = (uint32_t)M ^ 0x80000000u;
+  const uint32_t before = ex > m0 ? ex : m0;
+  const uint32_t all = wave_read(inc, 63);
+  M = (int32_t)((all > m0 ? all : m0) ^ 0x80000000u);
+  return valid && u >= before;
+}
+
+}  // namespace gqf

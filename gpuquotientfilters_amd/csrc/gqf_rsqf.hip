@@ -14,7 +14,7 @@
 // reference on any table (including the history-dependent layouts its insert
 // leaves).  Build / insert / delete produce the canonical layout, which is
 // what the reference insert produces when fed fingerprints in ascending order.
-#include "gqf_rebuild.hpp"
+#include "gqf_local.hpp"
 
 #include <type_traits>
 
@@ -233,6 +233,7 @@ __global__ __launch_bounds__(256) void k_rsqf_lookup(RsqfDev f, uint32_t q, cons
 // same way, one run at a time).
 constexpr uint32_t RD_BLOCKS = 64;
 constexpr uint32_t RD_SLOTS = RD_BLOCKS * 64;
+static_assert(RD_SLOTS == LW_SLOTS, "k_wm_bounds cuts batches at these windows");
 constexpr uint32_t RD_THREADS = 256;  // 16 slots per thread
 constexpr uint32_t RD_LIST = RD_SLOTS + 1;
 
@@ -1025,22 +1026,6 @@ __device__ __forceinline__ void wm_cnt_add(uint32_t* s_cnt, uint32_t p, uint32_t
 }
 __device__ __forceinline__ uint32_t wm_cnt_get(const uint32_t* s_cnt, uint32_t p) {
   return (s_cnt[p >> 1] >> (16 * (p & 1))) & 0xFFFFu;
-}
-
-// Each window's range of B: bstart[x] = first fingerprint with quotient >=
-// RD_SLOTS x (x = 0 .. W), 8 lanes per window (group8_search).  Also resets
-// the counters the insert uses.
-constexpr uint32_t WB_LANES = 8;
-template <typename K>
-__global__ __launch_bounds__(256) void k_wm_bounds(const K* __restrict__ B, uint32_t n, uint32_t r, uint32_t W,
-                                                   uint32_t* __restrict__ bstart, uint32_t* __restrict__ ctr) {
-  if (blockIdx.x == 0 && threadIdx.x >= CTR_OP && threadIdx.x < CTR_TOTAL) ctr[threadIdx.x] = 0u;
-  const uint32_t gt = blockIdx.x * 256 + threadIdx.x;
-  const uint32_t x = gt / WB_LANES;
-  // every lane stays for the ballots; groups past W search an empty range
-  const uint64_t key = ((uint64_t)x * RD_SLOTS) << r;
-  const uint32_t b = group8_search(0u, x <= W ? n : 0u, [&](uint32_t m) { return (uint64_t)B[m] < key; });
-  if (gt % WB_LANES == 0 && x <= W) bstart[x] = b;
 }
 
 // Window w's scan state (agg[w]) from the entry counts of its quotients;

@@ -1190,291 +1190,4 @@ __global__ __launch_bounds__(256) void k_sqf_decode(const uint8_t* __restrict__ 
   for (uint32_t k = tid; k < nout; k += 256) out[bI + k] = s_out[k];
 }
 
-// ---------------------------------------------------------------- localized insert
-// A batch that is small next to the table is inserted by rewriting only the
-// regions it changes (insert keep rule only).  In a canonical table the
-// occupied slots after inserting a sorted batch are what linear probing
-// gives: key i takes the first empty slot at or after max(h_i, p_{i-1} + 1)
-// (h_i: its quotient).  With E(x) = the empty slots before x, that slot is
-// the j_i-th empty slot, j_i = max(E(h_i), j_{i-1} + 1) -- the location
-// recurrence over empty ranks, scanned with the same state as locations.  A
-// boundary is an empty or unshifted slot (no run crosses it); key i's region
-// starts at the last boundary at or before h_i, and a key whose boundary lies
-// after the previous key's slot starts a new region, which ends at the last
-// slot its keys take.  Slots before a region and after it keep their entries,
-// so every region is decoded, merged with its keys and re-encoded in place,
-// each by one thread.  A key's slot past the last empty slot, or a region
-// longer than PI_LEN_CAP, sends the call to the full rebuild instead (flags).
-// E(x) and the j-th empty slot come from per-region and per-64-slot-window
-// prefixes plus one 64-slot bitmask, so each key costs a few loads.
-constexpr uint32_t PI_REGION = 4096;        // slots per counting region (64 windows of 64)
-constexpr uint32_t PI_LEN_CAP = 1u << 16;   // longest region a thread rewrites
-constexpr uint32_t PI_SCAN_CAP = 1u << 16;  // longest backward scan to a boundary
-// Automatic choice: batches of at most PI_AUTO_MAX keys and S / 256 of the
-// table.  Measured on a q=26 r=5 table (ms per call, localized / rebuild):
-// at fill 0.45, 2^14 keys 0.43 / 0.57, 2^16 0.43 / 0.55, 2^18 0.50 / 0.55;
-// at fill 0.75, 2^16 0.64 / 0.63, 2^17 0.68 / 0.62 -- its regions grow with
-// the fill, and one thread rewrites each.
-constexpr uint32_t PI_AUTO_MAX = 65536;
-constexpr uint32_t PI_MIN_RATIO = 256;
-
-template <int BPE>
-__device__ __forceinline__ void sqf_put(uint8_t* __restrict__ t, uint32_t i, uint32_t e) {
-  uint8_t* p = t + (size_t)i * BPE;
-#pragma unroll
-  for (int b = 0; b < BPE; ++b) p[b] = (uint8_t)(e >> (8 * (BPE - 1 - b)));
-}
-
-// Empty slots per region (rcnt) and, per 64-slot window, the empty slots of
-// its region before it (wpre, 16 bits).
-template <int BPE>
-__global__ __launch_bounds__(256) void k_pi_count(const uint8_t* __restrict__ t, uint32_t S, uint16_t* __restrict__ wpre,
-                                                  uint32_t* __restrict__ rcnt) {
-  __shared__ uint32_t s_tmp4[4];
-  const uint32_t s0 = blockIdx.x * PI_REGION + threadIdx.x * 16;
-  uint32_t e[16];
-  sqf_load16<BPE>(t, S, s0, e);
-  uint32_t c = 0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) c += (s0 + (uint32_t)j < S && (e[j] & 7u) == 0) ? 1u : 0u;
-  uint32_t tot;
-  const uint32_t pre = block256_excl_scan(c, s_tmp4, &tot);
-  if ((threadIdx.x & 3) == 0 && s0 < S) wpre[s0 >> 6] = (uint16_t)pre;  // the window's first thread
-  if (threadIdx.x == 0) rcnt[blockIdx.x] = tot;
-}
-
-// Bit j set: slot 64 w + j is empty (*empty) / a boundary -- empty or
-// unshifted, so that no run crosses it (*bound).  Slots past S: neither.
-template <int BPE>
-__device__ __forceinline__ void pi_masks64(const uint8_t* __restrict__ t, uint32_t S, uint32_t w, uint64_t* empty,
-                                           uint64_t* bound) {
-  uint64_t em = 0, bd = 0;
-#pragma unroll
-  for (uint32_t c = 0; c < 4; ++c) {
-    uint32_t e[16];
-    sqf_load16<BPE>(t, S, 64 * w + 16 * c, e);
-#pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-      if (64 * w + 16 * c + j < S) {
-        em |= (uint64_t)((e[j] & 7u) == 0) << (16 * c + j);
-        bd |= (uint64_t)((e[j] & 1u) == 0) << (16 * c + j);
-      }
-    }
-  }
-  *empty = em;
-  *bound = bd;
-}
-
-// Empty slots before window w (ER: exclusive region prefix of rcnt).
-__device__ __forceinline__ uint32_t pi_empties_before_window(const uint16_t* __restrict__ wpre,
-                                                             const uint32_t* __restrict__ ER, uint32_t w) {
-  return ER[w / (PI_REGION / 64)] + wpre[w];
-}
-
-// The j-th empty slot (0-based), known to lie at or after slot h: windows
-// are walked forward from h's (usually it is there or in the next one).
-template <int BPE>
-__device__ uint32_t pi_select_empty(const uint8_t* __restrict__ t, uint32_t S, const uint16_t* __restrict__ wpre,
-                                    const uint32_t* __restrict__ ER, uint32_t h, uint32_t j) {
-  const uint32_t wend = (S + 63) / 64;
-  uint32_t w = h >> 6;
-  if (w >= wend) return S;
-  uint32_t g = pi_empties_before_window(wpre, ER, w);
-  for (; w < wend; ++w) {
-    uint64_t em, bd;
-    pi_masks64<BPE>(t, S, w, &em, &bd);
-    const uint32_t c = (uint32_t)__popcll(em);
-    if (g + c > j) return 64 * w + select_bit64(em, j - g + 1);
-    g += c;
-  }
-  return S;  // not reached for a consistent count
-}
-
-// Per key: empties before its quotient, and its region's boundary (the last
-// boundary slot at or before it).
-template <int BPE>
-__global__ __launch_bounds__(256) void k_pi_keys(const uint8_t* __restrict__ t, uint32_t S, uint32_t q, uint32_t r,
-                                                 const uint32_t* __restrict__ B, uint32_t nb,
-                                                 const uint16_t* __restrict__ wpre, const uint32_t* __restrict__ ER,
-                                                 uint32_t* __restrict__ E, uint32_t* __restrict__ s0,
-                                                 uint32_t* __restrict__ flags) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb) return;
-  const uint32_t h = (B[i] >> r) & (uint32_t)mask64(q);
-  uint32_t w = h >> 6;
-  uint64_t em, bd;
-  pi_masks64<BPE>(t, S, w, &em, &bd);
-  const uint64_t below = (1ull << (h & 63)) - 1ull;
-  E[i] = pi_empties_before_window(wpre, ER, w) + (uint32_t)__popcll(em & below);
-  uint64_t m = bd & (below | (1ull << (h & 63)));  // boundaries at or before h
-  uint32_t steps = 0;
-  while (!m && w > 0) {
-    --w;
-    pi_masks64<BPE>(t, S, w, &em, &bd);
-    m = bd;
-    if (++steps * 64 > PI_SCAN_CAP) {
-      atomicOr(flags, 1u);
-      break;
-    }
-  }
-  s0[i] = m ? 64 * w + 63 - (uint32_t)__clzll(m) : 0u;
-}
-
-// Chunk states of the slot-rank recurrence (RB_TILE keys per workgroup, as
-// the rebuild's location scan; the "quotient" of key i is E_i).
-[[maybe_unused]] static __global__ __launch_bounds__(RB_THREADS) void k_pi_jagg(const uint32_t* __restrict__ E, uint32_t nb,
-                                                        uint4* __restrict__ agg) {
-  __shared__ uint4 s_wave[RB_WAVES + 1];
-  const uint32_t i0 = blockIdx.x * RB_TILE + threadIdx.x * RB_ITEMS;
-  RS a = rs_none();
-#pragma unroll
-  for (int k = 0; k < RB_ITEMS; ++k)
-    if (i0 + k < nb) rs_push(a, E[i0 + k]);
-  RS ex;
-  const RS sub = rs_block(a, &ex, s_wave);
-  if (threadIdx.x == 0) agg[blockIdx.x] = rs_pack(sub);
-}
-
-// Each key's empty rank j_i = max(E_i, j_{i-1} + 1), from the chunk prefixes
-// of the rank scan (RB_TILE keys per workgroup).
-[[maybe_unused]] static __global__ __launch_bounds__(RB_THREADS) void k_pi_ranks(const uint32_t* __restrict__ E,
-                                                                                 uint32_t nb,
-                                                                                 const uint4* __restrict__ pre,
-                                                                                 const uint32_t* __restrict__ ER,
-                                                                                 uint32_t R, uint32_t* __restrict__ J,
-                                                                                 uint32_t* __restrict__ flags) {
-  __shared__ uint4 s_wave[RB_WAVES + 1];
-  const uint32_t tid = threadIdx.x, i0 = blockIdx.x * RB_TILE + tid * RB_ITEMS;
-  const uint32_t total = ER[R];
-  uint32_t e[RB_ITEMS];
-  RS a = rs_none();
-#pragma unroll
-  for (int k = 0; k < RB_ITEMS; ++k) {
-    e[k] = i0 + k < nb ? E[i0 + k] : 0u;
-    if (i0 + k < nb) rs_push(a, e[k]);
-  }
-  RS ex;
-  (void)rs_block(a, &ex, s_wave);
-  uint32_t lp = rs_combine(rs_unpack(pre[blockIdx.x]), ex).lp;
-#pragma unroll
-  for (int k = 0; k < RB_ITEMS; ++k) {
-    if (i0 + k < nb) {
-      lp = lp + 1u > e[k] + 1u ? lp + 1u : e[k] + 1u;
-      if (lp - 1u >= total) atomicOr(flags, 2u);  // no empty slot left: the full rebuild decides
-      J[i0 + k] = lp - 1u;
-    }
-  }
-}
-
-// One thread per key: its slot p_i (the j_i-th empty slot, at or after its
-// quotient) and whether it heads a region (i == 0 or s0_i > p_{i-1}; the
-// previous key's slot is selected again here rather than waited for).
-template <int BPE>
-__global__ __launch_bounds__(256) void k_pi_pos(const uint8_t* __restrict__ t, uint32_t S, uint32_t q, uint32_t r,
-                                                const uint32_t* __restrict__ B, const uint32_t* __restrict__ J,
-                                                const uint32_t* __restrict__ s0, uint32_t nb,
-                                                const uint16_t* __restrict__ wpre, const uint32_t* __restrict__ ER,
-                                                uint32_t R, uint32_t* __restrict__ P, uint8_t* __restrict__ head) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb) return;
-  const uint32_t total = ER[R], mq = (uint32_t)mask64(q);
-  const uint32_t j = J[i];
-  const uint32_t p = j < total ? pi_select_empty<BPE>(t, S, wpre, ER, (B[i] >> r) & mq, j) : S;
-  P[i] = p;
-  bool h = true;
-  if (i > 0) {
-    const uint32_t jp = J[i - 1];
-    const uint32_t pp = jp < total ? pi_select_empty<BPE>(t, S, wpre, ER, (B[i - 1] >> r) & mq, jp) : S;
-    h = s0[i] > pp;
-  }
-  head[i] = h ? 1 : 0;
-}
-
-// Region of each head key: its keys [i, rend_i) and a length check.
-[[maybe_unused]] static __global__ __launch_bounds__(256) void k_pi_regions(const uint32_t* __restrict__ s0, const uint32_t* __restrict__ P,
-                                                    const uint8_t* __restrict__ head, uint32_t nb,
-                                                    uint32_t* __restrict__ rend, uint32_t* __restrict__ flags) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb || !head[i]) return;
-  uint32_t k = i + 1;
-  while (k < nb && !head[k] && k - i < PI_LEN_CAP) ++k;
-  rend[i] = k;
-  if ((k < nb && !head[k]) || P[k - 1] - s0[i] + 1u > PI_LEN_CAP) atomicOr(flags, 4u);
-}
-
-[[maybe_unused]] static __global__ void k_pi_init(uint32_t* __restrict__ rcnt_last, uint32_t* __restrict__ flags) {
-  if (threadIdx.x == 0) {
-    *rcnt_last = 0u;
-    *flags = 0u;
-  }
-}
-
-// One thread per region [s0_i, P[rend_i - 1]]: decode its entries into the
-// slot-indexed scratch, merge the region's keys (insert rule: a key equal
-// to the entry before it is dropped), write every slot of the region (elements
-// and zeros), then the occupied bits of its run heads.  (One workgroup per
-// 4096-slot window rewriting its regions from an LDS copy was measured
-// slower: the windows run in rounds, each as long as its longest region,
-// where one thread per key keeps every region in flight at once.)
-template <int BPE>
-__global__ __launch_bounds__(256) void k_pi_write(uint8_t* __restrict__ t, uint32_t S, uint32_t r,
-                                                  const uint32_t* __restrict__ B, uint32_t nb,
-                                                  const uint32_t* __restrict__ s0, const uint32_t* __restrict__ P,
-                                                  const uint8_t* __restrict__ head, const uint32_t* __restrict__ rend,
-                                                  uint32_t* __restrict__ scratch, uint32_t* __restrict__ flags) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb || !head[i]) return;
-  const uint32_t lo = s0[i], kend = rend[i], hi = P[kend - 1];
-  const uint32_t rmask = (1u << r) - 1u;
-  // decode: an unshifted entry starts a run at its own slot; a shifted run
-  // start takes the next occupied quotient after the current one
-  uint32_t m = 0, qcur = 0;
-  for (uint32_t x = lo; x <= hi; ++x) {
-    const uint32_t ex = sqf_get<BPE>(t, S, x);
-    if ((ex & 7u) == 0) continue;
-    if (!(ex & 1u)) {
-      qcur = x;
-    } else if (!(ex & 2u)) {
-      uint32_t y = qcur + 1;
-      while (y <= hi && !(sqf_get<BPE>(t, S, y) & 4u)) ++y;
-      if (y > hi) {
-        atomicOr(flags, 8u);  // inconsistent table: leave the region as it was
-        return;
-      }
-      qcur = y;
-    }
-    scratch[lo + m++] = (qcur << r) | (ex >> 3);
-  }
-  // merge + encode; pass 0 writes elements and zeros, pass 1 the occupied bits
-  for (int pass = 0; pass < 2; ++pass) {
-    uint32_t ia = 0, ib = i, next = lo, lastq = 0xFFFFFFFFu;
-    int64_t loc = (int64_t)lo - 1;
-    uint64_t prevfp = ~0ull;
-    while (ia < m || ib < kend) {
-      const bool takeA = ib >= kend || (ia < m && scratch[lo + ia] <= B[ib]);
-      const uint32_t v = takeA ? scratch[lo + ia++] : B[ib++];
-      const bool keep = takeA || prevfp != (uint64_t)v;
-      prevfp = v;
-      if (!keep) continue;
-      const uint32_t fq = v >> r;
-      loc = (int64_t)fq > loc + 1 ? (int64_t)fq : loc + 1;
-      if (loc > (int64_t)hi) {
-        atomicOr(flags, 8u);  // not reached: the region holds its layout
-        break;
-      }
-      if (pass == 0) {
-        for (; next < (uint32_t)loc; ++next) sqf_put<BPE>(t, next, 0u);
-        sqf_put<BPE>(t, (uint32_t)loc, ((v & rmask) << 3) | (fq == lastq ? 2u : 0u) | ((uint32_t)loc != fq ? 1u : 0u));
-        next = (uint32_t)loc + 1;
-      } else if (fq != lastq) {
-        uint8_t* b = t + (size_t)fq * BPE + (BPE - 1);  // the element's low byte holds the flags
-        *b = (uint8_t)(*b | 4u);
-      }
-      lastq = fq;
-    }
-    if (pass == 0)
-      for (; next <= hi; ++next) sqf_put<BPE>(t, next, 0u);
-  }
-}
-
 }  // namespace gqf

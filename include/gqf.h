@@ -83,13 +83,12 @@ int gqf_sqf_get_hash(void);
 /* How gqf_sqf_insert (insert, quotientFilter.cu:1184) of the calling thread
  * updates the table.  No reference counterpart: the results are the same
  * either way; only the work differs.
- *   AUTO     localized for batches of at most 65536 keys (and S/256), else
- *            the rebuild;
+ *   AUTO     localized for batches of up to 1/32 of the slots (1/80 in
+ *            tables below 2^25 slots), else the rebuild;
  *   REBUILD  decode the table, merge the sorted batch, rebuild every slot;
- *   LOCAL    rewrite only the regions the batch changes, between the last
- *            empty-or-unshifted slot before each key and the last slot its
- *            keys take; a region longer than 2^16 slots, or a batch that
- *            does not fit, falls back to the rebuild. */
+ *   LOCAL    update in place only the slots from each key's quotient to the
+ *            empty slot it takes; batches too dense for that (and slots wider
+ *            than 2 bytes) fall back to the rebuild. */
 enum gqf_insert_path { GQF_INSERT_AUTO = 0, GQF_INSERT_REBUILD = 1, GQF_INSERT_LOCAL = 2 };
 gqf_status gqf_sqf_set_insert_path(int path);
 int gqf_sqf_get_insert_path(void);
