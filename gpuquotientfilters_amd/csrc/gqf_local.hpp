@@ -55,6 +55,10 @@ constexpr uint32_t LW_MAX_WINDOWS = RBS_PER * 64;  // one state per window: the 
 //             fill 0.8   2^10 keys 0.057 / 0.317   2^21 0.312 / 0.414   2^22 0.612 / 0.457
 //   q=22 r=5  fill 0.75  2^13 keys 0.061 / 0.098   2^16 0.087 / 0.097   2^18 0.179 / 0.103
 //   q=19 r=13 fill 0.8   2^10 keys 0.049 / 0.073   2^13 0.089 / 0.086   2^16 0.118 / 0.091
+// Deletes:
+//   q=26 r=5  fill 0.75  2^10 keys 0.056 / 0.314   2^20 0.182 / 0.370   2^21 0.316 / 0.423
+//             fill 0.8   2^20 keys 0.204 / 0.390   2^21 0.385 / 0.441
+//   q=22 r=5  fill 0.75  2^10 keys 0.050 / 0.079   2^13 0.075 / 0.092
 static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8192ull * LW_SLOTS) ? 32 : 80) <= slots; }
 
 static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }

@@ -359,14 +359,24 @@ static gqf_status sqf_delete_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
   GQF_TRY(cs.begin(stream));
   DeviceState& ds = *cs.ds;
   const uint32_t un = (uint32_t)n;
-  GQF_TRY(ws_reserve(ds, sort_workspace_bytes(un, 4, false) + sqf_decode_bytes(g) + aligned_bytes(g.S + 1) +
-                             rebuild_ws_bytes(g.S) + packed_ws_bytes(g)));
+  const bool local = un > 0 && sqf_local_fits(qf, g) && lw_auto(un, g.S);
+  const size_t full = sqf_decode_bytes(g) + aligned_bytes(g.S + 1) + rebuild_ws_bytes(g.S);
+  GQF_TRY(ws_reserve(ds, sort_workspace_bytes(un, 4, false) + packed_ws_bytes(g) +
+                             std::max(full, local ? sqf_local_bytes(g, un) : 0)));
   Arena ar(ds.ws, ds.ws_cap);
   uint32_t* D = nullptr;
   GQF_TRY(radix_sort<uint32_t>(cs.stream, ar, d_keys, true, (g.q + g.r) | sqf_hash_flag(), nullptr, false, un, 0, g.q + g.r, &D,
                                nullptr, &ds));
   gqf_sqf wq;
   GQF_TRY(work_table(cs.stream, ar, qf, g, true, &wq));
+  if (local) {
+    const size_t mark = ar.used;
+    GQF_TRY(sqf_local<false>(cs.stream, ds.counters, ar, wq, g, D, un));
+    finish_table(cs.stream, qf, wq, g, ds.counters);
+    GQF_TRY(cs.end(ms, true));
+    if (ds.h_pinned[CTR_MISC] == 0) return GQF_OK;
+    ar.used = mark;  // nothing was written: the rebuild takes over
+  }
   uint32_t* A;
   const uint32_t* m_dev = nullptr;
   GQF_TRY(sqf_decode(cs.stream, ar, wq, g, &A, &m_dev));

@@ -181,8 +181,8 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
     }
   }
   if (lane == 0) {
-    const int32_t a = (int32_t)nk - (int32_t)e;
-    int32_t b = nk ? M + a : 0;
+    const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
+    int32_t b = INS && nk ? M + a : 0;
     if (b < 0) b = 0;
     st[w] = lw_pack(LW{a, b, last ? base + last : 0u});
     if (!INS) fb[w] = (uint16_t)first;
@@ -202,7 +202,9 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
 // wave's longest region (dependent LDS reads) times the waves per CU: 2^20
 // keys into q=26 r=5 at fill 0.75 take 77 us, 559 us when the lanes walked
 // element bytes one by one (1.9 and 0.26 TB/s of table bytes read and
-// written); the rebuild's decode, state and write passes take 250 us.
+// written); the rebuild's decode, state and write passes take 250 us.  As
+// many deletes take 104 us, 160 when every run start that moves was paired
+// with its quotient one by one; decode, mark and rebuild take 290 us.
 constexpr uint32_t SL_HALO = 16;
 constexpr uint32_t SL_BLOCKS = 64 + SL_HALO;
 
@@ -361,23 +363,33 @@ struct SlPlanes {
     const uint32_t l = next(p + 1, [&](uint32_t w) { return ~(uint64_t)shf[w]; }) - 1;
     const bool first = p == s, more = l > p && bit(cont, p + 1);
     const uint32_t pw = p >> 6, lw = l >> 6;
-    // the run starts among them, in order, belong to the occupied quotients
-    // after fq: one that comes to its own quotient is no longer shifted
-    uint32_t qw = fw;
-    uint64_t om = occ[fw] & ~upto(fq & 63);
+    // the j-th run start among them belongs to the j-th occupied quotient
+    // after fq: it comes to its own quotient z (and is no longer shifted) iff
+    // z is occupied and R, the occupied quotients of (fq, z] less the run
+    // starts up to z, is 0 there.  R falls only at run starts on unoccupied
+    // slots, so 16 slots with fewer of those than R are passed at once.
+    int32_t R = 0;
+    for (uint32_t w = fw; w <= pw; ++w) {
+      const uint64_t sel = (w == fw ? ~upto(fq & 63) : ~0ull) & (w == pw ? ~from(p & 63) : ~0ull);
+      R += __builtin_popcountll(occ[w] & sel);
+    }
     for (uint32_t w = pw; w <= lw; ++w) {
       const uint64_t reg = (w == pw ? from(p & 63) : ~0ull) & (w == lw ? upto(l & 63) : ~0ull);
       const uint64_t gap = w == lw ? 1ull << (l & 63) : 0ull;  // becomes empty
       const uint64_t old = cont[w];
       uint64_t c = ((old >> 1) | (w < lw ? (uint64_t)cont[w + 1] << 63 : 0ull)) & ~gap, z = ~gap;
-      uint64_t heads = ~c & ~gap & reg;
-      while (heads) {
-        while (!om && qw + 1 < end / 64) om = occ[++qw];
-        if (!om) break;  // not reached: every run has its quotient
-        const uint64_t h = heads & (0 - heads);
-        if (qw == w && (om & (0 - om)) == h) z &= ~h;
-        heads ^= h;
-        om &= om - 1ull;
+      const uint64_t heads = ~c & ~gap & reg;
+      const uint64_t own = occ[w] & reg & (w == fw ? ~upto(fq & 63) : ~0ull);
+      for (uint32_t k = 0; k < 64; k += 16) {
+        const uint32_t h = (uint32_t)(heads >> k) & 0xFFFFu, o = (uint32_t)(own >> k) & 0xFFFFu;
+        if (R <= (int32_t)__builtin_popcount(h & ~o)) {
+          for (uint32_t m = h & o; m; m &= m - 1u) {
+            const uint32_t up = m ^ (m - 1u);  // up to the candidate's bit
+            if (R + (int32_t)__builtin_popcount(o & up) == (int32_t)__builtin_popcount(h & up))
+              z &= ~((uint64_t)(m & (0u - m)) << k);
+          }
+        }
+        R += (int32_t)__builtin_popcount(o) - (int32_t)__builtin_popcount(h);
       }
       if (w == pw && first && more) {  // the run's next entry becomes its first
         const uint64_t pb = 1ull << (p & 63);

@@ -112,3 +112,49 @@ def test_sqf_local_insert_hot_and_edges():
         f.insert(dev(b))
         fps = insert_set(fps, O.fingerprints(b, q, r))
         sqf_equal(f, sqf_table(fps, q, r))
+
+
+@pytest.mark.parametrize("q,r,alpha,dup", CASES)
+def test_sqf_local_delete(q, r, alpha, dup):
+    """Stored keys, keys that are not stored, repeated keys, several copies."""
+    say("sqf local delete", q, r, alpha, dup)
+    keys = O.mt19937(320 + q, O.key_count(alpha, q))
+    if dup:
+        keys = np.concatenate([keys[:-50], keys[:25], keys[:25]])
+    f = G.SQF(q, r)
+    f.bulk_build(dev(keys), NoDuplicates=not dup)
+    fps = O.fingerprints(keys, q, r)
+    if not dup:
+        fps = np.unique(fps)
+    S = G.SQF.num_slots(q)
+    other = O.mt19937(321 + q, S)
+    at = local = 0
+    for n in [1, 2, 63, 64, 65, 1000, S // 400 + 1, S // 82]:
+        n = min(n, S // 82)
+        if n <= 0:
+            break
+        b = np.concatenate([keys[at:at + n - n // 3], keys[at:at + n // 6], other[at:at + n // 6]])
+        at += n
+        names = _kernels(lambda: f.superclusterDeletes(dev(b)))
+        local += any("k_sl_apply" in x for x in names) and not any("k_rb_write" in x for x in names)
+        fps = delete_multiset(fps, O.fingerprints(b, q, r))
+        sqf_equal(f, sqf_table(fps, q, r))
+    assert local >= 2
+
+
+def test_sqf_local_delete_hot_and_edges():
+    q, r = 16, 5
+    say("sqf local delete edges", q, r)
+    cand = O.mt19937(330, 1 << 19)
+    fq = O.fingerprints(cand, q, r) >> np.uint64(r)
+    edge = cand[(fq % 4096 >= 4056) | (fq % 4096 < 8)]
+    ends = cand[(fq < 3) | (fq >= (1 << q) - 3)]
+    base = np.concatenate([O.mt19937(331, O.key_count(0.6, q)), edge[:2500], ends[:30], np.full(90, cand[5])])
+    f = G.SQF(q, r)
+    f.bulk_build(dev(base), NoDuplicates=False)
+    fps = O.fingerprints(base, q, r)
+    for b in [edge[:800], ends[:40], np.full(30, cand[5]), np.full(70, cand[5]), edge[800:1600], base[:800],
+              edge[1600:2400]]:
+        f.superclusterDeletes(dev(b))
+        fps = delete_multiset(fps, O.fingerprints(b, q, r))
+        sqf_equal(f, sqf_table(fps, q, r))
