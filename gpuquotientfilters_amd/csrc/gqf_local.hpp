@@ -35,7 +35,9 @@
 // and the call takes its general path: more than LW_KEYS keys in a window,
 // a whole aligned group
 // of 64 keys without a head, fewer than LW_SPILL empty slots in a
-// window (clusters longer than a window), an overflow above LW_SPILL.
+// window (clusters longer than a window), an overflow above LW_SPILL, too
+// few regions (lw_scan).  After such a batch the next 4, 8, ... 256 of its
+// kind on the stream go straight to the general path.
 #pragma once
 
 #include "gqf_rebuild.hpp"
@@ -59,27 +61,45 @@ constexpr uint32_t LW_MAX_WINDOWS = RBS_PER * 64;  // one state per window: the 
 //   q=26 r=5  fill 0.75  2^10 keys 0.056 / 0.314   2^20 0.182 / 0.370   2^21 0.316 / 0.423
 //             fill 0.8   2^20 keys 0.204 / 0.390   2^21 0.385 / 0.441
 //   q=22 r=5  fill 0.75  2^10 keys 0.050 / 0.079   2^13 0.075 / 0.092
+// RSQF inserts, localized / by windows:
+//   q=26 r=8  fill 0.5   2^10 keys 0.072 / 0.195   2^18 0.144 / 0.382   2^21 0.262 / 0.440
+//             fill 0.8   2^10 keys 0.072 / 0.293   2^18 0.158 / 0.392   2^20 0.232 / 0.400
+//   q=24 r=5  fill 0.7   2^10 keys 0.058 / 0.145   2^16 0.088 / 0.197
+//   q=22 r=8  fill 0.8   2^10 keys 0.055 / 0.073   2^13 0.070 / 0.084
 static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8192ull * LW_SLOTS) ? 32 : 80) <= slots; }
+
+// Whether the stream's next batch of this kind (LocalKind) tries the
+// localized form, and what came of it.
+static inline bool lw_try(DeviceState& ds, LocalKind k) {
+  if (!ds.local_skip[k]) return true;
+  --ds.local_skip[k];
+  return false;
+}
+static inline void lw_report(DeviceState& ds, LocalKind k, bool done) {
+  uint32_t& bo = ds.local_backoff[k];
+  bo = done ? 0 : (bo ? (bo < 256 ? 2 * bo : 256) : 4);
+  ds.local_skip[k] = bo;
+}
 
 static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }
 
-// Scan state of a window: overflow map x -> max(x + a, b) (insert), and 1 +
-// the last boundary slot (delete; 0: none).
+// Scan state of a window: overflow map x -> max(x + a, b) (insert), 1 + the
+// last boundary slot (delete; 0: none), and the keys that start a region.
 struct LW {
   int32_t a, b;
-  uint32_t lb;
+  uint32_t lb, heads;
 };
 __host__ __device__ __forceinline__ LW lw_combine(LW x, LW y) {
   const int32_t b = x.b + y.a;
-  return LW{x.a + y.a, b > y.b ? b : y.b, x.lb > y.lb ? x.lb : y.lb};
+  return LW{x.a + y.a, b > y.b ? b : y.b, x.lb > y.lb ? x.lb : y.lb, x.heads + y.heads};
 }
-__device__ __forceinline__ LW lw_none() { return LW{0, 0, 0u}; }
-__device__ __forceinline__ uint4 lw_pack(LW x) { return make_uint4((uint32_t)x.a, (uint32_t)x.b, x.lb, 0u); }
-__device__ __forceinline__ LW lw_unpack(uint4 w) { return LW{(int32_t)w.x, (int32_t)w.y, w.z}; }
+__device__ __forceinline__ LW lw_none() { return LW{0, 0, 0u, 0u}; }
+__device__ __forceinline__ uint4 lw_pack(LW x) { return make_uint4((uint32_t)x.a, (uint32_t)x.b, x.lb, x.heads); }
+__device__ __forceinline__ LW lw_unpack(uint4 w) { return LW{(int32_t)w.x, (int32_t)w.y, w.z, w.w}; }
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ LW lw_dpp(LW x) {
   return LW{(int32_t)dpp_u32<CTRL, ROW_MASK>(0u, (uint32_t)x.a), (int32_t)dpp_u32<CTRL, ROW_MASK>(0u, (uint32_t)x.b),
-            dpp_u32<CTRL, ROW_MASK>(0u, x.lb)};
+            dpp_u32<CTRL, ROW_MASK>(0u, x.lb), dpp_u32<CTRL, ROW_MASK>(0u, x.heads)};
 }
 __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
   LW inc = x;
@@ -89,7 +109,8 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
   inc = lw_combine(lw_dpp<DPP_ROW_SHR | 8>(inc), inc);
   inc = lw_combine(lw_dpp<DPP_ROW_BCAST15, 0xA>(inc), inc);
   inc = lw_combine(lw_dpp<DPP_ROW_BCAST31, 0xC>(inc), inc);
-  *total = LW{(int32_t)wave_read((uint32_t)inc.a, 63), (int32_t)wave_read((uint32_t)inc.b, 63), wave_read(inc.lb, 63)};
+  *total = LW{(int32_t)wave_read((uint32_t)inc.a, 63), (int32_t)wave_read((uint32_t)inc.b, 63), wave_read(inc.lb, 63),
+              wave_read(inc.heads, 63)};
   return lw_dpp<DPP_WAVE_SHR1>(inc);
 }
 // Inclusive maximum over the lanes of a wave.
@@ -106,7 +127,13 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
 
 // Exclusive scan of the window states in two launches (as rb_scan): pre[w] =
 // {keys that overflow into window w, 1 + the last boundary before it}.  More
-// than LW_SPILL of the former, or any past the last window, raise the flag.
+// than LW_SPILL of the former, or any past the last window, raise the flag;
+// so do fewer than 3 regions per 4 of the n keys (batches of at least a key
+// per window): long clusters and several keys in each make a wave wait for a
+// few lanes.  RSQF q=26 r=8 inserts without that rule, ms per call, localized
+// / by windows, with the keys per region:
+//   fill 0.8  2^20 keys 0.235 / 0.399 (1.20)  2^21 0.429 / 0.453 (1.39)
+//   fill 0.9  2^18 keys 0.307 / 0.401 (1.17)  2^20 0.950 / 0.412 (1.67)
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_reduce(const uint4* __restrict__ st, uint32_t W,
                                                                             uint4* __restrict__ part) {
   __shared__ uint4 s_wave[16];
@@ -124,7 +151,7 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
 
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W,
                                                                           const uint4* __restrict__ part,
-                                                                          uint2* __restrict__ pre,
+                                                                          uint2* __restrict__ pre, uint32_t n,
                                                                           uint32_t* __restrict__ ctr) {
   __shared__ uint4 s_wave[17];  // wave aggregates, then their prefixes; [16] = carry
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
@@ -152,13 +179,14 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
   bool bad = o > LW_SPILL;
   if (i + 1 == W) {
     const LW all = lw_combine(p, x);
-    bad = bad || (all.a > all.b ? all.a : all.b) > 0;
+    bad = bad || (all.a > all.b ? all.a : all.b) > 0 || (n >= W && (uint64_t)all.heads * 4 < (uint64_t)n * 3);
   }
   if (bad) ctr[CTR_MISC] = 1u;
 }
 
 static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
-static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre, uint32_t* ctr) {
+static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre, uint32_t n,
+                                 uint32_t* ctr) {
   const uint32_t P = (W + RBS_PER - 1) / RBS_PER;
   uint4* part = ar.take<uint4>(P ? P : 1);
   if (ar.used > ar.cap) {
@@ -166,7 +194,7 @@ static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint
     return GQF_ERR_INVALID;
   }
   GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part);
-  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, ctr);
+  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, n, ctr);
   return GQF_OK;
 }
 

@@ -14,7 +14,7 @@
 // reference on any table (including the history-dependent layouts its insert
 // leaves).  Build / insert / delete produce the canonical layout, which is
 // what the reference insert produces when fed fingerprints in ascending order.
-#include "gqf_local.hpp"
+#include "gqf_rsqf_local.hpp"
 
 #include <type_traits>
 
@@ -1741,14 +1741,81 @@ static gqf_status rsqf_insert_win(hipStream_t s, DeviceState& ds, Arena& ar, con
   return GQF_OK;
 }
 
+// Workspace of the localized insert or delete (beside the batch's sort).
+static size_t rsqf_local_ws(const RsqfGeom& g, uint32_t n) {
+  const uint32_t W = rd_windows(g.nb);
+  return aligned_bytes((size_t)W * 8) + 256 + scan_rows_bytes(W, 2) + aligned_bytes(((size_t)W + 1) * 4) +
+         aligned_bytes((size_t)n * 4) + aligned_bytes((size_t)g.nb * 8) + aligned_bytes((size_t)W * 2) +
+         aligned_bytes((size_t)W * 16) + aligned_bytes((size_t)W * 8) + lw_scan_bytes(W) + 2048;
+}
+static bool rsqf_local_fits(const RsqfGeom& g, uint32_t n) {
+  return n > 0 && rd_windows(g.nb) <= LW_MAX_WINDOWS && lw_auto(n, g.cap);
+}
+
+// The localized insert (INS) or delete of the sorted fingerprints B.  Leaves
+// ctr[CTR_MISC] != 0, and the table untouched, when the batch does not fit
+// that form.
+template <typename K, bool INS>
+static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gqf_rsqf& f, const K* B, uint32_t n) {
+  const RsqfGeom g = rgeom(f);
+  const RsqfDev d = rdev(f);
+  const uint32_t W = rd_windows(g.nb);
+  uint32_t* wp = ar.take<uint32_t>((size_t)W * 2);
+  uint32_t* tot = ar.take<uint32_t>(4);
+  uint32_t* bstart = ar.take<uint32_t>((size_t)W + 1);
+  uint32_t* key = ar.take<uint32_t>(n);
+  uint64_t* empty = ar.take<uint64_t>(g.nb);
+  uint16_t* fb = ar.take<uint16_t>(W);
+  uint4* st = ar.take<uint4>(W);
+  uint2* pre = ar.take<uint2>(W);
+  if (ar.used > ar.cap) {
+    set_error("internal: localized update workspace overflow");
+    return GQF_ERR_INVALID;
+  }
+  const double mb = (double)g.nb * 16;  // occupieds + run ends
+  GQF_LAUNCH_B(mb, k_rd_pop, dim3((W + 3) / 4), dim3(256), 0, s, d.meta, g.nb, W, wp, (uint32_t*)nullptr, 0u);
+  GQF_TRY(scan_rows<2>(s, ar, wp, W, tot));
+  GQF_LAUNCH((k_wm_bounds<K>), dim3(((W + 1) * WB_LANES + 255) / 256), dim3(256), 0, s, B, n, g.r, W, bstart,
+             ds.counters);
+  GQF_LAUNCH_B(mb + (double)n * (sizeof(K) + 4), (k_rl_plan<K, INS>), dim3(W), dim3(64), 0, s, d.meta, g.nb, g.r, wp, B,
+               bstart, W, key, empty, fb, st, ds.counters);
+  GQF_TRY(lw_scan(s, ar, st, W, pre, n, ds.counters));
+  uint64_t* meta = reinterpret_cast<uint64_t*>(f.blocks);
+  uint64_t* remg = reinterpret_cast<uint64_t*>(reinterpret_cast<uint8_t*>(f.blocks) + rsqf_meta_bytes(g.nb));
+  const double wb = (double)rsqf_dev_bytes(g.q, g.r) + (double)n * (sizeof(K) + 4 + 256);
+  if (g.r == 8)
+    GQF_LAUNCH_B(wb, (k_rl_apply<K, 8, INS>), dim3(W), dim3(64), 0, s, meta, remg, g.nb, g.r, B, n, bstart, W, pre, key,
+                 empty, fb, ds.counters);
+  else
+    GQF_LAUNCH_B(wb, (k_rl_apply<K, 0, INS>), dim3(W), dim3(64), 0, s, meta, remg, g.nb, g.r, B, n, bstart, W, pre, key,
+                 empty, fb, ds.counters);
+  return GQF_OK;
+}
+
+// The in-place inserts: localized where the batch is small (local; *done:
+// the call has ended), else window by window.  d_out: the keys' slots.
+static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out);
 template <typename K>
-static gqf_status rsqf_insert_win_t(const gqf_rsqf& f, uint32_t n, const uint32_t* keys, CallScope& cs) {
+static gqf_status rsqf_insert_win_t(const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* d_out, CallScope& cs,
+                                    bool local, bool* done, float* ms) {
   DeviceState& ds = *cs.ds;
   const RsqfGeom g = rgeom(f);
-  GQF_TRY(ws_reserve(ds, sort_workspace_bytes(n, sizeof(K), false) + rsqf_win_ws(g)));
+  GQF_TRY(ws_reserve(ds, sort_workspace_bytes(n, sizeof(K), false) +
+                             std::max(rsqf_win_ws(g), local ? rsqf_local_ws(g, n) : (size_t)0)));
   Arena ar(ds.ws, ds.ws_cap);
   K* B;
   GQF_TRY(radix_sort<K>(cs.stream, ar, keys, true, g.bits, nullptr, false, n, 0, g.bits, &B, nullptr, cs.ds));
+  *done = false;
+  if (local) {
+    const size_t mark = ar.used;
+    GQF_TRY((rsqf_local<K, true>(cs.stream, ds, ar, f, B, n)));
+    if (d_out) launch_rlookup(cs.stream, f, n, keys, d_out);
+    GQF_TRY(cs.end(ms, true));
+    *done = ds.h_pinned[CTR_MISC] == 0;
+    lw_report(ds, LOCAL_RSQF_INSERT, *done);
+    if (*done) return GQF_OK;
+    ar.used = mark;  // nothing was written
+  }
   return rsqf_insert_win<K>(cs.stream, ds, ar, f, B, n);
 }
 
@@ -1856,9 +1923,17 @@ static gqf_status rsqf_insert_call(gqf_rsqf cqf, int n, const uint32_t* d_keys, 
   if (n > 0 && rsqf_insert_path() != GQF_INSERT_REBUILD && rsqf_win_fits(rgeom(cqf))) {
     CallScope cs;
     GQF_TRY(cs.begin(stream));
-    if (!wide) GQF_TRY(rsqf_insert_win_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs));
-    else GQF_TRY(rsqf_insert_win_t<uint64_t>(cqf, (uint32_t)n, d_keys, cs));
-    if (d_out) launch_rlookup(cs.stream, cqf, (uint32_t)n, d_keys, reinterpret_cast<uint32_t*>(d_out));
+    uint32_t* out = reinterpret_cast<uint32_t*>(d_out);
+    const bool local = rsqf_insert_path() == GQF_INSERT_AUTO && rsqf_local_fits(rgeom(cqf), (uint32_t)n) &&
+                       lw_try(*cs.ds, LOCAL_RSQF_INSERT);
+    bool done = false;
+    if (!wide) GQF_TRY(rsqf_insert_win_t<uint32_t>(cqf, (uint32_t)n, d_keys, out, cs, local, &done, ms));
+    else GQF_TRY(rsqf_insert_win_t<uint64_t>(cqf, (uint32_t)n, d_keys, out, cs, local, &done, ms));
+    if (done) {
+      if (lp_end) *lp_end = 0;  // read only when a batch does not fit
+      return GQF_OK;
+    }
+    if (d_out) launch_rlookup(cs.stream, cqf, (uint32_t)n, d_keys, out);
     const gqf_status st = cs.end(&ms_win, true);
     if (st != GQF_OK && st != GQF_ERR_CAPACITY) return st;
     // a window the windowed path cannot take: nothing was written, rebuild
@@ -1973,8 +2048,12 @@ size_t gqf_rsqf_workspace_bytes(gqf_rsqf cqf, int op, int n, int sorted) {
   const uint32_t un = (uint32_t)n;
   (void)sorted;
   if (op == GQF_OP_LOOKUP) return 0;
-  if (op == GQF_OP_INSERT) return wide ? rsqf_insert_ws<uint64_t>(g, un) : rsqf_insert_ws<uint32_t>(g, un);
-  if (op == GQF_OP_DELETE) return wide ? rsqf_delete_ws<uint64_t>(g, un) : rsqf_delete_ws<uint32_t>(g, un);
+  const size_t local =
+      rsqf_local_fits(g, un) ? sort_workspace_bytes(un, wide ? 8 : 4, false) + rsqf_local_ws(g, un) : 0;
+  if (op == GQF_OP_INSERT)
+    return std::max(local, wide ? rsqf_insert_ws<uint64_t>(g, un) : rsqf_insert_ws<uint32_t>(g, un));
+  if (op == GQF_OP_DELETE)
+    return std::max(local, wide ? rsqf_delete_ws<uint64_t>(g, un) : rsqf_delete_ws<uint32_t>(g, un));
   return 0;
 }
 

@@ -58,6 +58,9 @@ struct ProfRec {
   double dper;
 };
 
+// Kinds of localized updates (gqf_local.hpp).
+enum LocalKind : int { LOCAL_SQF_INSERT = 0, LOCAL_SQF_DELETE, LOCAL_RSQF_INSERT, LOCAL_RSQF_DELETE, LOCAL_KINDS };
+
 // Execution context of one (device, stream) pair: workspace arena, device
 // counters and their pinned mirror, timing events.  Calls on the same stream
 // are serialized by the context's mutex; calls on different streams run
@@ -82,6 +85,8 @@ struct DeviceState {
   // pair per key width: 32-bit (SQF, AP hash) and 64-bit (wide) fingerprints
   // crowd differently.
   uint32_t crowd_skip[2] = {0, 0}, crowd_backoff[2] = {0, 0};
+  // likewise after a batch that the localized updates handed over, per kind
+  uint32_t local_skip[LOCAL_KINDS] = {}, local_backoff[LOCAL_KINDS] = {};
   // per-launch timing (gqf_profile_enable): event pool and launches to resolve
   hipEvent_t* pool = nullptr;
   size_t pool_size = 0, pool_used = 0;

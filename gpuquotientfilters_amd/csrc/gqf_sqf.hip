@@ -300,7 +300,7 @@ static gqf_status sqf_local_t(hipStream_t s, uint32_t* ctr, Arena& ar, const gqf
   GQF_LAUNCH((k_wm_bounds<uint32_t>), dim3(((W + 1) * WB_LANES + 255) / 256), dim3(256), 0, s, B, n, g.r, W, bstart, ctr);
   GQF_LAUNCH_B((double)g.bytes + (double)n * 6, (k_sl_plan<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S, g.r, B,
                bstart, W, el, fb, st, ctr);
-  GQF_TRY(lw_scan(s, ar, st, W, pre, ctr));
+  GQF_TRY(lw_scan(s, ar, st, W, pre, n, ctr));
   GQF_LAUNCH_B(2.0 * (double)g.bytes + (double)n * 6, (k_sl_apply<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S,
                g.r, B, n, bstart, W, pre, el, fb, ctr);
   return GQF_OK;
@@ -323,7 +323,7 @@ static gqf_status sqf_insert_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
   const uint32_t un = (uint32_t)n;
   const int path = sqf_insert_path();
   const bool local = mode == KEEP_TAGGED_INSERT && un > 0 && path != GQF_INSERT_REBUILD && sqf_local_fits(qf, g) &&
-                     (path == GQF_INSERT_LOCAL || lw_auto(un, g.S));
+                     (path == GQF_INSERT_LOCAL || (lw_auto(un, g.S) && lw_try(ds, LOCAL_SQF_INSERT)));
   const size_t full = sqf_decode_bytes(g) + rebuild_ws_bytes((uint64_t)g.S + un);
   GQF_TRY(ws_reserve(ds, sort_workspace_bytes(un, 4, false) + packed_ws_bytes(g) +
                              std::max(full, local ? sqf_local_bytes(g, un) : 0)));
@@ -338,7 +338,9 @@ static gqf_status sqf_insert_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
     GQF_TRY(sqf_local<true>(cs.stream, ds.counters, ar, wq, g, B, un));
     finish_table(cs.stream, qf, wq, g, ds.counters);
     GQF_TRY(cs.end(ms, true));
-    if (ds.h_pinned[CTR_MISC] == 0) return GQF_OK;
+    const bool done = ds.h_pinned[CTR_MISC] == 0;
+    lw_report(ds, LOCAL_SQF_INSERT, done);
+    if (done) return GQF_OK;
     ar.used = mark;  // nothing was written: the rebuild takes over
   }
   uint32_t* A;
@@ -359,7 +361,7 @@ static gqf_status sqf_delete_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
   GQF_TRY(cs.begin(stream));
   DeviceState& ds = *cs.ds;
   const uint32_t un = (uint32_t)n;
-  const bool local = un > 0 && sqf_local_fits(qf, g) && lw_auto(un, g.S);
+  const bool local = un > 0 && sqf_local_fits(qf, g) && lw_auto(un, g.S) && lw_try(ds, LOCAL_SQF_DELETE);
   const size_t full = sqf_decode_bytes(g) + aligned_bytes(g.S + 1) + rebuild_ws_bytes(g.S);
   GQF_TRY(ws_reserve(ds, sort_workspace_bytes(un, 4, false) + packed_ws_bytes(g) +
                              std::max(full, local ? sqf_local_bytes(g, un) : 0)));
@@ -374,7 +376,9 @@ static gqf_status sqf_delete_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
     GQF_TRY(sqf_local<false>(cs.stream, ds.counters, ar, wq, g, D, un));
     finish_table(cs.stream, qf, wq, g, ds.counters);
     GQF_TRY(cs.end(ms, true));
-    if (ds.h_pinned[CTR_MISC] == 0) return GQF_OK;
+    const bool done = ds.h_pinned[CTR_MISC] == 0;
+    lw_report(ds, LOCAL_SQF_DELETE, done);
+    if (done) return GQF_OK;
     ar.used = mark;  // nothing was written: the rebuild takes over
   }
   uint32_t* A;

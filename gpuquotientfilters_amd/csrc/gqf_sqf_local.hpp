@@ -123,7 +123,7 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
     // not read: what overflows into it is absorbed by the window before, and
     // a boundary of that window separates keys on both sides
     if (lane == 0) {
-      st[w] = lw_pack(LW{-LW_SPILL, 0, base + 1});
+      st[w] = lw_pack(LW{-LW_SPILL, 0, base + 1, 0u});
       if (!INS) fb[w] = 0;
     }
     return;
@@ -155,6 +155,7 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
   __syncthreads();
   bool bad = nk > LW_KEYS || (INS ? e < (uint32_t)LW_SPILL && w + 1 < W : first == LW_SLOTS);
   int32_t M = 0;
+  uint32_t heads = 0;
   if (!bad) {
     uint32_t prev = 0;  // delete: 1 + the key before the group (0: none)
     for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
@@ -177,14 +178,16 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
         head = on && lb > p;  // boundary lb - 1 after the key p - 1
         if (on) el[b0 + k] = head ? 1 : 0;
       }
-      if (k0 + 64 <= nk && __ballot(head) == 0) bad = true;
+      const uint64_t hm = __ballot(head);
+      heads += (uint32_t)__popcll(hm);
+      if (k0 + 64 <= nk && hm == 0) bad = true;
     }
   }
   if (lane == 0) {
     const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
     int32_t b = INS && nk ? M + a : 0;
     if (b < 0) b = 0;
-    st[w] = lw_pack(LW{a, b, last ? base + last : 0u});
+    st[w] = lw_pack(LW{a, b, last ? base + last : 0u, heads});
     if (!INS) fb[w] = (uint16_t)first;
     if (bad) ctr[CTR_MISC] = 1u;
   }

@@ -94,7 +94,9 @@ gqf_status gqf_sqf_set_insert_path(int path);
 int gqf_sqf_get_insert_path(void);
 /* The same choice for this thread's RSQF inserts (no reference counterpart;
  * the results are equal, only the work differs):
- *   AUTO, LOCAL  rewrite the table in place, window by window (4096 slots:
+ *   AUTO     small batches (up to 1/32 of the slots, 1/80 in tables below
+ *            2^25 slots) update only the slots they change; others as LOCAL;
+ *   LOCAL    rewrite the table in place, window by window (4096 slots:
  *            each window's stored entries decoded from its run ends, merged
  *            with its batch entries, laid out from its incoming location);
  *            a window of more than 8192 merged entries, or runs crossing a

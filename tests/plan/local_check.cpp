@@ -11,6 +11,7 @@
 #include <set>
 #include <vector>
 
+#include "../../gpuquotientfilters_amd/csrc/gqf_rsqf_local.hpp"
 #include "../../gpuquotientfilters_amd/csrc/gqf_sqf_local.hpp"
 
 using namespace gqf;
@@ -117,8 +118,134 @@ static std::vector<uint32_t> on_planes(const std::vector<uint32_t>& t, const std
   return x;
 }
 
+// RSQF: nb blocks, the canonical bits, remainders and offsets of sorted
+// fingerprints (loc_i = max(fq_i, loc_{i-1} + 1)).
+struct Rs {
+  std::vector<unsigned long long> occ, ends, rem;
+  std::vector<uint32_t> off;
+  uint32_t nb, r;
+  Rs(uint32_t nb_, uint32_t r_) : occ(nb_, 0), ends(nb_, 0), rem((size_t)nb_ * r_ + 1, 0), off(nb_, 0), nb(nb_), r(r_) {}
+  bool fill(const std::vector<uint64_t>& fps) {
+    int64_t loc = -1, last = -1;
+    std::vector<int64_t> L(nb, -1);  // last location of a quotient below the block
+    for (uint64_t f : fps) {
+      const int64_t q = (int64_t)(f >> r);
+      if (q != last && last >= 0) ends[(size_t)loc >> 6] |= 1ull << (loc & 63);
+      loc = std::max(q, loc + 1);
+      if (loc >= 64 * (int64_t)nb) return false;
+      occ[(size_t)q >> 6] |= 1ull << (q & 63);
+      for (uint32_t k = 0; k < r; ++k) {
+        const uint64_t b = (uint64_t)loc * r + k;
+        rem[b >> 6] |= (unsigned long long)((f >> k) & 1ull) << (b & 63);
+      }
+      for (size_t j = (size_t)(q >> 6) + 1; j < nb; ++j) L[j] = loc;
+      last = q;
+    }
+    if (last >= 0) ends[(size_t)loc >> 6] |= 1ull << (loc & 63);
+    for (uint32_t j = 0; j < nb; ++j) off[j] = L[j] >= 64 * (int64_t)j ? (uint32_t)(L[j] - 64 * (int64_t)j + 1) & 0xFFu : 0u;
+    return true;
+  }
+  bool operator==(const Rs& o) const { return occ == o.occ && ends == o.ends && rem == o.rem && off == o.off; }
+};
+
+template <int R>
+static void rsqf_case(std::mt19937& g, uint32_t r) {
+  const uint32_t q = 6 + g() % 6, nb = (1u << q) / 64 + 1, S = 64 * nb;
+  const uint32_t n = (uint32_t)(g() % 100 * (1u << q) / 100), m = 1 + g() % (1 + (1u << q) / 4);
+  const uint64_t fm = (1ull << (q + r)) - 1;
+  std::vector<uint64_t> base, batch;
+  for (uint32_t i = 0; i < n; ++i) base.push_back(g() & fm);
+  std::sort(base.begin(), base.end());
+  for (uint32_t i = 0; i < m; ++i) batch.push_back(base.size() && g() % 2 ? base[g() % base.size()] : g() & fm);
+  if (g() % 3 == 0)
+    for (uint32_t i = 0; i < m; i += 1 + g() % 3) batch[i] = batch[0];
+  std::sort(batch.begin(), batch.end());
+  Rs t(nb, r);
+  if (!t.fill(base)) return;
+  // D at every slot, empty slots, boundaries
+  std::vector<uint32_t> E(S + 1), D(S + 1), empties, lb(S);
+  std::vector<unsigned long long> em(nb, 0);
+  int32_t d = 0;
+  for (uint32_t s = 0, l = 0; s < S; ++s) {
+    E[s] = (uint32_t)empties.size();
+    D[s] = (uint32_t)d;
+    if (d == 0) l = s + 1;
+    lb[s] = l;
+    d += (int32_t)((t.occ[s >> 6] >> (s & 63)) & 1ull);
+    if (d == 0) {
+      empties.push_back(s);
+      em[s >> 6] |= 1ull << (s & 63);
+    }
+    d -= (int32_t)((t.ends[s >> 6] >> (s & 63)) & 1ull);
+  }
+  auto run = [&](bool ins, const std::vector<uint32_t>& heads) {
+    Rs x(t);
+    std::vector<int32_t> off(nb, 0);
+    RlPlanes<R> P;
+    P.occ = x.occ.data(), P.ends = x.ends.data(), P.rem = x.rem.data(), P.empty = em.data(), P.off = off.data();
+    P.end = S, P.r = r, P.dirty[0] = P.dirty[1] = 0;
+    std::vector<uint32_t> order(heads.size());
+    for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
+    std::shuffle(order.begin(), order.end(), g);
+    for (uint32_t i : order) {
+      const uint32_t kb = i + 1 < heads.size() ? heads[i + 1] : m;
+      const uint32_t a = (uint32_t)(batch[heads[i]] >> r);
+      uint32_t e = a - 1;
+      for (uint32_t k = heads[i]; k < kb; ++k) {
+        const uint32_t fq = (uint32_t)(batch[k] >> r), fr = (uint32_t)batch[k] & ((1u << r) - 1u);
+        if (ins) {
+          e = P.next(em.data(), e + 1);
+          P.insert(fq, fr, a, D[a], e);
+        } else {
+          P.erase(fq, fr, a, D[a]);
+        }
+      }
+    }
+    for (uint32_t j = 0; j < nb; ++j) {
+      const bool changed = x.occ[j] != t.occ[j] || x.ends[j] != t.ends[j] || off[j] != 0;
+      if (changed && !((P.dirty[j >> 6] >> (j & 63)) & 1ull)) fail("rsqf change outside the marked blocks", j, q);
+      x.off[j] = (x.off[j] + (uint32_t)off[j]) & 0xFFu;
+    }
+    return x;
+  };
+  {
+    std::vector<uint64_t> all(base);
+    all.insert(all.end(), batch.begin(), batch.end());
+    std::sort(all.begin(), all.end());
+    std::vector<uint32_t> heads;
+    bool fits = true;
+    int64_t J = -1;
+    for (uint32_t k = 0; k < m; ++k) {
+      const int64_t e = E[batch[k] >> r];
+      if (J < e) heads.push_back(k);
+      J = std::max(J + 1, e);
+      fits = fits && J < (int64_t)empties.size();
+    }
+    Rs want(nb, r);
+    if (fits != want.fill(all)) fail("rsqf fits", q, r);
+    if (fits && !(run(true, heads) == want)) fail("rsqf insert", q, r);
+  }
+  {
+    std::multiset<uint64_t> ms(base.begin(), base.end());
+    for (uint64_t b : batch) {
+      auto p = ms.find(b);
+      if (p != ms.end()) ms.erase(p);
+    }
+    std::vector<uint32_t> heads;
+    for (uint32_t k = 0; k < m; ++k)
+      if (k == 0 || lb[batch[k] >> r] > (uint32_t)(batch[k - 1] >> r) + 1) heads.push_back(k);
+    Rs want(nb, r);
+    (void)want.fill(std::vector<uint64_t>(ms.begin(), ms.end()));
+    if (!(run(false, heads) == want)) fail("rsqf delete", q, r);
+  }
+}
+
 int main() {
   std::mt19937 g(7);
+  for (int it = 0; it < 1500; ++it) {
+    rsqf_case<8>(g, 8);
+    rsqf_case<0>(g, 1 + g() % 16);
+  }
   for (int it = 0; it < 6000; ++it) {
     const uint32_t q = 3 + g() % 9, r = 1 + g() % 9;
     const uint32_t S = (uint32_t)((double)(1u << q) * 1.1);
@@ -198,7 +325,7 @@ int main() {
   }
   // the window states' composition against the recurrence, key by key
   for (int it = 0; it < 2000; ++it) {
-    LW p{0, 0, 0u};
+    LW p{0, 0, 0u, 0u};
     int64_t o = 0;
     for (int w = 0; w < 20; ++w) {
       const int32_t e = (int32_t)(g() % 40), nk = (int32_t)(g() % 30);
@@ -213,7 +340,7 @@ int main() {
       }
       o = std::max<int64_t>(0, c - e);
       const int32_t a = nk - e;
-      p = lw_combine(p, LW{a, std::max(0, nk ? M + a : 0), 0u});
+      p = lw_combine(p, LW{a, std::max(0, nk ? M + a : 0), 0u, 0u});
       if (std::max(p.a, p.b) != o) fail("state", (uint32_t)w, (uint32_t)o);
     }
   }

@@ -69,6 +69,7 @@ CASES = [(13, 5, 0.5, False), (16, 5, 0.75, False), (18, 5, 0.85, True), (16, 13
 @pytest.mark.parametrize("q,r,alpha,dup", CASES)
 def test_sqf_local_insert(q, r, alpha, dup):
     say("sqf local insert", q, r, alpha, dup)
+    st = G.Stream()  # a context of its own: no batch of it has been handed over yet
     keys = O.mt19937(300 + q, O.key_count(alpha, q))
     if dup:
         keys = np.concatenate([keys[:-50], keys[:50]])
@@ -87,11 +88,12 @@ def test_sqf_local_insert(q, r, alpha, dup):
             break
         b = np.concatenate([pool[at:at + n - n // 4], keys[at:at + n // 4]])
         at += n
-        names = _kernels(lambda: f.insert(dev(b)))
+        names = _kernels(lambda: f.insert(dev(b), stream=st))
         local += any("k_sl_apply" in x for x in names) and not any("k_rb_write" in x for x in names)
         fps = insert_set(fps, O.fingerprints(b, q, r))
         sqf_equal(f, sqf_table(fps, q, r))
     assert local >= 2  # the localized form ran, and alone
+    st.destroy()
 
 
 def test_sqf_local_insert_hot_and_edges():
@@ -118,6 +120,7 @@ def test_sqf_local_insert_hot_and_edges():
 def test_sqf_local_delete(q, r, alpha, dup):
     """Stored keys, keys that are not stored, repeated keys, several copies."""
     say("sqf local delete", q, r, alpha, dup)
+    st = G.Stream()
     keys = O.mt19937(320 + q, O.key_count(alpha, q))
     if dup:
         keys = np.concatenate([keys[:-50], keys[:25], keys[:25]])
@@ -135,11 +138,12 @@ def test_sqf_local_delete(q, r, alpha, dup):
             break
         b = np.concatenate([keys[at:at + n - n // 3], keys[at:at + n // 6], other[at:at + n // 6]])
         at += n
-        names = _kernels(lambda: f.superclusterDeletes(dev(b)))
+        names = _kernels(lambda: f.superclusterDeletes(dev(b), stream=st))
         local += any("k_sl_apply" in x for x in names) and not any("k_rb_write" in x for x in names)
         fps = delete_multiset(fps, O.fingerprints(b, q, r))
         sqf_equal(f, sqf_table(fps, q, r))
     assert local >= 2
+    st.destroy()
 
 
 def test_sqf_local_delete_hot_and_edges():
@@ -158,3 +162,68 @@ def test_sqf_local_delete_hot_and_edges():
         f.superclusterDeletes(dev(b))
         fps = delete_multiset(fps, O.fingerprints(b, q, r))
         sqf_equal(f, sqf_table(fps, q, r))
+
+
+# ---------------------------------------------------------------- RSQF
+RCASES = [(13, 8, 0.5), (16, 8, 0.8), (18, 8, 0.9), (16, 16, 0.9), (17, 5, 0.85), (16, 11, 0.8), (20, 13, 0.5),
+          (15, 1, 0.5), (25, 8, 0.1)]
+
+
+def rsqf_table(fps, q, r):
+    st, t = O.rsqf_canon(np.sort(fps), q, r)
+    assert st == O.OK
+    return t
+
+
+def rsqf_equal(f, want):
+    got = f.dump()
+    assert (got == want).all(), np.flatnonzero(got != want)[:8]
+
+
+@pytest.mark.parametrize("q,r,alpha", RCASES)
+def test_rsqf_local_insert(q, r, alpha):
+    say("rsqf local insert", q, r, alpha)
+    st = G.Stream()
+    keys = O.mt19937(340 + q + r, O.key_count(alpha, q))
+    f = G.RSQF(q, r)
+    f.bulk_build(dev(keys))
+    fps = O.fingerprints(keys, q, r)
+    S = 1 << q
+    pool = O.mt19937(341 + q, S)
+    at = local = 0
+    for n in [1, 2, 63, 64, 65, 1000, S // 400 + 1, S // 82]:
+        n = min(n, S // 82)
+        b = np.concatenate([pool[at:at + n - n // 4], keys[at:at + n // 4]])
+        at += n
+        if len(b) == 0:
+            continue
+        out = G.DeviceArray.empty(len(b))
+        names = _kernels(lambda: f.insert(dev(b), out, stream=st))
+        ran = any("k_rl_apply" in x for x in names)
+        alone = not any("k_wm_write" in x or "k_rr_write" in x for x in names)
+        local += ran and alone
+        fps = np.concatenate([fps, O.fingerprints(b, q, r)])
+        want = rsqf_table(fps, q, r)
+        rsqf_equal(f, want)
+        assert (out.to_host() == O.rsqf_lookup_keys(want, q, r, b)).all()
+    assert local >= 2
+    st.destroy()
+
+
+def test_rsqf_local_insert_hot_and_edges():
+    q, r = 16, 8
+    say("rsqf local insert edges", q, r)
+    cand = O.mt19937(350, 1 << 19)
+    fq = O.fingerprints(cand, q, r) >> np.uint64(r)
+    edge = cand[((fq % 4096 >= 4056) | (fq % 4096 < 8)) & (fq < (1 << q) - 64)]  # the last block overflows
+    ends = cand[(fq < 3) | (fq >= (1 << q) - 3)]
+    base = np.concatenate([O.mt19937(351, O.key_count(0.6, q)), edge[:1500]])
+    f = G.RSQF(q, r)
+    f.bulk_build(dev(base))
+    fps = O.fingerprints(base, q, r)
+    # (30 copies: one region; 70 and 300: a wave of copies and more, handed over)
+    for b in [edge[1500:2200], ends[:40], np.full(30, cand[0]), np.full(70, cand[1]), np.full(300, cand[1]),
+              edge[2200:2900], np.concatenate([np.full(40, cand[1]), edge[2900:3000]])]:
+        f.insert(dev(b))
+        fps = np.concatenate([fps, O.fingerprints(b, q, r)])
+        rsqf_equal(f, rsqf_table(fps, q, r))
