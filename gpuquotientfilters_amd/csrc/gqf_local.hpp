@@ -66,6 +66,10 @@ constexpr uint32_t LW_MAX_WINDOWS = RBS_PER * 64;  // one state per window: the 
 //             fill 0.8   2^10 keys 0.072 / 0.293   2^18 0.158 / 0.392   2^20 0.232 / 0.400
 //   q=24 r=5  fill 0.7   2^10 keys 0.058 / 0.145   2^16 0.088 / 0.197
 //   q=22 r=8  fill 0.8   2^10 keys 0.055 / 0.073   2^13 0.070 / 0.084
+// RSQF deletes, localized / rebuild:
+//   q=26 r=8  fill 0.5   2^10 keys 0.077 / 0.375   2^18 0.155 / 0.419   2^21 0.288 / 0.497
+//             fill 0.8   2^10 keys 0.083 / 0.472   2^18 0.216 / 0.549   2^20 0.333 / 0.574
+//   q=24 r=5  fill 0.7   2^10 keys 0.062 / 0.182   2^16 0.110 / 0.191
 static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8192ull * LW_SLOTS) ? 32 : 80) <= slots; }
 
 // Whether the stream's next batch of this kind (LocalKind) tries the
@@ -128,12 +132,7 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
 // Exclusive scan of the window states in two launches (as rb_scan): pre[w] =
 // {keys that overflow into window w, 1 + the last boundary before it}.  More
 // than LW_SPILL of the former, or any past the last window, raise the flag;
-// so do fewer than 3 regions per 4 of the n keys (batches of at least a key
-// per window): long clusters and several keys in each make a wave wait for a
-// few lanes.  RSQF q=26 r=8 inserts without that rule, ms per call, localized
-// / by windows, with the keys per region:
-//   fill 0.8  2^20 keys 0.235 / 0.399 (1.20)  2^21 0.429 / 0.453 (1.39)
-//   fill 0.9  2^18 keys 0.307 / 0.401 (1.17)  2^20 0.950 / 0.412 (1.67)
+// so do fewer regions than min_heads (lw_min_heads).
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_reduce(const uint4* __restrict__ st, uint32_t W,
                                                                             uint4* __restrict__ part) {
   __shared__ uint4 s_wave[16];
@@ -151,7 +150,7 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
 
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W,
                                                                           const uint4* __restrict__ part,
-                                                                          uint2* __restrict__ pre, uint32_t n,
+                                                                          uint2* __restrict__ pre, uint32_t min_heads,
                                                                           uint32_t* __restrict__ ctr) {
   __shared__ uint4 s_wave[17];  // wave aggregates, then their prefixes; [16] = carry
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
@@ -179,14 +178,26 @@ __device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
   bool bad = o > LW_SPILL;
   if (i + 1 == W) {
     const LW all = lw_combine(p, x);
-    bad = bad || (all.a > all.b ? all.a : all.b) > 0 || (n >= W && (uint64_t)all.heads * 4 < (uint64_t)n * 3);
+    bad = bad || (all.a > all.b ? all.a : all.b) > 0 || all.heads < min_heads;
   }
   if (bad) ctr[CTR_MISC] = 1u;
 }
 
+// The regions a batch must have, 24 (insert) or 25 (delete) per 32 keys
+// where there is a key per window: long clusters with several keys in each
+// make a wave wait for a few lanes.  RSQF q=26 r=8 without that rule, ms per
+// call, localized / general path, and the keys per region:
+//   insert  fill 0.8   2^20 keys 0.235 / 0.399 (1.20)   2^21 0.429 / 0.453 (1.39)
+//           fill 0.9   2^18 keys 0.307 / 0.401 (1.17)   2^20 0.950 / 0.412 (1.67)
+//   delete  fill 0.85  2^20 keys 0.515 / 0.597 (1.27)
+//           fill 0.9   2^18 keys 0.458 / 0.601 (1.18)   2^19 0.688 / 0.611 (1.29)
+static inline uint32_t lw_min_heads(bool insert, uint32_t n, uint32_t W) {
+  return n < W ? 0u : (uint32_t)((uint64_t)n * (insert ? 24 : 25) / 32);
+}
+
 static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
-static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre, uint32_t n,
-                                 uint32_t* ctr) {
+static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre,
+                                 uint32_t min_heads, uint32_t* ctr) {
   const uint32_t P = (W + RBS_PER - 1) / RBS_PER;
   uint4* part = ar.take<uint4>(P ? P : 1);
   if (ar.used > ar.cap) {
@@ -194,7 +205,7 @@ static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint
     return GQF_ERR_INVALID;
   }
   GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part);
-  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, n, ctr);
+  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, min_heads, ctr);
   return GQF_OK;
 }
 

@@ -1779,7 +1779,7 @@ static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gq
              ds.counters);
   GQF_LAUNCH_B(mb + (double)n * (sizeof(K) + 4), (k_rl_plan<K, INS>), dim3(W), dim3(64), 0, s, d.meta, g.nb, g.r, wp, B,
                bstart, W, key, empty, fb, st, ds.counters);
-  GQF_TRY(lw_scan(s, ar, st, W, pre, n, ds.counters));
+  GQF_TRY(lw_scan(s, ar, st, W, pre, lw_min_heads(INS, n, W), ds.counters));
   uint64_t* meta = reinterpret_cast<uint64_t*>(f.blocks);
   uint64_t* remg = reinterpret_cast<uint64_t*>(reinterpret_cast<uint8_t*>(f.blocks) + rsqf_meta_bytes(g.nb));
   const double wb = (double)rsqf_dev_bytes(g.q, g.r) + (double)n * (sizeof(K) + 4 + 256);
@@ -1853,6 +1853,23 @@ static gqf_status rsqf_delete_t(const gqf_rsqf& f, uint32_t n, const uint32_t* k
     GQF_LAUNCH_BC(0.0, m_dev, dper, (k_delete_mark<K, false>), dim3((mcap + DM_TILE - 1) / DM_TILE), dim3(DM_THREADS),
                   0, cs.stream, A, mcap, m_dev, D, n, keep, (const uint32_t*)nullptr);
   return rsqf_rebuild<K, KEEP_FLAGS, false>(cs.stream, ds, ar, f, A, mcap, m_dev, (const K*)nullptr, 0u, keep, hb);
+}
+
+// The localized delete: *done, or the table is untouched.
+template <typename K>
+static gqf_status rsqf_delete_local_t(const gqf_rsqf& f, uint32_t n, const uint32_t* keys, CallScope& cs, bool* done,
+                                      float* ms) {
+  DeviceState& ds = *cs.ds;
+  const RsqfGeom g = rgeom(f);
+  GQF_TRY(ws_reserve(ds, sort_workspace_bytes(n, sizeof(K), false) + rsqf_local_ws(g, n)));
+  Arena ar(ds.ws, ds.ws_cap);
+  K* D;
+  GQF_TRY(radix_sort<K>(cs.stream, ar, keys, true, g.bits, nullptr, false, n, 0, g.bits, &D, nullptr, cs.ds));
+  GQF_TRY((rsqf_local<K, false>(cs.stream, ds, ar, f, D, n)));
+  GQF_TRY(cs.end(ms, true));
+  *done = ds.h_pinned[CTR_MISC] == 0;
+  lw_report(ds, LOCAL_RSQF_DELETE, *done);
+  return GQF_OK;
 }
 
 // Keys left out of a partial insert: fingerprint >= cut -> -1.
@@ -2015,9 +2032,20 @@ gqf_status gqf_rsqf_insert_report(gqf_rsqf cqf, int n, const uint32_t* d_keys, i
 
 gqf_status gqf_rsqf_delete(gqf_rsqf cqf, int n, const uint32_t* d_keys, gqf_stream stream, float* ms) {
   GQF_TRY(rsqf_args(cqf, n, d_keys));
+  const bool wide = cqf.qbits + cqf.rbits > 32;
   CallScope cs;
   GQF_TRY(cs.begin(stream));
-  if (cqf.qbits + cqf.rbits <= 32) GQF_TRY(rsqf_delete_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs));
+  float t0 = 0.f;
+  if (rsqf_local_fits(rgeom(cqf), (uint32_t)n) && lw_try(*cs.ds, LOCAL_RSQF_DELETE)) {
+    bool done = false;
+    if (!wide) GQF_TRY(rsqf_delete_local_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs, &done, &t0));
+    else GQF_TRY(rsqf_delete_local_t<uint64_t>(cqf, (uint32_t)n, d_keys, cs, &done, &t0));
+    if (done) {
+      if (ms) *ms = t0;
+      return GQF_OK;
+    }
+  }
+  if (!wide) GQF_TRY(rsqf_delete_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs));
   else GQF_TRY(rsqf_delete_t<uint64_t>(cqf, (uint32_t)n, d_keys, cs));
   return cs.end(ms, true);
 }

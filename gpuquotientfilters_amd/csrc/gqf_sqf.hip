@@ -300,7 +300,7 @@ static gqf_status sqf_local_t(hipStream_t s, uint32_t* ctr, Arena& ar, const gqf
   GQF_LAUNCH((k_wm_bounds<uint32_t>), dim3(((W + 1) * WB_LANES + 255) / 256), dim3(256), 0, s, B, n, g.r, W, bstart, ctr);
   GQF_LAUNCH_B((double)g.bytes + (double)n * 6, (k_sl_plan<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S, g.r, B,
                bstart, W, el, fb, st, ctr);
-  GQF_TRY(lw_scan(s, ar, st, W, pre, n, ctr));
+  GQF_TRY(lw_scan(s, ar, st, W, pre, lw_min_heads(INS, n, W), ctr));
   GQF_LAUNCH_B(2.0 * (double)g.bytes + (double)n * 6, (k_sl_apply<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S,
                g.r, B, n, bstart, W, pre, el, fb, ctr);
   return GQF_OK;

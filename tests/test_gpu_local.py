@@ -227,3 +227,48 @@ def test_rsqf_local_insert_hot_and_edges():
         f.insert(dev(b))
         fps = np.concatenate([fps, O.fingerprints(b, q, r)])
         rsqf_equal(f, rsqf_table(fps, q, r))
+
+
+@pytest.mark.parametrize("q,r,alpha", RCASES)
+def test_rsqf_local_delete(q, r, alpha):
+    """Stored keys, keys that are not stored, repeated keys, several copies."""
+    say("rsqf local delete", q, r, alpha)
+    st = G.Stream()
+    keys = O.mt19937(360 + q + r, O.key_count(alpha, q))
+    keys = np.concatenate([keys[:-50], keys[:25], keys[:25]])
+    f = G.RSQF(q, r)
+    f.bulk_build(dev(keys))
+    fps = O.fingerprints(keys, q, r)
+    S = 1 << q
+    other = O.mt19937(361 + q, S)
+    at = local = 0
+    for n in [1, 2, 63, 64, 65, 1000, S // 400 + 1, S // 82]:
+        n = min(n, S // 82)
+        b = np.concatenate([keys[at:at + n - n // 3], keys[at:at + n // 6], other[at:at + n // 6]])
+        at += n
+        if len(b) == 0:
+            continue
+        names = _kernels(lambda: f.deleteGPU(dev(b), stream=st))
+        local += any("k_rl_apply" in x for x in names) and not any("k_rr_write" in x for x in names)
+        fps = delete_multiset(fps, O.fingerprints(b, q, r))
+        rsqf_equal(f, rsqf_table(fps, q, r))
+    assert local >= 2
+    st.destroy()
+
+
+def test_rsqf_local_delete_hot_and_edges():
+    q, r = 16, 8
+    say("rsqf local delete edges", q, r)
+    cand = O.mt19937(370, 1 << 19)
+    fq = O.fingerprints(cand, q, r) >> np.uint64(r)
+    edge = cand[((fq % 4096 >= 4056) | (fq % 4096 < 8)) & (fq < (1 << q) - 64)]
+    ends = cand[(fq < 3) | (fq >= (1 << q) - 3)]
+    base = np.concatenate([O.mt19937(371, O.key_count(0.6, q)), edge[:2500], ends[:30], np.full(90, cand[5])])
+    f = G.RSQF(q, r)
+    f.bulk_build(dev(base))
+    fps = O.fingerprints(base, q, r)
+    for b in [edge[:700], ends[:40], np.full(30, cand[5]), np.full(70, cand[5]), edge[700:1400], base[:700],
+              edge[1400:2100]]:
+        f.deleteGPU(dev(b))
+        fps = delete_multiset(fps, O.fingerprints(b, q, r))
+        rsqf_equal(f, rsqf_table(fps, q, r))
