@@ -115,6 +115,17 @@ __device__ __forceinline__ uint64_t wave_incl_add64(uint64_t x) {
   x += dpp_u64<DPP_ROW_BCAST31, 0xC>(0ull, x);
   return x;
 }
+// Inclusive maximum over the lanes of a wave.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
+  auto mx = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 1>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 2>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 4>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_SHR | 8>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_BCAST15, 0xA>(0u, x));
+  x = mx(x, dpp_u32<DPP_ROW_BCAST31, 0xC>(0u, x));
+  return x;
+}
 __device__ __forceinline__ uint32_t wave_read(uint32_t x, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)x, lane);
 }

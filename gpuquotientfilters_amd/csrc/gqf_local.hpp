@@ -72,19 +72,6 @@ constexpr uint32_t LW_MAX_WINDOWS = RBS_PER * 64;  // one state per window: the 
 //   q=24 r=5  fill 0.7   2^10 keys 0.062 / 0.182   2^16 0.110 / 0.191
 static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8192ull * LW_SLOTS) ? 32 : 80) <= slots; }
 
-// Whether the stream's next batch of this kind (LocalKind) tries the
-// localized form, and what came of it.
-static inline bool lw_try(DeviceState& ds, LocalKind k) {
-  if (!ds.local_skip[k]) return true;
-  --ds.local_skip[k];
-  return false;
-}
-static inline void lw_report(DeviceState& ds, LocalKind k, bool done) {
-  uint32_t& bo = ds.local_backoff[k];
-  bo = done ? 0 : (bo ? (bo < 256 ? 2 * bo : 256) : 4);
-  ds.local_skip[k] = bo;
-}
-
 static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }
 
 // Scan state of a window: overflow map x -> max(x + a, b) (insert), 1 + the
@@ -117,18 +104,6 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
               wave_read(inc.heads, 63)};
   return lw_dpp<DPP_WAVE_SHR1>(inc);
 }
-// Inclusive maximum over the lanes of a wave.
-__device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
-  auto mx = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
-  x = mx(x, dpp_u32<DPP_ROW_SHR | 1>(0u, x));
-  x = mx(x, dpp_u32<DPP_ROW_SHR | 2>(0u, x));
-  x = mx(x, dpp_u32<DPP_ROW_SHR | 4>(0u, x));
-  x = mx(x, dpp_u32<DPP_ROW_SHR | 8>(0u, x));
-  x = mx(x, dpp_u32<DPP_ROW_BCAST15, 0xA>(0u, x));
-  x = mx(x, dpp_u32<DPP_ROW_BCAST31, 0xC>(0u, x));
-  return x;
-}
-
 // Exclusive scan of the window states in two launches (as rb_scan): pre[w] =
 // {keys that overflow into window w, 1 + the last boundary before it}.  More
 // than LW_SPILL of the former, or any past the last window, raise the flag;

@@ -14,6 +14,7 @@
 // reference on any table (including the history-dependent layouts its insert
 // leaves).  Build / insert / delete produce the canonical layout, which is
 // what the reference insert produces when fed fingerprints in ascending order.
+#include "gqf_dbuild.hpp"
 #include "gqf_rsqf_local.hpp"
 
 #include <type_traits>
@@ -1664,6 +1665,26 @@ static gqf_status rsqf_build_t(const gqf_rsqf& f, uint32_t n, const uint32_t* ke
   return rsqf_rebuild<K, KEEP_ALL, false>(cs.stream, ds, ar, f, sorted, n, nullptr, (const K*)nullptr, 0u, nullptr);
 }
 
+// The build by runs; leaves ctr[CTR_MISC] != 0, and the table untouched, when
+// the keys do not fit that form.
+template <bool WIDE>
+static gqf_status rsqf_build_runs(const gqf_rsqf& f, const PsPlan& p, uint32_t n, const uint32_t* keys, CallScope& cs) {
+  DeviceState& ds = *cs.ds;
+  const RsqfGeom g = rgeom(f);
+  Arena ar(ds.ws, ds.ws_cap);
+  DbRuns d;
+  GQF_TRY((db_runs<WIDE>(cs.stream, ar, p, keys, g.bits, n, g.r, false, g.cap, ds.counters, &d)));
+  uint8_t* meta = reinterpret_cast<uint8_t*>(f.blocks);
+  const double wb = (double)rsqf_dev_bytes(g.q, g.r) + (double)n + (double)((uint64_t)1 << g.q);
+  if (g.r == 8)
+    GQF_LAUNCH_B(wb, k_db_rsqf<8>, dim3(p.ngroups), dim3(PS_THREADS), 0, cs.stream, meta, meta + rsqf_meta_bytes(g.nb), g.r,
+                 d.gsize, p.cap, p.qb, d.counts, d.rems, d.th, d.agg, d.spill, p.ngroups, ds.counters);
+  else
+    GQF_LAUNCH_B(wb, k_db_rsqf<0>, dim3(p.ngroups), dim3(PS_THREADS), 0, cs.stream, meta, meta + rsqf_meta_bytes(g.nb), g.r,
+                 d.gsize, p.cap, p.qb, d.counts, d.rems, d.th, d.agg, d.spill, p.ngroups, ds.counters);
+  return GQF_OK;
+}
+
 template <typename K>
 static size_t rsqf_insert_ws(const RsqfGeom& g, uint32_t n) {
   return rsqf_decode_ws(g, sizeof(K)) + sort_workspace_bytes(n, sizeof(K), false) + rsqf_rebuild_ws(g.cap + n);
@@ -1925,6 +1946,16 @@ gqf_status gqf_rsqf_bulk_build(gqf_rsqf cqf, int n, const uint32_t* d_keys, gqf_
   GQF_TRY(rsqf_args(cqf, n, d_keys));
   CallScope cs;
   GQF_TRY(cs.begin(stream));
+  PsPlan p;
+  if (ps_plan((uint64_t)n, cqf.qbits, cqf.rbits, PS_SPARSE_RSQF, &p) && lw_try(*cs.ds, LOCAL_RSQF_BUILD) &&
+      ws_try_reserve(*cs.ds, ps_bytes(p))) {
+    if (cqf.qbits + cqf.rbits <= 32) GQF_TRY(rsqf_build_runs<false>(cqf, p, (uint32_t)n, d_keys, cs));
+    else GQF_TRY(rsqf_build_runs<true>(cqf, p, (uint32_t)n, d_keys, cs));
+    const gqf_status st = cs.end(ms, true);
+    const bool done = cs.ds->h_pinned[CTR_MISC] == 0;
+    lw_report(*cs.ds, LOCAL_RSQF_BUILD, done);
+    if (done) return st;
+  }
   if (cqf.qbits + cqf.rbits <= 32) GQF_TRY(rsqf_build_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs));
   else GQF_TRY(rsqf_build_t<uint64_t>(cqf, (uint32_t)n, d_keys, cs));
   return cs.end(ms, true);

@@ -58,8 +58,12 @@ struct ProfRec {
   double dper;
 };
 
-// Kinds of localized updates (gqf_local.hpp).
-enum LocalKind : int { LOCAL_SQF_INSERT = 0, LOCAL_SQF_DELETE, LOCAL_RSQF_INSERT, LOCAL_RSQF_DELETE, LOCAL_KINDS };
+// Kinds of calls whose fast form (gqf_local.hpp, gqf_dbuild.hpp) may hand a
+// batch over to the general one.
+enum LocalKind : int {
+  LOCAL_SQF_INSERT = 0, LOCAL_SQF_DELETE, LOCAL_RSQF_INSERT, LOCAL_RSQF_DELETE, LOCAL_SQF_BUILD, LOCAL_RSQF_BUILD,
+  LOCAL_KINDS
+};
 
 // Execution context of one (device, stream) pair: workspace arena, device
 // counters and their pinned mirror, timing events.  Calls on the same stream
@@ -85,7 +89,7 @@ struct DeviceState {
   // pair per key width: 32-bit (SQF, AP hash) and 64-bit (wide) fingerprints
   // crowd differently.
   uint32_t crowd_skip[2] = {0, 0}, crowd_backoff[2] = {0, 0};
-  // likewise after a batch that the localized updates handed over, per kind
+  // likewise after a batch that a fast form handed over, per kind
   uint32_t local_skip[LOCAL_KINDS] = {}, local_backoff[LOCAL_KINDS] = {};
   // per-launch timing (gqf_profile_enable): event pool and launches to resolve
   hipEvent_t* pool = nullptr;
@@ -94,12 +98,31 @@ struct DeviceState {
   size_t pending_size = 0, pending_used = 0;
 };
 
+// Whether the stream's next call of this kind tries its fast form, and what
+// came of it.
+inline bool lw_try(DeviceState& ds, LocalKind k) {
+  if (!ds.local_skip[k]) return true;
+  --ds.local_skip[k];
+  return false;
+}
+inline void lw_report(DeviceState& ds, LocalKind k, bool done) {
+  uint32_t& bo = ds.local_backoff[k];
+  bo = done ? 0 : (bo ? (bo < 256 ? 2 * bo : 256) : 4);
+  ds.local_skip[k] = bo;
+}
+
 // The context of the calling thread's current device and `stream`, created
 // on first use (contexts live until the process ends).
 gqf_status device_state(hipStream_t stream, DeviceState** out);
 // Bytes a workspace grows to when a call needs `bytes` more than it holds.
 size_t ws_alloc_bytes(size_t bytes);
 gqf_status ws_reserve(DeviceState& ds, size_t bytes);
+// The same for a form that another one can stand in for.
+inline bool ws_try_reserve(DeviceState& ds, size_t bytes) {
+  if (ws_reserve(ds, bytes) == GQF_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
 
 // Bump allocator over the workspace of one call.
 struct Arena {

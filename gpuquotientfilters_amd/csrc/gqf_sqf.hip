@@ -11,6 +11,7 @@
 //   [decode table] -> [hash + radix sort keys] -> [merge / mark] ->
 //   layout scan (locations) -> table writer (every slot written once).
 // Lookups are the reference's run walk (quotientFilter.cu:172-196, 320-357).
+#include "gqf_dbuild.hpp"
 #include "gqf_sqf_local.hpp"
 
 #include <algorithm>
@@ -211,6 +212,24 @@ static gqf_status sqf_build_launch(hipStream_t s, Arena& ar, uint32_t* counters,
   return launch_rebuild<KEEP_ALL, false>(s, counters, ar, qf, g, sorted, un, nullptr, nullptr, 0, nullptr);
 }
 
+// The build without a sort (gqf_dbuild.hpp).  Leaves ctr[CTR_MISC] != 0, and
+// the table untouched, when the keys do not fit that form.
+static gqf_status sqf_build_runs(hipStream_t s, Arena& ar, uint32_t* ctr, const gqf_sqf& wq, const SqfGeom& g,
+                                 const PsPlan& p, uint32_t un, const uint32_t* d_keys, int no_dup) {
+  DbRuns d;
+  GQF_TRY((db_runs<false>(s, ar, p, d_keys, (g.q + g.r) | sqf_hash_flag(), un, g.r, no_dup != 0, (uint64_t)g.S, ctr, &d)));
+  const double wb = (double)g.bytes + (double)un + (double)((uint64_t)1 << g.q);
+  if (g.bpe == 1)
+    GQF_LAUNCH_B(wb, k_db_sqf<1>, dim3(p.ngroups), dim3(PS_THREADS), 0, s, wq.table, g.S, d.gsize, p.cap, p.qb, d.counts, d.rems,
+                 d.th, d.agg, d.spill, p.ngroups, ctr);
+  else
+    GQF_LAUNCH_B(wb, k_db_sqf<2>, dim3(p.ngroups), dim3(PS_THREADS), 0, s, wq.table, g.S, d.gsize, p.cap, p.qb, d.counts, d.rems,
+                 d.th, d.agg, d.spill, p.ngroups, ctr);
+  GQF_LAUNCH(k_sqf_clear_tail, dim3(1024), dim3(256), 0, s, wq.table, g.bpe, g.bytes, ctr, 4, (const uint32_t*)nullptr, 0u,
+             1u << g.q);
+  return GQF_OK;
+}
+
 static gqf_status sqf_build_impl(const gqf_sqf& qf, int n, const uint32_t* d_keys, int no_dup, gqf_stream stream,
                                  float* ms) {
   GQF_TRY(sqf_check(qf));
@@ -220,10 +239,24 @@ static gqf_status sqf_build_impl(const gqf_sqf& qf, int n, const uint32_t* d_key
   GQF_TRY(cs.begin(stream));
   DeviceState& ds = *cs.ds;
   const uint32_t un = (uint32_t)n;
-  GQF_TRY(ws_reserve(ds, sqf_build_ws_bytes(un, true) + packed_ws_bytes(g)));
+  PsPlan p;
+  bool runs = g.bpe <= 2 && ps_plan(un, g.q, g.r, PS_SPARSE_SQF, &p) && lw_try(ds, LOCAL_SQF_BUILD);
+  const size_t sort_ws = sqf_build_ws_bytes(un, true) + packed_ws_bytes(g);
+  if (runs) runs = ws_try_reserve(ds, std::max(sort_ws, ps_bytes(p) + packed_ws_bytes(g)));
+  GQF_TRY(ws_reserve(ds, sort_ws));
   Arena ar(ds.ws, ds.ws_cap);
   gqf_sqf wq;
   GQF_TRY(work_table(cs.stream, ar, qf, g, false, &wq));
+  if (runs) {
+    const size_t mark = ar.used;
+    GQF_TRY(sqf_build_runs(cs.stream, ar, ds.counters, wq, g, p, un, d_keys, no_dup));
+    finish_table(cs.stream, qf, wq, g, ds.counters);
+    const gqf_status st = cs.end(ms, true);
+    const bool done = ds.h_pinned[CTR_MISC] == 0;
+    lw_report(ds, LOCAL_SQF_BUILD, done);
+    if (done) return st;
+    ar.used = mark;  // nothing was written: the sort takes over
+  }
   GQF_TRY(sqf_build_launch(cs.stream, ar, ds.counters, wq, g, un, d_keys, no_dup, &ds));
   finish_table(cs.stream, qf, wq, g, ds.counters);
   return cs.end(ms, true);  // a layout that does not fit is detected before any write

@@ -74,7 +74,8 @@ __host__ __device__ __forceinline__ uint32_t sqf_get_packed(const uint32_t* __re
 
 // Wide table -> packed words, one word per thread: the slots whose bits
 // overlap word j, shifted into place.  With ctr, nothing is written when the
-// call's capacity flag is set (the wide table then holds no result).
+// call's capacity or hand-over flag is set (the wide table then holds no
+// result).
 [[maybe_unused]] static __global__ __launch_bounds__(256) void k_sqf_pack(const uint16_t* __restrict__ wide,
                                                                         uint32_t S, uint32_t width,
                                                                         uint32_t* __restrict__ packed,
@@ -82,7 +83,7 @@ __host__ __device__ __forceinline__ uint32_t sqf_get_packed(const uint32_t* __re
                                                                         const uint32_t* __restrict__ ctr) {
   const uint32_t j = blockIdx.x * 256u + threadIdx.x;
   if (j >= nwords) return;
-  if (ctr && (ctr[CTR_ERR] & DEV_ERR_CAPACITY)) return;
+  if (ctr && ((ctr[CTR_ERR] & DEV_ERR_CAPACITY) || ctr[CTR_MISC])) return;
   const uint64_t b0 = (uint64_t)j * 32;
   uint32_t acc = 0;
   for (uint64_t s = b0 / width; s < S && s * width < b0 + 32; ++s) {
@@ -932,19 +933,22 @@ __global__ __launch_bounds__(RB_THREADS, 6) void k_rb_write(uint8_t* __restrict_
 // cleared after a capacity error.
 // mode 0: the tail; 1: the whole table; 2: the whole table iff the rebuild
 // is sparse (N * 8 < S, then the writer skips windows of zeros); 3: the tail
-// iff it is not.  N = *n_dev (when given) + n_add.
+// iff it is not; 4: from slot S on, or from the slot after the last entry if
+// that is later.  N = *n_dev (when given) + n_add.
 [[maybe_unused]] static __global__ __launch_bounds__(256) void k_sqf_clear_tail(uint8_t* __restrict__ t, uint32_t bpe, uint64_t tbytes,
                                                         const uint32_t* __restrict__ ctr, int mode,
                                                         const uint32_t* __restrict__ n_dev, uint32_t n_add,
                                                         uint32_t S) {
   if (ctr[CTR_ERR]) return;  // capacity error: the table stays as it was
-  if (mode >= 2) {
+  if (mode == 4 && ctr[CTR_MISC]) return;  // handed over: nothing was written
+  if (mode == 2 || mode == 3) {
     const uint64_t N = (uint64_t)(n_dev ? *n_dev : 0u) + n_add;
     const bool sparse = N * 8 < (uint64_t)S;
     if (sparse != (mode == 2)) return;
   }
   const int whole_table = mode == 1 || mode == 2;
-  const uint64_t b0 = whole_table ? 0ull : (uint64_t)ctr[CTR_MISC + 3] * bpe;
+  const uint32_t tail = mode == 4 && S > ctr[CTR_MISC + 3] ? S : ctr[CTR_MISC + 3];
+  const uint64_t b0 = whole_table ? 0ull : (uint64_t)tail * bpe;
   const uint64_t a0 = (b0 + 15) & ~15ull, a1 = tbytes & ~15ull;
   const uint64_t tid = blockIdx.x * 256ull + threadIdx.x, nth = (uint64_t)gridDim.x * 256;
   if (a0 >= a1) {
