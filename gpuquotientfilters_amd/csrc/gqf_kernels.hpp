@@ -679,7 +679,8 @@ k_rs_downsweep(const void* __restrict__ in_keys, const uint32_t* __restrict__ in
                              s_hist, s_run, s_base, s_tmp);
 }
 
-// Every pass of a sort of at most SORT_TILE keys in one workgroup: the keys
+// Every pass of a sort of at most SORT_TILE keys in one workgroup (hashed keys
+// of up to 32 bits take k_rs_one): the keys
 // (and values) stay in registers and LDS between passes; each pass ranks them
 // stably as k_rs_downsweep does (ballots within a wave, then waves in order)
 // and scatters them within LDS.  Key j sits at position wid*1024 + i*64 +
@@ -763,7 +764,8 @@ __global__ __launch_bounds__(SORT_THREADS) void k_rs_small(const void* __restric
 // A keys-only sort with the stream's context replaces the 8-bit passes of
 // the chunked sort by a partition on the top bits and one LDS sort per group
 // of keys:
-//   * 4097 .. 256 * SEG_GROUP_AVG keys: one chunked pass on the top 8 bits
+//   * 16385 (fingerprints past 32 bits: 4097) .. 256 * SEG_GROUP_AVG keys
+//     (fewer: k_rs_one, k_rs_small): one chunked pass on the top 8 bits
 //     of the key range (a stable partition into 256 segments), then
 //     k_rs_seg, one workgroup per segment, sorts the bits below in LDS with
 //     every 4-bit counting pass of the tile sort back to back.  4 launches
@@ -1126,6 +1128,103 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg_slow(K* __restrict__ key
   }
 }
 
+// A keys-only sort of at most ONE_TILE keys by their bits [0, nbits) (nbits <=
+// 32, no bits above) in one workgroup, hashed as read: the bucket method of
+// k_rs_seg with 2^ONE_BB buckets.  One launch: 10000 keys take 10.8 us, where
+// the partition and the segment sort take 35 (4 launches); 4000 keys 6,
+// where 8-bit passes of ballots (k_rs_small) take 21 -- every pass is a chain
+// of LDS accesses that one workgroup cannot hide.
+constexpr int ONE_THREADS = 1024;
+constexpr uint32_t ONE_TILE = ONE_THREADS * SORT_ITEMS;  // 16384 keys
+constexpr uint32_t ONE_BB = 14;
+template <typename K>
+__global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restrict__ in, K* __restrict__ out, uint32_t n,
+                                                        uint32_t fp_bits, uint32_t nbits) {
+  constexpr int T = ONE_THREADS, W = T / 64;
+  __shared__ __align__(16) uint32_t s_keys[ONE_TILE];
+  __shared__ __align__(16) uint32_t s_c[(1u << ONE_BB) / 2];  // bucket counters / cursors; the counting passes' table
+  __shared__ uint32_t s_tmp[W];
+  static_assert(sizeof(s_c) >= 16 * T * sizeof(uint16_t), "the counting passes' table fits");
+  const uint32_t tid = threadIdx.x;
+  const uint32_t bsh = nbits > ONE_BB ? nbits - ONE_BB : 0u;
+  uint4* c4 = reinterpret_cast<uint4*>(s_c) + 2 * tid;  // this thread's 16 counters
+  c4[0] = c4[1] = make_uint4(0u, 0u, 0u, 0u);
+  // key i is in[4 T (i / 4) + 4 tid + i % 4]
+  uint32_t k[SORT_ITEMS];
+#pragma unroll
+  for (int i = 0; i < SORT_ITEMS; ++i) {
+    const uint32_t at = 4 * T * (i / 4) + 4 * tid + (i & 3);
+    k[i] = at < n ? (uint32_t)sort_load_key<K, true>(in, at, fp_bits) : 0u;
+  }
+  auto each = [&](auto f) {
+#pragma unroll
+    for (uint32_t c = 0; c < SORT_ITEMS / 4; ++c)
+      if (4 * T * c < n) {
+#pragma unroll
+        for (uint32_t i = 4 * c; i < 4 * c + 4; ++i)
+          if (4 * T * c + 4 * tid + (i & 3) < n) f(k[i]);
+      }
+  };
+  __syncthreads();
+  each([&](uint32_t x) {
+    const uint32_t b = x >> bsh;
+    atomicAdd(&s_c[b >> 1], 1u << (16 * (b & 1u)));
+  });
+  __syncthreads();
+  {
+    uint32_t w[8];
+    {
+      const uint4 x = c4[0], y = c4[1];
+      w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w, w[4] = y.x, w[5] = y.y, w[6] = y.z, w[7] = y.w;
+    }
+    uint32_t sum = 0, mx = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+      const uint32_t lo = w[i] & 0xFFFFu, hi = w[i] >> 16;
+      sum += lo + hi;
+      mx = lo > mx ? lo : mx;
+      mx = hi > mx ? hi : mx;
+    }
+    uint32_t run = block_excl_scan<T>(sum, s_tmp);
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+      const uint32_t lo = run, c = w[i];
+      run += c & 0xFFFFu;
+      w[i] = lo | (run << 16);
+      run += c >> 16;
+    }
+    c4[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    c4[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    if (__syncthreads_or(mx > SEG_RANK_MAX)) {  // crowded buckets
+#pragma unroll
+      for (int i = 0; i < SORT_ITEMS; ++i) {
+        const uint32_t at = 4 * T * (i / 4) + 4 * tid + (i & 3);
+        if (at < n) out[at] = (K)k[i];
+      }
+      __syncthreads();
+      seg_counting_sort<K, T>(out, n, nbits, s_keys, reinterpret_cast<uint16_t*>(s_c), s_tmp);
+      return;
+    }
+  }
+  each([&](uint32_t x) {
+    const uint32_t b = x >> bsh, hs = 16 * (b & 1u);
+    s_keys[(atomicAdd(&s_c[b >> 1], 1u << hs) >> hs) & 0xFFFFu] = x;
+  });
+  __syncthreads();
+  // counter b now holds the end of bucket b
+  const uint16_t* s_c16 = reinterpret_cast<const uint16_t*>(s_c);
+  for (uint32_t p = tid; p < n; p += T) {
+    const uint32_t x = s_keys[p], b = x >> bsh;
+    const uint32_t st = b ? s_c16[b - 1] : 0u, en = s_c16[b];
+    uint32_t rank = st;
+    for (uint32_t j = st; j < en; ++j) {
+      const uint32_t y = s_keys[j];
+      rank += (y < x || (y == x && j < p)) ? 1u : 0u;
+    }
+    out[rank] = (K)x;
+  }
+}
+
 // Chunks of the segmented pass over n keys (each segment adds at most one
 // partial chunk).
 inline uint32_t seg_chunks2(uint64_t n, uint32_t chunk) { return (uint32_t)((n + chunk - 1) / chunk) + 256u; }
@@ -1176,6 +1275,12 @@ gqf_status radix_sort(hipStream_t s, Arena& ar, const void* in, bool hash, uint3
   if (n == 0) {
     *keys_out = kb[0];
     if (vals_out) *vals_out = vb[0];
+    return GQF_OK;
+  }
+  if (hash && !with_vals && lo_bit == 0 && hi_bit <= 32 && n <= ONE_TILE) {
+    GQF_LAUNCH_B((double)n * (4.0 + sizeof(K)), k_rs_one<K>, dim3(1), dim3(ONE_THREADS), 0, s,
+                 reinterpret_cast<const uint32_t*>(in), kb[0], n, fp_bits, hi_bit);
+    *keys_out = kb[0];
     return GQF_OK;
   }
   if (n <= (uint32_t)SORT_TILE) {
