@@ -1,8 +1,8 @@
 // gqf_serve.hip -- the serving loop: a timed request stream over resident
 // filters, admission against a device-memory budget, and continuous batching.
-// Host C++ only (no kernels).  The scheduler knows nothing of HIP: each call
-// goes through an executor -- the RSQF one at the end of this file, or one
-// the caller supplies (gqf_serve_run).
+// The scheduler knows nothing of HIP: each call goes through an executor --
+// the RSQF one at the end of this file, or one the caller supplies
+// (gqf_serve_run).
 //
 // Workers: with coalescing, one worker per filter (its own host thread and,
 // in the RSQF executor, its own stream); without, one worker for everything.
@@ -261,6 +261,77 @@ gqf_status check_requests(int nfilters, const gqf_request* reqs, int nreqs, cons
   return GQF_OK;
 }
 
+// ---------------------------------------------------------------- gather / scatter
+// The keys of a coalesced call's requests end to end, or its results back to
+// them: one launch per MV_MAX requests with their buffers as kernel arguments.
+// (A copy per request kept the device busy for 2 us and the host for about 4,
+// the latter under a lock that all workers' launches share: 514 copies of a
+// 300-request backlog took a third of its time.)
+constexpr int MV_MAX = 192;
+constexpr uint32_t MV_TILE = 1024;  // keys per workgroup
+struct MvSegs {
+  uint32_t* p[MV_MAX];
+  uint32_t end[MV_MAX];  // of the request's keys in the flat buffer, from the launch's first key on
+};
+static_assert(sizeof(MvSegs) <= 3072, "kernel arguments");
+template <bool GATHER>
+__global__ __launch_bounds__(256) void k_mv(MvSegs s, uint32_t* __restrict__ flat, uint32_t n) {
+  uint32_t at = blockIdx.x * MV_TILE;
+  // the request of the tile's first key: the first that ends past it
+  uint32_t lo = 0, hi = MV_MAX - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) / 2;
+    if (s.end[mid] > at) hi = mid;
+    else lo = mid + 1;
+  }
+  const uint32_t stop = at + MV_TILE < n ? at + MV_TILE : n;
+  // (uniform: every request of the tile in turn)
+  for (uint32_t r = lo; at < stop; ++r) {
+    const uint32_t e = s.end[r] < stop ? s.end[r] : stop;
+    uint32_t* p = s.p[r] - (r ? s.end[r - 1] : 0u);  // (of the launch's first key)
+    for (uint32_t i = at + threadIdx.x; i < e; i += 256) {
+      if (GATHER) flat[i] = p[i];
+      else p[i] = flat[i];
+    }
+    at = e;
+  }
+}
+// Requests b[0 .. nb) <-> flat; requests without keys are left out.
+template <bool GATHER>
+gqf_status mv_requests(hipStream_t s, gqf_request** b, int nb, uint32_t* flat) {
+  MvSegs m;
+  for (int i = 0; i < nb;) {
+    int k = 0;
+    uint64_t n = 0;
+    for (; i < nb && k < MV_MAX && n + (uint64_t)b[i]->n <= 0xFFFFFFFFull; ++i) {
+      if (!b[i]->n) continue;
+      n += (uint64_t)b[i]->n;
+      m.p[k] = GATHER ? const_cast<uint32_t*>(b[i]->d_keys) : reinterpret_cast<uint32_t*>(b[i]->d_out);
+      m.end[k++] = (uint32_t)n;
+    }
+    for (int j = k; j < MV_MAX; ++j) {
+      m.p[j] = nullptr;
+      m.end[j] = 0xFFFFFFFFu;
+    }
+    if (n)
+      GQF_LAUNCH_B((double)n * 8.0, k_mv<GATHER>, dim3((uint32_t)((n + MV_TILE - 1) / MV_TILE)), dim3(256), 0, s, m, flat,
+                   (uint32_t)n);
+    flat += n;
+  }
+  GQF_HIP(hipGetLastError());
+  return GQF_OK;
+}
+// Whether result buffers overlap (the later request's results then stand).
+bool mv_overlap(gqf_request** b, int nb) {
+  std::vector<std::pair<uintptr_t, uintptr_t>> v;
+  for (int i = 0; i < nb; ++i)
+    if (b[i]->n) v.emplace_back(reinterpret_cast<uintptr_t>(b[i]->d_out), reinterpret_cast<uintptr_t>(b[i]->d_out + b[i]->n));
+  std::sort(v.begin(), v.end());
+  for (size_t i = 1; i < v.size(); ++i)
+    if (v[i].first < v[i - 1].second) return true;
+  return false;
+}
+
 // ---------------------------------------------------------------- RSQF executor
 // Worker w owns a stream (its calls' workspace lives in the stream's
 // context) and, coalescing, gather buffers for keys and lookup results.
@@ -332,16 +403,16 @@ struct RsqfExec {
       GQF_HIP(hipMalloc((void**)&x.out, n * 4));
       x.cap = n;
     }
-    size_t at = 0;
-    for (int i = 0; i < nb; ++i) {
-      const size_t k = (size_t)b[i]->n;
-      if (k) GQF_HIP(hipMemcpyAsync(x.keys + at, b[i]->d_keys, k * 4, hipMemcpyDeviceToDevice, hs));
-      at += k;
-    }
+    GQF_TRY(mv_requests<true>(hs, b, nb, x.keys));
     if (op == GQF_OP_INSERT) return gqf_rsqf_insert(fl, (int)n, x.keys, nullptr, x.st, &ms);
     if (op == GQF_OP_DELETE) return gqf_rsqf_delete(fl, (int)n, x.keys, x.st, &ms);
     GQF_TRY(gqf_rsqf_lookup(fl, sorted, (int)n, x.keys, x.out, x.st, &ms));
-    at = 0;
+    if (!mv_overlap(b, nb)) {
+      GQF_TRY(mv_requests<false>(hs, b, nb, reinterpret_cast<uint32_t*>(x.out)));
+      GQF_HIP(hipStreamSynchronize(hs));
+      return GQF_OK;
+    }
+    size_t at = 0;
     for (int i = 0; i < nb; ++i) {
       const size_t k = (size_t)b[i]->n;
       if (k) GQF_HIP(hipMemcpyAsync(b[i]->d_out, x.out + at, k * 4, hipMemcpyDeviceToDevice, hs));
