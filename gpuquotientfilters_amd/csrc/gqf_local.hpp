@@ -84,6 +84,9 @@ __host__ __device__ __forceinline__ LW lw_combine(LW x, LW y) {
   const int32_t b = x.b + y.a;
   return LW{x.a + y.a, b > y.b ? b : y.b, x.lb > y.lb ? x.lb : y.lb, x.heads + y.heads};
 }
+// b of a window that the localized form does not take: an overflow that no
+// window absorbs.
+constexpr int32_t LW_BAD = 1 << 28;
 __device__ __forceinline__ LW lw_none() { return LW{0, 0, 0u, 0u}; }
 __device__ __forceinline__ uint4 lw_pack(LW x) { return make_uint4((uint32_t)x.a, (uint32_t)x.b, x.lb, x.heads); }
 __device__ __forceinline__ LW lw_unpack(uint4 w) { return LW{(int32_t)w.x, (int32_t)w.y, w.z, w.w}; }
@@ -104,14 +107,74 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
               wave_read(inc.heads, 63)};
   return lw_dpp<DPP_WAVE_SHR1>(inc);
 }
-// Exclusive scan of the window states in two launches (as rb_scan): pre[w] =
-// {keys that overflow into window w, 1 + the last boundary before it}.  More
-// than LW_SPILL of the former, or any past the last window, raise the flag;
-// so do fewer regions than min_heads (lw_min_heads).
+// Exclusive scan of the window states: pre[w] = {keys that overflow into
+// window w, 1 + the last boundary before it}.  More than LW_SPILL of the
+// former, or any past the last window (LW_BAD is both), raise the flag, in the
+// counters and in host memory (report); so do fewer regions than min_heads
+// (lw_min_heads).  Resets the counters before.  One workgroup and one launch
+// for up to LW_ONE windows a thread (5.2 us for 4097; a loop over more of them
+// took 34 us for 16385), two launches as rb_scan for more (7 us).
+constexpr uint32_t LW_ONE = 8;
+__device__ __forceinline__ void lw_raise(uint32_t* ctr, uint32_t* report) {
+  ctr[CTR_MISC] = 1u;
+  __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// Stores window w's prefix; whether it or (the last window) the end is bad.
+__device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t W, uint2* __restrict__ pre, uint32_t min_heads) {
+  const int32_t o = p.a > p.b ? p.a : p.b;  // the map of the windows before, at 0
+  pre[w] = make_uint2(o > 0 ? (uint32_t)o : 0u, p.lb);
+  if (w + 1 < W) return o > LW_SPILL;
+  const LW all = lw_combine(p, x);
+  return o > LW_SPILL || (all.a > all.b ? all.a : all.b) > 0 || all.heads < min_heads;
+}
+[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_one(const uint4* __restrict__ st, uint32_t W,
+                                                                         uint2* __restrict__ pre, uint32_t min_heads,
+                                                                         uint32_t* __restrict__ ctr,
+                                                                         uint32_t* __restrict__ report) {
+  __shared__ uint4 s_wave[16];
+  __shared__ uint4 s_st[1024 * (LW_ONE + 1)];  // a thread's windows, one word of 16 bytes apart (banks)
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (tid >= CTR_OP && tid < CTR_TOTAL) ctr[tid] = 0u;
+  const uint32_t w0 = tid * LW_ONE;
+  uint4 x[LW_ONE];
+#pragma unroll
+  for (uint32_t j = 0; j < LW_ONE; ++j) x[j] = j * 1024 + tid < W ? st[j * 1024 + tid] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+  for (uint32_t j = 0; j < LW_ONE; ++j) {
+    const uint32_t i = j * 1024 + tid;
+    s_st[i + i / LW_ONE] = x[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < LW_ONE; ++j) x[j] = s_st[w0 + tid + j];
+  LW own = lw_unpack(x[0]);
+#pragma unroll
+  for (uint32_t j = 1; j < LW_ONE; ++j) own = lw_combine(own, lw_unpack(x[j]));
+  LW wt;
+  const LW ex = lw_wave_excl(own, &wt);
+  if (lane == 0) s_wave[wid] = lw_pack(wt);
+  __syncthreads();  // (orders the counters' reset as well)
+  if (wid == 0) {
+    LW tot;
+    const LW xe = lw_wave_excl(lane < 16 ? lw_unpack(s_wave[lane]) : lw_none(), &tot);
+    if (lane < 16) s_wave[lane] = lw_pack(xe);
+  }
+  __syncthreads();
+  LW p = lw_combine(lw_unpack(s_wave[wid]), ex);
+  bool bad = false;
+#pragma unroll
+  for (uint32_t j = 0; j < LW_ONE; ++j) {
+    if (w0 + j < W) bad |= lw_put(p, lw_unpack(x[j]), w0 + j, W, pre, min_heads);
+    p = lw_combine(p, lw_unpack(x[j]));
+  }
+  if (bad) lw_raise(ctr, report);
+}
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_reduce(const uint4* __restrict__ st, uint32_t W,
-                                                                            uint4* __restrict__ part) {
+                                                                            uint4* __restrict__ part,
+                                                                            uint32_t* __restrict__ ctr) {
   __shared__ uint4 s_wave[16];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
+  if (blockIdx.x == 0 && tid >= CTR_OP && tid < CTR_TOTAL) ctr[tid] = 0u;
   LW t;
   (void)lw_wave_excl(i < W ? lw_unpack(st[i]) : lw_none(), &t);
   if (lane == 0) s_wave[wid] = lw_pack(t);
@@ -126,7 +189,8 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W,
                                                                           const uint4* __restrict__ part,
                                                                           uint2* __restrict__ pre, uint32_t min_heads,
-                                                                          uint32_t* __restrict__ ctr) {
+                                                                          uint32_t* __restrict__ ctr,
+                                                                          uint32_t* __restrict__ report) {
   __shared__ uint4 s_wave[17];  // wave aggregates, then their prefixes; [16] = carry
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
   const LW x = i < W ? lw_unpack(st[i]) : lw_none();
@@ -147,15 +211,7 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
   }
   __syncthreads();
   if (i >= W) return;
-  const LW p = lw_combine(lw_unpack(s_wave[wid]), ex);
-  const int32_t o = p.a > p.b ? p.a : p.b;  // the map of the windows before, at 0
-  pre[i] = make_uint2(o > 0 ? (uint32_t)o : 0u, p.lb);
-  bool bad = o > LW_SPILL;
-  if (i + 1 == W) {
-    const LW all = lw_combine(p, x);
-    bad = bad || (all.a > all.b ? all.a : all.b) > 0 || all.heads < min_heads;
-  }
-  if (bad) ctr[CTR_MISC] = 1u;
+  if (lw_put(lw_combine(lw_unpack(s_wave[wid]), ex), x, i, W, pre, min_heads)) lw_raise(ctr, report);
 }
 
 // The regions a batch must have, 24 (insert) or 25 (delete) per 32 keys
@@ -171,17 +227,38 @@ static inline uint32_t lw_min_heads(bool insert, uint32_t n, uint32_t W) {
 }
 
 static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
-static inline gqf_status lw_scan(hipStream_t s, Arena& ar, const uint4* st, uint32_t W, uint2* pre,
-                                 uint32_t min_heads, uint32_t* ctr) {
+static inline gqf_status lw_scan(hipStream_t s, DeviceState& ds, Arena& ar, const uint4* st, uint32_t W, uint2* pre,
+                                 uint32_t min_heads) {
   const uint32_t P = (W + RBS_PER - 1) / RBS_PER;
   uint4* part = ar.take<uint4>(P ? P : 1);
   if (ar.used > ar.cap) {
     set_error("internal: window scan workspace overflow");
     return GQF_ERR_INVALID;
   }
-  GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part);
-  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, min_heads, ctr);
+  *reinterpret_cast<volatile uint32_t*>(ds.h_local) = 0u;
+  if (W <= LW_ONE * 1024) {
+    GQF_LAUNCH(k_lw_one, dim3(1), dim3(1024), 0, s, st, W, pre, min_heads, ds.counters, ds.d_local);
+    return GQF_OK;
+  }
+  GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part, ds.counters);
+  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, min_heads, ds.counters, ds.d_local);
   return GQF_OK;
+}
+// After the call's work: whether the localized form took the batch.
+static inline bool lw_done(DeviceState& ds) { return *reinterpret_cast<volatile uint32_t*>(ds.h_local) == 0u; }
+
+// Entries of the sorted batch with quotients below the windows w - 1, w and
+// w + 1 (the calling wave's three searches, 8 lanes each).
+template <typename K>
+__device__ __forceinline__ void lw_bounds(const K* __restrict__ B, uint32_t n, uint32_t r, uint32_t w, uint32_t* prev,
+                                          uint32_t* b0, uint32_t* b1) {
+  const uint32_t g = (threadIdx.x & 63) / 8, x = w + g - 1;  // (w = 0: no window before)
+  const bool on = g < 3 && (w || g);
+  const uint64_t key = ((uint64_t)x * LW_SLOTS) << r;
+  const uint32_t b = group8_search(0u, on ? n : 0u, [&](uint32_t m) { return (uint64_t)B[m] < key; });
+  *prev = wave_read(b, 0);
+  *b0 = wave_read(b, 8);
+  *b1 = wave_read(b, 16);
 }
 
 // Each window's range of the sorted batch: bstart[x] = first fingerprint with

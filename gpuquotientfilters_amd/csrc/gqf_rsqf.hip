@@ -1765,7 +1765,7 @@ static gqf_status rsqf_insert_win(hipStream_t s, DeviceState& ds, Arena& ar, con
 // Workspace of the localized insert or delete (beside the batch's sort).
 static size_t rsqf_local_ws(const RsqfGeom& g, uint32_t n) {
   const uint32_t W = rd_windows(g.nb);
-  return aligned_bytes((size_t)W * 8) + 256 + scan_rows_bytes(W, 2) + aligned_bytes(((size_t)W + 1) * 4) +
+  return aligned_bytes((size_t)W * 4) + aligned_bytes((size_t)((W + 63) / 64) * 4) + aligned_bytes(((size_t)W + 1) * 4) +
          aligned_bytes((size_t)n * 4) + aligned_bytes((size_t)g.nb * 8) + aligned_bytes((size_t)W * 2) +
          aligned_bytes((size_t)W * 16) + aligned_bytes((size_t)W * 8) + lw_scan_bytes(W) + 2048;
 }
@@ -1781,8 +1781,8 @@ static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gq
   const RsqfGeom g = rgeom(f);
   const RsqfDev d = rdev(f);
   const uint32_t W = rd_windows(g.nb);
-  uint32_t* wp = ar.take<uint32_t>((size_t)W * 2);
-  uint32_t* tot = ar.take<uint32_t>(4);
+  uint32_t* dw = ar.take<uint32_t>(W);
+  uint32_t* gs = ar.take<uint32_t>((W + 63) / 64);
   uint32_t* bstart = ar.take<uint32_t>((size_t)W + 1);
   uint32_t* key = ar.take<uint32_t>(n);
   uint64_t* empty = ar.take<uint64_t>(g.nb);
@@ -1794,13 +1794,10 @@ static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gq
     return GQF_ERR_INVALID;
   }
   const double mb = (double)g.nb * 16;  // occupieds + run ends
-  GQF_LAUNCH_B(mb, k_rd_pop, dim3((W + 3) / 4), dim3(256), 0, s, d.meta, g.nb, W, wp, (uint32_t*)nullptr, 0u);
-  GQF_TRY(scan_rows<2>(s, ar, wp, W, tot));
-  GQF_LAUNCH((k_wm_bounds<K>), dim3(((W + 1) * WB_LANES + 255) / 256), dim3(256), 0, s, B, n, g.r, W, bstart,
-             ds.counters);
-  GQF_LAUNCH_B(mb + (double)n * (sizeof(K) + 4), (k_rl_plan<K, INS>), dim3(W), dim3(64), 0, s, d.meta, g.nb, g.r, wp, B,
-               bstart, W, key, empty, fb, st, ds.counters);
-  GQF_TRY(lw_scan(s, ar, st, W, pre, lw_min_heads(INS, n, W), ds.counters));
+  GQF_LAUNCH_B(mb, k_rl_pop<K>, dim3((W + 63) / 64), dim3(1024), 0, s, d.meta, g.nb, W, B, n, g.r, bstart, dw, gs);
+  GQF_LAUNCH_B(mb + (double)n * (sizeof(K) + 4), (k_rl_plan<K, INS>), dim3(W), dim3(64), 0, s, d.meta, g.nb, g.r, dw, gs, B,
+               bstart, W, key, empty, fb, st);
+  GQF_TRY(lw_scan(s, ds, ar, st, W, pre, lw_min_heads(INS, n, W)));
   uint64_t* meta = reinterpret_cast<uint64_t*>(f.blocks);
   uint64_t* remg = reinterpret_cast<uint64_t*>(reinterpret_cast<uint8_t*>(f.blocks) + rsqf_meta_bytes(g.nb));
   const double wb = (double)rsqf_dev_bytes(g.q, g.r) + (double)n * (sizeof(K) + 4 + 256);
@@ -1831,8 +1828,8 @@ static gqf_status rsqf_insert_win_t(const gqf_rsqf& f, uint32_t n, const uint32_
     const size_t mark = ar.used;
     GQF_TRY((rsqf_local<K, true>(cs.stream, ds, ar, f, B, n)));
     if (d_out) launch_rlookup(cs.stream, f, n, keys, d_out);
-    GQF_TRY(cs.end(ms, true));
-    *done = ds.h_pinned[CTR_MISC] == 0;
+    GQF_TRY(cs.end(ms, false));
+    *done = lw_done(ds);
     lw_report(ds, LOCAL_RSQF_INSERT, *done);
     if (*done) return GQF_OK;
     ar.used = mark;  // nothing was written
@@ -1887,8 +1884,8 @@ static gqf_status rsqf_delete_local_t(const gqf_rsqf& f, uint32_t n, const uint3
   K* D;
   GQF_TRY(radix_sort<K>(cs.stream, ar, keys, true, g.bits, nullptr, false, n, 0, g.bits, &D, nullptr, cs.ds));
   GQF_TRY((rsqf_local<K, false>(cs.stream, ds, ar, f, D, n)));
-  GQF_TRY(cs.end(ms, true));
-  *done = ds.h_pinned[CTR_MISC] == 0;
+  GQF_TRY(cs.end(ms, false));
+  *done = lw_done(ds);
   lw_report(ds, LOCAL_RSQF_DELETE, *done);
   return GQF_OK;
 }

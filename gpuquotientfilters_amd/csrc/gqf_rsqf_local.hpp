@@ -228,18 +228,56 @@ struct RlPlanes {
 };
 
 // ---------------------------------------------------------------- plan
-// One wave per window, a lane per block.  wp: the exclusive occupied and
-// run-end counts of every window.  key[i]: insert E_k within the window,
-// delete 1 iff a boundary of the window lies after the key before it and at
-// or before it; D above (RL_E_BITS).  Insert: empty[block] of the windows
+// Window w's occupied quotients less its run ends (dw) and their sums over
+// groups of 64 windows (gs), 64 windows per workgroup; the windows' ranges of
+// the sorted batch (bstart).
+template <typename K>
+__global__ __launch_bounds__(1024) void k_rl_pop(const uint64_t* __restrict__ meta, uint32_t nb, uint32_t W,
+                                                 const K* __restrict__ B, uint32_t n, uint32_t r,
+                                                 uint32_t* __restrict__ bstart, uint32_t* __restrict__ dw,
+                                                 uint32_t* __restrict__ gs) {
+  __shared__ uint32_t s_sum[16];
+  const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6, w0 = blockIdx.x * 64 + 4 * wid;
+  uint4 x[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t b = (w0 + i) * 64 + lane;
+    x[i] = b < nb ? reinterpret_cast<const uint4*>(meta)[2 * (size_t)b] : make_uint4(0u, 0u, 0u, 0u);
+  }
+  {
+    const uint32_t w = w0 + lane / 8;
+    const bool on = lane < 32 && w < W;
+    const uint64_t key = ((uint64_t)w * LW_SLOTS) << r;
+    const uint32_t b = group8_search(0u, on ? n : 0u, [&](uint32_t m) { return (uint64_t)B[m] < key; });
+    if (on && (lane & 7) == 0) bstart[w] = b;
+    if (blockIdx.x == 0 && threadIdx.x == 0) bstart[W] = n;
+  }
+  uint32_t sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t d = wave_read(wave_incl_add((uint32_t)__popc(x[i].x) + (uint32_t)__popc(x[i].y) -
+                                               (uint32_t)__popc(x[i].z) - (uint32_t)__popc(x[i].w)), 63);
+    if (lane == 0 && w0 + i < W) dw[w0 + i] = d;
+    sum += d;
+  }
+  if (lane == 0) s_sum[wid] = sum;
+  __syncthreads();
+  if (wid == 0) {
+    const uint32_t a = wave_read(wave_incl_add(lane < 16 ? s_sum[lane] : 0u), 63);
+    if (lane == 0) gs[blockIdx.x] = a;
+  }
+}
+
+// One wave per window, a lane per block.  dw, gs: from k_rl_pop.  key[i]:
+// insert E_k within the window, delete 1 iff a boundary of the window lies
+// after the key before it and at or before it; D above (RL_E_BITS).  Insert: empty[block] of the windows
 // read; delete: fb[w] = the window's first boundary (LW_SLOTS: none).
 template <typename K, bool INS>
 __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ meta, uint32_t nb, uint32_t r,
-                                                const uint32_t* __restrict__ wp, const K* __restrict__ B,
-                                                const uint32_t* __restrict__ bstart, uint32_t W,
+                                                const uint32_t* __restrict__ dw, const uint32_t* __restrict__ gs,
+                                                const K* __restrict__ B, const uint32_t* __restrict__ bstart, uint32_t W,
                                                 uint32_t* __restrict__ key, uint64_t* __restrict__ empty,
-                                                uint16_t* __restrict__ fb, uint4* __restrict__ st,
-                                                uint32_t* __restrict__ ctr) {
+                                                uint16_t* __restrict__ fb, uint4* __restrict__ st) {
   __shared__ uint64_t s_mask[64], s_occ[64], s_end[64];
   __shared__ uint32_t s_pre[64];
   __shared__ int32_t s_D[64];
@@ -264,7 +302,12 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
     end = ((uint64_t)x.w << 32) | x.z;
   }
   const uint32_t step = (uint32_t)__popcll(occ) - (uint32_t)__popcll(end);
-  int32_t D = (int32_t)(wp[2 * (size_t)w] - wp[2 * (size_t)w + 1] + wave_incl_add(step) - step);
+  // runs that begin before the window's quotients' and end in or past it: the
+  // sums of the 64-window groups before, and of the windows of its own
+  uint32_t d = (w & ~63u) + lane < w ? dw[(w & ~63u) + lane] : 0u;
+  for (uint32_t i = lane; i < w / 64; i += 64) d += gs[i];
+  d = wave_read(wave_incl_add(d), 63);
+  int32_t D = (int32_t)(d + wave_incl_add(step) - step);
   s_occ[lane] = occ;
   s_end[lane] = end;
   s_D[lane] = D;
@@ -342,11 +385,12 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       if (k0 + 64 <= nk && hm == 0) bad = true;
     }
   }
-  if (bad) ctr[CTR_MISC] = 1u;
+  bad = __any(bad);
   if (lane == 0) {
     const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
     int32_t b = INS && nk ? M + a : 0;
     if (b < 0) b = 0;
+    if (bad) b = LW_BAD;
     st[w] = lw_pack(LW{a, b, last ? base + last : 0u, heads});
     if (!INS) fb[w] = (uint16_t)first;
   }

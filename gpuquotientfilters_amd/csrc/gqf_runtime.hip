@@ -62,6 +62,8 @@ gqf_status device_state(hipStream_t stream, DeviceState** out) {
   GQF_HIP(hipEventCreate(&ds->ev1));
   GQF_HIP(hipHostMalloc((void**)&ds->h_crowd, 64, hipHostMallocMapped | hipHostMallocCoherent));
   GQF_HIP(hipHostGetDevicePointer((void**)&ds->d_crowd, ds->h_crowd, 0));
+  ds->h_local = ds->h_crowd + 8;
+  ds->d_local = ds->d_crowd + 8;
   GQF_HIP(hipEventCreateWithFlags(&ds->ev_crowd, hipEventDisableTiming));
   GQF_HIP(hipDeviceSynchronize());
   ds->device = dev;

@@ -84,6 +84,10 @@ struct DeviceState {
   uint32_t* h_crowd = nullptr;
   uint32_t* d_crowd = nullptr;
   hipEvent_t ev_crowd = nullptr;
+  // the same kind of word for localized updates: raised when a batch is
+  // handed over (saves the copy of the counters)
+  uint32_t* h_local = nullptr;
+  uint32_t* d_local = nullptr;
   // after a crowded sort the next crowd_skip sorts take the chunked passes
   // directly; crowd_backoff doubles with every crowded probe in a row.  One
   // pair per key width: 32-bit (SQF, AP hash) and 64-bit (wide) fingerprints

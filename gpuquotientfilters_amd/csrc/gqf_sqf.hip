@@ -318,7 +318,7 @@ static size_t sqf_local_bytes(const SqfGeom& g, uint32_t n) {
 // ctr[CTR_MISC] != 0, and the table untouched, when the batch does not fit
 // that form.
 template <int BPE, bool INS>
-static gqf_status sqf_local_t(hipStream_t s, uint32_t* ctr, Arena& ar, const gqf_sqf& wq, const SqfGeom& g,
+static gqf_status sqf_local_t(hipStream_t s, DeviceState& ds, Arena& ar, const gqf_sqf& wq, const SqfGeom& g,
                               const uint32_t* B, uint32_t n) {
   const uint32_t W = lw_windows(g.S);
   uint32_t* bstart = ar.take<uint32_t>((size_t)W + 1);
@@ -330,19 +330,18 @@ static gqf_status sqf_local_t(hipStream_t s, uint32_t* ctr, Arena& ar, const gqf
     set_error("internal: localized update workspace overflow");
     return GQF_ERR_INVALID;
   }
-  GQF_LAUNCH((k_wm_bounds<uint32_t>), dim3(((W + 1) * WB_LANES + 255) / 256), dim3(256), 0, s, B, n, g.r, W, bstart, ctr);
-  GQF_LAUNCH_B((double)g.bytes + (double)n * 6, (k_sl_plan<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S, g.r, B,
-               bstart, W, el, fb, st, ctr);
-  GQF_TRY(lw_scan(s, ar, st, W, pre, lw_min_heads(INS, n, W), ctr));
+  GQF_LAUNCH_B((double)g.bytes + (double)n * 6, (k_sl_plan<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S, g.r, B, n,
+               bstart, W, el, fb, st);
+  GQF_TRY(lw_scan(s, ds, ar, st, W, pre, lw_min_heads(INS, n, W)));
   GQF_LAUNCH_B(2.0 * (double)g.bytes + (double)n * 6, (k_sl_apply<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S,
-               g.r, B, n, bstart, W, pre, el, fb, ctr);
+               g.r, B, n, bstart, W, pre, el, fb, ds.counters);
   return GQF_OK;
 }
 template <bool INS>
-static gqf_status sqf_local(hipStream_t s, uint32_t* ctr, Arena& ar, const gqf_sqf& wq, const SqfGeom& g,
+static gqf_status sqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gqf_sqf& wq, const SqfGeom& g,
                             const uint32_t* B, uint32_t n) {
-  if (g.bpe == 1) return sqf_local_t<1, INS>(s, ctr, ar, wq, g, B, n);
-  return sqf_local_t<2, INS>(s, ctr, ar, wq, g, B, n);
+  if (g.bpe == 1) return sqf_local_t<1, INS>(s, ds, ar, wq, g, B, n);
+  return sqf_local_t<2, INS>(s, ds, ar, wq, g, B, n);
 }
 
 static gqf_status sqf_insert_impl(const gqf_sqf& qf, int n, const uint32_t* d_keys, int mode, gqf_stream stream,
@@ -368,10 +367,10 @@ static gqf_status sqf_insert_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
   GQF_TRY(work_table(cs.stream, ar, qf, g, true, &wq));
   if (local) {
     const size_t mark = ar.used;
-    GQF_TRY(sqf_local<true>(cs.stream, ds.counters, ar, wq, g, B, un));
+    GQF_TRY(sqf_local<true>(cs.stream, ds, ar, wq, g, B, un));
     finish_table(cs.stream, qf, wq, g, ds.counters);
-    GQF_TRY(cs.end(ms, true));
-    const bool done = ds.h_pinned[CTR_MISC] == 0;
+    GQF_TRY(cs.end(ms, false));
+    const bool done = lw_done(ds);
     lw_report(ds, LOCAL_SQF_INSERT, done);
     if (done) return GQF_OK;
     ar.used = mark;  // nothing was written: the rebuild takes over
@@ -406,10 +405,10 @@ static gqf_status sqf_delete_impl(const gqf_sqf& qf, int n, const uint32_t* d_ke
   GQF_TRY(work_table(cs.stream, ar, qf, g, true, &wq));
   if (local) {
     const size_t mark = ar.used;
-    GQF_TRY(sqf_local<false>(cs.stream, ds.counters, ar, wq, g, D, un));
+    GQF_TRY(sqf_local<false>(cs.stream, ds, ar, wq, g, D, un));
     finish_table(cs.stream, qf, wq, g, ds.counters);
-    GQF_TRY(cs.end(ms, true));
-    const bool done = ds.h_pinned[CTR_MISC] == 0;
+    GQF_TRY(cs.end(ms, false));
+    const bool done = lw_done(ds);
     lw_report(ds, LOCAL_SQF_DELETE, done);
     if (done) return GQF_OK;
     ar.used = mark;  // nothing was written: the rebuild takes over

@@ -111,15 +111,21 @@ __host__ __device__ __forceinline__ void sl_erase(A& a, uint32_t S, uint32_t fq,
 // state's last boundary.
 template <int BPE, bool INS>
 __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, uint32_t S, uint32_t r,
-                                                const uint32_t* __restrict__ B, const uint32_t* __restrict__ bstart,
-                                                uint32_t W, uint16_t* __restrict__ el, uint16_t* __restrict__ fb,
-                                                uint4* __restrict__ st, uint32_t* __restrict__ ctr) {
+                                                const uint32_t* __restrict__ B, uint32_t n,
+                                                uint32_t* __restrict__ bstart, uint32_t W, uint16_t* __restrict__ el,
+                                                uint16_t* __restrict__ fb, uint4* __restrict__ st) {
   __shared__ uint64_t s_mask[64];
   __shared__ uint16_t s_pre[64];
   const uint32_t w = blockIdx.x, lane = threadIdx.x;
-  const uint32_t b0 = bstart[w], nk = bstart[w + 1] - b0;
+  uint32_t bp, b0, nk;
+  lw_bounds(B, n, r, w, &bp, &b0, &nk);
+  nk -= b0;
+  if (lane == 0) {
+    bstart[w] = b0;
+    if (w + 1 == W) bstart[W] = b0 + nk;
+  }
   const uint32_t base = w * LW_SLOTS;
-  if (nk == 0 && (w == 0 || bstart[w - 1] == b0)) {
+  if (nk == 0 && (w == 0 || bp == b0)) {
     // not read: what overflows into it is absorbed by the window before, and
     // a boundary of that window separates keys on both sides
     if (lane == 0) {
@@ -187,9 +193,9 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
     const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
     int32_t b = INS && nk ? M + a : 0;
     if (b < 0) b = 0;
+    if (bad) b = LW_BAD;
     st[w] = lw_pack(LW{a, b, last ? base + last : 0u, heads});
     if (!INS) fb[w] = (uint16_t)first;
-    if (bad) ctr[CTR_MISC] = 1u;
   }
 }
 
