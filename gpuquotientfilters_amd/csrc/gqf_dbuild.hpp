@@ -121,6 +121,15 @@ __device__ __forceinline__ void ps_each(uint32_t tn, F f) {
   if (threadIdx.x >= CTR_OP && threadIdx.x < CTR_TOTAL) ctr[threadIdx.x] = 0u;
 }
 
+// Where a tile's keys went: key p of the tile in order of digits (d: its own)
+// lies at place base[tile][d] + p of d's region, the digit's first key of the
+// tile is p = first[tile][d], and key i of all is its tile's place[i].
+struct PsBack {
+  uint16_t* place;
+  uint32_t* base;
+  uint16_t* first;
+};
+
 // Tiles blockIdx.x, + gridDim.x, ... to their groups, each a region of `cap`
 // keys in `out`: every key takes its rank in its digit from an LDS counter,
 // one global atomic per digit reserves the tile's places (in flight while
@@ -133,12 +142,13 @@ __device__ __forceinline__ void ps_each(uint32_t tn, F f) {
 // the tile (two workgroups per CU, runs of 8 keys) 355 us.  The next tile is
 // loaded before this one is written; interleaving its hashes with the stores
 // gained nothing.
-template <bool WIDE>
+//   BACK leaves the way back to the keys' order (gqf_plookup.hpp).
+template <bool WIDE, bool BACK>
 __global__ __launch_bounds__(PS_THREADS) void k_ps_scatter(const uint32_t* __restrict__ keys, uint32_t n,
                                                            uint32_t fp_bits, uint32_t shift, uint32_t nd,
                                                            uint32_t hbits, uint32_t tile, uint32_t cap,
                                                            uint32_t* __restrict__ gsize, uint32_t* __restrict__ out,
-                                                           uint32_t* __restrict__ ctr) {
+                                                           uint32_t* __restrict__ ctr, PsBack back) {
   __shared__ uint32_t s_key[PS_TILE];
   __shared__ uint32_t s_cnt[PS_ND], s_base[PS_ND];
   __shared__ uint32_t s_tmp[PS_THREADS / 64];
@@ -173,7 +183,23 @@ __global__ __launch_bounds__(PS_THREADS) void k_ps_scatter(const uint32_t* __res
     __syncthreads();
 #pragma unroll
     for (uint32_t i = 0; i < PS_ITEMS; ++i)
-      if (dr[i] != 0xFFFFFFFFu) s_key[s_cnt[dr[i] >> 16] + (dr[i] & 0xFFFFu)] = w[i];
+      if (dr[i] != 0xFFFFFFFFu) {
+        const uint32_t p = s_cnt[dr[i] >> 16] + (dr[i] & 0xFFFFu);
+        s_key[p] = w[i];
+        if (BACK) dr[i] = p;
+      }
+    if (BACK) {
+#pragma unroll
+      for (uint32_t i = 0; i < PS_ITEMS; i += 4)
+        if (ps_at(i) < tn)  // (the last four may be part of one: place has room)
+          *reinterpret_cast<uint2*>(back.place + t0 + ps_at(i)) =
+              make_uint2((dr[i] & 0xFFFFu) | dr[i + 1] << 16, (dr[i + 2] & 0xFFFFu) | dr[i + 3] << 16);
+      if (d0 < nd) {
+        const uint64_t row = (t0 / tile) * nd + d0;
+        *reinterpret_cast<uint2*>(back.base + row) = make_uint2(b0 - e, b1 - (e + c.x));
+        *reinterpret_cast<uint32_t*>(back.first + row) = e | (e + c.x) << 16;
+      }
+    }
     if (d0 < nd) {
       *reinterpret_cast<uint2*>(s_base + d0) = make_uint2(b0 - e, b1 - (e + c.x));
       if (b0 + c.x > cap || b1 + c.y > cap) ctr[CTR_MISC] = 1u;  // a group is full: its further keys are not written
@@ -816,8 +842,8 @@ static gqf_status db_runs(hipStream_t s, Arena& ar, const PsPlan& p, const uint3
   }
   o->gsize = gsize;
   GQF_LAUNCH(k_ps_reset, dim3(1), dim3(PS_THREADS), 0, s, gsize, nd, ctr);
-  GQF_LAUNCH_B((double)n * 8.0, k_ps_scatter<WIDE>, dim3(p.wgs), dim3(PS_THREADS), 0, s, keys, n, fp_bits, p.shift, nd,
-               hbits, p.tile, p.cap, gsize, mid, ctr);
+  GQF_LAUNCH_B((double)n * 8.0, (k_ps_scatter<WIDE, false>), dim3(p.wgs), dim3(PS_THREADS), 0, s, keys, n, fp_bits,
+               p.shift, nd, hbits, p.tile, p.cap, gsize, mid, ctr, PsBack{});
   const double rb = (double)n * 5.0 + (double)((uint64_t)1 << (p.qb + p.gb));
   if (unique)
     GQF_LAUNCH_B(rb, k_db_runs<true>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, p.cap, p.qb, r, o->counts, o->rems,

@@ -387,6 +387,8 @@ __device__ __forceinline__ uint4 ld16_dw(const uint32_t* p) {
   return x;
 }
 
+__device__ __forceinline__ void st16_dw(uint32_t* p, uint4 x) { __builtin_memcpy(p, &x, 16); }
+
 // Thread t's 16 consecutive entries [16t, 16t+16) of the sub-tile at t0
 // (tile_n of them valid; the rest become all-ones padding); whole groups
 // load as 16-byte words.

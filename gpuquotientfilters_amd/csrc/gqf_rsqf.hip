@@ -14,7 +14,7 @@
 // reference on any table (including the history-dependent layouts its insert
 // leaves).  Build / insert / delete produce the canonical layout, which is
 // what the reference insert produces when fed fingerprints in ascending order.
-#include "gqf_dbuild.hpp"
+#include "gqf_plookup.hpp"
 #include "gqf_rsqf_local.hpp"
 
 #include <type_traits>
@@ -1897,11 +1897,161 @@ __global__ __launch_bounds__(256) void k_rk_mark(const uint32_t* __restrict__ ke
   if (i < n && fingerprint(keys[i], bits) >= cut) out[i] = RS_NOT_FOUND;
 }
 
+// ---------------------------------------------------------------- large lookups
+// Large batches by groups (gqf_plookup.hpp): the group's blocks in LDS, one
+// before them (a walk reads the slot before its quotient's) and PL_BLOCKS_FWD
+// past them (run ends that lie there).
+constexpr uint32_t PL_BLOCKS_FWD = 8, PL_BLOCKS = DB_NQ / 64 + 1 + PL_BLOCKS_FWD;
+struct RsqfLds {
+  const uint32_t *o, *e;  // occupied and run-end words, 32 slots each
+  const uint8_t *off, *rem;
+  uint32_t words, r, none;  // words loaded; past them: PL_PENDING or not found
+};
+// rsqf_lookup_one's walk for the quotient at `at` in the loaded slots: the
+// slot, counted in them.  The run end is found in 32-bit words from the
+// block's offset on (blocks and 64-bit selects: 138 us at 2^24 keys), and
+// one-byte remainders are compared four at a time.
+template <int R>
+__device__ __forceinline__ uint32_t rsqf_lds_walk(const RsqfLds& f, uint32_t at, uint32_t fr) {
+  uint32_t w = at >> 5;
+  const uint32_t occ = f.o[w] << (31u - (at & 31u));  // (the quotient's bit on top)
+  if (!(occ >> 31)) return RS_NOT_FOUND;
+  uint32_t k = (uint32_t)__popc(occ) + ((w & 1) ? (uint32_t)__popc(f.o[w - 1]) : 0u);
+  uint32_t s = (at & ~63u) + f.off[at >> 6];
+  w = s >> 5;
+  if (w >= f.words) return f.none;
+  uint32_t x = f.e[w] & (~0u << (s & 31u)), c;
+  while ((c = (uint32_t)__popc(x)) < k) {
+    k -= c;
+    if (++w >= f.words) return f.none;
+    x = f.e[w];
+  }
+  s = 32 * w + pl_select(x, k);
+  if (R != 8) {
+    for (;;) {
+      const uint32_t bit = s * f.r, b = bit >> 3;
+      const uint32_t cur = ((f.rem[b] | (uint32_t)f.rem[b + 1] << 8) >> (bit & 7)) & ((1u << f.r) - 1u);  // (r <= 8)
+      if (cur == fr) return s;
+      if (cur < fr || s <= at) return RS_NOT_FOUND;
+      --s;
+      if ((f.e[s >> 5] >> (s & 31u)) & 1u) return RS_NOT_FOUND;
+    }
+  }
+  const uint32_t* rem = reinterpret_cast<const uint32_t*>(f.rem);
+  const uint32_t ff = fr * 0x00010001u | 0x01000100u;
+  for (;;) {
+    // slots s - 3 .. s, those of the run: down to `at` and the run end before (s >= 64)
+    const uint32_t y = __builtin_amdgcn_alignbyte(rem[((s - 3) >> 2) + 1], rem[(s - 3) >> 2], (s - 3) & 3u);
+    const uint32_t before = pl_bits(f.e, s - 4) & 15u;  // run ends at s - 4 .. s - 1
+    // entries of the run among the four, and whether it goes on
+    uint32_t nv = before >> 1 ? (uint32_t)__builtin_clz(before << 28) + 1u : 4u;
+    bool more = before == 0;
+    const uint32_t left = s >= at ? s - at + 1u : 1u;
+    if (left <= nv) nv = left, more = false;
+    // bytes <= fr, by their top bits
+    const uint32_t me = (ff - (y & 0x00FF00FFu)) & 0x01000100u, mo = (ff - ((y >> 8) & 0x00FF00FFu)) & 0x01000100u;
+    const uint32_t m = ((me >> 1) | (mo << 7)) & (~0u << (8 * (4u - nv)));
+    if (m) {
+      const uint32_t p = (uint32_t)__builtin_clz(m) >> 3;  // slots below s
+      return ((y >> (24u - 8u * p)) & 0xFFu) == fr ? s - p : RS_NOT_FOUND;
+    }
+    if (!more) return RS_NOT_FOUND;
+    s -= 4;
+  }
+}
+struct RsqfWalk {
+  RsqfDev f;
+  uint32_t q;
+  __device__ __forceinline__ uint32_t operator()(uint32_t key) const {
+    const uint64_t fp = fingerprint(key, q + f.r);
+    return rsqf_lookup_one<0>(f, (uint32_t)((fp >> f.r) & mask64(q)), (uint32_t)(fp & ((1u << f.r) - 1u)));
+  }
+};
+
+template <int R>
+__global__ __launch_bounds__(PL_THREADS) void k_pl_rsqf(RsqfDev f, uint32_t qb, const uint32_t* __restrict__ gsize,
+                                                        uint32_t cap, uint32_t* __restrict__ io) {
+  __shared__ __align__(8) uint32_t s_occ[2 * PL_BLOCKS + 2], s_end[2 * PL_BLOCKS + 2];
+  __shared__ __align__(16) uint32_t s_rem[PL_BLOCKS * (R ? 2 * R : 16) + 4];
+  __shared__ uint8_t s_off[PL_BLOCKS];
+  const uint32_t r = R ? (uint32_t)R : f.r, t = threadIdx.x;
+  const uint32_t g = blockIdx.x, m = gsize[g] < cap ? gsize[g] : cap;
+  if (m == 0) return;
+  // blocks b0 .. nb - 1 (group 0: an empty one stands before block 0)
+  const uint32_t first = g << (qb - 6), b0 = first - 1u, skip = first ? 0u : 1u;
+  const uint32_t end = first + (1u << (qb - 6)) + PL_BLOCKS_FWD, nb = end < f.nb ? end : f.nb;
+  for (uint32_t b = t; b < nb - b0; b += PL_THREADS) {
+    uint4 x = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t o = 0;
+    if (b >= skip) {
+      const uint4* p = reinterpret_cast<const uint4*>(f.meta) + 2 * (size_t)(b0 + b);
+      x = p[0];
+      o = reinterpret_cast<const uint32_t*>(p)[4];
+    }
+    *reinterpret_cast<uint2*>(s_occ + 2 * b) = make_uint2(x.x, x.y);
+    *reinterpret_cast<uint2*>(s_end + 2 * b) = make_uint2(x.z, x.w);
+    s_off[b] = (uint8_t)o;
+  }
+  const uint2* src = reinterpret_cast<const uint2*>(f.rem + (size_t)(first - 1u + skip) * 8 * r);
+  for (uint32_t i = t + skip * r; i < (nb - b0) * r; i += PL_THREADS)
+    reinterpret_cast<uint2*>(s_rem)[i] = src[i - skip * r];
+  __syncthreads();
+  const RsqfLds l{s_occ, s_end, s_off, reinterpret_cast<const uint8_t*>(s_rem), 2 * (nb - b0), r,
+                  nb < f.nb ? PL_PENDING : RS_NOT_FOUND};
+  uint32_t* p = io + (uint64_t)g * cap;
+  const uint32_t qmask = (1u << qb) - 1u, rmask = (1u << r) - 1u;
+  pl_each(p, m, [&](uint32_t key) {
+    const uint32_t a = rsqf_lds_walk<R>(l, ((key >> r) & qmask) + 64u, key & rmask);
+    return a >= PL_PENDING ? a : a + 64u * b0;
+  });
+}
+
+// *done: the answers are on their way; otherwise the direct walk is asked for.
+static gqf_status rsqf_pl_lookup(hipStream_t s, DeviceState& ds, const gqf_rsqf& f, uint32_t n, const uint32_t* keys,
+                                 uint32_t* out, bool may_grow, bool* done) {
+  PlPlan pl;
+  *done = pl_plan(n, f.qbits, f.rbits, PL_QMIN_RSQF, &pl) && lw_try(ds, LOCAL_RSQF_LOOKUP) &&
+          (pl_bytes(pl, n) <= ds.ws_cap || (may_grow && ws_try_reserve(ds, pl_bytes(pl, n))));
+  if (!*done) return GQF_OK;
+  const RsqfDev d = rdev(f);
+  const uint32_t bits = f.qbits + f.rbits;
+  const double b = (double)d.nb * (32 + 8 * f.rbits) + (double)n * 8.0;
+  auto walks = [&](const uint32_t* gsize, uint32_t cap, uint32_t* io) {
+    if (f.rbits == 8) GQF_LAUNCH_B(b, k_pl_rsqf<8>, dim3(pl.p.ngroups), dim3(PL_THREADS), 0, s, d, pl.p.qb, gsize, cap, io);
+    else GQF_LAUNCH_B(b, k_pl_rsqf<0>, dim3(pl.p.ngroups), dim3(PL_THREADS), 0, s, d, pl.p.qb, gsize, cap, io);
+  };
+  if (bits > 32) return pl_lookup<true>(s, ds, pl, keys, bits, n, out, RsqfWalk{d, f.qbits}, walks);
+  return pl_lookup<false>(s, ds, pl, keys, bits, n, out, RsqfWalk{d, f.qbits}, walks);
+}
+
 static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out) {
   const RsqfDev d = rdev(f);
   const dim3 grid((n + 255) / 256);
   if (f.rbits == 8) GQF_LAUNCH_B((double)n * (8 + 128), k_rsqf_lookup<8>, grid, dim3(256), 0, s, d, f.qbits, keys, n, out);
   else GQF_LAUNCH_B((double)n * (8 + 128), k_rsqf_lookup<0>, grid, dim3(256), 0, s, d, f.qbits, keys, n, out);
+}
+
+gqf_status rsqf_lookup_call(const gqf_rsqf& f, int n, const uint32_t* d_keys, int32_t* d_out, gqf_stream stream,
+                            float* ms, bool may_grow) {
+  GQF_TRY(rsqf_args(f, n, d_keys));
+  if (n > 0 && !d_out) {
+    set_error("output array is NULL");
+    return GQF_ERR_INVALID;
+  }
+  CallScope cs;
+  GQF_TRY(cs.begin(stream));
+  uint32_t* out = reinterpret_cast<uint32_t*>(d_out);
+  if (n > 0) {
+    bool done;
+    GQF_TRY(rsqf_pl_lookup(cs.stream, *cs.ds, f, (uint32_t)n, d_keys, out, may_grow, &done));
+    if (done) {
+      GQF_TRY(cs.end(ms, false));
+      pl_report(*cs.ds, LOCAL_RSQF_LOOKUP);
+      return GQF_OK;
+    }
+    launch_rlookup(cs.stream, f, (uint32_t)n, d_keys, out);
+  }
+  return cs.end(ms, false);
 }
 
 }  // namespace gqf
@@ -2080,21 +2230,10 @@ gqf_status gqf_rsqf_delete(gqf_rsqf cqf, int n, const uint32_t* d_keys, gqf_stre
 
 gqf_status gqf_rsqf_lookup(gqf_rsqf cqf, int sorted, int n, const uint32_t* d_keys, int32_t* d_out, gqf_stream stream,
                            float* ms) {
-  GQF_TRY(rsqf_args(cqf, n, d_keys));
-  if (n > 0 && !d_out) {
-    set_error("output array is NULL");
-    return GQF_ERR_INVALID;
-  }
-  CallScope cs;
-  GQF_TRY(cs.begin(stream));
-  uint32_t* out = reinterpret_cast<uint32_t*>(d_out);
-  if (n > 0) {
-    // sorted or not, the same per-key walk: sorting the keys first costs
-    // more than the locality it buys on MI355X (measured up to 1.6 GB tables)
-    (void)sorted;
-    launch_rlookup(cs.stream, cqf, (uint32_t)n, d_keys, out);
-  }
-  return cs.end(ms, false);
+  // sorted or not, the same walk: a full sort of the keys costs more than
+  // the locality it buys on MI355X (measured up to 1.6 GB tables)
+  (void)sorted;
+  return rsqf_lookup_call(cqf, n, d_keys, d_out, stream, ms, true);
 }
 
 size_t gqf_rsqf_workspace_bytes(gqf_rsqf cqf, int op, int n, int sorted) {

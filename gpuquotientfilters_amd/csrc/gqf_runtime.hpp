@@ -58,11 +58,11 @@ struct ProfRec {
   double dper;
 };
 
-// Kinds of calls whose fast form (gqf_local.hpp, gqf_dbuild.hpp) may hand a
+// Kinds of calls whose fast form (gqf_local.hpp, gqf_dbuild.hpp, gqf_plookup.hpp) may hand a
 // batch over to the general one.
 enum LocalKind : int {
   LOCAL_SQF_INSERT = 0, LOCAL_SQF_DELETE, LOCAL_RSQF_INSERT, LOCAL_RSQF_DELETE, LOCAL_SQF_BUILD, LOCAL_RSQF_BUILD,
-  LOCAL_KINDS
+  LOCAL_SQF_LOOKUP, LOCAL_RSQF_LOOKUP, LOCAL_KINDS
 };
 
 // Execution context of one (device, stream) pair: workspace arena, device
@@ -142,6 +142,11 @@ struct Arena {
   }
 };
 __host__ __device__ inline size_t aligned_bytes(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+
+// gqf_rsqf_lookup; may_grow: the stream's workspace may be enlarged for it
+// (otherwise the call makes do with what is there).
+gqf_status rsqf_lookup_call(const gqf_rsqf& f, int n, const uint32_t* d_keys, int32_t* d_out, gqf_stream stream,
+                            float* ms, bool may_grow);
 
 // ---------------------------------------------------------------- kernel timing
 // When enabled (gqf_profile_enable), every launch is bracketed by two events

@@ -390,7 +390,7 @@ struct RsqfExec {
     float ms = 0.f;
     if (nb == 1) {
       const gqf_request& r = *b[0];
-      if (op == GQF_OP_LOOKUP) return gqf_rsqf_lookup(fl, sorted, r.n, r.d_keys, r.d_out, x.st, &ms);
+      if (op == GQF_OP_LOOKUP) return rsqf_lookup_call(fl, r.n, r.d_keys, r.d_out, x.st, &ms, false);
       if (op == GQF_OP_INSERT) return gqf_rsqf_insert(fl, r.n, r.d_keys, nullptr, x.st, &ms);
       return gqf_rsqf_delete(fl, r.n, r.d_keys, x.st, &ms);
     }
@@ -406,7 +406,7 @@ struct RsqfExec {
     GQF_TRY(mv_requests<true>(hs, b, nb, x.keys));
     if (op == GQF_OP_INSERT) return gqf_rsqf_insert(fl, (int)n, x.keys, nullptr, x.st, &ms);
     if (op == GQF_OP_DELETE) return gqf_rsqf_delete(fl, (int)n, x.keys, x.st, &ms);
-    GQF_TRY(gqf_rsqf_lookup(fl, sorted, (int)n, x.keys, x.out, x.st, &ms));
+    GQF_TRY(rsqf_lookup_call(fl, (int)n, x.keys, x.out, x.st, &ms, false));
     if (!mv_overlap(b, nb)) {
       GQF_TRY(mv_requests<false>(hs, b, nb, reinterpret_cast<uint32_t*>(x.out)));
       GQF_HIP(hipStreamSynchronize(hs));

@@ -11,7 +11,7 @@
 //   [decode table] -> [hash + radix sort keys] -> [merge / mark] ->
 //   layout scan (locations) -> table writer (every slot written once).
 // Lookups are the reference's run walk (quotientFilter.cu:172-196, 320-357).
-#include "gqf_dbuild.hpp"
+#include "gqf_plookup.hpp"
 #include "gqf_sqf_local.hpp"
 
 #include <algorithm>
@@ -553,13 +553,25 @@ gqf_status gqf_sqf_lookup(gqf_sqf qf, int sorted, int n, const uint32_t* d_keys,
   if (un) {
     // 64-slot windows need 16-byte aligned tables (hipMalloc gives 256)
     const bool win = (reinterpret_cast<uintptr_t>(qf.table) & 15u) == 0;
-    // The sorted variant (launchSortedLookups) runs the same per-key walk
-    // without sorting the keys first: the results are the same by
-    // construction, and on MI355X sorting 2^24 keys costs more than the
-    // locality it buys (tables up to 147 MB; the RSQF up to 1.6 GB).
+    // The sorted variant (launchSortedLookups) runs the same walks without a
+    // full sort of the keys: the results are the same by construction, and on
+    // MI355X sorting 2^24 keys costs more than the locality it buys.
     (void)sorted;
     const dim3 grid((un + 255) / 256);
     const double b = (double)un * (8 + 64);
+    PlPlan pl;
+    if (g.bpe == 1 && !g.packed && win && pl_plan(un, g.q, g.r, PL_QMIN_SQF, &pl) && lw_try(*cs.ds, LOCAL_SQF_LOOKUP) &&
+        (pl_bytes(pl, un) <= cs.ds->ws_cap || ws_try_reserve(*cs.ds, pl_bytes(pl, un)))) {
+      GQF_TRY(pl_lookup<false>(cs.stream, *cs.ds, pl, d_keys, (g.q + g.r) | sqf_hash_flag(), un, d_out,
+                               SqfWalk{qf.table, g.S, g.q, g.r, sqf_hash_flag()},
+                               [&](const uint32_t* gsize, uint32_t cap, uint32_t* io) {
+                                 GQF_LAUNCH_B((double)g.bytes + (double)un * 8.0, k_pl_sqf, dim3(pl.p.ngroups),
+                                              dim3(PL_THREADS), 0, cs.stream, qf.table, g.S, pl.p.qb, g.r, gsize, cap, io);
+                               }));
+      GQF_TRY(cs.end(ms, false));
+      pl_report(*cs.ds, LOCAL_SQF_LOOKUP);
+      return GQF_OK;
+    }
     if (g.packed) GQF_LAUNCH_B(b, k_sqf_lookup_packed, grid, dim3(256), 0, cs.stream, reinterpret_cast<const uint32_t*>(qf.table), g.S, g.q, g.r, d_keys, un, d_out, sqf_hash_flag());
     else if (g.bpe == 1 && win) GQF_LAUNCH_B(b, (k_sqf_lookup<1, true>), grid, dim3(256), 0, cs.stream, qf.table, g.S, g.q, g.r, d_keys, un, d_out, sqf_hash_flag());
     else if (g.bpe == 2 && win) GQF_LAUNCH_B(b, (k_sqf_lookup<2, true>), grid, dim3(256), 0, cs.stream, qf.table, g.S, g.q, g.r, d_keys, un, d_out, sqf_hash_flag());

@@ -255,7 +255,9 @@ gqf_status gqf_rsqf_delete(gqf_rsqf cqf, int n, const uint32_t* d_keys, gqf_stre
                            float* ms);
 
 /* Device workspace (bytes) a call of `op` (gqf_op) over n keys reserves on
- * its stream's context (lookups: none; `sorted` is kept for the signature).
+ * its stream's context (lookups: none that they need -- those of several
+ * million keys use about 10 bytes per key where the device has them --;
+ * `sorted` is kept for the signature).
  * No reference counterpart (the reference allocates per call). */
 size_t gqf_rsqf_workspace_bytes(gqf_rsqf cqf, int op, int n, int sorted);
 
