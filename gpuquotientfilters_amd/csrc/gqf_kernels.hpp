@@ -771,7 +771,9 @@ __global__ __launch_bounds__(SORT_THREADS) void k_rs_small(const void* __restric
 //     of the key range (a stable partition into 256 segments), then
 //     k_rs_seg, one workgroup per segment, sorts the bits below in LDS with
 //     every 4-bit counting pass of the tile sort back to back.  4 launches
-//     instead of 12 (31-bit fingerprints) or 15 (34-bit ones).
+//     instead of 12 (31-bit fingerprints) or 15 (34-bit ones).  Where the
+//     workspace has room for a region per segment, k_rs_place puts the keys
+//     there in one pass, and 2 launches are left.
 //   * more keys: a second chunked pass over the segments on the next b2 bits
 //     (k_rs_upsweep_seg, k_rs_segbase, k_rs_downsweep_seg: each chunk lies in
 //     one segment, and the digit bases count within the segment), so that
@@ -997,6 +999,59 @@ __device__ __forceinline__ void seg_counting_sort(K* __restrict__ seg, uint32_t 
   for (uint32_t p = tid; p < m; p += T) seg[p] = high | (K)s_keys[ts_swz<4>(p)];
 }
 
+// Keys to the regions of their segments (top 8 bits of the fingerprint, region
+// d: `cap` keys from d cap on) in one pass: every key takes its rank in its
+// tile from an LDS counter and every tile its places with one global atomic
+// per segment.  Order within a region is of no account to k_rs_seg.  place:
+// segment sizes and a ticket, zero before; the last tile to reserve its
+// places tells the host whether every region has room (1) or not (2: keys
+// past it are dropped) while the keys are still being written.
+//   Stores of 4 or 8 bytes anywhere: the L2 merges them, and up to 2 M keys
+// it holds them.  Against the counted partition (k_rs_upsweep, k_rs_rowscan,
+// k_rs_downsweep) this saves two launches and a second read and hash: 98 K
+// keys 7.3 us for 24, 2^20 keys 15 us for 30 (LDS atomics and the scattered
+// stores, in about equal parts), 2^18 64-bit fingerprints 10 us for 37.
+constexpr uint32_t PLACE_WORDS = 257;
+constexpr int PLACE_THREADS = 512;
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(PLACE_THREADS) void k_rs_place(const uint32_t* __restrict__ in, uint32_t n, uint32_t fp_bits,
+                                                            uint32_t shift, uint32_t cap, uint32_t* __restrict__ place,
+                                                            K* __restrict__ regions, uint32_t* __restrict__ room) {
+  __shared__ uint32_t s_cnt[256];
+  const uint32_t t = threadIdx.x, t0 = blockIdx.x * PLACE_THREADS * ITEMS;
+  if (t < 256) s_cnt[t] = 0u;
+  K k[ITEMS];
+  uint32_t d[ITEMS], rank[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t at = t0 + i * PLACE_THREADS + t;
+    k[i] = at < n ? sort_load_key<K, true>(in, at, fp_bits) : (K)0;
+    d[i] = at < n ? (uint32_t)(k[i] >> shift) : 256u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) rank[i] = d[i] < 256 ? atomicAdd(&s_cnt[d[i]], 1u) : 0u;
+  __syncthreads();
+  bool full = false;
+  if (t < 256) {
+    const uint32_t c = s_cnt[t], b = c ? atomicAdd(&place[t], c) : 0u;
+    s_cnt[t] = b;
+    full = b + c > cap;
+  }
+  const int any = __syncthreads_or(full);
+  if (t == 0) {
+    // low half: tiles so far; high half: those that met a full region
+    const uint32_t v = atomicAdd(&place[256], any ? 0x10001u : 1u) + (any ? 0x10001u : 1u);
+    if ((v & 0xFFFFu) == gridDim.x) __hip_atomic_store(room, v >> 16 ? 2u : 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (d[i] < 256) {
+      const uint32_t at = s_cnt[d[i]] + rank[i];
+      if (at < cap) regions[(size_t)d[i] * cap + at] = k[i];
+    }
+}
+
 // One group per workgroup, sorted in place by its bits [0, nbits) (nbits <=
 // 32; the bits above are equal within the group): the keys' top SEG_BB bits
 // of the range pick one of SEG_NBK buckets (LDS counters; the scanned starts
@@ -1009,11 +1064,15 @@ __device__ __forceinline__ void seg_counting_sort(K* __restrict__ seg, uint32_t 
 // group ids) for k_rs_seg_slow, which keeps this kernel at 40 registers and
 // four workgroups per CU.  A group above SEG_TILE is never launched here
 // (the host sorts crowded keys with the chunked passes) and is left alone.
+//   regions (k_rs_place; else null): segment g is the gsize[g] keys from g cap
+// on, at most cap, and goes to its place in `keys`; the counters `next` of
+// the stream's next such sort are cleared.
 template <typename K, bool INLINE>
 __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, const uint32_t* __restrict__ digit_totals,
                                                         const uint32_t* __restrict__ gstart,
                                                         const uint32_t* __restrict__ gsize, uint32_t nbits,
-                                                        uint32_t* __restrict__ slow) {
+                                                        uint32_t* __restrict__ slow, const K* __restrict__ regions,
+                                                        uint32_t cap, uint32_t* __restrict__ next) {
   constexpr int T = SEG_THREADS, W = T / 64;
   __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
   __shared__ __align__(16) uint16_t s_cnt[INLINE ? 16 * T : 8];  // the counting passes' count table
@@ -1023,8 +1082,14 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, co
   const uint32_t tid = threadIdx.x;
   uint32_t c0, m;
   seg_group<T>(blockIdx.x, digit_totals, gstart, gsize, &c0, &m, s_tmp, s_seg);
-  if (m <= 1 || m > (uint32_t)SEG_TILE) return;  // the whole workgroup
+  if (INLINE && regions) {
+    if (blockIdx.x == 0 && tid < PLACE_WORDS) next[tid] = 0u;
+    if (m > cap) return;  // the host sorts these keys otherwise
+  }
+  const bool moved = INLINE && regions;
+  if ((m <= 1 && !moved) || m == 0 || m > (uint32_t)SEG_TILE) return;  // the whole workgroup
   K* seg = keys + c0;
+  const K* from = moved ? regions + (size_t)blockIdx.x * cap : seg;
   const uint32_t lmask = nbits >= 32 ? 0xFFFFFFFFu : (1u << nbits) - 1u;
   const uint32_t i0 = tid * SORT_ITEMS;
   const uint32_t nreal = m > i0 ? (m - i0 < SORT_ITEMS ? m - i0 : SORT_ITEMS) : 0u;
@@ -1032,11 +1097,11 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, co
   uint32_t k[SORT_ITEMS];
   {
     K kk[SORT_ITEMS];
-    ts_load_keys<K, false>(seg, 0, m, 0u, kk);
+    ts_load_keys<K, false>(from, 0, m, 0u, kk);
 #pragma unroll
     for (int i = 0; i < SORT_ITEMS; ++i) k[i] = (uint32_t)kk[i] & lmask;
   }
-  const K high = seg[0] & ~(K)lmask;
+  const K high = from[0] & ~(K)lmask;
   for (uint32_t i = tid; i < SEG_NBK / 2; i += T) s_c[i] = 0u;
   __syncthreads();
 #pragma unroll
@@ -1080,6 +1145,10 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, co
 #pragma unroll
     for (uint32_t i = 0; i < PT / 4; ++i) c4[i] = make_uint4(st[4 * i], st[4 * i + 1], st[4 * i + 2], st[4 * i + 3]);
     if (__syncthreads_or(mx > SEG_RANK_MAX)) {  // also orders the bucket starts
+      if (moved) {
+        for (uint32_t i = tid; i < m; i += T) seg[i] = from[i];
+        __syncthreads();
+      }
       if (INLINE) seg_counting_sort<K, T>(seg, m, nbits, s_keys, s_cnt, s_tmp);
       else if (tid == 0) slow[1 + atomicAdd(&slow[0], 1u)] = blockIdx.x;
       return;
@@ -1246,6 +1315,61 @@ inline size_t sort_workspace_bytes(uint64_t n, size_t key_bytes, bool vals, bool
   return b;
 }
 
+// The sort of up to 256 * SEG_GROUP_AVG keys through regions, from `scratch` on:
+// memory that the arena gives out after the sort, so it needs no workspace of
+// its own; *done is false, and nothing but scratch written, where that has
+// too little room, or a segment holds more keys than its region (then the
+// stream's next sorts of this width leave the attempt out, for a while).
+//   The host waits for the word that the partition writes halfway, not for
+// an event behind it.
+template <typename K>
+gqf_status place_sort(hipStream_t s, const Arena& ar, DeviceState& ds, const uint32_t* in, uint32_t n, uint32_t fp_bits,
+                      uint32_t hi_bit, K* out, K* scratch, bool* done) {
+  *done = false;
+  const LocalKind kind = sizeof(K) == 8 ? LOCAL_PLACE_U64 : LOCAL_PLACE_U32;
+  const uint64_t have = (uint64_t)(ar.base + ar.cap - reinterpret_cast<char*>(scratch)) / (256 * sizeof(K));
+  const uint32_t mean = n / 256;
+  uint32_t s6 = 64;  // 6 sigma and a little
+  while ((uint64_t)(s6 - 64) * (s6 - 64) < 36ull * mean) s6 += 8;
+  uint64_t cap = 4ull * mean + 512;  // uneven keys are welcome where there is room
+  cap = (cap < have ? cap : have) & ~15ull;
+  if (cap > (uint64_t)SEG_TILE) cap = SEG_TILE;
+  if (cap < mean + s6 || !lw_try(ds, kind)) return GQF_OK;
+  uint32_t* place = ds.place[ds.place_turn];
+  ds.place_turn ^= 1u;
+  volatile uint32_t* room = ds.h_crowd;
+  *room = 0u;
+  const uint32_t shift = hi_bit - 8, c = (uint32_t)cap;
+  const double bytes = (double)n * (4.0 + sizeof(K));
+  // 256 tiles at most: a workgroup per CU, and 256 of them to a segment's counter
+#define GQF_RS_PLACE(I_)                                                                                             \
+  GQF_LAUNCH_B(bytes, (k_rs_place<K, I_>), dim3((n + I_ * PLACE_THREADS - 1) / (I_ * PLACE_THREADS)),                \
+               dim3(PLACE_THREADS), 0, s, in, n, fp_bits, shift, c, place, scratch, ds.d_crowd)
+  if (n <= 256u * PLACE_THREADS) GQF_RS_PLACE(1);
+  else if (n <= 512u * PLACE_THREADS) GQF_RS_PLACE(2);
+  else if (n <= 1024u * PLACE_THREADS) GQF_RS_PLACE(4);
+  else if (n <= 2048u * PLACE_THREADS) GQF_RS_PLACE(8);
+  else GQF_RS_PLACE(16);
+#undef GQF_RS_PLACE
+  GQF_LAUNCH_B((double)n * 2.0 * sizeof(K), (k_rs_seg<K, true>), dim3(256), dim3(SEG_THREADS), 0, s, out, place,
+               (const uint32_t*)nullptr, (const uint32_t*)nullptr, shift, (uint32_t*)nullptr, (const K*)scratch, c,
+               ds.place[ds.place_turn]);
+  uint32_t v;
+  for (uint32_t i = 1; (v = *room) == 0u; ++i) {
+    __builtin_ia32_pause();
+    if (i & 0xFFFFu) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    GQF_HIP(e);
+    if ((v = *room) != 0u) break;
+    set_error("internal: the sort's partition ended without an answer");
+    return GQF_ERR_HIP;
+  }
+  *done = v == 1u;
+  lw_report(ds, kind, *done);
+  return GQF_OK;
+}
+
 // LSD radix sort of n keys over bits [lo_bit, hi_bit).  When hash is set, the
 // input is raw uint32 keys, fingerprinted (fp_bits) as they are read in the
 // first pass.  vals: nullptr + with_vals -> the original index is carried.
@@ -1300,6 +1424,15 @@ gqf_status radix_sort(hipStream_t s, Arena& ar, const void* in, bool hash, uint3
     *keys_out = kb[0];
     if (vals_out) *vals_out = vb[0];
     return GQF_OK;
+  }
+  if (ds && hash && !with_vals && lo_bit == 0 && hi_bit >= 16 && hi_bit - 8 <= 32 && seg_bits2(n) == 0) {
+    bool done;
+    GQF_TRY(place_sort<K>(s, ar, *ds, reinterpret_cast<const uint32_t*>(in), n, fp_bits, hi_bit, kb[0], kb[1], &done));
+    if (done) {
+      *keys_out = kb[0];
+      if (vals_out) *vals_out = nullptr;
+      return GQF_OK;
+    }
   }
   const void* src = in;
   const uint32_t* vsrc = in_vals;
@@ -1373,12 +1506,13 @@ gqf_status radix_sort(hipStream_t s, Arena& ar, const void* in, bool hash, uint3
     if (!crowded) {
       if (seg2) {
         GQF_LAUNCH_B((double)n * 2.0 * sizeof(K), (k_rs_seg<K, false>), dim3(ngroups), dim3(SEG_THREADS), 0, s, out,
-                     (const uint32_t*)nullptr, gstart, gsize, nbits, slow);
+                     (const uint32_t*)nullptr, gstart, gsize, nbits, slow, (const K*)nullptr, 0u, (uint32_t*)nullptr);
         GQF_LAUNCH(k_rs_seg_slow<K>, dim3(SEG_SLOW_GRID), dim3(SEG_THREADS), 0, s, out, (const uint32_t*)nullptr,
                    gstart, gsize, nbits, (const uint32_t*)slow);
       } else {
         GQF_LAUNCH_B((double)n * 2.0 * sizeof(K), (k_rs_seg<K, true>), dim3(256), dim3(SEG_THREADS), 0, s, out, dbase,
-                     (const uint32_t*)nullptr, (const uint32_t*)nullptr, nbits, (uint32_t*)nullptr);
+                     (const uint32_t*)nullptr, (const uint32_t*)nullptr, nbits, (uint32_t*)nullptr, (const K*)nullptr, 0u,
+                     (uint32_t*)nullptr);
       }
       *keys_out = out;
       if (vals_out) *vals_out = nullptr;

@@ -55,8 +55,12 @@ gqf_status device_state(hipStream_t stream, DeviceState** out) {
       return GQF_OK;
     }
   DeviceState* ds = new DeviceState();
-  GQF_HIP(hipMalloc((void**)&ds->counters, CTR_TOTAL * sizeof(uint32_t)));
-  GQF_HIP(hipMemset(ds->counters, 0, CTR_TOTAL * sizeof(uint32_t)));
+  constexpr size_t PLACE_AT = 64, PLACE_STRIDE = 320;  // (257 words each, on lines of their own)
+  static_assert(CTR_TOTAL <= PLACE_AT, "the counters come first");
+  GQF_HIP(hipMalloc((void**)&ds->counters, (PLACE_AT + 2 * PLACE_STRIDE) * sizeof(uint32_t)));
+  GQF_HIP(hipMemset(ds->counters, 0, (PLACE_AT + 2 * PLACE_STRIDE) * sizeof(uint32_t)));
+  ds->place[0] = ds->counters + PLACE_AT;
+  ds->place[1] = ds->place[0] + PLACE_STRIDE;
   GQF_HIP(hipHostMalloc((void**)&ds->h_pinned, CTR_TOTAL * sizeof(uint32_t), hipHostMallocDefault));
   GQF_HIP(hipEventCreate(&ds->ev0));
   GQF_HIP(hipEventCreate(&ds->ev1));

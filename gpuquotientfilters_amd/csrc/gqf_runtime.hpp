@@ -62,7 +62,7 @@ struct ProfRec {
 // batch over to the general one.
 enum LocalKind : int {
   LOCAL_SQF_INSERT = 0, LOCAL_SQF_DELETE, LOCAL_RSQF_INSERT, LOCAL_RSQF_DELETE, LOCAL_SQF_BUILD, LOCAL_RSQF_BUILD,
-  LOCAL_SQF_LOOKUP, LOCAL_RSQF_LOOKUP, LOCAL_KINDS
+  LOCAL_SQF_LOOKUP, LOCAL_RSQF_LOOKUP, LOCAL_PLACE_U32, LOCAL_PLACE_U64, LOCAL_KINDS
 };
 
 // Execution context of one (device, stream) pair: workspace arena, device
@@ -88,6 +88,10 @@ struct DeviceState {
   // handed over (saves the copy of the counters)
   uint32_t* h_local = nullptr;
   uint32_t* d_local = nullptr;
+  // counters of the sorts through regions (place_sort), zero before use: each
+  // sort clears the other set for the next one
+  uint32_t* place[2] = {nullptr, nullptr};
+  uint32_t place_turn = 0;
   // after a crowded sort the next crowd_skip sorts take the chunked passes
   // directly; crowd_backoff doubles with every crowded probe in a row.  One
   // pair per key width: 32-bit (SQF, AP hash) and 64-bit (wide) fingerprints
