@@ -129,8 +129,27 @@ gqf_status ws_reserve(DeviceState& ds, size_t bytes) {
   if (ds.ws) GQF_HIP(hipFree(ds.ws));
   ds.ws = nullptr;
   ds.ws_cap = 0;
-  GQF_HIP(hipMalloc((void**)&ds.ws, cap));
+  hipError_t e = hipMalloc((void**)&ds.ws, cap);
+  if (e == hipErrorOutOfMemory && serve_release_idle()) {
+    (void)hipGetLastError();
+    e = hipMalloc((void**)&ds.ws, cap);
+  }
+  if (e != hipSuccess) ds.ws = nullptr;
+  GQF_HIP(e);
   ds.ws_cap = cap;
+  return GQF_OK;
+}
+
+gqf_status ws_trim(gqf_stream s) {
+  int dev = 0;
+  GQF_HIP(hipGetDevice(&dev));
+  DeviceState* ds = find_state(reinterpret_cast<hipStream_t>(s), dev);
+  if (!ds) return GQF_OK;
+  std::lock_guard<std::mutex> lk(ds->mu);
+  GQF_HIP(hipStreamSynchronize(ds->stream));
+  if (ds->ws) GQF_HIP(hipFree(ds->ws));
+  ds->ws = nullptr;
+  ds->ws_cap = 0;
   return GQF_OK;
 }
 
@@ -431,16 +450,8 @@ gqf_status gqf_stream_workspace_bytes(gqf_stream s, size_t* bytes) {
 }
 
 gqf_status gqf_stream_trim(gqf_stream s) {
-  int dev = 0;
-  GQF_HIP(hipGetDevice(&dev));
-  DeviceState* ds = find_state(reinterpret_cast<hipStream_t>(s), dev);
-  if (!ds) return GQF_OK;
-  std::lock_guard<std::mutex> lk(ds->mu);
-  GQF_HIP(hipStreamSynchronize(ds->stream));
-  if (ds->ws) GQF_HIP(hipFree(ds->ws));
-  ds->ws = nullptr;
-  ds->ws_cap = 0;
-  return GQF_OK;
+  (void)serve_release_idle();
+  return ws_trim(s);
 }
 
 size_t gqf_workspace_alloc_bytes(size_t bytes) { return bytes ? ws_alloc_bytes(bytes) : 0; }

@@ -125,6 +125,11 @@ gqf_status device_state(hipStream_t stream, DeviceState** out);
 // Bytes a workspace grows to when a call needs `bytes` more than it holds.
 size_t ws_alloc_bytes(size_t bytes);
 gqf_status ws_reserve(DeviceState& ds, size_t bytes);
+// Releases the workspace of a stream's context.
+gqf_status ws_trim(gqf_stream s);
+// Releases the serving loop's idle workers of the current device (kept from
+// one run to the next); whether there were any.
+bool serve_release_idle();
 // The same for a form that another one can stand in for.
 inline bool ws_try_reserve(DeviceState& ds, size_t bytes) {
   if (ws_reserve(ds, bytes) == GQF_OK) return true;

@@ -82,13 +82,15 @@ struct Scheduler {
         running++;
         return true;
       }
-      // release what an idle worker holds
+      // release what an idle worker holds, and our own last (a run may begin
+      // with what its workers held at the end of another)
       int v = -1;
       for (int i = 0; i < nworkers; ++i)
         if (i != w && state[(size_t)i] == IDLE && held[(size_t)i] > 0) {
           v = i;
           break;
         }
+      if (v < 0 && running == 0 && trimming == 0 && held[(size_t)w] > 0) v = w;
       if (v >= 0) {
         state[(size_t)v] = TRIMMING;
         trimming++;
@@ -338,6 +340,7 @@ bool mv_overlap(gqf_request** b, int nb) {
 struct RsqfExec {
   const gqf_rsqf* f = nullptr;
   int sorted = 0;
+  bool tight = false;  // the budget leaves no room for more than the calls need
   struct W {
     gqf_stream st = nullptr;
     uint32_t* keys = nullptr;
@@ -347,6 +350,9 @@ struct RsqfExec {
   std::vector<W> w;
 
   static size_t stage_bytes(size_t cap) { return cap * 8; }
+  // Keys the gather buffers grow to for a call of n (every free waits for the
+  // device, and so for the other workers' calls).
+  size_t stage_room(size_t n) const { return tight ? n : n + n / 2; }
 
   static size_t grow(void* u, int wi, int filter, int op, uint64_t n, int coalesced) {
     RsqfExec& e = *static_cast<RsqfExec*>(u);
@@ -355,7 +361,7 @@ struct RsqfExec {
     size_t have = 0;
     (void)gqf_stream_workspace_bytes(x.st, &have);
     size_t g = need > have ? ws_alloc_bytes(need) - have : 0;
-    if (coalesced && n > x.cap) g += stage_bytes((size_t)n) - stage_bytes(x.cap);
+    if (coalesced && n > x.cap) g += stage_bytes(e.stage_room((size_t)n)) - stage_bytes(x.cap);
     return g;
   }
   static size_t held(void* u, int wi) {
@@ -368,10 +374,10 @@ struct RsqfExec {
   static void trim(void* u, int wi) {
     RsqfExec& e = *static_cast<RsqfExec*>(u);
     W& x = e.w[(size_t)wi];
-    (void)gqf_stream_trim(x.st);
+    (void)ws_trim(x.st);
     e.free_stage(x);
   }
-  void free_stage(W& x) {
+  static void free_stage(W& x) {
     if (x.keys) (void)hipFree(x.keys);
     if (x.out) (void)hipFree(x.out);
     x.keys = nullptr;
@@ -399,9 +405,10 @@ struct RsqfExec {
     if (n > x.cap) {
       GQF_HIP(hipStreamSynchronize(hs));
       free_stage(x);
-      GQF_HIP(hipMalloc((void**)&x.keys, n * 4));
-      GQF_HIP(hipMalloc((void**)&x.out, n * 4));
-      x.cap = n;
+      const size_t cap = stage_room(n);
+      GQF_HIP(hipMalloc((void**)&x.keys, cap * 4));
+      GQF_HIP(hipMalloc((void**)&x.out, cap * 4));
+      x.cap = cap;
     }
     GQF_TRY(mv_requests<true>(hs, b, nb, x.keys));
     if (op == GQF_OP_INSERT) return gqf_rsqf_insert(fl, (int)n, x.keys, nullptr, x.st, &ms);
@@ -423,7 +430,88 @@ struct RsqfExec {
   }
 };
 
+// Workers between runs: a stream, its context and what both hold.  Making and
+// freeing them took a third of a run of 300 requests (every free waits for
+// the device, and so for the other workers' calls).  At most IDLE_MAX of them
+// are kept, IDLE_BYTES in all, oldest taken first; a worker is one run's alone
+// while it is taken.  Given back by serve_release_idle.
+struct IdleWorker {
+  int device;
+  RsqfExec::W w;
+  size_t bytes;
+};
+constexpr size_t IDLE_MAX = 16, IDLE_BYTES = (size_t)256 << 20;
+static std::mutex g_idle_mu;
+static std::vector<IdleWorker>* g_idle = nullptr;
+
+static gqf_status worker_end(RsqfExec::W& x) {
+  RsqfExec::free_stage(x);
+  gqf_status st = GQF_OK;
+  if (x.st) st = gqf_stream_destroy(x.st);
+  x.st = nullptr;
+  return st;
+}
+// bare: holding nothing.
+static gqf_status worker_take(RsqfExec::W* x, bool bare) {
+  int dev = 0;
+  GQF_HIP(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    for (size_t i = 0; g_idle && i < g_idle->size(); ++i)
+      if ((*g_idle)[i].device == dev) {
+        *x = (*g_idle)[i].w;
+        g_idle->erase(g_idle->begin() + (long)i);
+        break;
+      }
+  }
+  if (!x->st) return gqf_stream_create(&x->st);
+  if (bare) {
+    RsqfExec::free_stage(*x);
+    GQF_TRY(ws_trim(x->st));
+  }
+  return GQF_OK;
+}
+static gqf_status worker_put(RsqfExec::W& x) {
+  int dev = 0;
+  GQF_HIP(hipGetDevice(&dev));
+  if (!x.st) return worker_end(x);
+  size_t bytes = 0;
+  (void)gqf_stream_workspace_bytes(x.st, &bytes);
+  bytes += RsqfExec::stage_bytes(x.cap);
+  {
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    if (!g_idle) g_idle = new std::vector<IdleWorker>();
+    size_t held = bytes;
+    for (const IdleWorker& w : *g_idle) held += w.bytes;
+    if (g_idle->size() < IDLE_MAX && held <= IDLE_BYTES) {
+      g_idle->push_back({dev, x, bytes});
+      x = RsqfExec::W();
+      return GQF_OK;
+    }
+  }
+  return worker_end(x);
+}
+
 }  // namespace
+
+bool serve_release_idle() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::vector<IdleWorker> mine;
+  {
+    std::lock_guard<std::mutex> lk(g_idle_mu);
+    for (size_t i = 0; g_idle && i < g_idle->size();)
+      if ((*g_idle)[i].device == dev) {
+        mine.push_back((*g_idle)[i]);
+        g_idle->erase(g_idle->begin() + (long)i);
+      } else {
+        ++i;
+      }
+  }
+  for (IdleWorker& w : mine) (void)worker_end(w.w);
+  return !mine.empty();
+}
+
 }  // namespace gqf
 
 using namespace gqf;
@@ -460,10 +548,11 @@ gqf_status gqf_rsqf_serve(gqf_rsqf* filters, int nfilters, gqf_request* reqs, in
   RsqfExec e;
   e.f = filters;
   e.sorted = cfg->sorted_lookups;
+  e.tight = cfg->hbm_budget < resident || cfg->hbm_budget - resident < 2 * IDLE_BYTES;
   e.w.resize(cfg->coalesce ? (size_t)nfilters : 1);
   gqf_status st = GQF_OK;
   for (RsqfExec::W& x : e.w)
-    if (st == GQF_OK) st = gqf_stream_create(&x.st);
+    if (st == GQF_OK) st = worker_take(&x, e.tight);
   if (st == GQF_OK) {
     gqf_serve_executor ex{&e, &RsqfExec::grow, &RsqfExec::held, &RsqfExec::trim, &RsqfExec::run};
     Scheduler s;
@@ -474,11 +563,8 @@ gqf_status gqf_rsqf_serve(gqf_rsqf* filters, int nfilters, gqf_request* reqs, in
     st = s.run(reqs, nreqs, stats);
   }
   for (RsqfExec::W& x : e.w) {
-    e.free_stage(x);
-    if (x.st) {
-      const gqf_status d = gqf_stream_destroy(x.st);
-      if (st == GQF_OK) st = d;
-    }
+    const gqf_status d = st == GQF_OK ? worker_put(x) : worker_end(x);
+    if (st == GQF_OK) st = d;
   }
   return st;
 }

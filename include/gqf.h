@@ -361,7 +361,8 @@ gqf_status gqf_stream_create(gqf_stream* out);
 /* Waits for the stream, releases its workspace and destroys it. */
 gqf_status gqf_stream_destroy(gqf_stream s);
 /* Workspace currently held for calls on the stream (grow-only until trimmed),
- * and its release. */
+ * and its release (with that of the serving loop's idle workers on the
+ * device: their streams and up to 256 MiB of buffers stay for the next run). */
 gqf_status gqf_stream_workspace_bytes(gqf_stream s, size_t* bytes);
 gqf_status gqf_stream_trim(gqf_stream s);
 /* What a workspace grows to when a call needs `bytes` more than it holds. */
