@@ -58,8 +58,8 @@ static gqf_status work_table(hipStream_t s, Arena& ar, const gqf_sqf& qf, const 
     return GQF_ERR_INVALID;
   }
   if (load)
-    GQF_LAUNCH_B((double)g.pwords * 4 + (double)g.bytes, k_sqf_unpack, dim3((g.S + 255) / 256), dim3(256), 0, s,
-                 reinterpret_cast<const uint32_t*>(qf.table), g.S, g.r + 3, reinterpret_cast<uint16_t*>(out->table));
+    GQF_LAUNCH_B((double)g.pwords * 4 + (double)g.bytes, k_sqf_unpack, dim3((g.S + 2047) / 2048), dim3(256), 0, s,
+                 reinterpret_cast<const uint32_t*>(qf.table), g.pwords, g.S, g.r + 3, reinterpret_cast<uint16_t*>(out->table));
   return GQF_OK;
 }
 // Packs the wide copy back into the caller's table (packed widths only);
@@ -67,7 +67,8 @@ static gqf_status work_table(hipStream_t s, Arena& ar, const gqf_sqf& qf, const 
 static void finish_table(hipStream_t s, const gqf_sqf& qf, const gqf_sqf& work, const SqfGeom& g,
                          const uint32_t* ctr) {
   if (!g.packed) return;
-  GQF_LAUNCH_B((double)g.bytes + (double)g.pwords * 4, k_sqf_pack, dim3((g.pwords + 255) / 256), dim3(256), 0, s,
+  GQF_LAUNCH_B((double)g.bytes + (double)g.pwords * 4, k_sqf_pack,
+               dim3((uint32_t)(((uint64_t)g.pwords / (g.r + 3) + 1 + 63) / 64)), dim3(64), 0, s,
                reinterpret_cast<const uint16_t*>(work.table), g.S, g.r + 3, reinterpret_cast<uint32_t*>(qf.table),
                g.pwords, ctr);
 }
