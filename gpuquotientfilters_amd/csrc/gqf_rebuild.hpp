@@ -200,7 +200,8 @@ static_assert(RB_MAX_CHUNKS <= 64 * RBS_PER, "the apply kernel combines at most 
   if (i < G) agg[i] = rs_pack(rs_combine(rs_unpack(s_wave[wid]), ex));
 }
 
-// Host side: the two launches, with their partials taken from the arena.
+// Host side: the two launches (one up to 1024 states), with their partials
+// taken from the arena.
 static inline gqf_status rb_scan(hipStream_t s, Arena& ar, uint4* agg, uint32_t G, uint64_t S, uint32_t* ctr,
                                  uint4* total) {
   const uint32_t P = (G + RBS_PER - 1) / RBS_PER;
@@ -209,7 +210,8 @@ static inline gqf_status rb_scan(hipStream_t s, Arena& ar, uint4* agg, uint32_t 
     set_error("internal: rebuild workspace overflow");
     return GQF_ERR_INVALID;
   }
-  GQF_LAUNCH(k_rb_scan_reduce, dim3(P), dim3(RBS_PER), 0, s, agg, G, part);
+  // (one workgroup has no aggregates before it)
+  if (P > 1) GQF_LAUNCH(k_rb_scan_reduce, dim3(P), dim3(RBS_PER), 0, s, agg, G, part);
   GQF_LAUNCH(k_rb_scan_apply, dim3(P), dim3(RBS_PER), 0, s, agg, G, part, S, ctr, total);
   return GQF_OK;
 }

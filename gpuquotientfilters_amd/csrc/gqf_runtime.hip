@@ -61,7 +61,8 @@ gqf_status device_state(hipStream_t stream, DeviceState** out) {
   GQF_HIP(hipMemset(ds->counters, 0, (PLACE_AT + 2 * PLACE_STRIDE) * sizeof(uint32_t)));
   ds->place[0] = ds->counters + PLACE_AT;
   ds->place[1] = ds->place[0] + PLACE_STRIDE;
-  GQF_HIP(hipHostMalloc((void**)&ds->h_pinned, CTR_TOTAL * sizeof(uint32_t), hipHostMallocDefault));
+  GQF_HIP(hipHostMalloc((void**)&ds->h_pinned, CTR_TOTAL * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+  GQF_HIP(hipHostGetDevicePointer((void**)&ds->d_pinned, ds->h_pinned, 0));
   GQF_HIP(hipEventCreate(&ds->ev0));
   GQF_HIP(hipEventCreate(&ds->ev1));
   GQF_HIP(hipHostMalloc((void**)&ds->h_crowd, 64, hipHostMallocMapped | hipHostMallocCoherent));
@@ -241,6 +242,10 @@ void prof_resolve(DeviceState& ds) {
   ds.pool_used = 0;
 }
 
+static __global__ __launch_bounds__(64) void k_ctr_out(const uint32_t* __restrict__ ctr, uint32_t* __restrict__ host) {
+  if (threadIdx.x < CTR_TOTAL) host[threadIdx.x] = ctr[threadIdx.x];
+}
+
 gqf_status CallScope::begin(gqf_stream s) {
   stream = reinterpret_cast<hipStream_t>(s);
   GQF_TRY(device_state(stream, &ds));
@@ -260,8 +265,8 @@ CallScope::~CallScope() {
 
 gqf_status CallScope::end(float* ms, bool check_device_err) {
   if (check_device_err) {
-    GQF_HIP(hipMemcpyAsync(ds->h_pinned, ds->counters, CTR_TOTAL * sizeof(uint32_t),
-                           hipMemcpyDeviceToHost, stream));
+    // (a copy of 64 bytes takes the queue and the host longer than a kernel)
+    hipLaunchKernelGGL(k_ctr_out, dim3(1), dim3(64), 0, stream, ds->counters, ds->d_pinned);
   }
   GQF_HIP(hipEventRecord(ds->ev1, stream));
   GQF_HIP(hipEventSynchronize(ds->ev1));

@@ -76,7 +76,8 @@ struct DeviceState {
   char* ws = nullptr;               // workspace arena (grow-only)
   size_t ws_cap = 0;
   uint32_t* counters = nullptr;     // CTR_TOTAL device counters
-  uint32_t* h_pinned = nullptr;     // pinned host mirror of the counters
+  uint32_t* h_pinned = nullptr;     // pinned host mirror of the counters (host and device views)
+  uint32_t* d_pinned = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // sort probe: a word of host-coherent pinned memory (host and device views)
   // that a sort's row scan raises when its top-digit segments are too large

@@ -179,11 +179,9 @@ static gqf_status launch_rebuild(hipStream_t s, uint32_t* counters, Arena& ar, c
   else if (g.bpe == 3) GQF_RB_WRITE(3);
   else GQF_RB_WRITE(4);
 #undef GQF_RB_WRITE
-  if (precleared != 1)
-    GQF_LAUNCH(k_sqf_clear_tail, dim3(1024), dim3(256), 0, s, qf.table, g.bpe, g.bytes, counters, post_mode, na_dev,
-               nadd, g.S);
-  GQF_LAUNCH(k_sqf_fixup, dim3(p.nsub + 1), dim3(64), 0, s, qf.table, g.bpe, fix, fix_cnt, fix_more, counters,
-             p.nsub, (uint32_t)(N + 1), na_dev, nadd);
+  const uint32_t tail = precleared != 1 ? (uint32_t)std::min<uint64_t>(1024, g.bytes / 16384 + 1) : 0u;
+  GQF_LAUNCH(k_sqf_finish, dim3((p.nsub + 1 + 3) / 4 + tail), dim3(256), 0, s, qf.table, g.bpe, fix, fix_cnt, fix_more,
+             counters, p.nsub, (uint32_t)(N + 1), na_dev, nadd, g.bytes, post_mode, g.S);
   return GQF_OK;
 }
 

@@ -486,7 +486,7 @@ __global__ __launch_bounds__(256) void k_sqf_lookup(const uint8_t* __restrict__ 
 //               window, each thread the slots up to its own last entry from
 //               registers; slots past the last entry are cleared by
 //               k_sqf_clear_tail.  An occupied bit that falls in an earlier
-//               sub-tile's range goes to a fix-up list (k_sqf_fixup).
+//               sub-tile's range goes to a fix-up list (k_sqf_finish).
 // Replaces the location and write stages of the three reference builds
 // (quotientFilter.cu:788-857, 985-1038, 1492-1539), the merge rebuild
 // (quotientFilter.cu:1651-1719) and the end states of insert /
@@ -985,10 +985,10 @@ __global__ __launch_bounds__(RB_THREADS, 6) void k_rb_write(uint8_t* __restrict_
 // is sparse (N * 8 < S, then the writer skips windows of zeros); 3: the tail
 // iff it is not; 4: from slot S on, or from the slot after the last entry if
 // that is later.  N = *n_dev (when given) + n_add.
-[[maybe_unused]] static __global__ __launch_bounds__(256) void k_sqf_clear_tail(uint8_t* __restrict__ t, uint32_t bpe, uint64_t tbytes,
-                                                        const uint32_t* __restrict__ ctr, int mode,
-                                                        const uint32_t* __restrict__ n_dev, uint32_t n_add,
-                                                        uint32_t S) {
+__device__ __forceinline__ void sqf_clear_tail(uint8_t* __restrict__ t, uint32_t bpe, uint64_t tbytes,
+                                               const uint32_t* __restrict__ ctr, int mode,
+                                               const uint32_t* __restrict__ n_dev, uint32_t n_add, uint32_t S,
+                                               uint32_t block, uint32_t blocks) {
   if (ctr[CTR_ERR]) return;  // capacity error: the table stays as it was
   if (mode == 4 && ctr[CTR_MISC]) return;  // handed over: nothing was written
   if (mode == 2 || mode == 3) {
@@ -1000,7 +1000,7 @@ __global__ __launch_bounds__(RB_THREADS, 6) void k_rb_write(uint8_t* __restrict_
   const uint32_t tail = mode == 4 && S > ctr[CTR_MISC + 3] ? S : ctr[CTR_MISC + 3];
   const uint64_t b0 = whole_table ? 0ull : (uint64_t)tail * bpe;
   const uint64_t a0 = (b0 + 15) & ~15ull, a1 = tbytes & ~15ull;
-  const uint64_t tid = blockIdx.x * 256ull + threadIdx.x, nth = (uint64_t)gridDim.x * 256;
+  const uint64_t tid = block * 256ull + threadIdx.x, nth = (uint64_t)blocks * 256;
   if (a0 >= a1) {
     for (uint64_t b = b0 + tid; b < tbytes; b += nth) t[b] = 0;
     return;
@@ -1011,6 +1011,12 @@ __global__ __launch_bounds__(RB_THREADS, 6) void k_rb_write(uint8_t* __restrict_
   const uint64_t nw = (a1 - a0) / 16;
   for (uint64_t i = tid; i < nw; i += nth) w[i] = make_uint4(0u, 0u, 0u, 0u);
 }
+[[maybe_unused]] static __global__ __launch_bounds__(256) void k_sqf_clear_tail(uint8_t* __restrict__ t, uint32_t bpe, uint64_t tbytes,
+                                                        const uint32_t* __restrict__ ctr, int mode,
+                                                        const uint32_t* __restrict__ n_dev, uint32_t n_add,
+                                                        uint32_t S) {
+  sqf_clear_tail(t, bpe, tbytes, ctr, mode, n_dev, n_add, S, blockIdx.x, gridDim.x);
+}
 
 // Occupied bits that rebuild tiles could not place in their own ranges: one
 // workgroup per tile's slots, plus the shared overflow list.
@@ -1020,15 +1026,23 @@ __device__ __forceinline__ void sqf_set_occupied(uint8_t* t, uint32_t bpe, uint3
   atomicOr(word, 4u << (8 * (uint32_t)(byte & 3)));
 }
 
-[[maybe_unused]] static __global__ __launch_bounds__(64) void k_sqf_fixup(uint8_t* __restrict__ t, uint32_t bpe,
+// The workgroups past the lists' (with tail) clear the slots past the last
+// entry, which no list reaches: one launch for both.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void k_sqf_finish(uint8_t* __restrict__ t, uint32_t bpe,
                                                   const uint32_t* __restrict__ fix,
                                                   const uint32_t* __restrict__ fix_cnt,
                                                   const uint32_t* __restrict__ fix_more,
                                                   const uint32_t* __restrict__ ctr, uint32_t tiles,
                                                   uint32_t fix_cap, const uint32_t* __restrict__ n_dev,
-                                                  uint32_t n_add) {
+                                                  uint32_t n_add, uint64_t tbytes, int mode, uint32_t S) {
+  const uint32_t lists = (tiles + 1 + 3) / 4;  // workgroups, a wave per list
+  if (blockIdx.x >= lists) {
+    sqf_clear_tail(t, bpe, tbytes, ctr, mode, n_dev, n_add, S, blockIdx.x - lists, gridDim.x - lists);
+    return;
+  }
   if (ctr[CTR_ERR]) return;  // capacity error: the table stays as it was
-  const uint32_t tile = blockIdx.x;
+  const uint32_t tile = 4 * blockIdx.x + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (tile > tiles) return;
   if (n_dev) {  // the grid covers an upper bound: sub-tiles past the entries have no list
     const uint64_t N = (uint64_t)*n_dev + n_add;
     const uint64_t used = (N + RB_TILE - 1) / RB_TILE;
@@ -1036,11 +1050,11 @@ __device__ __forceinline__ void sqf_set_occupied(uint8_t* t, uint32_t bpe, uint3
   }
   if (tile < tiles) {
     const uint32_t c = fix_cnt[tile];
-    for (uint32_t i = threadIdx.x; i < c; i += 64) sqf_set_occupied(t, bpe, fix[(uint64_t)tile * RB_FIX + i]);
+    for (uint32_t i = lane; i < c; i += 64) sqf_set_occupied(t, bpe, fix[(uint64_t)tile * RB_FIX + i]);
   } else {
     uint32_t n = ctr[CTR_MISC + 2];  // shared overflow list length
     if (n > fix_cap) n = fix_cap;
-    for (uint32_t i = threadIdx.x; i < n; i += 64) sqf_set_occupied(t, bpe, fix_more[i]);
+    for (uint32_t i = lane; i < n; i += 64) sqf_set_occupied(t, bpe, fix_more[i]);
   }
 }
 
