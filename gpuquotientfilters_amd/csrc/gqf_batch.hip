@@ -3,7 +3,10 @@
 // A batch holds F SQFs (same r, any q) and, back to back in one device array
 // each, their build keys and their lookup keys.  Every stage of the build
 // pipeline is one launch over all filters:
-//   segmented LSD radix sort   chunks never cross a filter; per 8-bit digit:
+//   segmented radix sort       chunks never cross a filter; one pass on every
+//                              filter's top 8 bits, then its groups of digits
+//                              in LDS (filters past 1.9 M keys: a pass per 8
+//                              bits from the lowest).  A pass:
 //                              upsweep (chunk histograms), row scan (prefix
 //                              of every digit over all chunks), per-filter
 //                              digit bases (a filter's count of digit d is a
@@ -53,6 +56,19 @@ struct BTile {
 };
 
 // ---------------------------------------------------------------- segmented sort
+// Batches whose filters have up to 256 * SEG_GROUP_AVG keys take one pass on
+// every filter's own top 8 bits (BS_TOP) and then sort groups of neighbouring
+// digits, about 4096 keys each, in LDS: two reads and writes of the keys
+// instead of one per 8 bits.  48 filters of q = 12 .. 20, 6 M keys: 94 us, four
+// passes 200.
+constexpr uint32_t BS_TOP = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t bs_shift(uint32_t shift, uint32_t bits) {
+  const uint32_t b = bits & 0xFFu;
+  return shift != BS_TOP ? shift : b > 8 ? b - 8 : 0u;
+}
+struct BGroup {
+  uint32_t f, d0, d1, nbits;  // filter, its digits [d0, d1), bits below those all keys share
+};
 template <bool HASH>
 __global__ __launch_bounds__(256) void k_bs_upsweep(const uint32_t* __restrict__ in, const BChunk* __restrict__ ch,
                                                     const BFilter* __restrict__ flt, uint32_t shift, uint32_t G,
@@ -63,6 +79,7 @@ __global__ __launch_bounds__(256) void k_bs_upsweep(const uint32_t* __restrict__
   __syncthreads();
   const BChunk c = ch[blockIdx.x];
   const uint32_t bits = flt[c.f].bits;
+  shift = bs_shift(shift, bits);
   for (uint32_t t0 = c.begin; t0 < c.end; t0 += SORT_TILE) {
     uint32_t k[SORT_ITEMS];
 #pragma unroll
@@ -94,23 +111,19 @@ __global__ __launch_bounds__(256) void k_bs_digitbase(const uint32_t* __restrict
   dbase[(uint64_t)f * 256 + d] = block256_excl_scan(p1 - p0, tmp, nullptr);
 }
 
+// LDS of a stable pass over tiles of SORT_TILE keys.
+struct BsLds {
+  uint32_t run[256], wcnt[4 * 256], lstart[256], tmp[4], keys[SORT_TILE];
+};
+// The keys [begin, end) of `in` by one digit, in order: a key of digit d to
+// s_run[d] and on.
 template <bool HASH>
-__global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                      const BChunk* __restrict__ ch, const BFilter* __restrict__ flt,
-                                                      uint32_t shift, uint32_t G, const uint32_t* __restrict__ hist,
-                                                      const uint32_t* __restrict__ dbase, uint32_t n_total) {
-  __shared__ uint32_t s_run[256];
-  __shared__ uint32_t s_wcnt[4 * 256];
-  __shared__ uint32_t s_lstart[256];
-  __shared__ uint32_t s_tmp[4];
-  __shared__ uint32_t s_keys[SORT_TILE];
+__device__ __forceinline__ void bs_tiles(const uint32_t* in, uint32_t* out, uint32_t begin, uint32_t end, uint32_t bits,
+                                         uint32_t shift, uint32_t n_total, BsLds& l) {
+  uint32_t *s_run = l.run, *s_wcnt = l.wcnt, *s_lstart = l.lstart, *s_tmp = l.tmp, *s_keys = l.keys;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const BChunk c = ch[blockIdx.x];
-  const BFilter fl = flt[c.f];
-  s_run[tid] = fl.key0 + dbase[(uint64_t)c.f * 256 + tid] + hist[(uint64_t)tid * G + blockIdx.x] -
-               hist[(uint64_t)tid * G + c.head];
   const uint64_t lt = (1ull << lane) - 1ull;
-  for (uint32_t t0 = c.begin; t0 < c.end; t0 += SORT_TILE) {
+  for (uint32_t t0 = begin; t0 < end; t0 += SORT_TILE) {
     for (int i = tid; i < 4 * 256; i += 256) s_wcnt[i] = 0;
     __syncthreads();
     const uint32_t base = t0 + (uint32_t)wid * (SORT_ITEMS * 64) + lane;
@@ -119,7 +132,7 @@ __global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict
     for (int i = 0; i < SORT_ITEMS; ++i) {
       const uint32_t idx = base + (uint32_t)i * 64;
       // padding keys (all ones) take the last digit and rank after real keys
-      k[i] = idx < c.end ? (HASH ? fingerprint32(in[idx], fl.bits) : in[idx]) : 0xFFFFFFFFu;
+      k[i] = idx < end ? (HASH ? fingerprint32(in[idx], bits) : in[idx]) : 0xFFFFFFFFu;
     }
     uint32_t rk[SORT_ITEMS];
 #pragma unroll
@@ -151,7 +164,7 @@ __global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict
       s_keys[s_lstart[d] + s_wcnt[wid * 256 + d] + rk[i]] = k[i];
     }
     __syncthreads();
-    const uint32_t tile_n = c.end - t0 < (uint32_t)SORT_TILE ? c.end - t0 : (uint32_t)SORT_TILE;
+    const uint32_t tile_n = end - t0 < (uint32_t)SORT_TILE ? end - t0 : (uint32_t)SORT_TILE;
 #pragma unroll
     for (int i = 0; i < SORT_ITEMS; ++i) {
       const uint32_t p = tid + i * SORT_THREADS;
@@ -164,6 +177,83 @@ __global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict
     }
     __syncthreads();
     s_run[tid] += total;
+    __syncthreads();
+  }
+}
+
+template <bool HASH>
+__global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                      const BChunk* __restrict__ ch, const BFilter* __restrict__ flt,
+                                                      uint32_t shift, uint32_t G, const uint32_t* __restrict__ hist,
+                                                      const uint32_t* __restrict__ dbase, uint32_t n_total) {
+  __shared__ BsLds l;
+  const int tid = threadIdx.x;
+  const BChunk c = ch[blockIdx.x];
+  const BFilter fl = flt[c.f];
+  l.run[tid] = fl.key0 + dbase[(uint64_t)c.f * 256 + tid] + hist[(uint64_t)tid * G + blockIdx.x] -
+               hist[(uint64_t)tid * G + c.head];
+  bs_tiles<HASH>(in, out, c.begin, c.end, fl.bits, bs_shift(shift, fl.bits), n_total, l);
+}
+
+__device__ __forceinline__ void bs_range(const BGroup& g, const BFilter* __restrict__ flt, const uint32_t* __restrict__ dbase,
+                                         uint32_t* begin, uint32_t* end) {
+  const uint32_t k0 = flt[g.f].key0;
+  *begin = k0 + dbase[(uint64_t)g.f * 256 + g.d0];
+  *end = k0 + (g.d1 < 256 ? dbase[(uint64_t)g.f * 256 + g.d1] : flt[g.f].nkeys);
+}
+// Group blockIdx.x in place; one of more keys than LDS holds, or with a
+// crowded bucket, goes to `big` (count, then group ids).
+[[maybe_unused]] static __global__ __launch_bounds__(SEG_THREADS) void k_bs_groups(uint32_t* __restrict__ keys,
+                                                                                 const BGroup* __restrict__ grp,
+                                                                                 const BFilter* __restrict__ flt,
+                                                                                 const uint32_t* __restrict__ dbase,
+                                                                                 uint32_t* __restrict__ big) {
+  __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
+  __shared__ __align__(16) uint32_t s_c[SEG_NBK / 2];
+  __shared__ uint32_t s_tmp[SEG_THREADS / 64];
+  const BGroup g = grp[blockIdx.x];
+  uint32_t begin, end;
+  bs_range(g, flt, dbase, &begin, &end);
+  if (end - begin <= 1) return;
+  if (end - begin > (uint32_t)SEG_TILE) {
+    if (threadIdx.x == 0) big[1 + atomicAdd(&big[0], 1u)] = blockIdx.x;
+    return;
+  }
+  if (!seg_bucket_sort<uint32_t, false>(keys + begin, keys + begin, end - begin, g.nbits, s_keys, nullptr, s_c, s_tmp) &&
+      threadIdx.x == 0)
+    big[1 + atomicAdd(&big[0], 1u)] = blockIdx.x;
+}
+// The groups left (crowded digits: many copies of a few keys), one workgroup
+// each: 8-bit passes between the group's ranges of a and b.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void k_bs_big(uint32_t* a, uint32_t* b,
+                                                                      const BGroup* __restrict__ grp,
+                                                                      const BFilter* __restrict__ flt,
+                                                                      const uint32_t* __restrict__ dbase,
+                                                                      const uint32_t* __restrict__ big, uint32_t n_total) {
+  __shared__ BsLds l;
+  __shared__ uint32_t s_hist[256];
+  const uint32_t tid = threadIdx.x, n = big[0];
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const BGroup g = grp[big[1 + i]];
+    uint32_t begin, end;
+    bs_range(g, flt, dbase, &begin, &end);
+    uint32_t *src = a, *dst = b;
+    for (uint32_t shift = 0; shift < g.nbits; shift += 8) {
+      s_hist[tid] = 0u;
+      __syncthreads();
+      for (uint32_t k = begin + tid; k < end; k += 256) atomicAdd(&s_hist[(src[k] >> shift) & 255u], 1u);
+      __syncthreads();
+      l.run[tid] = begin + block256_excl_scan(s_hist[tid], l.tmp, nullptr);
+      __syncthreads();
+      bs_tiles<false>(src, dst, begin, end, 0u, shift, n_total, l);
+      __threadfence_block();
+      __syncthreads();
+      uint32_t* t = src;
+      src = dst;
+      dst = t;
+    }
+    if (src != a)
+      for (uint32_t k = begin + tid; k < end; k += 256) a[k] = src[k];
     __syncthreads();
   }
 }
@@ -384,16 +474,34 @@ __global__ __launch_bounds__(256) void k_bi_count(const BFilter* __restrict__ fl
   idx[i] = make_uint2(o, r);
 }
 
-// Filter blockIdx.x: exclusive scan of its entries in place, 1024 at a time.
+// Filter blockIdx.x: exclusive scan of its entries in place, BI_SEG per thread
+// and the next ones on their way (1024 entries per round, loaded when their
+// turn came, took 22 us for q = 20, 18 rounds of one load's latency; this, 16).
+constexpr uint32_t BI_SEG = 8;
 __global__ __launch_bounds__(1024) void k_bi_scan(const uint32_t* __restrict__ woff, uint2* __restrict__ idx) {
   __shared__ uint32_t s_w[2][16];
   const uint32_t f = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const uint32_t b0 = woff[f], b1 = woff[f + 1];
   uint32_t co = 0, cr = 0;  // carries
-  for (uint32_t base = b0; base < b1; base += 1024) {
-    const uint32_t i = base + tid;
-    const uint2 x = i < b1 ? idx[i] : make_uint2(0u, 0u);
-    const uint32_t io = wave_incl_add(x.x), ir = wave_incl_add(x.y);
+  uint2 x[BI_SEG];
+  auto load = [&](uint32_t base) {
+#pragma unroll
+    for (uint32_t k = 0; k < BI_SEG; ++k) {
+      const uint32_t i = base + BI_SEG * tid + k;
+      x[k] = i < b1 ? idx[i] : make_uint2(0u, 0u);
+    }
+  };
+  load(b0);
+  for (uint32_t base = b0; base < b1; base += 1024 * BI_SEG) {
+    uint2 sum = make_uint2(0u, 0u), ex[BI_SEG];
+#pragma unroll
+    for (uint32_t k = 0; k < BI_SEG; ++k) {
+      ex[k] = sum;
+      sum.x += x[k].x;
+      sum.y += x[k].y;
+    }
+    load(base + 1024 * BI_SEG);
+    const uint32_t io = wave_incl_add(sum.x), ir = wave_incl_add(sum.y);
     if (lane == 63) {
       s_w[0][wid] = io;
       s_w[1][wid] = ir;
@@ -408,7 +516,12 @@ __global__ __launch_bounds__(1024) void k_bi_scan(const uint32_t* __restrict__ w
       to += a;
       tr += c;
     }
-    if (i < b1) idx[i] = make_uint2(co + po + io - x.x, cr + pr + ir - x.y);
+    const uint32_t so = co + po + io - sum.x, sr = cr + pr + ir - sum.y;
+#pragma unroll
+    for (uint32_t k = 0; k < BI_SEG; ++k) {
+      const uint32_t i = base + BI_SEG * tid + k;
+      if (i < b1) idx[i] = make_uint2(so + ex[k].x, sr + ex[k].y);
+    }
     co += to;
     cr += tr;
     __syncthreads();
@@ -469,6 +582,9 @@ struct SqfBatch {
   BChunk* d_ch = nullptr;
   uint32_t *d_fchunk = nullptr, *d_poff = nullptr, *d_hist = nullptr, *d_tot = nullptr, *d_dbase = nullptr;
   uint32_t *d_k0 = nullptr, *d_k1 = nullptr;
+  BGroup* d_grp = nullptr;
+  uint32_t* d_big = nullptr;  // count and ids of the groups k_bs_groups leaves
+  uint32_t ngroups = 0;       // 0: the 8-bit passes
   uint4* d_agg = nullptr;
   uint32_t *d_fix = nullptr, *d_fixcnt = nullptr, *d_more = nullptr, *d_moren = nullptr;
   uint32_t *d_ferr = nullptr, *d_fend = nullptr;
@@ -543,15 +659,15 @@ static void batch_index_launch(SqfBatch& b) {
 static void batch_build_launch(SqfBatch& b) {
   hipStream_t s = b.stream;
   const uint32_t F = (uint32_t)b.F;
-  GQF_LAUNCH(k_bb_reset, dim3(64), dim3(256), 0, s, b.d_ferr, 3 * F);  // ferr, fend, more_n
+  GQF_LAUNCH(k_bb_reset, dim3(64), dim3(256), 0, s, b.d_ferr, 3 * F + 1);  // ferr, fend, more_n, the count in big
   if (b.N == 0) {
     GQF_LAUNCH(k_bb_clear_tail, dim3(64, F), dim3(256), 0, s, b.d_flt, b.d_ferr, b.d_fend, b.bpe);
     return;
   }
   const uint32_t* src = b.d_keys;
   uint32_t* buf[2] = {b.d_k0, b.d_k1};
-  for (uint32_t p = 0; p < b.npass; ++p) {
-    const uint32_t shift = 8 * p;
+  for (uint32_t p = 0; p < (b.ngroups ? 1u : b.npass); ++p) {
+    const uint32_t shift = b.ngroups ? BS_TOP : 8 * p;
     uint32_t* dst = buf[p & 1];
     if (p == 0)
       GQF_LAUNCH_B((double)b.N * 4, k_bs_upsweep<true>, dim3(b.G), dim3(256), 0, s, src, b.d_ch, b.d_flt, shift, b.G,
@@ -569,6 +685,11 @@ static void batch_build_launch(SqfBatch& b) {
       GQF_LAUNCH_B((double)b.N * 8, k_bs_downsweep<false>, dim3(b.G), dim3(256), 0, s, src, dst, b.d_ch, b.d_flt,
                    shift, b.G, b.d_hist, b.d_dbase, b.N);
     src = dst;
+  }
+  if (b.ngroups) {
+    GQF_LAUNCH_B((double)b.N * 8, k_bs_groups, dim3(b.ngroups), dim3(SEG_THREADS), 0, s, buf[0], b.d_grp, b.d_flt,
+                 b.d_dbase, b.d_big);
+    GQF_LAUNCH(k_bs_big, dim3(256), dim3(256), 0, s, buf[0], buf[1], b.d_grp, b.d_flt, b.d_dbase, b.d_big, b.N);
   }
   const uint32_t* A = src;
   if (b.no_dup)
@@ -762,6 +883,19 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   }
   b->nsub = (uint32_t)tl.size();
   b->npass = (maxbits + 7) / 8;
+  // groups of the top-digit form: about 4096 keys each
+  std::vector<BGroup> grp;
+  bool groups = b->npass >= 3;
+  for (int f = 0; f < count; ++f) {
+    const BFilter& x = hf[(size_t)f];
+    groups = groups && x.nkeys <= 256 * SEG_GROUP_AVG;
+    uint32_t gb = 0;
+    while (gb < 8 && x.nkeys > (4096u << gb)) ++gb;
+    const uint32_t span = 256u >> gb, bits = x.bits & 0xFFu, low = bits > 8 ? bits - 8 : 0u;
+    for (uint32_t d = 0; x.nkeys && d < 256; d += span)
+      grp.push_back({(uint32_t)f, d, d + span, std::min(low + 8 - gb, 32u)});
+  }
+  if (groups) b->ngroups = (uint32_t)grp.size();
   std::vector<BChunk> ch;
   std::vector<uint32_t> fchunk;
   b->gmax = std::max<uint32_t>(batch_chunks(*b, 1, ch, fchunk), 1);
@@ -778,8 +912,8 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
                o_dbase = take((size_t)4 * 256 * count), o_k0 = take((size_t)4 * b->N), o_k1 = take((size_t)4 * b->N),
                o_agg = take((size_t)16 * b->nsub), o_fix = take((size_t)4 * RB_FIX * b->nsub),
                o_fixcnt = take((size_t)4 * b->nsub), o_more = take((size_t)4 * ((size_t)b->N + count)),
-               o_state = take((size_t)4 * 3 * count), o_woff = take(4 * ((size_t)count + 1)),
-               o_idx = take((size_t)8 * nidx);
+               o_state = take((size_t)4 * (3 * (size_t)count + 1 + b->ngroups)), o_woff = take(4 * ((size_t)count + 1)),
+               o_idx = take((size_t)8 * nidx), o_grp = take(sizeof(BGroup) * b->ngroups);
   GQF_HIP(hipMalloc((void**)&b->mem, off));
   char* m = b->mem;
   b->d_flt = reinterpret_cast<BFilter*>(m + o_flt);
@@ -796,7 +930,9 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   b->d_fix = reinterpret_cast<uint32_t*>(m + o_fix);
   b->d_fixcnt = reinterpret_cast<uint32_t*>(m + o_fixcnt);
   b->d_more = reinterpret_cast<uint32_t*>(m + o_more);
+  b->d_grp = reinterpret_cast<BGroup*>(m + o_grp);
   b->d_ferr = reinterpret_cast<uint32_t*>(m + o_state);
+  b->d_big = b->d_ferr + 3 * (size_t)count;
   b->d_fend = b->d_ferr + count;
   b->d_moren = b->d_fend + count;
   b->d_woff = reinterpret_cast<uint32_t*>(m + o_woff);
@@ -805,6 +941,8 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   std::vector<uint32_t> poff32((size_t)count + 1);
   for (int f = 0; f <= count; ++f) poff32[(size_t)f] = (uint32_t)b->poff[(size_t)f];
   GQF_HIP(hipMemcpyAsync(b->d_flt, hf.data(), hf.size() * sizeof(BFilter), hipMemcpyHostToDevice, b->stream));
+  if (b->ngroups)
+    GQF_HIP(hipMemcpyAsync(b->d_grp, grp.data(), grp.size() * sizeof(BGroup), hipMemcpyHostToDevice, b->stream));
   if (!tl.empty())
     GQF_HIP(hipMemcpyAsync(b->d_tl, tl.data(), tl.size() * sizeof(BTile), hipMemcpyHostToDevice, b->stream));
   GQF_HIP(hipMemcpyAsync(b->d_poff, poff32.data(), poff32.size() * 4, hipMemcpyHostToDevice, b->stream));

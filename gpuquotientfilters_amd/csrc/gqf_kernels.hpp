@@ -1052,44 +1052,13 @@ __global__ __launch_bounds__(PLACE_THREADS) void k_rs_place(const uint32_t* __re
     }
 }
 
-// One group per workgroup, sorted in place by its bits [0, nbits) (nbits <=
-// 32; the bits above are equal within the group): the keys' top SEG_BB bits
-// of the range pick one of SEG_NBK buckets (LDS counters; the scanned starts
-// then serve as cursors that place every key in its bucket), and every key's
-// place is its bucket's start plus the bucket's smaller keys.  With hashed
-// keys a bucket holds ~3 keys.  A group with a bucket of more than
-// SEG_RANK_MAX keys (many copies of a few keys) takes the 4-bit counting
-// passes instead: in the same workgroup (INLINE: grids of one workgroup per
-// CU, where occupancy does not matter), or appended to `slow` (count, then
-// group ids) for k_rs_seg_slow, which keeps this kernel at 40 registers and
-// four workgroups per CU.  A group above SEG_TILE is never launched here
-// (the host sorts crowded keys with the chunked passes) and is left alone.
-//   regions (k_rs_place; else null): segment g is the gsize[g] keys from g cap
-// on, at most cap, and goes to its place in `keys`; the counters `next` of
-// the stream's next such sort are cleared.
+// The m keys (1 .. SEG_TILE) at `from`, alike above bit nbits, to `seg` (or in
+// place) in order.  False: a crowded bucket, nothing written (not INLINE).
 template <typename K, bool INLINE>
-__global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, const uint32_t* __restrict__ digit_totals,
-                                                        const uint32_t* __restrict__ gstart,
-                                                        const uint32_t* __restrict__ gsize, uint32_t nbits,
-                                                        uint32_t* __restrict__ slow, const K* __restrict__ regions,
-                                                        uint32_t cap, uint32_t* __restrict__ next) {
-  constexpr int T = SEG_THREADS, W = T / 64;
-  __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
-  __shared__ __align__(16) uint16_t s_cnt[INLINE ? 16 * T : 8];  // the counting passes' count table
-  __shared__ __align__(16) uint32_t s_c[SEG_NBK / 2];  // bucket counters / cursors, 16 bits each
-  __shared__ uint32_t s_tmp[W];
-  __shared__ uint32_t s_seg[2];
+__device__ __forceinline__ bool seg_bucket_sort(K* seg, const K* from, uint32_t m, uint32_t nbits, uint32_t* s_keys,
+                                                uint16_t* s_cnt, uint32_t* s_c, uint32_t* s_tmp) {
+  constexpr int T = SEG_THREADS;
   const uint32_t tid = threadIdx.x;
-  uint32_t c0, m;
-  seg_group<T>(blockIdx.x, digit_totals, gstart, gsize, &c0, &m, s_tmp, s_seg);
-  if (INLINE && regions) {
-    if (blockIdx.x == 0 && tid < PLACE_WORDS) next[tid] = 0u;
-    if (m > cap) return;  // the host sorts these keys otherwise
-  }
-  const bool moved = INLINE && regions;
-  if ((m <= 1 && !moved) || m == 0 || m > (uint32_t)SEG_TILE) return;  // the whole workgroup
-  K* seg = keys + c0;
-  const K* from = moved ? regions + (size_t)blockIdx.x * cap : seg;
   const uint32_t lmask = nbits >= 32 ? 0xFFFFFFFFu : (1u << nbits) - 1u;
   const uint32_t i0 = tid * SORT_ITEMS;
   const uint32_t nreal = m > i0 ? (m - i0 < SORT_ITEMS ? m - i0 : SORT_ITEMS) : 0u;
@@ -1145,13 +1114,13 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, co
 #pragma unroll
     for (uint32_t i = 0; i < PT / 4; ++i) c4[i] = make_uint4(st[4 * i], st[4 * i + 1], st[4 * i + 2], st[4 * i + 3]);
     if (__syncthreads_or(mx > SEG_RANK_MAX)) {  // also orders the bucket starts
-      if (moved) {
+      if (!INLINE) return false;
+      if (seg != from) {
         for (uint32_t i = tid; i < m; i += T) seg[i] = from[i];
         __syncthreads();
       }
-      if (INLINE) seg_counting_sort<K, T>(seg, m, nbits, s_keys, s_cnt, s_tmp);
-      else if (tid == 0) slow[1 + atomicAdd(&slow[0], 1u)] = blockIdx.x;
-      return;
+      seg_counting_sort<K, T>(seg, m, nbits, s_keys, s_cnt, s_tmp);
+      return true;
     }
   }
 #pragma unroll
@@ -1174,6 +1143,49 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, co
     }
     seg[rank] = high | (K)x;  // within the group's lines: merged in L2
   }
+  return true;
+}
+
+// One group per workgroup, sorted in place by its bits [0, nbits) (nbits <=
+// 32; the bits above are equal within the group): the keys' top SEG_BB bits
+// of the range pick one of SEG_NBK buckets (LDS counters; the scanned starts
+// then serve as cursors that place every key in its bucket), and every key's
+// place is its bucket's start plus the bucket's smaller keys.  With hashed
+// keys a bucket holds ~3 keys.  A group with a bucket of more than
+// SEG_RANK_MAX keys (many copies of a few keys) takes the 4-bit counting
+// passes instead: in the same workgroup (INLINE: grids of one workgroup per
+// CU, where occupancy does not matter), or appended to `slow` (count, then
+// group ids) for k_rs_seg_slow, which keeps this kernel at 40 registers and
+// four workgroups per CU.  A group above SEG_TILE is never launched here
+// (the host sorts crowded keys with the chunked passes) and is left alone.
+//   regions (k_rs_place; else null): segment g is the gsize[g] keys from g cap
+// on, at most cap, and goes to its place in `keys`; the counters `next` of
+// the stream's next such sort are cleared.
+template <typename K, bool INLINE>
+__global__ __launch_bounds__(SEG_THREADS) void k_rs_seg(K* __restrict__ keys, const uint32_t* __restrict__ digit_totals,
+                                                        const uint32_t* __restrict__ gstart,
+                                                        const uint32_t* __restrict__ gsize, uint32_t nbits,
+                                                        uint32_t* __restrict__ slow, const K* __restrict__ regions,
+                                                        uint32_t cap, uint32_t* __restrict__ next) {
+  constexpr int T = SEG_THREADS, W = T / 64;
+  __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
+  __shared__ __align__(16) uint16_t s_cnt[INLINE ? 16 * T : 8];  // the counting passes' count table
+  __shared__ __align__(16) uint32_t s_c[SEG_NBK / 2];  // bucket counters / cursors, 16 bits each
+  __shared__ uint32_t s_tmp[W];
+  __shared__ uint32_t s_seg[2];
+  const uint32_t tid = threadIdx.x;
+  uint32_t c0, m;
+  seg_group<T>(blockIdx.x, digit_totals, gstart, gsize, &c0, &m, s_tmp, s_seg);
+  if (INLINE && regions) {
+    if (blockIdx.x == 0 && tid < PLACE_WORDS) next[tid] = 0u;
+    if (m > cap) return;  // the host sorts these keys otherwise
+  }
+  const bool moved = INLINE && regions;
+  if ((m <= 1 && !moved) || m == 0 || m > (uint32_t)SEG_TILE) return;  // the whole workgroup
+  K* seg = keys + c0;
+  const K* from = moved ? regions + (size_t)blockIdx.x * cap : seg;
+  if (!seg_bucket_sort<K, INLINE>(seg, from, m, nbits, s_keys, s_cnt, s_c, s_tmp) && tid == 0)
+    slow[1 + atomicAdd(&slow[0], 1u)] = blockIdx.x;
 }
 
 // The groups k_rs_seg left (slow[0] of them, ids after it): the 4-bit

@@ -103,7 +103,7 @@ __host__ __device__ __forceinline__ uint32_t sqf_get_packed(const uint32_t* __re
 // Wide table -> packed words, 32 slots (`width` words) per thread.  With ctr,
 // nothing is written when the call's capacity or hand-over flag is set (the
 // wide table then holds no result).  A word per thread, its slots found by
-// division, took 10 us for 4.6 M slots of 12 bits; this, 6 us
+// division, took 10 us for 4.6 M slots of 12 bits; this, 6.
 [[maybe_unused]] static __global__ __launch_bounds__(64) void k_sqf_pack(const uint16_t* __restrict__ wide, uint32_t S,
                                                                        uint32_t width, uint32_t* __restrict__ packed,
                                                                        uint32_t nwords, const uint32_t* __restrict__ ctr) {
