@@ -59,8 +59,8 @@ struct BTile {
 // Batches whose filters have up to 256 * SEG_GROUP_AVG keys take one pass on
 // every filter's own top 8 bits (BS_TOP) and then sort groups of neighbouring
 // digits, about 4096 keys each, in LDS: two reads and writes of the keys
-// instead of one per 8 bits.  48 filters of q = 12 .. 20, 6 M keys: 94 us, four
-// passes 200.
+// instead of one per 8 bits (the autotuner times both).  48 filters of q = 12
+// .. 20, 6 M keys: 94 us, four passes 200.
 constexpr uint32_t BS_TOP = 0xFFFFFFFFu;
 __device__ __forceinline__ uint32_t bs_shift(uint32_t shift, uint32_t bits) {
   const uint32_t b = bits & 0xFFu;
@@ -951,6 +951,17 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   // autotune the sort chunk size on the build (the tables are rebuilt from
   // the batch keys each time: the last run leaves them built)
   const int pers[4] = {1, 2, 4, 8};
+  // groups or 8-bit passes: keys with many copies of a few (Zipf ranks) leave
+  // groups that one workgroup each has to sort
+  if (b->ngroups) {
+    const uint32_t ng = b->ngroups;
+    float tg = 0.f, tp = 0.f;
+    GQF_TRY(batch_upload_chunks(*b, 1));
+    GQF_TRY(time_on_stream(*b, batch_build_launch, 2, &tg));
+    b->ngroups = 0;
+    GQF_TRY(time_on_stream(*b, batch_build_launch, 2, &tp));
+    if (tg <= tp) b->ngroups = ng;
+  }
   float best = 1e30f;
   int best_per = 1;
   for (int per : pers) {
