@@ -17,7 +17,7 @@
 // key costs one LDS atomic, two reads and one byte store after the partition,
 // and what remains is a byte per quotient and one per key.  Fingerprints of
 // 33 and 34 bits are partitioned as their low words.  53.7 M keys into 2^26
-// quotients: SQF (r = 5, NoDup) 790 -> 505 us, RSQF (r = 8) 1380 -> 475 us.
+// quotients: SQF (r = 5, NoDup) 790 -> 474 us, RSQF (r = 8) 1380 -> 470 us.
 //   Groups of more keys than they have room for, runs past 255 entries (hot
 // keys), more than 255 keys in 32 neighbouring quotients and spills past 512
 // slots raise ctr[CTR_MISC] before the table is written, and the call takes
@@ -311,7 +311,7 @@ constexpr uint32_t DB_LIST = 128;  // listed runs per wave
 // per run (up to 8 entries in registers, longer runs in a loop).  Repeats
 // (UNIQUE) are dropped from the bytes at the end.
 //   A thread sorting its own 32 quotients' runs in place costs its wave the
-// longest run at every quotient: 342 us for 53.7 M keys; this: 225 us, 155 us
+// longest run at every quotient: 342 us for 53.7 M keys; this: 201 us, 151 us
 // with repeats kept.  Bound by instructions and LDS accesses in about equal
 // parts (rank, placing and sorting 15, 15 and 25% of the time).
 template <bool UNIQUE>
@@ -423,19 +423,24 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   // for theirs)
   RS a = rs_none();
   {
-    uint32_t o[DB_Q / 4], n = sum;  // kept entries before each quotient, of the thread
-    {
+    uint32_t n = sum;
+    uint32_t last = 0;  // the last occupied quotient: the last whose count is not 0
+    auto offsets = [&](uint32_t (&o)[DB_Q / 4]) {
       const uint4 x = c4[2 * t], y = c4[2 * t + 1];
       o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w, o[4] = y.x, o[5] = y.y, o[6] = y.z, o[7] = y.w;
-    }
-    uint32_t last = 0;  // the last occupied quotient: the last whose count is not 0
+    };
+    {
+      uint32_t o[DB_Q / 4];
+      offsets(o);
 #pragma unroll
-    for (uint32_t w = 0; w < DB_Q / 4; ++w) {
-      const uint32_t c = ((o[w] >> 8) | ((w + 1 < DB_Q / 4 ? o[w + 1] : sum) << 24)) - o[w];
-      if (c) last = 4 * w + ((31u - (uint32_t)__builtin_clz(c)) >> 3);
+      for (uint32_t w = 0; w < DB_Q / 4; ++w) {
+        const uint32_t c = ((o[w] >> 8) | ((w + 1 < DB_Q / 4 ? o[w + 1] : sum) << 24)) - o[w];
+        if (c) last = 4 * w + ((31u - (uint32_t)__builtin_clz(c)) >> 3);
+      }
     }
     if (UNIQUE) {
-      // the offsets past every repeat fall by one
+      // the offsets past every repeat fall by one (in LDS: a loop over them in
+      // registers spilled 26, 330 MB of scratch at 53.7 M keys)
       for (uint32_t z0 = first & ~31u; z0 < first + sum; z0 += 32) {
         uint32_t lost = ~s_keep[z0 >> 5];
         if (z0 < first) lost &= ~0u << (first - z0);
@@ -443,17 +448,22 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
         for (; lost; lost &= lost - 1u) {
           const uint32_t z = z0 + (uint32_t)__builtin_ctz(lost) - first - (sum - n);  // its place among the kept so far
           const uint32_t s = z * 0x01010101u;
-#pragma unroll
-          for (uint32_t w = 0; w < DB_Q / 4; ++w) {
-            // bytes of o above z
-            const uint32_t lo = (o[w] | 0x80808080u) - (s & 0x7F7F7F7Fu) - 0x01010101u;  // top bits: low 7 bits of o > those of s
-            const uint32_t gt = ((o[w] & ~s) | (~(o[w] ^ s) & lo)) & 0x80808080u;
-            o[w] -= gt >> 7;
+          // bytes of x above z
+          auto fall = [&](uint32_t x) {
+            const uint32_t lo = (x | 0x80808080u) - (s & 0x7F7F7F7Fu) - 0x01010101u;  // top bits: low 7 bits of x > those of s
+            return x - ((((x & ~s) | (~(x ^ s) & lo)) & 0x80808080u) >> 7);
+          };
+#pragma unroll 1
+          for (uint32_t h = 2 * t; h < 2 * t + 2; ++h) {
+            const uint4 x = c4[h];
+            c4[h] = make_uint4(fall(x.x), fall(x.y), fall(x.z), fall(x.w));
           }
           --n;
         }
       }
     }
+    uint32_t o[DB_Q / 4];  // kept entries before each quotient, of the thread
+    offsets(o);
     uint32_t kc[DB_Q / 4];
     int32_t mx = -256;
 #pragma unroll
