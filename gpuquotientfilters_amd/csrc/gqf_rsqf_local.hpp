@@ -19,7 +19,10 @@
 
 namespace gqf {
 
-constexpr uint32_t RL_HALO = 48;  // blocks of the next window that a region may reach
+// Blocks of the next window that a region may reach.  45: 10,204 bytes of LDS
+// per deleting wave, 16 of them per CU (48: 15; steps of 2^18 keys 339 us, now
+// 330).
+constexpr uint32_t RL_HALO = 45;
 constexpr uint32_t RL_BLOCKS = 64 + RL_HALO;
 constexpr uint32_t RL_E_BITS = 13;  // a key's word: E_k or the head bit, D above
 

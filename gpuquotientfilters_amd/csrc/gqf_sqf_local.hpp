@@ -207,14 +207,14 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
 // remainders: a lane changes bits of its own region only, by xor.  Slots are
 // relative to the window.
 //   One wave per window: a batch of 1/64 of the slots has a region for most
-// lanes, and 8 KB of LDS leave room for 19 waves per CU.  The time is the
+// lanes, and 8 KB of LDS leave room for 21 waves per CU.  The time is the
 // wave's longest region (dependent LDS reads) times the waves per CU: 2^20
 // keys into q=26 r=5 at fill 0.75 take 77 us, 559 us when the lanes walked
 // element bytes one by one (1.9 and 0.26 TB/s of table bytes read and
 // written); the rebuild's decode, state and write passes take 250 us.  As
 // many deletes take 104 us, 160 when every run start that moves was paired
 // with its quotient one by one; decode, mark and rebuild take 290 us.
-constexpr uint32_t SL_HALO = 16;
+constexpr uint32_t SL_HALO = 11;  // 7.6 KB of LDS, 21 waves per CU (16: 8.1 KB; 2^20-key steps 309 us, now 300)
 constexpr uint32_t SL_BLOCKS = 64 + SL_HALO;
 
 __host__ __device__ __forceinline__ void lds_xor(unsigned long long* p, uint64_t d) {
