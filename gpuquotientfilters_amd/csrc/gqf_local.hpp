@@ -120,7 +120,8 @@ __device__ __forceinline__ void lw_raise(uint32_t* ctr, uint32_t* report) {
   __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // Stores window w's prefix; whether it or (the last window) the end is bad.
-__device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t W, uint2* __restrict__ pre, uint32_t min_heads) {
+__host__ __device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t W, uint2* __restrict__ pre,
+                                                uint32_t min_heads) {
   const int32_t o = p.a > p.b ? p.a : p.b;  // the map of the windows before, at 0
   pre[w] = make_uint2(o > 0 ? (uint32_t)o : 0u, p.lb);
   if (w + 1 < W) return o > LW_SPILL;

@@ -26,6 +26,15 @@ constexpr uint32_t RL_HALO = 45;
 constexpr uint32_t RL_BLOCKS = 64 + RL_HALO;
 constexpr uint32_t RL_E_BITS = 13;  // a key's word: E_k or the head bit, D above
 
+// Whether a region that overflows into a window ends in the blocks held of it
+// (`room` empty slots there): it takes a slot for each of the at most LW_SPILL
+// keys of the windows before and for each of the window's keys that it takes
+// with it -- those before the first with E_k - k >= LW_SPILL, at most
+// (`chained`: the first with E_k - k >= the overflow starts a region).
+__host__ __device__ __forceinline__ bool rl_holds(uint32_t chained, uint32_t room) {
+  return (uint32_t)LW_SPILL + chained <= room;
+}
+
 __host__ __device__ __forceinline__ void rl_xor(unsigned long long* p, uint64_t d) {
 #ifdef __HIP_DEVICE_COMPILE__
   if (d) atomicXor(p, (unsigned long long)d);
@@ -122,7 +131,7 @@ struct RlPlanes {
         y = p;
       }
     }
-    if (p > e || y > e || e >= end) return;  // not reached
+    if (p > e || y > e || e >= end) return;  // not reached: the region is held
     if (!stored) rl_xor(&occ[fw], 1ull << (fq & 63));
     // run ends of [y, e]: those of [y, e) move up by one; slot y ends a run
     // iff the quotient is new
@@ -332,15 +341,16 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
   if (blk >= nb) mask = 0;
   s_mask[lane] = mask;
   uint32_t e = 0, first = LW_SLOTS, last = 0;
+  uint32_t room = ~0u, chained = nk;  // insert: what a region that overflows into the window finds, and takes
   bool bad = nk > LW_KEYS;
   if (INS) {
     if (blk < nb) empty[blk] = mask;
     const uint32_t c = (uint32_t)__popcll(mask), inc = wave_incl_add(c);
     s_pre[lane] = inc - c;
     e = wave_read(inc, 63);
-    // what overflows into the window must find room in the blocks a region
-    // may reach
-    if (w + 1 < W) bad = bad || e < (uint32_t)LW_SPILL || (after && wave_read(inc, RL_HALO - 1) < (uint32_t)LW_SPILL);
+    if (w + 1 < W) bad = bad || e < (uint32_t)LW_SPILL;
+    // (a last window of fewer blocks is held whole)
+    if (after && nb > w * 64 + RL_HALO) room = wave_read(inc, RL_HALO - 1);
   } else {
     const uint32_t own = mask ? 64 * lane + 64 - (uint32_t)__clzll(mask) : 0u;
     const uint32_t inc = wave_incl_max(own);
@@ -372,7 +382,10 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       uint32_t info;
       if (INS) {
         info = s_pre[bk] + (uint32_t)__popcll(m & below);
-        head = lw_insert_head((int32_t)info - (int32_t)k, on, M);
+        const int32_t v = (int32_t)info - (int32_t)k;
+        head = lw_insert_head(v, on, M);
+        const uint64_t past = __ballot(on && v >= LW_SPILL);
+        if (past && chained == nk) chained = k0 + (uint32_t)__builtin_ctzll(past);
       } else {
         const uint64_t at = m & (below | (1ull << (rel & 63u)));
         const uint32_t lb = at ? 64 * bk + 64 - (uint32_t)__clzll(at) : s_pre[bk];
@@ -388,7 +401,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       if (k0 + 64 <= nk && hm == 0) bad = true;
     }
   }
-  bad = __any(bad);
+  bad = __any(bad || (INS && !rl_holds(chained, room)));
   if (lane == 0) {
     const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
     int32_t b = INS && nk ? M + a : 0;
@@ -479,7 +492,7 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
       for (; need > 1; --need) em &= em - 1ull;
       for (;;) {  // the empty slot that the region's last key takes
         while (em == 0 && c + 1 < nb && c + 1 < bw + RL_BLOCKS) em = empty[++c];
-        if (em == 0) break;  // not reached: the plan found room
+        if (em == 0) break;  // not reached: the plan found room (rl_holds)
         hi = 64 * (c - bw) + (uint32_t)__builtin_ctzll(em);
         em &= em - 1ull;
         if (k1 >= n || (uint32_t)(B[k1] >> rr) > base + hi) break;
@@ -523,7 +536,7 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
     for (uint32_t k = ka; k < kb; ++k) {
       const uint32_t x = (uint32_t)(B[k] - kbase);
       const uint32_t fq = (uint32_t)((B[k] - kbase) >> rr);
-      if (fq >= m.end) break;  // not reached
+      if (fq >= m.end) break;  // not reached: hi covers the region's keys
       if (INS) {
         e = m.next(s_empty, e + 1);
         m.insert(fq, x & rmask, a, D, e);

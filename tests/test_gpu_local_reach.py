@@ -1,0 +1,96 @@
+"""Localized inserts whose region runs from one window into the next: up to 64
+keys that the first has no room for, and the keys of the second that it takes
+with it, where the second has few empty slots in its first blocks.  Every key
+has to be there, wherever the call's rules draw the line."""
+import numpy as np
+import pytest
+
+import gpuquotientfilters_amd as G
+import oracle as O
+from gpu_helpers import dev, require_gpu, say
+from test_gpu_local import _kernels, insert_set, rsqf_equal, rsqf_table, sqf_equal, sqf_table
+
+pytestmark = pytest.mark.gpu
+
+Q, W0 = 20, 5 * 4096  # more windows than batch keys; the window that overflows
+HALO = 45 * 64        # slots of the next window that a region may reach (RSQF)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    require_gpu()
+
+
+def key_of_quotient(q, r, lo, hi):
+    """A key for every quotient of [lo, hi)."""
+    keys = O.mt19937(7, 1 << 24)
+    fq = (O.fingerprints(keys, q, r) >> np.uint64(r)).astype(np.int64)
+    sel = np.flatnonzero((fq >= lo) & (fq < hi))
+    u, first = np.unique(fq[sel], return_index=True)
+    assert len(u) == hi - lo
+    return keys[sel[first]]
+
+
+def crowded(r, empties, x, c):
+    """Stored keys and a batch: slot W0 + 4095 and, in the next window's first
+    HALO slots, all but `empties` are taken; x copies of the former's key and c
+    keys past the 22nd of those empty slots."""
+    lo, nxt = W0 + 4095, W0 + 4096
+    key = key_of_quotient(Q, r, lo, nxt + HALO)
+    s = np.arange(HALO)
+    gap = HALO // empties
+    stored = np.concatenate([key[:1], key[1:][(s % gap != 0) | (s // gap >= empties)]])
+    batch = np.concatenate([np.repeat(key[:1], x), key[1 + 1000:1 + 1000 + 40 * c:40]])
+    return stored, batch
+
+
+@pytest.mark.parametrize("x,c", [(64, 0), (63, 1), (63, 2), (64, 1), (64, 7), (60, 20), (65, 1), (40, 3)])
+@pytest.mark.parametrize("empties", [64, 72])
+def test_rsqf_insert_across_a_window(x, c, empties):
+    r = 8
+    say("rsqf insert across a window", x, c, empties)
+    st = G.Stream()
+    stored, batch = crowded(r, empties, x, c)
+    f = G.RSQF(Q, r)
+    f.bulk_build(dev(stored))
+    names = _kernels(lambda: f.insert(dev(batch), stream=st))
+    fps = np.concatenate([O.fingerprints(stored, Q, r), O.fingerprints(batch, Q, r)])
+    rsqf_equal(f, rsqf_table(fps, Q, r))
+    if x <= 64 and 64 + c <= empties:  # there is room for the most that can come: no other form is needed
+        assert any("k_rl_apply" in k for k in names) and not any("k_wm_write" in k for k in names)
+    # what is left in place after the same keys are deleted again
+    f.deleteGPU(dev(batch), stream=st)
+    left = np.sort(fps)
+    at = np.searchsorted(left, np.sort(O.fingerprints(batch, Q, r)), side="left")
+    keep = np.ones(len(left), bool)
+    for a in at:
+        while not keep[a]:
+            a += 1
+        keep[a] = False
+    rsqf_equal(f, rsqf_table(left[keep], Q, r))
+    st.destroy()
+
+
+@pytest.mark.parametrize("x,c", [(64, 0), (63, 2), (64, 20), (30, 20)])
+def test_sqf_insert_across_a_window(x, c):
+    """The SQF stores a fingerprint once: x different remainders at the quotient."""
+    r = 8  # packed slots
+    say("sqf insert across a window", x, c)
+    st = G.Stream()
+    keys = O.mt19937(9, 1 << 24)
+    fp = O.fingerprints(keys, Q, r)
+    fq = (fp >> np.uint64(r)).astype(np.int64)
+    lo = W0 + 4095
+    sel = np.flatnonzero((fq >= lo) & (fq < lo + 1 + HALO))
+    _, first = np.unique(fq[sel], return_index=True)
+    key = keys[sel[first]]
+    near = np.flatnonzero((fq > lo - 30) & (fq <= lo))  # about 16 keys a quotient
+    s = np.arange(HALO)
+    stored = np.concatenate([keys[near[-40:]], key[1:][(s % 45 != 0) | (s // 45 >= 64)]])
+    batch = np.concatenate([keys[near[:x]], key[1 + 1000:1 + 1000 + 40 * c:40]])
+    f = G.SQF(Q, r)
+    f.bulk_build(dev(stored))
+    f.insert(dev(batch), stream=st)
+    fps = np.unique(insert_set(np.unique(O.fingerprints(stored, Q, r)), O.fingerprints(batch, Q, r)))
+    sqf_equal(f, sqf_table(fps, Q, r))
+    st.destroy()

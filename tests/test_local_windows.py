@@ -1,0 +1,23 @@
+"""The RSQF's localized updates, window by window, on the CPU: what the plan
+accepts fits the blocks that a wave holds (tests/plan/window_check.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_accepted_batches_stay_in_the_blocks_held(tmp_path):
+    exe = str(tmp_path / "window_check")
+    src = os.path.join(ROOT, "tests", "plan", "window_check.cpp")
+    cmd = [HIPCC, "--cuda-host-only", "-std=c++17", "-O1", "-Xclang", "-target-feature", "-Xclang",
+           "-packed-fp32-ops", src, "-o", exe]
+    p = subprocess.run(cmd, capture_output=True, text=True)
+    assert p.returncode == 0, p.stderr[-2000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "windows ok" in r.stdout, r.stdout[-2000:]
