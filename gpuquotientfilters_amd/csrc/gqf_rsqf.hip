@@ -206,11 +206,13 @@ __global__ __launch_bounds__(256) void k_rsqf_count(RsqfDev f, uint32_t q, const
                                (uint32_t)(fp & ((1u << f.r) - 1u)));
 }
 
-template <int R>
-__global__ __launch_bounds__(256) void k_rsqf_lookup(RsqfDev f, uint32_t q, const uint32_t* __restrict__ keys,
-                                                     uint32_t n, uint32_t* __restrict__ out) {
+// GATED: the answers of an insert, left out where its batch was handed over
+// (ctr[CTR_MISC]): out may be keys, which the next form still needs.
+template <int R, bool GATED>
+__global__ __launch_bounds__(256) void k_rsqf_lookup(RsqfDev f, uint32_t q, const uint32_t* keys, uint32_t n, uint32_t* out,
+                                                     const uint32_t* __restrict__ ctr) {
   const uint64_t i = blockIdx.x * 256ull + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || (GATED && ctr[CTR_MISC])) return;
   const uint64_t fp = fingerprint(keys[i], q + f.r);
   out[i] = rsqf_lookup_one<R>(f, (uint32_t)((fp >> f.r) & mask64(q)), (uint32_t)(fp & ((1u << f.r) - 1u)));
 }
@@ -1812,7 +1814,8 @@ static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gq
 
 // The in-place inserts: localized where the batch is small (local; *done:
 // the call has ended), else window by window.  d_out: the keys' slots.
-static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out);
+static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out,
+                           const uint32_t* gate = nullptr);
 template <typename K>
 static gqf_status rsqf_insert_win_t(const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* d_out, CallScope& cs,
                                     bool local, bool* done, float* ms) {
@@ -1827,7 +1830,7 @@ static gqf_status rsqf_insert_win_t(const gqf_rsqf& f, uint32_t n, const uint32_
   if (local) {
     const size_t mark = ar.used;
     GQF_TRY((rsqf_local<K, true>(cs.stream, ds, ar, f, B, n)));
-    if (d_out) launch_rlookup(cs.stream, f, n, keys, d_out);
+    if (d_out) launch_rlookup(cs.stream, f, n, keys, d_out, ds.counters);
     GQF_TRY(cs.end(ms, false));
     *done = lw_done(ds);
     lw_report(ds, LOCAL_RSQF_INSERT, *done);
@@ -2024,11 +2027,18 @@ static gqf_status rsqf_pl_lookup(hipStream_t s, DeviceState& ds, const gqf_rsqf&
   return pl_lookup<false>(s, ds, pl, keys, bits, n, out, RsqfWalk{d, f.qbits}, walks);
 }
 
-static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out) {
+// gate: the stream's counters, where the call's form may have handed the batch over.
+static void launch_rlookup(hipStream_t s, const gqf_rsqf& f, uint32_t n, const uint32_t* keys, uint32_t* out,
+                           const uint32_t* gate) {
   const RsqfDev d = rdev(f);
   const dim3 grid((n + 255) / 256);
-  if (f.rbits == 8) GQF_LAUNCH_B((double)n * (8 + 128), k_rsqf_lookup<8>, grid, dim3(256), 0, s, d, f.qbits, keys, n, out);
-  else GQF_LAUNCH_B((double)n * (8 + 128), k_rsqf_lookup<0>, grid, dim3(256), 0, s, d, f.qbits, keys, n, out);
+  const double b = (double)n * (8 + 128);
+#define GQF_RLOOKUP(R_, G_) GQF_LAUNCH_B(b, (k_rsqf_lookup<R_, G_>), grid, dim3(256), 0, s, d, f.qbits, keys, n, out, gate)
+  if (f.rbits == 8 && gate) GQF_RLOOKUP(8, true);
+  else if (f.rbits == 8) GQF_RLOOKUP(8, false);
+  else if (gate) GQF_RLOOKUP(0, true);
+  else GQF_RLOOKUP(0, false);
+#undef GQF_RLOOKUP
 }
 
 gqf_status rsqf_lookup_call(const gqf_rsqf& f, int n, const uint32_t* d_keys, int32_t* d_out, gqf_stream stream,
@@ -2128,7 +2138,7 @@ static gqf_status rsqf_insert_call(gqf_rsqf cqf, int n, const uint32_t* d_keys, 
       if (lp_end) *lp_end = 0;  // read only when a batch does not fit
       return GQF_OK;
     }
-    if (d_out) launch_rlookup(cs.stream, cqf, (uint32_t)n, d_keys, out);
+    if (d_out) launch_rlookup(cs.stream, cqf, (uint32_t)n, d_keys, out, cs.ds->counters);
     const gqf_status st = cs.end(&ms_win, true);
     if (st != GQF_OK && st != GQF_ERR_CAPACITY) return st;
     // a window the windowed path cannot take: nothing was written, rebuild
