@@ -303,9 +303,11 @@ static gqf_status sqf_merge_into(CallScope& cs, Arena& ar, const gqf_sqf& qf, co
 }
 
 // Localized inserts and deletes: tables of 1- and 2-byte slots (packed widths
-// are worked on as 2-byte ones) on a 16-byte boundary.
+// are worked on as 2-byte ones) on a 4-byte boundary (their 16-byte loads and
+// stores need no more).  A table 4 bytes off a 16-byte boundary, q=26 r=5 at
+// fill 0.7, 10 / 60000 keys: 350 / 382 us by the rebuild, 36 / 73 localized.
 static bool sqf_local_fits(const gqf_sqf& wq, const SqfGeom& g) {
-  return g.bpe <= 2 && lw_windows(g.S) <= LW_MAX_WINDOWS && (g.packed || (reinterpret_cast<uintptr_t>(wq.table) & 15u) == 0);
+  return g.bpe <= 2 && lw_windows(g.S) <= LW_MAX_WINDOWS && (g.packed || (reinterpret_cast<uintptr_t>(wq.table) & 3u) == 0);
 }
 static size_t sqf_local_bytes(const SqfGeom& g, uint32_t n) {
   const uint32_t W = lw_windows(g.S);

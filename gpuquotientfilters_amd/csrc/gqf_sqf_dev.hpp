@@ -243,10 +243,12 @@ template <int BPE>
 __host__ __device__ __forceinline__ void sqf_win_load(const uint8_t* __restrict__ t, uint32_t S, uint32_t w, SqfWin<BPE>& W) {
   const uint64_t s0 = (uint64_t)w * 64;
   if (s0 + 64 <= S) {
-    const uint4* p = reinterpret_cast<const uint4*>(t + s0 * BPE);
+    // (memcpy: multi-dword loads need dword alignment only)
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(t + s0 * BPE);
 #pragma unroll
     for (int k = 0; k < 4 * BPE; ++k) {
-      const uint4 x = p[k];
+      uint4 x;
+      __builtin_memcpy(&x, p + 4 * k, 16);
       W.raw[4 * k] = x.x;
       W.raw[4 * k + 1] = x.y;
       W.raw[4 * k + 2] = x.z;

@@ -650,7 +650,7 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
     if (s >= lo && s + 15 <= last) {
 #pragma unroll
       for (int k = 0; k < BPE; ++k)
-        reinterpret_cast<uint4*>(d)[k] = make_uint4(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]);
+        st16_dw(reinterpret_cast<uint32_t*>(d) + 4 * k, make_uint4(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]));
     } else {
 #pragma unroll
       for (uint32_t j = 0; j < 16 * BPE; ++j) {
