@@ -43,6 +43,7 @@ struct Scheduler {
   enum State : char { IDLE = 0, RUNNING = 1, TRIMMING = 2 };
   std::vector<char> state;                    // per worker
   std::vector<size_t> held;                   // bytes each worker holds
+  std::vector<size_t> left;                   // bytes its last release left: no release gives these back
   int running = 0;   // calls in flight
   int trimming = 0;  // workers being released
   bool closing = false;
@@ -86,11 +87,11 @@ struct Scheduler {
       // with what its workers held at the end of another)
       int v = -1;
       for (int i = 0; i < nworkers; ++i)
-        if (i != w && state[(size_t)i] == IDLE && held[(size_t)i] > 0) {
+        if (i != w && state[(size_t)i] == IDLE && held[(size_t)i] > left[(size_t)i]) {
           v = i;
           break;
         }
-      if (v < 0 && running == 0 && trimming == 0 && held[(size_t)w] > 0) v = w;
+      if (v < 0 && running == 0 && trimming == 0 && held[(size_t)w] > left[(size_t)w]) v = w;
       if (v >= 0) {
         state[(size_t)v] = TRIMMING;
         trimming++;
@@ -98,7 +99,7 @@ struct Scheduler {
         ex.trim(ex.user, v);
         const size_t h = ex.held_bytes(ex.user, v);
         lk.lock();
-        held[(size_t)v] = h;
+        held[(size_t)v] = left[(size_t)v] = h;
         state[(size_t)v] = IDLE;
         trimming--;
         cv.notify_all();
@@ -176,6 +177,7 @@ struct Scheduler {
     q.assign((size_t)nworkers, {});
     state.assign((size_t)nworkers, IDLE);
     held.assign((size_t)nworkers, 0);
+    left.assign((size_t)nworkers, 0);
     for (int i = 0; i < nworkers; ++i) held[(size_t)i] = ex.held_bytes(ex.user, i);
     for (int i = 0; i < nreqs; ++i) {
       reqs[i].status = GQF_OK;
