@@ -36,6 +36,7 @@ struct Scheduler {
   gqf_serve_executor ex{};
   int nfilters = 0, nworkers = 0;
   size_t resident = 0;
+  bool roomy = false;  // the executor knows calls with room to spare (coalesced = 2), which no call needs
   uint64_t max_batch = 0;
   std::mutex mu;
   std::condition_variable cv;                 // queue changes and call completions
@@ -74,8 +75,10 @@ struct Scheduler {
         cv.wait(lk);
         continue;
       }
-      const size_t grow = ex.grow_bytes(ex.user, w, b[0]->filter, b[0]->op, n, coalesced ? 1 : 0);
       const size_t u = used();
+      size_t grow = ex.grow_bytes(ex.user, w, b[0]->filter, b[0]->op, n, coalesced ? (roomy ? 2 : 1) : 0);
+      if (coalesced && roomy && u + grow > cfg.hbm_budget)
+        grow = ex.grow_bytes(ex.user, w, b[0]->filter, b[0]->op, n, 1);
       if (u + grow <= cfg.hbm_budget) {
         held[(size_t)w] += grow;
         peak = std::max(peak, u + grow);
@@ -342,19 +345,16 @@ bool mv_overlap(gqf_request** b, int nb) {
 struct RsqfExec {
   const gqf_rsqf* f = nullptr;
   int sorted = 0;
-  bool tight = false;  // the budget leaves no room for more than the calls need
   struct W {
     gqf_stream st = nullptr;
     uint32_t* keys = nullptr;
     int32_t* out = nullptr;
     size_t cap = 0;  // keys the gather buffers hold
+    size_t room = 0;  // keys that the admitted call makes them hold
   };
   std::vector<W> w;
 
   static size_t stage_bytes(size_t cap) { return cap * 8; }
-  // Keys the gather buffers grow to for a call of n (every free waits for the
-  // device, and so for the other workers' calls).
-  size_t stage_room(size_t n) const { return tight ? n : n + n / 2; }
 
   static size_t grow(void* u, int wi, int filter, int op, uint64_t n, int coalesced) {
     RsqfExec& e = *static_cast<RsqfExec*>(u);
@@ -363,7 +363,10 @@ struct RsqfExec {
     size_t have = 0;
     (void)gqf_stream_workspace_bytes(x.st, &have);
     size_t g = need > have ? ws_alloc_bytes(need) - have : 0;
-    if (coalesced && n > x.cap) g += stage_bytes(e.stage_room((size_t)n)) - stage_bytes(x.cap);
+    // gather buffers for half as many keys again where there is room (2):
+    // every free waits for the device, and so for the other workers' calls
+    x.room = coalesced == 2 ? (size_t)(n + n / 2) : (size_t)n;
+    if (coalesced && n > x.cap) g += stage_bytes(x.room) - stage_bytes(x.cap);
     return g;
   }
   static size_t held(void* u, int wi) {
@@ -407,7 +410,7 @@ struct RsqfExec {
     if (n > x.cap) {
       GQF_HIP(hipStreamSynchronize(hs));
       free_stage(x);
-      const size_t cap = stage_room(n);
+      const size_t cap = std::max(x.room, n);
       GQF_HIP(hipMalloc((void**)&x.keys, cap * 4));
       GQF_HIP(hipMalloc((void**)&x.out, cap * 4));
       x.cap = cap;
@@ -550,11 +553,12 @@ gqf_status gqf_rsqf_serve(gqf_rsqf* filters, int nfilters, gqf_request* reqs, in
   RsqfExec e;
   e.f = filters;
   e.sorted = cfg->sorted_lookups;
-  e.tight = cfg->hbm_budget < resident || cfg->hbm_budget - resident < 2 * IDLE_BYTES;
+  // little room: the workers begin with nothing, and take what their calls need
+  const bool tight = cfg->hbm_budget < resident || cfg->hbm_budget - resident < 2 * IDLE_BYTES;
   e.w.resize(cfg->coalesce ? (size_t)nfilters : 1);
   gqf_status st = GQF_OK;
   for (RsqfExec::W& x : e.w)
-    if (st == GQF_OK) st = worker_take(&x, e.tight);
+    if (st == GQF_OK) st = worker_take(&x, tight);
   if (st == GQF_OK) {
     gqf_serve_executor ex{&e, &RsqfExec::grow, &RsqfExec::held, &RsqfExec::trim, &RsqfExec::run};
     Scheduler s;
@@ -562,6 +566,7 @@ gqf_status gqf_rsqf_serve(gqf_rsqf* filters, int nfilters, gqf_request* reqs, in
     s.ex = ex;
     s.nfilters = nfilters;
     s.resident = resident;
+    s.roomy = !tight;
     st = s.run(reqs, nreqs, stats);
   }
   for (RsqfExec::W& x : e.w) {
