@@ -135,8 +135,10 @@ gqf_status ws_reserve(DeviceState& ds, size_t bytes) {
     (void)hipGetLastError();
     e = hipMalloc((void**)&ds.ws, cap);
   }
-  if (e != hipSuccess) ds.ws = nullptr;
-  GQF_HIP(e);
+  if (e != hipSuccess) {
+    ds.ws = nullptr;
+    return hip_fail(e, "hipMalloc of the workspace", __FILE__, __LINE__);
+  }
   ds.ws_cap = cap;
   return GQF_OK;
 }

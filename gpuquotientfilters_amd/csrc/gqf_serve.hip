@@ -382,6 +382,23 @@ struct RsqfExec {
     (void)ws_trim(x.st);
     e.free_stage(x);
   }
+  // Gather buffers for `cap` keys; the idle workers of other runs make room
+  // where the device has none.
+  static gqf_status stage_malloc(W& x, size_t cap) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < 2; ++i) {
+      e = hipMalloc((void**)&x.keys, cap * 4);
+      if (e != hipSuccess) x.keys = nullptr;
+      else if ((e = hipMalloc((void**)&x.out, cap * 4)) != hipSuccess) x.out = nullptr;
+      if (e == hipSuccess) break;
+      (void)hipGetLastError();
+      free_stage(x);
+      if (e != hipErrorOutOfMemory || !serve_release_idle()) break;
+    }
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc of gather buffers", __FILE__, __LINE__);
+    x.cap = cap;
+    return GQF_OK;
+  }
   static void free_stage(W& x) {
     if (x.keys) (void)hipFree(x.keys);
     if (x.out) (void)hipFree(x.out);
@@ -410,10 +427,9 @@ struct RsqfExec {
     if (n > x.cap) {
       GQF_HIP(hipStreamSynchronize(hs));
       free_stage(x);
-      const size_t cap = std::max(x.room, n);
-      GQF_HIP(hipMalloc((void**)&x.keys, cap * 4));
-      GQF_HIP(hipMalloc((void**)&x.out, cap * 4));
-      x.cap = cap;
+      gqf_status st = stage_malloc(x, std::max(x.room, n));
+      if (st == GQF_ERR_NOMEM && x.room > n) st = stage_malloc(x, n);
+      GQF_TRY(st);
     }
     GQF_TRY(mv_requests<true>(hs, b, nb, x.keys));
     if (op == GQF_OP_INSERT) return gqf_rsqf_insert(fl, (int)n, x.keys, nullptr, x.st, &ms);
