@@ -36,6 +36,10 @@ struct Scheduler {
   gqf_serve_executor ex{};
   int nfilters = 0, nworkers = 0;
   size_t resident = 0;
+  // bytes that stay beside the run (idle workers of other runs), and their
+  // release; none: null
+  size_t (*spare_bytes)() = nullptr;
+  bool (*spare_release)() = nullptr;
   bool roomy = false;  // the executor knows calls with room to spare (coalesced = 2), which no call needs
   uint64_t max_batch = 0;
   std::mutex mu;
@@ -59,7 +63,7 @@ struct Scheduler {
   int worker_of(int filter) const { return cfg.coalesce ? filter : 0; }
 
   size_t used() const {
-    size_t u = resident;
+    size_t u = resident + (spare_bytes ? spare_bytes() : 0);
     for (size_t h : held) u += h;
     return u;
   }
@@ -86,8 +90,18 @@ struct Scheduler {
         running++;
         return true;
       }
-      // release what an idle worker holds, and our own last (a run may begin
-      // with what its workers held at the end of another)
+      // release what is beside the run, then what an idle worker holds, and our
+      // own last (a run may begin with what its workers held at the end of
+      // another)
+      if (spare_bytes && spare_bytes() > 0) {
+        trimming++;
+        lk.unlock();
+        (void)spare_release();
+        lk.lock();
+        trimming--;
+        cv.notify_all();
+        continue;
+      }
       int v = -1;
       for (int i = 0; i < nworkers; ++i)
         if (i != w && state[(size_t)i] == IDLE && held[(size_t)i] > left[(size_t)i]) {
@@ -455,7 +469,9 @@ struct RsqfExec {
 // freeing them took a third of a run of 300 requests (every free waits for
 // the device, and so for the other workers' calls).  At most IDLE_MAX of them
 // are kept, IDLE_BYTES in all, oldest taken first; a worker is one run's alone
-// while it is taken.  Given back by serve_release_idle.
+// while it is taken.  A run counts the idle ones of its device within its
+// budget.  Given back by serve_release_idle: when a run needs their bytes, when
+// the device refuses an allocation, by gqf_stream_trim.
 struct IdleWorker {
   int device;
   RsqfExec::W w;
@@ -511,6 +527,18 @@ static gqf_status worker_put(RsqfExec::W& x) {
     }
   }
   return worker_end(x);
+}
+
+// What the idle workers of the current device hold.
+static size_t idle_bytes() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> lk(g_idle_mu);
+  size_t n = 0;
+  if (g_idle)
+    for (const IdleWorker& w : *g_idle)
+      if (w.device == dev) n += w.bytes;
+  return n;
 }
 
 }  // namespace
@@ -583,6 +611,8 @@ gqf_status gqf_rsqf_serve(gqf_rsqf* filters, int nfilters, gqf_request* reqs, in
     s.nfilters = nfilters;
     s.resident = resident;
     s.roomy = !tight;
+    s.spare_bytes = &idle_bytes;
+    s.spare_release = &serve_release_idle;
     st = s.run(reqs, nreqs, stats);
   }
   for (RsqfExec::W& x : e.w) {

@@ -385,9 +385,9 @@ size_t gqf_workspace_alloc_bytes(size_t bytes);
  *   coalesce == 0  plain execution: one call per request, in arrival order,
  *                  on one stream.
  * Admission: a call starts when the filter tables, the workspaces the
- * workers hold and the call's own need (workspace growth, gather buffers) fit
- * hbm_budget; otherwise it waits for running calls to finish, releasing the
- * workspaces of idle workers.  A request that cannot fit on its own is
+ * workers hold, what idle workers of earlier runs keep and the call's own need
+ * (workspace growth, gather buffers) fit hbm_budget; otherwise it waits for
+ * running calls to finish, releasing what idle workers hold.  A request that cannot fit on its own is
  * rejected (status GQF_ERR_NOMEM) and the loop goes on. */
 enum gqf_op { GQF_OP_LOOKUP = 0, GQF_OP_INSERT = 1, GQF_OP_DELETE = 2 };
 

@@ -197,11 +197,31 @@ static int refused() {
   return 0;
 }
 
+// A run with fewer filters than the one before: the workers that it does not
+// take count, and are given up when the budget needs their bytes.
+static int idle() {
+  Run a(3, 60 * MB / 8, 4, (size_t)1 << 40);
+  CHECK(a.all_ok() && g_used >= 150 * MB);
+  Run b(1, 100 * MB / 8, 4, 800 * MB);  // there is room: they stay
+  CHECK(b.all_ok() && b.one_call(1));
+  CHECK(b.stats.peak_bytes >= b.max_used && b.max_used <= 800 * MB && b.max_used >= 230 * MB);
+  Run c(1, 590 * MB / 8, 4, 600 * MB);
+  CHECK(c.all_ok() && c.one_call(1));
+  CHECK(c.max_used <= 600 * MB && c.stats.peak_bytes <= 600 * MB);
+  (void)serve_release_idle();
+  Run d(3, 60 * MB / 8, 4, (size_t)1 << 40);
+  Run e(1, 4 * MB / 8, 4, 100 * MB);  // a tight budget, below what stayed
+  CHECK(d.all_ok() && e.all_ok());
+  CHECK(e.stats.peak_bytes <= 100 * MB && g_used <= 100 * MB);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   int rc = 2;
   if (name == "exact") rc = exact();
   if (name == "refused") rc = refused();
+  if (name == "idle") rc = idle();
   (void)serve_release_idle();
   if (rc == 0 && g_used != 0) {
     std::printf("FAIL %zu bytes left\n", g_used);

@@ -26,7 +26,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["exact", "refused"])
+@pytest.mark.parametrize("scenario", ["exact", "refused", "idle"])
 def test_serving_memory(check, scenario):
     r = subprocess.run([check, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and scenario + " ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
