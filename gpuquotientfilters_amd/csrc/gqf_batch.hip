@@ -61,7 +61,13 @@ struct BTile {
 // digits, about 4096 keys each, in LDS: two reads and writes of the keys
 // instead of one per 8 bits (the autotuner times both).  48 filters of q = 12
 // .. 20, 6 M keys: 94 us, four passes 200.
+//   Keys are refilled in place, so a batch tuned on uniform keys may meet
+// crowded ones (many copies of a few).  A group of more keys than LDS holds
+// raises BS_HANDED before any key has moved: the kernels that follow leave
+// every table alone and the call launches the 8-bit passes (as do the batch's
+// next builds, for a while).
 constexpr uint32_t BS_TOP = 0xFFFFFFFFu;
+constexpr uint32_t BS_HANDED = 0x80000000u;  // in `left`, and then every filter's error word
 __device__ __forceinline__ uint32_t bs_shift(uint32_t shift, uint32_t bits) {
   const uint32_t b = bits & 0xFFu;
   return shift != BS_TOP ? shift : b > 8 ? b - 8 : 0u;
@@ -69,6 +75,12 @@ __device__ __forceinline__ uint32_t bs_shift(uint32_t shift, uint32_t bits) {
 struct BGroup {
   uint32_t f, d0, d1, nbits;  // filter, its digits [d0, d1), bits below those all keys share
 };
+// log2 of the groups of a filter of so many keys.
+__host__ __device__ inline uint32_t bs_group_bits(uint32_t nkeys) {
+  uint32_t gb = 0;
+  while (gb < 8 && nkeys > (4096u << gb)) ++gb;
+  return gb;
+}
 template <bool HASH>
 __global__ __launch_bounds__(256) void k_bs_upsweep(const uint32_t* __restrict__ in, const BChunk* __restrict__ ch,
                                                     const BFilter* __restrict__ flt, uint32_t shift, uint32_t G,
@@ -100,15 +112,24 @@ __global__ __launch_bounds__(256) void k_bs_upsweep(const uint32_t* __restrict__
 // dbase[f][d] = keys of filter f with a smaller digit: the filter's count of
 // digit d is (row prefix at its next filter's first chunk) - (row prefix at
 // its own first chunk), with the row total standing in past the last chunk.
+// left (the form by groups; else null): whether a group is too large.
 __global__ __launch_bounds__(256) void k_bs_digitbase(const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals,
                                                       const uint32_t* __restrict__ fchunk, uint32_t G,
-                                                      uint32_t* __restrict__ dbase) {
-  __shared__ uint32_t tmp[4];
+                                                      const BFilter* __restrict__ flt, uint32_t* __restrict__ dbase,
+                                                      uint32_t* __restrict__ left) {
+  __shared__ uint32_t tmp[4], s_base[257];
   const uint32_t f = blockIdx.x, d = threadIdx.x;
   const uint32_t c0 = fchunk[f], c1 = fchunk[f + 1];
   const uint32_t p0 = c0 < G ? hist[(uint64_t)d * G + c0] : totals[d];
   const uint32_t p1 = c1 < G ? hist[(uint64_t)d * G + c1] : totals[d];
-  dbase[(uint64_t)f * 256 + d] = block256_excl_scan(p1 - p0, tmp, nullptr);
+  const uint32_t base = block256_excl_scan(p1 - p0, tmp, nullptr);
+  dbase[(uint64_t)f * 256 + d] = base;
+  if (!left) return;
+  s_base[d] = base;
+  if (d == 255) s_base[256] = base + p1 - p0;
+  __syncthreads();
+  const uint32_t span = 256u >> bs_group_bits(flt[f].nkeys);
+  if ((d & (span - 1u)) == 0 && s_base[d + span] - s_base[d] > (uint32_t)SEG_TILE) atomicOr(left, BS_HANDED);
 }
 
 // LDS of a stable pass over tiles of SORT_TILE keys.
@@ -185,11 +206,14 @@ template <bool HASH>
 __global__ __launch_bounds__(256) void k_bs_downsweep(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                       const BChunk* __restrict__ ch, const BFilter* __restrict__ flt,
                                                       uint32_t shift, uint32_t G, const uint32_t* __restrict__ hist,
-                                                      const uint32_t* __restrict__ dbase, uint32_t n_total) {
+                                                      const uint32_t* __restrict__ dbase, uint32_t n_total,
+                                                      const uint32_t* __restrict__ left) {
   __shared__ BsLds l;
   const int tid = threadIdx.x;
+  const uint32_t handed = left ? *left : 0u;  // (asked for before the loads that follow, used after)
   const BChunk c = ch[blockIdx.x];
   const BFilter fl = flt[c.f];
+  if (handed) return;
   l.run[tid] = fl.key0 + dbase[(uint64_t)c.f * 256 + tid] + hist[(uint64_t)tid * G + blockIdx.x] -
                hist[(uint64_t)tid * G + c.head];
   bs_tiles<HASH>(in, out, c.begin, c.end, fl.bits, bs_shift(shift, fl.bits), n_total, l);
@@ -201,60 +225,48 @@ __device__ __forceinline__ void bs_range(const BGroup& g, const BFilter* __restr
   *begin = k0 + dbase[(uint64_t)g.f * 256 + g.d0];
   *end = k0 + (g.d1 < 256 ? dbase[(uint64_t)g.f * 256 + g.d1] : flt[g.f].nkeys);
 }
-// Group blockIdx.x in place; one of more keys than LDS holds, or with a
-// crowded bucket, goes to `big` (count, then group ids).
+// Group blockIdx.x in place; one with a crowded bucket goes to `left` (count,
+// then group ids).
 [[maybe_unused]] static __global__ __launch_bounds__(SEG_THREADS) void k_bs_groups(uint32_t* __restrict__ keys,
                                                                                  const BGroup* __restrict__ grp,
                                                                                  const BFilter* __restrict__ flt,
                                                                                  const uint32_t* __restrict__ dbase,
-                                                                                 uint32_t* __restrict__ big) {
+                                                                                 uint32_t* __restrict__ left) {
   __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
   __shared__ __align__(16) uint32_t s_c[SEG_NBK / 2];
   __shared__ uint32_t s_tmp[SEG_THREADS / 64];
+  const uint32_t handed = *left & BS_HANDED;
   const BGroup g = grp[blockIdx.x];
   uint32_t begin, end;
   bs_range(g, flt, dbase, &begin, &end);
-  if (end - begin <= 1) return;
-  if (end - begin > (uint32_t)SEG_TILE) {
-    if (threadIdx.x == 0) big[1 + atomicAdd(&big[0], 1u)] = blockIdx.x;
-    return;
-  }
+  if (end - begin <= 1 || end - begin > (uint32_t)SEG_TILE || handed) return;
   if (!seg_bucket_sort<uint32_t, false>(keys + begin, keys + begin, end - begin, g.nbits, s_keys, nullptr, s_c, s_tmp) &&
       threadIdx.x == 0)
-    big[1 + atomicAdd(&big[0], 1u)] = blockIdx.x;
+    left[1 + atomicAdd(&left[0], 1u)] = blockIdx.x;
 }
-// The groups left (crowded digits: many copies of a few keys), one workgroup
-// each: 8-bit passes between the group's ranges of a and b.
-[[maybe_unused]] static __global__ __launch_bounds__(256) void k_bs_big(uint32_t* a, uint32_t* b,
-                                                                      const BGroup* __restrict__ grp,
-                                                                      const BFilter* __restrict__ flt,
-                                                                      const uint32_t* __restrict__ dbase,
-                                                                      const uint32_t* __restrict__ big, uint32_t n_total) {
-  __shared__ BsLds l;
-  __shared__ uint32_t s_hist[256];
-  const uint32_t tid = threadIdx.x, n = big[0];
+// The groups left: 4-bit counting passes in LDS.  A build that was handed over
+// says so in every filter's error word.
+[[maybe_unused]] static __global__ __launch_bounds__(SEG_THREADS) void k_bs_crowded(uint32_t* __restrict__ keys,
+                                                                                  const BGroup* __restrict__ grp,
+                                                                                  const BFilter* __restrict__ flt,
+                                                                                  const uint32_t* __restrict__ dbase,
+                                                                                  const uint32_t* __restrict__ left,
+                                                                                  uint32_t* __restrict__ ferr, uint32_t F) {
+  __shared__ __align__(16) uint32_t s_keys[SEG_TILE];
+  __shared__ __align__(16) uint16_t s_cnt[16 * SEG_THREADS];
+  __shared__ uint32_t s_tmp[SEG_THREADS / 64];
+  const uint32_t n = left[0];
+  if (n & BS_HANDED) {
+    if (blockIdx.x == 0)
+      for (uint32_t f = threadIdx.x; f < F; f += SEG_THREADS) ferr[f] = BS_HANDED;
+    return;
+  }
   for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const BGroup g = grp[big[1 + i]];
+    const BGroup g = grp[left[1 + i]];
     uint32_t begin, end;
     bs_range(g, flt, dbase, &begin, &end);
-    uint32_t *src = a, *dst = b;
-    for (uint32_t shift = 0; shift < g.nbits; shift += 8) {
-      s_hist[tid] = 0u;
-      __syncthreads();
-      for (uint32_t k = begin + tid; k < end; k += 256) atomicAdd(&s_hist[(src[k] >> shift) & 255u], 1u);
-      __syncthreads();
-      l.run[tid] = begin + block256_excl_scan(s_hist[tid], l.tmp, nullptr);
-      __syncthreads();
-      bs_tiles<false>(src, dst, begin, end, 0u, shift, n_total, l);
-      __threadfence_block();
-      __syncthreads();
-      uint32_t* t = src;
-      src = dst;
-      dst = t;
-    }
-    if (src != a)
-      for (uint32_t k = begin + tid; k < end; k += 256) a[k] = src[k];
-    __syncthreads();
+    seg_counting_sort<uint32_t, SEG_THREADS>(keys + begin, end - begin, g.nbits, s_keys, s_cnt, s_tmp);
+    __syncthreads();  // s_keys is read before the next group writes it
   }
 }
 
@@ -360,7 +372,7 @@ __global__ __launch_bounds__(1024) void k_bb_scan(uint4* __restrict__ agg, uint3
           const uint32_t f = tl[i].f;
           const uint32_t lp = run.s.lp, S = flt[f].S;
           fend[f] = lp < S ? lp : S;  // the slot after the filter's last entry
-          if (lp > S) ferr[f] = DEV_ERR_CAPACITY;
+          if (lp > S) ferr[f] |= DEV_ERR_CAPACITY;
         }
       }
     }
@@ -583,8 +595,9 @@ struct SqfBatch {
   uint32_t *d_fchunk = nullptr, *d_poff = nullptr, *d_hist = nullptr, *d_tot = nullptr, *d_dbase = nullptr;
   uint32_t *d_k0 = nullptr, *d_k1 = nullptr;
   BGroup* d_grp = nullptr;
-  uint32_t* d_big = nullptr;  // count and ids of the groups k_bs_groups leaves
-  uint32_t ngroups = 0;       // 0: the 8-bit passes
+  uint32_t* d_left = nullptr;  // count and ids of the groups k_bs_groups leaves, BS_HANDED
+  uint32_t ngroups = 0;        // 0: the 8-bit passes
+  uint32_t skip = 0, backoff = 0;  // builds that take the passes after one that was handed over
   uint4* d_agg = nullptr;
   uint32_t *d_fix = nullptr, *d_fixcnt = nullptr, *d_more = nullptr, *d_moren = nullptr;
   uint32_t *d_ferr = nullptr, *d_fend = nullptr;
@@ -596,7 +609,7 @@ struct SqfBatch {
   int sort_per = 1;     // sub-tiles per sort chunk
   int lk_block = 256, lk_ipt = 1;
   std::vector<float> tune_sort_ms, tune_lookup_ms;
-  hipGraphExec_t g_build = nullptr, g_lookup = nullptr;
+  hipGraphExec_t g_build = nullptr, g_passes = nullptr, g_lookup = nullptr;  // (g_passes: after a hand-over)
   int build_nodes = 0, lookup_nodes = 0;
   std::vector<uint32_t> h_err;
 };
@@ -659,13 +672,14 @@ static void batch_index_launch(SqfBatch& b) {
 static void batch_build_launch(SqfBatch& b) {
   hipStream_t s = b.stream;
   const uint32_t F = (uint32_t)b.F;
-  GQF_LAUNCH(k_bb_reset, dim3(64), dim3(256), 0, s, b.d_ferr, 3 * F + 1);  // ferr, fend, more_n, the count in big
+  GQF_LAUNCH(k_bb_reset, dim3(64), dim3(256), 0, s, b.d_ferr, 3 * F + 1);  // ferr, fend, more_n, the count in left
   if (b.N == 0) {
     GQF_LAUNCH(k_bb_clear_tail, dim3(64, F), dim3(256), 0, s, b.d_flt, b.d_ferr, b.d_fend, b.bpe);
     return;
   }
   const uint32_t* src = b.d_keys;
   uint32_t* buf[2] = {b.d_k0, b.d_k1};
+  uint32_t* left = b.ngroups ? b.d_left : nullptr;
   for (uint32_t p = 0; p < (b.ngroups ? 1u : b.npass); ++p) {
     const uint32_t shift = b.ngroups ? BS_TOP : 8 * p;
     uint32_t* dst = buf[p & 1];
@@ -677,19 +691,21 @@ static void batch_build_launch(SqfBatch& b) {
                    b.G, b.d_hist);
     GQF_LAUNCH(k_rs_rowscan, dim3(256), dim3(1024), 0, s, b.d_hist, b.G, b.d_tot, (uint32_t*)nullptr, 0u,
                (uint32_t*)nullptr);
-    GQF_LAUNCH(k_bs_digitbase, dim3(F), dim3(256), 0, s, b.d_hist, b.d_tot, b.d_fchunk, b.G, b.d_dbase);
+    GQF_LAUNCH(k_bs_digitbase, dim3(F), dim3(256), 0, s, b.d_hist, b.d_tot, b.d_fchunk, b.G, b.d_flt, b.d_dbase,
+               left);
     if (p == 0)
       GQF_LAUNCH_B((double)b.N * 8, k_bs_downsweep<true>, dim3(b.G), dim3(256), 0, s, src, dst, b.d_ch, b.d_flt,
-                   shift, b.G, b.d_hist, b.d_dbase, b.N);
+                   shift, b.G, b.d_hist, b.d_dbase, b.N, left);
     else
       GQF_LAUNCH_B((double)b.N * 8, k_bs_downsweep<false>, dim3(b.G), dim3(256), 0, s, src, dst, b.d_ch, b.d_flt,
-                   shift, b.G, b.d_hist, b.d_dbase, b.N);
+                   shift, b.G, b.d_hist, b.d_dbase, b.N, left);
     src = dst;
   }
   if (b.ngroups) {
     GQF_LAUNCH_B((double)b.N * 8, k_bs_groups, dim3(b.ngroups), dim3(SEG_THREADS), 0, s, buf[0], b.d_grp, b.d_flt,
-                 b.d_dbase, b.d_big);
-    GQF_LAUNCH(k_bs_big, dim3(256), dim3(256), 0, s, buf[0], buf[1], b.d_grp, b.d_flt, b.d_dbase, b.d_big, b.N);
+                 b.d_dbase, left);
+    GQF_LAUNCH(k_bs_crowded, dim3(std::min(b.ngroups, 512u)), dim3(SEG_THREADS), 0, s, buf[0], b.d_grp, b.d_flt, b.d_dbase,
+               left, b.d_ferr, F);
   }
   const uint32_t* A = src;
   if (b.no_dup)
@@ -717,6 +733,13 @@ static void batch_build_launch(SqfBatch& b) {
   GQF_LAUNCH(k_bb_clear_tail, dim3(64, F), dim3(256), 0, s, b.d_flt, b.d_ferr, b.d_fend, b.bpe);
   GQF_LAUNCH(k_bb_fixup, dim3(b.nsub + F), dim3(64), 0, s, b.d_tl, b.d_flt, b.d_ferr, b.d_fix, b.d_fixcnt, b.d_more,
              b.d_moren, b.nsub, b.bpe);
+}
+
+static void batch_passes_launch(SqfBatch& b) {
+  const uint32_t ng = b.ngroups;
+  b.ngroups = 0;
+  batch_build_launch(b);
+  b.ngroups = ng;
 }
 
 // The lookups: first the window index of every table as it is now (a
@@ -787,9 +810,10 @@ static gqf_status capture(SqfBatch& b, void (*fn)(SqfBatch&), hipGraphExec_t* ex
 static void batch_release(SqfBatch& b) {
   if (b.stream) (void)hipStreamSynchronize(b.stream);
   if (b.g_build) (void)hipGraphExecDestroy(b.g_build);
+  if (b.g_passes) (void)hipGraphExecDestroy(b.g_passes);
   if (b.g_lookup) (void)hipGraphExecDestroy(b.g_lookup);
   if (b.mem) (void)hipFree(b.mem);
-  b.g_build = b.g_lookup = nullptr;
+  b.g_build = b.g_passes = b.g_lookup = nullptr;
   b.mem = nullptr;
   if (b.own_stream && b.stream) (void)gqf_stream_destroy(reinterpret_cast<gqf_stream>(b.stream));
   b.stream = nullptr;
@@ -889,9 +913,7 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   for (int f = 0; f < count; ++f) {
     const BFilter& x = hf[(size_t)f];
     groups = groups && x.nkeys <= 256 * SEG_GROUP_AVG;
-    uint32_t gb = 0;
-    while (gb < 8 && x.nkeys > (4096u << gb)) ++gb;
-    const uint32_t span = 256u >> gb, bits = x.bits & 0xFFu, low = bits > 8 ? bits - 8 : 0u;
+    const uint32_t gb = bs_group_bits(x.nkeys), span = 256u >> gb, bits = x.bits & 0xFFu, low = bits > 8 ? bits - 8 : 0u;
     for (uint32_t d = 0; x.nkeys && d < 256; d += span)
       grp.push_back({(uint32_t)f, d, d + span, std::min(low + 8 - gb, 32u)});
   }
@@ -932,7 +954,7 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   b->d_more = reinterpret_cast<uint32_t*>(m + o_more);
   b->d_grp = reinterpret_cast<BGroup*>(m + o_grp);
   b->d_ferr = reinterpret_cast<uint32_t*>(m + o_state);
-  b->d_big = b->d_ferr + 3 * (size_t)count;
+  b->d_left = b->d_ferr + 3 * (size_t)count;
   b->d_fend = b->d_ferr + count;
   b->d_moren = b->d_fend + count;
   b->d_woff = reinterpret_cast<uint32_t*>(m + o_woff);
@@ -952,15 +974,17 @@ static gqf_status batch_create(SqfBatch* b, const gqf_sqf* filters, int count, i
   // the batch keys each time: the last run leaves them built)
   const int pers[4] = {1, 2, 4, 8};
   // groups or 8-bit passes: keys with many copies of a few (Zipf ranks) leave
-  // groups that one workgroup each has to sort
+  // crowded groups, or are handed over
   if (b->ngroups) {
     const uint32_t ng = b->ngroups;
     float tg = 0.f, tp = 0.f;
     GQF_TRY(batch_upload_chunks(*b, 1));
     GQF_TRY(time_on_stream(*b, batch_build_launch, 2, &tg));
+    GQF_HIP(hipMemcpyAsync(b->h_err.data(), b->d_ferr, 4, hipMemcpyDeviceToHost, b->stream));
+    GQF_HIP(hipStreamSynchronize(b->stream));
     b->ngroups = 0;
     GQF_TRY(time_on_stream(*b, batch_build_launch, 2, &tp));
-    if (tg <= tp) b->ngroups = ng;
+    if (tg <= tp && !(b->h_err[0] & BS_HANDED)) b->ngroups = ng;
   }
   float best = 1e30f;
   int best_per = 1;
@@ -1036,10 +1060,32 @@ gqf_status gqf_sqf_batch_build(gqf_sqf_batch h, int use_graph, int* filter_statu
   SqfBatch& b = h->b;
   CallScope cs;
   GQF_TRY(cs.begin(reinterpret_cast<gqf_stream>(b.stream)));
-  if (use_graph) GQF_HIP(hipGraphLaunch(b.g_build, b.stream));
-  else batch_build_launch(b);
-  GQF_HIP(hipMemcpyAsync(b.h_err.data(), b.d_ferr, (size_t)b.F * 4, hipMemcpyDeviceToHost, b.stream));
-  GQF_TRY(cs.end(ms, false));
+  const bool groups = b.ngroups && b.skip == 0;
+  if (b.skip) --b.skip;
+  if (groups || !b.ngroups) {
+    if (use_graph) GQF_HIP(hipGraphLaunch(b.g_build, b.stream));
+    else batch_build_launch(b);
+    GQF_HIP(hipMemcpyAsync(b.h_err.data(), b.d_ferr, (size_t)b.F * 4, hipMemcpyDeviceToHost, b.stream));
+    GQF_TRY(cs.end(ms, false));
+  }
+  const bool handed = groups && (b.h_err[0] & BS_HANDED);
+  if (groups) {
+    b.backoff = handed ? (b.backoff ? std::min(2 * b.backoff, 256u) : 4u) : 0u;
+    b.skip = b.backoff;
+  }
+  if (handed || (b.ngroups && !groups)) {  // nothing was written
+    if (use_graph && !prof_enabled()) {  // (no timing events in a graph)
+      if (!b.g_passes) {
+        int nodes = 0;
+        GQF_TRY(capture(b, batch_passes_launch, &b.g_passes, &nodes));
+      }
+      GQF_HIP(hipGraphLaunch(b.g_passes, b.stream));
+    } else {
+      batch_passes_launch(b);
+    }
+    GQF_HIP(hipMemcpyAsync(b.h_err.data(), b.d_ferr, (size_t)b.F * 4, hipMemcpyDeviceToHost, b.stream));
+    GQF_TRY(cs.end(ms, false));
+  }
   bool any = false;
   for (int f = 0; f < b.F; ++f) {
     const int st = b.h_err[(size_t)f] ? GQF_ERR_CAPACITY : GQF_OK;
