@@ -48,7 +48,11 @@ struct PsPlan {
 // than 2^26 quotients (more digits than runs of stores allow), remainders
 // past a byte, more than `sparse` quotients per key (the passes over the
 // counts outweigh the sort: an SQF of q = 26 breaks even near 6, 288 : 256 us
-// at 8 M keys, 327 : 346 at 16 M; an RSQF near 32, 208 : 200 us at 2 M).
+// at 8 M keys, 327 : 346 at 16 M; an RSQF near 32, 208 : 200 us at 2 M), and
+// batches that uniform keys would hand over as well: groups with no room for
+// three standard deviations past their mean, or more than 208 keys per 32
+// quotients (their bytes count to 255).
+constexpr uint32_t PS_MEAN_MAX = PS_TILE - 640, DB_LOAD_MAX = 208;
 inline bool ps_plan(uint64_t n, uint32_t q, uint32_t r, uint32_t sparse, PsPlan* p) {
   if (n <= 256ull * 7600 || n * sparse < (1ull << q) || q < 20 || q > DB_QB + PS_GB_MAX || r > 8 || n >= (1ull << 30)) return false;
   p->gb = q > DB_QB + PS_GB_MIN ? q - DB_QB : PS_GB_MIN;
@@ -61,6 +65,7 @@ inline bool ps_plan(uint64_t n, uint32_t q, uint32_t r, uint32_t sparse, PsPlan*
   const uint64_t tiles = (n + p->tile - 1) / p->tile;
   p->wgs = (uint32_t)(tiles < 256 ? tiles : 256);
   const uint64_t mean = n >> p->gb, cap = (2 * mean + 2048 + 63) & ~63ull;
+  if (mean > PS_MEAN_MAX || 32 * n > ((uint64_t)DB_LOAD_MAX << q)) return false;
   p->cap = (uint32_t)(cap < PS_TILE ? cap : PS_TILE);
   return true;
 }
