@@ -207,7 +207,10 @@ __global__ __launch_bounds__(PS_THREADS) void k_ps_scatter(const uint32_t* __res
     }
     if (d0 < nd) {
       *reinterpret_cast<uint2*>(s_base + d0) = make_uint2(b0 - e, b1 - (e + c.x));
-      if (b0 + c.x > cap || b1 + c.y > cap) ctr[CTR_MISC] = 1u;  // a group is full: its further keys are not written
+      if (b0 + c.x > cap || b1 + c.y > cap) {  // a group is full: its further keys are not written
+        ctr[CTR_MISC] = 1u;
+        if (!BACK) gsize[nd] = 1u;
+      }
     }
     __syncthreads();
     const uint32_t tw = tn;
@@ -321,7 +324,7 @@ constexpr uint32_t DB_LIST = 128;  // listed runs per wave
 // parts (rank, placing and sorting 15, 15 and 25% of the time).
 template <bool UNIQUE>
 __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __restrict__ in,
-                                                           const uint32_t* __restrict__ gsize, uint32_t cap,
+                                                           const uint32_t* __restrict__ gsize, uint32_t nd, uint32_t cap,
                                                            uint32_t qb, uint32_t r, uint8_t* __restrict__ counts,
                                                            uint8_t* __restrict__ rems,
                                                            DbThread* __restrict__ th, uint4* __restrict__ agg,
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   const uint32_t t = threadIdx.x, lane = t & 63;
   const uint32_t shift = qb + r, lmask = (1u << shift) - 1u, rmask = (1u << r) - 1u;
   const uint32_t g = blockIdx.x, m = gsize[g];
-  if (m > cap) return;  // (uniform; reported by the partition)
+  if (gsize[nd]) return;  // (uniform) some group is too full: handed over
   uint4* c4 = reinterpret_cast<uint4*>(s_cnt);
   uint32_t k[PS_ITEMS];
   ps_load(in + (uint64_t)g * cap, m, k);
@@ -823,7 +826,7 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_rsqf(uint8_t* __restrict__
 // ---------------------------------------------------------------- host
 static inline size_t ps_bytes(const PsPlan& p) {
   const size_t room = (size_t)p.ngroups * p.cap;
-  return aligned_bytes(room * 4) + aligned_bytes((size_t)p.ngroups * 4) + aligned_bytes((size_t)1 << (p.qb + p.gb)) +
+  return aligned_bytes(room * 4) + aligned_bytes(((size_t)p.ngroups + 1) * 4) + aligned_bytes((size_t)1 << (p.qb + p.gb)) +
          aligned_bytes(room) +
          aligned_bytes((size_t)p.ngroups * PS_THREADS * sizeof(DbThread)) + aligned_bytes((size_t)p.ngroups * 16) +
          aligned_bytes(((size_t)p.ngroups + 1) * DB_SW * 4) +
@@ -845,7 +848,7 @@ static gqf_status db_runs(hipStream_t s, Arena& ar, const PsPlan& p, const uint3
   const uint32_t nd = p.ngroups, bits = p.shift + p.gb, hbits = bits > 32 ? bits - 32 : 0u;
   const size_t room = (size_t)nd * p.cap;
   uint32_t* mid = ar.take<uint32_t>(room);
-  uint32_t* gsize = ar.take<uint32_t>(nd);
+  uint32_t* gsize = ar.take<uint32_t>(nd + 1);  // and whether one is past its room
   o->counts = ar.take<uint8_t>((size_t)1 << (p.qb + p.gb));
   o->rems = ar.take<uint8_t>(room);
   o->th = ar.take<DbThread>((size_t)nd * PS_THREADS);
@@ -856,15 +859,15 @@ static gqf_status db_runs(hipStream_t s, Arena& ar, const PsPlan& p, const uint3
     return GQF_ERR_INVALID;
   }
   o->gsize = gsize;
-  GQF_LAUNCH(k_ps_reset, dim3(1), dim3(PS_THREADS), 0, s, gsize, nd, ctr);
+  GQF_LAUNCH(k_ps_reset, dim3(1), dim3(PS_THREADS), 0, s, gsize, nd + 1, ctr);
   GQF_LAUNCH_B((double)n * 8.0, (k_ps_scatter<WIDE, false>), dim3(p.wgs), dim3(PS_THREADS), 0, s, keys, n, fp_bits,
                p.shift, nd, hbits, p.tile, p.cap, gsize, mid, ctr, PsBack{});
   const double rb = (double)n * 5.0 + (double)((uint64_t)1 << (p.qb + p.gb));
   if (unique)
-    GQF_LAUNCH_B(rb, k_db_runs<true>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, p.cap, p.qb, r, o->counts, o->rems,
+    GQF_LAUNCH_B(rb, k_db_runs<true>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, nd, p.cap, p.qb, r, o->counts, o->rems,
                  o->th, o->agg, ctr);
   else
-    GQF_LAUNCH_B(rb, k_db_runs<false>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, p.cap, p.qb, r, o->counts, o->rems,
+    GQF_LAUNCH_B(rb, k_db_runs<false>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, nd, p.cap, p.qb, r, o->counts, o->rems,
                  o->th, o->agg, ctr);
   GQF_TRY(rb_scan(s, ar, o->agg, nd, slots, ctr, nullptr));
   GQF_LAUNCH(k_db_spill, dim3(nd), dim3(256), 0, s, o->counts, p.qb, o->agg, nd, o->spill, ctr);
