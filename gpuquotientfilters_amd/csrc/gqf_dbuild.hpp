@@ -247,15 +247,20 @@ __device__ __forceinline__ void db_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 // Sorts the n (2 at least) bytes of a run from p on (rem8 may be read three
-// bytes further); UNIQUE: clears the kept bits of repeats.
+// bytes further); UNIQUE: clears the kept bits of repeats and returns their
+// number.
 template <bool UNIQUE>
-__device__ __forceinline__ void db_sort_run(uint8_t* rem8, uint32_t p, uint32_t n, uint32_t* s_keep) {
+__device__ __forceinline__ uint32_t db_sort_run(uint8_t* rem8, uint32_t p, uint32_t n, uint32_t* s_keep) {
   auto order = [](uint32_t& a, uint32_t& b) {
     const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
     a = lo;
     b = hi;
   };
-  auto repeat = [&](uint32_t z) { atomicAnd(&s_keep[z >> 5], ~(1u << (z & 31))); };
+  uint32_t repeats = 0;
+  auto repeat = [&](uint32_t z) {
+    atomicAnd(&s_keep[z >> 5], ~(1u << (z & 31)));
+    ++repeats;
+  };
   if (n <= 4) {
     // a missing value is larger than any byte
     uint32_t x0 = rem8[p], x1 = rem8[p + 1], x2 = rem8[p + 2], x3 = rem8[p + 3];
@@ -301,6 +306,35 @@ __device__ __forceinline__ void db_sort_run(uint8_t* rem8, uint32_t p, uint32_t 
       for (uint32_t a = p + 1; a < p + n; ++a)
         if (rem8[a] == rem8[a - 1]) repeat(a);
   }
+  return repeats;
+}
+
+// The same by a wave, for a run of 2 .. 255 bytes: every byte's rank among
+// them, a few per lane.  A lane sorting 64 bytes of two values in place takes
+// 1000 dependent moves, and its wave waits; this takes 64 steps.
+constexpr uint32_t DB_LONG = 24;  // longer runs are sorted so
+template <bool UNIQUE>
+__device__ __forceinline__ void db_sort_long(uint8_t* rem8, uint32_t p, uint32_t n, uint8_t* tmp, uint32_t* s_keep) {
+  const uint32_t lane = threadIdx.x & 63;
+#pragma unroll 1
+  for (uint32_t i = lane; i - lane < n; i += 64) {
+    const uint32_t x = i < n ? (uint32_t)rem8[p + i] : 0x100u;
+    uint32_t rank = 0;
+#pragma unroll 4
+    for (uint32_t j = 0; j < n; ++j) {
+      const uint32_t y = rem8[p + j];
+      rank += y < x + (j < i ? 1u : 0u) ? 1u : 0u;
+    }
+    if (i < n) tmp[rank] = (uint8_t)x;
+  }
+  db_wave_sync();
+#pragma unroll 1
+  for (uint32_t i = lane; i < n; i += 64) {
+    const uint32_t x = tmp[i];
+    rem8[p + i] = (uint8_t)x;
+    if (UNIQUE && i && tmp[i - 1] == x) atomicAnd(&s_keep[(p + i) >> 5], ~(1u << ((p + i) & 31)));
+  }
+  db_wave_sync();
 }
 
 // A thread's 32 quotients on the way from k_db_runs to the table: the kept
@@ -310,20 +344,31 @@ struct DbThread {
   uint32_t kept, lp;
 };
 constexpr uint32_t DB_LIST = 128;  // listed runs per wave
+constexpr uint32_t DB_MANY = 8;    // repeats that one lane meets: many
 
 // Group blockIdx.x: counts[quotient] (kept entries), their remainders in
 // order (db_stream), th[1024 g + t], agg[g].
 //   LDS atomics give every key its rank in its run; a key's byte then goes to
 // run start + rank, in the order of arrival.  Every wave lists the runs of
 // several entries among its quotients and sorts 64 of them at a time, a lane
-// per run (up to 8 entries in registers, longer runs in a loop).  Repeats
+// per run (up to 8 entries in registers, up to 24 in a loop, longer runs by
+// the wave).  Repeats
 // (UNIQUE) are dropped from the bytes at the end.
 //   A thread sorting its own 32 quotients' runs in place costs its wave the
 // longest run at every quotient: 342 us for 53.7 M keys; this: 201 us, 151 us
 // with repeats kept.  Bound by instructions and LDS accesses in about equal
 // parts (rank, placing and sorting 15, 15 and 25% of the time).
-template <bool UNIQUE>
-__global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __restrict__ in,
+//   A thread takes Q quotients, a group's by its 1024 threads (32 for 2^15; with
+// 32 for 2^12 as well, two of sixteen waves had work).  Fewer than 2^15
+// quotients: 256 groups, one to a CU, with all its registers.
+//   MANY, for keys with many copies: runs past 24 entries are sorted by their
+// wave, and where a lane has met 8 repeats the offsets are recounted from the
+// kept bits instead of lowered past each.  Builds (NoDup) of 2^25 keys, q = 26,
+// so many copies of each on average: 1: 366 us (368 with MANY), 4: 715 -> 575,
+// 32: 1520 -> 706; the sort takes 573, 620 and 983.  q = 22, 2^21 keys: 32
+// copies 302 -> 118 (the sort 153); q = 20, 2^21 keys, 4 copies: 278 -> 119 (124).
+template <bool UNIQUE, uint32_t Q, bool MANY>
+__global__ __launch_bounds__(PS_THREADS, Q == DB_Q ? 8 : 4) void k_db_runs(const uint32_t* __restrict__ in,
                                                            const uint32_t* __restrict__ gsize, uint32_t nd, uint32_t cap,
                                                            uint32_t qb, uint32_t r, uint8_t* __restrict__ counts,
                                                            uint8_t* __restrict__ rems,
@@ -332,10 +377,12 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   __shared__ __align__(16) uint32_t s_cnt[DB_NQ / 4];    // counts, then offsets within a thread's range
   __shared__ __align__(16) uint32_t s_rem[PS_TILE / 4 + 4];  // remainder bytes
   __shared__ __align__(16) uint32_t s_keep[UNIQUE ? PS_TILE / 32 + 4 : 4];
+  constexpr uint32_t NW = Q / 4;  // a thread's counter words
   __shared__ uint16_t s_base[PS_THREADS + 1];
-  __shared__ uint16_t s_list[PS_THREADS / 64][DB_LIST];
+  __shared__ __align__(16) uint16_t s_list[PS_THREADS / 64][MANY ? DB_LIST + 64 : DB_LIST];  // (MANY: room for 255 bytes past 64)
   __shared__ uint32_t s_tmp[PS_THREADS / 64];
   __shared__ uint4 s_wave[PS_THREADS / 64 + 1];
+  __shared__ uint32_t s_many, s_handed;  // MANY: repeats enough to recount; handed over
   const uint32_t t = threadIdx.x, lane = t & 63;
   const uint32_t shift = qb + r, lmask = (1u << shift) - 1u, rmask = (1u << r) - 1u;
   const uint32_t g = blockIdx.x, m = gsize[g];
@@ -346,6 +393,7 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   c4[t] = make_uint4(0u, 0u, 0u, 0u);
   c4[PS_THREADS + t] = make_uint4(0u, 0u, 0u, 0u);
   if (UNIQUE) {
+    if (MANY && t == 0) s_many = 0u;
     s_keep[t] = ~0u;
     if (t < 4) s_keep[PS_TILE / 32 + t] = ~0u;
   }
@@ -361,20 +409,43 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   });
   __syncthreads();
   // this thread's quotients: counts, first key, offsets
+  uint32_t* own = s_cnt + NW * t;
+  auto words = [&](uint32_t (&o)[NW]) {
+    if constexpr (NW == 8) {
+      const uint4 x = c4[2 * t], y = c4[2 * t + 1];
+      o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w, o[4] = y.x, o[5] = y.y, o[6] = y.z, o[7] = y.w;
+    } else if constexpr (NW == 4) {
+      const uint4 x = c4[t];
+      o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w;
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < NW; ++j) o[j] = own[j];
+    }
+  };
+  auto put_words = [&](void* at, const uint32_t (&o)[NW]) {
+    if constexpr (NW >= 4) {
+#pragma unroll
+      for (uint32_t j = 0; j < NW; j += 4) reinterpret_cast<uint4*>(at)[j / 4] = make_uint4(o[j], o[j + 1], o[j + 2], o[j + 3]);
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < NW; ++j) reinterpret_cast<uint32_t*>(at)[j] = o[j];
+    }
+  };
   uint32_t first, sum = 0;
   {
-    const uint4 x = c4[2 * t], y = c4[2 * t + 1];
-    const uint32_t c[DB_Q / 4] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-    uint32_t o[DB_Q / 4];
+    uint32_t c[NW], o[NW];
+    words(c);
 #pragma unroll
-    for (uint32_t j = 0; j < DB_Q / 4; ++j) {
+    for (uint32_t j = 0; j < NW; ++j) {
       const uint32_t h = (c[j] & 0x00FF00FFu) + ((c[j] >> 8) & 0x00FF00FFu);
       o[j] = (c[j] * 0x01010100u) + (sum & 0xFFu) * 0x01010101u;  // bytes: sums of those below (if all are at most 255)
       sum += (h & 0xFFFFu) + (h >> 16);
     }
-    bad |= sum > 255u;
-    c4[2 * t] = make_uint4(o[0], o[1], o[2], o[3]);
-    c4[2 * t + 1] = make_uint4(o[4], o[5], o[6], o[7]);
+    uint32_t near = sum;  // of 32 neighbouring quotients
+#pragma unroll
+    for (uint32_t x = 1; x < DB_Q / Q; x *= 2) near += (uint32_t)__shfl_xor((int)near, (int)x);
+    bad |= near > 255u;
+    put_words(own, o);
     first = block_excl_scan<PS_THREADS>(sum, s_tmp);
     s_base[t] = (uint16_t)first;
     if (t == PS_THREADS - 1) s_base[PS_THREADS] = (uint16_t)(first + sum);
@@ -387,43 +458,66 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   const uint8_t* off8 = reinterpret_cast<const uint8_t*>(s_cnt);
   ps_each(m, [&](uint32_t i) {
     const uint32_t fq = (k[i] & lmask) >> r;
-    rem8[s_base[fq / DB_Q] + off8[fq] + (k[i] >> 24)] = (uint8_t)(k[i] & rmask);
+    rem8[s_base[fq / Q] + off8[fq] + (k[i] >> 24)] = (uint8_t)(k[i] & rmask);
   });
   // counts of the thread's quotients 4 w .. 4 w + 3, from the offsets
   auto cnt4 = [&](uint32_t w) {
-    const uint32_t o = s_cnt[DB_Q / 4 * t + w], nx = w + 1 < DB_Q / 4 ? s_cnt[DB_Q / 4 * t + w + 1] : sum;
+    const uint32_t o = own[w], nx = w + 1 < NW ? own[w + 1] : sum;
     return ((o >> 8) | (nx << 24)) - o;  // no byte borrows: offsets do not decrease
   };
+  // handed over by another group meanwhile (where all groups run at once)
+  if (Q < DB_Q && t == 0) s_handed = __hip_atomic_load(&ctr[CTR_MISC], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
+  if (Q < DB_Q && s_handed) return;  // (uniform)
   // runs of several entries
   {
     uint16_t* list = s_list[t >> 6];
-    uint32_t listed = 0, x = 0;  // (listed: the same in all lanes)
+    uint32_t listed = 0, x = 0, repeats = 0;  // (listed: the same in all lanes)
 #pragma unroll 1
     for (uint32_t j = 0;;) {
-      if (j < DB_Q) {
+      if (j < Q) {
         if ((j & 3) == 0) x = cnt4(j >> 2);
         const bool several = (x & 0xFFu) > 1;
         const uint64_t who = __ballot(several);
-        if (several) list[listed + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u))] = (uint16_t)(DB_Q * t + j);
+        if (several) list[listed + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u))] = (uint16_t)(Q * t + j);
         listed += (uint32_t)__popcll(who);
         x >>= 8;
         ++j;
       }
-      if (j < DB_Q && listed < 64) continue;
+      if (j < Q && listed < 64) continue;
       if (listed == 0) break;
       db_wave_sync();
       const uint32_t nl = listed < 64 ? listed : 64u;
       listed -= nl;
+      uint32_t longer = 0;  // a run's place and length (MANY)
       if (lane < nl) {
-        const uint32_t q = list[listed + lane], b0 = s_base[q / DB_Q], o = off8[q], p = b0 + o;
-        const uint32_t n = (q % DB_Q == DB_Q - 1 ? s_base[q / DB_Q + 1] - b0 : off8[q + 1]) - o;
-        db_sort_run<UNIQUE>(rem8, p, n, s_keep);
+        const uint32_t q = list[listed + lane], b0 = s_base[q / Q], o = off8[q], p = b0 + o;
+        const uint32_t n = (q % Q == Q - 1 ? s_base[q / Q + 1] - b0 : off8[q + 1]) - o;
+        if (MANY && n > DB_LONG) longer = p << 8 | n;
+        else repeats += db_sort_run<UNIQUE>(rem8, p, n, s_keep);
+      }
+      if (MANY) {
+        for (uint64_t who = __ballot(longer != 0); who; who &= who - 1ull) {
+          const uint32_t x = wave_read(longer, __builtin_ctzll(who));
+          db_sort_long<UNIQUE>(rem8, x >> 8, x & 0xFFu, reinterpret_cast<uint8_t*>(list + 64), s_keep);
+          repeats = DB_MANY;
+        }
       }
       db_wave_sync();
     }
+    if (MANY && UNIQUE && repeats >= DB_MANY) s_many = 1u;
   }
   __syncthreads();
+  // many repeats: the kept entries before every 32 (where the lists were)
+  uint16_t* s_pre = &s_list[0][0];
+  static_assert(sizeof(s_list) >= 2 * (PS_THREADS + 1), "the counts fit");
+  const bool many = MANY && UNIQUE && s_many != 0;  // (uniform)
+  if (many) {
+    const uint32_t c = (uint32_t)__popc(s_keep[t]), d = block_excl_scan<PS_THREADS>(c, s_tmp);
+    s_pre[t] = (uint16_t)d;
+    if (t == PS_THREADS - 1) s_pre[PS_THREADS] = (uint16_t)(d + c);
+    __syncthreads();
+  }
   // kept entries per quotient, and the thread's scan state: lp = kept +
   // max(quotient - kept entries before it) over the occupied quotients, four
   // quotients at a time (for an empty one the difference is no larger than
@@ -433,50 +527,65 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
   {
     uint32_t n = sum;
     uint32_t last = 0;  // the last occupied quotient: the last whose count is not 0
-    auto offsets = [&](uint32_t (&o)[DB_Q / 4]) {
-      const uint4 x = c4[2 * t], y = c4[2 * t + 1];
-      o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w, o[4] = y.x, o[5] = y.y, o[6] = y.z, o[7] = y.w;
-    };
     {
-      uint32_t o[DB_Q / 4];
-      offsets(o);
+      uint32_t o[NW];
+      words(o);
 #pragma unroll
-      for (uint32_t w = 0; w < DB_Q / 4; ++w) {
-        const uint32_t c = ((o[w] >> 8) | ((w + 1 < DB_Q / 4 ? o[w + 1] : sum) << 24)) - o[w];
+      for (uint32_t w = 0; w < NW; ++w) {
+        const uint32_t c = ((o[w] >> 8) | ((w + 1 < NW ? o[w + 1] : sum) << 24)) - o[w];
         if (c) last = 4 * w + ((31u - (uint32_t)__builtin_clz(c)) >> 3);
       }
     }
     if (UNIQUE) {
-      // the offsets past every repeat fall by one (in LDS: a loop over them in
-      // registers spilled 26, 330 MB of scratch at 53.7 M keys)
-      for (uint32_t z0 = first & ~31u; z0 < first + sum; z0 += 32) {
-        uint32_t lost = ~s_keep[z0 >> 5];
-        if (z0 < first) lost &= ~0u << (first - z0);
-        if (first + sum - z0 < 32) lost &= (1u << (first + sum - z0)) - 1u;
-        for (; lost; lost &= lost - 1u) {
-          const uint32_t z = z0 + (uint32_t)__builtin_ctz(lost) - first - (sum - n);  // its place among the kept so far
-          const uint32_t s = z * 0x01010101u;
-          // bytes of x above z
-          auto fall = [&](uint32_t x) {
-            const uint32_t lo = (x | 0x80808080u) - (s & 0x7F7F7F7Fu) - 0x01010101u;  // top bits: low 7 bits of x > those of s
-            return x - ((((x & ~s) | (~(x ^ s) & lo)) & 0x80808080u) >> 7);
-          };
+      if (many) {
+        // kept entries before position z of the group
+        auto kept = [&](uint32_t z) { return s_pre[z >> 5] + (uint32_t)__popc(s_keep[z >> 5] & ((1u << (z & 31)) - 1u)); };
+        const uint32_t k0 = kept(first);
+        n = kept(first + sum) - k0;
 #pragma unroll 1
-          for (uint32_t h = 2 * t; h < 2 * t + 2; ++h) {
-            const uint4 x = c4[h];
-            c4[h] = make_uint4(fall(x.x), fall(x.y), fall(x.z), fall(x.w));
+        for (uint32_t w = 0; w < NW; ++w) {
+          const uint32_t x = own[w];
+          uint32_t y = 0;
+#pragma unroll
+          for (uint32_t b = 0; b < 4; ++b) y |= (kept(first + ((x >> (8 * b)) & 0xFFu)) - k0) << (8 * b);
+          own[w] = y;
+        }
+      } else {
+        // the offsets past every repeat fall by one (in LDS: a loop over them in
+        // registers spilled 26, 330 MB of scratch at 53.7 M keys)
+        for (uint32_t z0 = first & ~31u; z0 < first + sum; z0 += 32) {
+          uint32_t lost = ~s_keep[z0 >> 5];
+          if (z0 < first) lost &= ~0u << (first - z0);
+          if (first + sum - z0 < 32) lost &= (1u << (first + sum - z0)) - 1u;
+          for (; lost; lost &= lost - 1u) {
+            const uint32_t z = z0 + (uint32_t)__builtin_ctz(lost) - first - (sum - n);  // its place among the kept so far
+            const uint32_t s = z * 0x01010101u;
+            // bytes of x above z
+            auto fall = [&](uint32_t x) {
+              const uint32_t lo = (x | 0x80808080u) - (s & 0x7F7F7F7Fu) - 0x01010101u;  // top bits: low 7 bits of x > those of s
+              return x - ((((x & ~s) | (~(x ^ s) & lo)) & 0x80808080u) >> 7);
+            };
+            if constexpr (NW >= 4) {
+#pragma unroll 1
+              for (uint32_t h = NW / 4 * t; h < NW / 4 * t + NW / 4; ++h) {
+                const uint4 x = c4[h];
+                c4[h] = make_uint4(fall(x.x), fall(x.y), fall(x.z), fall(x.w));
+              }
+            } else {
+              for (uint32_t w = 0; w < NW; ++w) own[w] = fall(own[w]);
+            }
+            --n;
           }
-          --n;
         }
       }
     }
-    uint32_t o[DB_Q / 4];  // kept entries before each quotient, of the thread
-    offsets(o);
-    uint32_t kc[DB_Q / 4];
+    uint32_t o[NW];  // kept entries before each quotient, of the thread
+    words(o);
+    uint32_t kc[NW];
     int32_t mx = -256;
 #pragma unroll
-    for (uint32_t w = 0; w < DB_Q / 4; ++w) {
-      kc[w] = ((o[w] >> 8) | ((w + 1 < DB_Q / 4 ? o[w + 1] : n) << 24)) - o[w];
+    for (uint32_t w = 0; w < NW; ++w) {
+      kc[w] = ((o[w] >> 8) | ((w + 1 < NW ? o[w + 1] : n) << 24)) - o[w];
 #pragma unroll
       for (uint32_t b = 0; b < 4; ++b) {
         const uint32_t q = 4 * w + b < last ? 4 * w + b : last;
@@ -484,17 +593,13 @@ __global__ __launch_bounds__(PS_THREADS, 8) void k_db_runs(const uint32_t* __res
         mx = v > mx ? v : mx;
       }
     }
-    const uint32_t fq0 = (g << qb) + DB_Q * t;
+    const uint32_t fq0 = (g << qb) + Q * t;
     if (n) a = RS{n, fq0 + (uint32_t)((int32_t)n + mx), fq0 + last + 1};
-    if (DB_Q * t < (1u << qb)) {
-      uint4* d = reinterpret_cast<uint4*>(counts + ((uint64_t)g << qb) + DB_Q * t);
-      d[0] = make_uint4(kc[0], kc[1], kc[2], kc[3]);
-      d[1] = make_uint4(kc[4], kc[5], kc[6], kc[7]);
-    }
+    put_words(counts + ((uint64_t)g << qb) + Q * t, kc);
   }
   RS ex;
   const RS all = rs_block_n<PS_THREADS / 64>(a, &ex, s_wave);
-  th[(uint64_t)g * PS_THREADS + t] = DbThread{ex.c, ex.lp};
+  if (Q * t % DB_Q == 0) th[(uint64_t)g * PS_THREADS + Q * t / DB_Q] = DbThread{ex.c, ex.lp};
   if (t == 0) agg[g] = rs_pack(all);
   if (UNIQUE && all.c != m) {  // (uniform) the kept bytes together: 32 keys per thread
     const uint4* s4 = reinterpret_cast<const uint4*>(s_rem);
@@ -540,6 +645,7 @@ __device__ __forceinline__ uint32_t db_lp(const uint4* __restrict__ pre, uint32_
   }
   const uint32_t c = *reinterpret_cast<const uint32_t*>(counts + q1 - 1024 + 4 * t);
   const uint32_t h = (c & 0x00FF00FFu) + ((c >> 8) & 0x00FF00FFu), sum = (h & 0xFFFFu) + (h >> 16);
+  if (((c & 0xFFu) > DB_LONG) | ((c >> 8 & 0xFFu) > DB_LONG) | ((c >> 16 & 0xFFu) > DB_LONG) | (c >> 24 > DB_LONG)) ctr[CTR_MISC + 2] = 1u;
   const uint32_t before = block_excl_scan<256>(sum, s_tmp);
   __shared__ uint32_t s_all;
   if (t == 255) s_all = before + sum;
@@ -833,6 +939,14 @@ static inline size_t ps_bytes(const PsPlan& p) {
          aligned_bytes(((p.ngroups + RBS_PER - 1) / RBS_PER) * 16) + 2048;
 }
 
+// After a build: whether the stream's next one may expect few repeats -- three
+// of four keys kept (NoDup), no run past DB_LONG entries among those that
+// k_db_spill reads.  Until a build has shown it, many are expected: the form
+// for many costs 1% on keys without, the other up to 60% on keys with.
+static inline bool db_few(const DeviceState& ds, uint32_t n, bool done) {
+  return done && (uint64_t)ds.h_pinned[CTR_COUNT] * 4 >= (uint64_t)n * 3 && ds.h_pinned[CTR_MISC + 2] == 0;
+}
+
 struct DbRuns {
   const uint32_t* gsize;
   uint8_t *counts, *rems;
@@ -841,10 +955,11 @@ struct DbRuns {
   uint32_t* spill;  // what reaches into every group
 };
 // Partition and runs of the raw keys; scans the locations (slots: the
-// table's).  WIDE: fingerprints of more than 32 bits.
+// table's).  WIDE: fingerprints of more than 32 bits.  few: the keys are
+// expected to hold few repeats (db_few).
 template <bool WIDE>
 static gqf_status db_runs(hipStream_t s, Arena& ar, const PsPlan& p, const uint32_t* keys, uint32_t fp_bits, uint32_t n,
-                          uint32_t r, bool unique, uint64_t slots, uint32_t* ctr, DbRuns* o) {
+                          uint32_t r, bool unique, bool few, uint64_t slots, uint32_t* ctr, DbRuns* o) {
   const uint32_t nd = p.ngroups, bits = p.shift + p.gb, hbits = bits > 32 ? bits - 32 : 0u;
   const size_t room = (size_t)nd * p.cap;
   uint32_t* mid = ar.take<uint32_t>(room);
@@ -863,12 +978,22 @@ static gqf_status db_runs(hipStream_t s, Arena& ar, const PsPlan& p, const uint3
   GQF_LAUNCH_B((double)n * 8.0, (k_ps_scatter<WIDE, false>), dim3(p.wgs), dim3(PS_THREADS), 0, s, keys, n, fp_bits,
                p.shift, nd, hbits, p.tile, p.cap, gsize, mid, ctr, PsBack{});
   const double rb = (double)n * 5.0 + (double)((uint64_t)1 << (p.qb + p.gb));
-  if (unique)
-    GQF_LAUNCH_B(rb, k_db_runs<true>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, nd, p.cap, p.qb, r, o->counts, o->rems,
-                 o->th, o->agg, ctr);
-  else
-    GQF_LAUNCH_B(rb, k_db_runs<false>, dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, nd, p.cap, p.qb, r, o->counts, o->rems,
-                 o->th, o->agg, ctr);
+#define GQF_DB_RUNS(U_, Q_, M_)                                                                                             \
+  GQF_LAUNCH_B(rb, (k_db_runs<U_, Q_, M_>), dim3(nd), dim3(PS_THREADS), 0, s, mid, gsize, nd, p.cap, p.qb, r, o->counts, o->rems, \
+               o->th, o->agg, ctr)
+#define GQF_DB_RUNS_Q(U_)                          \
+  do {                                             \
+    if (p.qb == 15 && few) GQF_DB_RUNS(U_, 32, false); \
+    else if (p.qb == 15) GQF_DB_RUNS(U_, 32, true);    \
+    else if (p.qb == 14) GQF_DB_RUNS(U_, 16, true);    \
+    else if (p.qb == 13) GQF_DB_RUNS(U_, 8, true);     \
+    else GQF_DB_RUNS(U_, 4, true);                     \
+  } while (0)
+  static_assert(DB_QB == 15, "the quotients of a thread: 2^qb / 1024");
+  if (unique) GQF_DB_RUNS_Q(true);
+  else GQF_DB_RUNS_Q(false);
+#undef GQF_DB_RUNS_Q
+#undef GQF_DB_RUNS
   GQF_TRY(rb_scan(s, ar, o->agg, nd, slots, ctr, nullptr));
   GQF_LAUNCH(k_db_spill, dim3(nd), dim3(256), 0, s, o->counts, p.qb, o->agg, nd, o->spill, ctr);
   return GQF_OK;

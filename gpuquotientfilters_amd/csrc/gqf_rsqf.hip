@@ -1675,7 +1675,7 @@ static gqf_status rsqf_build_runs(const gqf_rsqf& f, const PsPlan& p, uint32_t n
   const RsqfGeom g = rgeom(f);
   Arena ar(ds.ws, ds.ws_cap);
   DbRuns d;
-  GQF_TRY((db_runs<WIDE>(cs.stream, ar, p, keys, g.bits, n, g.r, false, g.cap, ds.counters, &d)));
+  GQF_TRY((db_runs<WIDE>(cs.stream, ar, p, keys, g.bits, n, g.r, false, ds.build_few[1], g.cap, ds.counters, &d)));
   uint8_t* meta = reinterpret_cast<uint8_t*>(f.blocks);
   const double wb = (double)rsqf_dev_bytes(g.q, g.r) + (double)n + (double)((uint64_t)1 << g.q);
   if (g.r == 8)
@@ -2111,6 +2111,7 @@ gqf_status gqf_rsqf_bulk_build(gqf_rsqf cqf, int n, const uint32_t* d_keys, gqf_
     const gqf_status st = cs.end(ms, true);
     const bool done = cs.ds->h_pinned[CTR_MISC] == 0;
     lw_report(*cs.ds, LOCAL_RSQF_BUILD, done);
+    cs.ds->build_few[1] = db_few(*cs.ds, (uint32_t)n, done);
     if (done) return st;
   }
   if (cqf.qbits + cqf.rbits <= 32) GQF_TRY(rsqf_build_t<uint32_t>(cqf, (uint32_t)n, d_keys, cs));

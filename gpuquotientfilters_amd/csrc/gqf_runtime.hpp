@@ -100,6 +100,8 @@ struct DeviceState {
   uint32_t crowd_skip[2] = {0, 0}, crowd_backoff[2] = {0, 0};
   // likewise after a batch that a fast form handed over, per kind
   uint32_t local_skip[LOCAL_KINDS] = {}, local_backoff[LOCAL_KINDS] = {};
+  // builds by runs: the stream's last one (SQF, RSQF) held few repeats
+  bool build_few[2] = {false, false};
   // per-launch timing (gqf_profile_enable): event pool and launches to resolve
   hipEvent_t* pool = nullptr;
   size_t pool_size = 0, pool_used = 0;

@@ -214,9 +214,9 @@ static gqf_status sqf_build_launch(hipStream_t s, Arena& ar, uint32_t* counters,
 // The build without a sort (gqf_dbuild.hpp).  Leaves ctr[CTR_MISC] != 0, and
 // the table untouched, when the keys do not fit that form.
 static gqf_status sqf_build_runs(hipStream_t s, Arena& ar, uint32_t* ctr, const gqf_sqf& wq, const SqfGeom& g,
-                                 const PsPlan& p, uint32_t un, const uint32_t* d_keys, int no_dup) {
+                                 const PsPlan& p, uint32_t un, const uint32_t* d_keys, int no_dup, bool few) {
   DbRuns d;
-  GQF_TRY((db_runs<false>(s, ar, p, d_keys, (g.q + g.r) | sqf_hash_flag(), un, g.r, no_dup != 0, (uint64_t)g.S, ctr, &d)));
+  GQF_TRY((db_runs<false>(s, ar, p, d_keys, (g.q + g.r) | sqf_hash_flag(), un, g.r, no_dup != 0, few, (uint64_t)g.S, ctr, &d)));
   const double wb = (double)g.bytes + (double)un + (double)((uint64_t)1 << g.q);
   if (g.bpe == 1)
     GQF_LAUNCH_B(wb, k_db_sqf<1>, dim3(p.ngroups), dim3(PS_THREADS), 0, s, wq.table, g.S, d.gsize, p.cap, p.qb, d.counts, d.rems,
@@ -248,11 +248,12 @@ static gqf_status sqf_build_impl(const gqf_sqf& qf, int n, const uint32_t* d_key
   GQF_TRY(work_table(cs.stream, ar, qf, g, false, &wq));
   if (runs) {
     const size_t mark = ar.used;
-    GQF_TRY(sqf_build_runs(cs.stream, ar, ds.counters, wq, g, p, un, d_keys, no_dup));
+    GQF_TRY(sqf_build_runs(cs.stream, ar, ds.counters, wq, g, p, un, d_keys, no_dup, ds.build_few[0]));
     finish_table(cs.stream, qf, wq, g, ds.counters);
     const gqf_status st = cs.end(ms, true);
     const bool done = ds.h_pinned[CTR_MISC] == 0;
     lw_report(ds, LOCAL_SQF_BUILD, done);
+    ds.build_few[0] = db_few(ds, un, done);
     if (done) return st;
     ar.used = mark;  // nothing was written: the sort takes over
   }

@@ -60,4 +60,5 @@ def test_runs_of_a_build_that_the_partition_hands_over(cls, no_dup):
         sqf_equal(f, sqf_table(fps, q, r, no_dup))
     else:
         rsqf_equal(f, rsqf_table(fps, q, r))
+    say("whole, handed", whole, handed)
     assert handed < whole / 2
