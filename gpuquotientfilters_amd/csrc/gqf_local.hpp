@@ -24,9 +24,9 @@
 //   delete  key k starts a region iff a boundary (a slot that is empty or
 //           whose entry is at its own quotient) lies after key k-1's quotient
 //           and at or before its own; the state is the last boundary.
-// A region that passes its window's end is followed into the table directly
-// by its lane; the next window's wave leaves those slots, and the keys there,
-// alone.  The 64-slot block where a window's first region starts may hold the
+// A region that passes its window's end is held with it, up to some blocks of
+// the next window; the next window's wave leaves those slots, and the keys
+// there, alone.  The 64-slot block where a window's first region starts may hold the
 // end of an earlier window's region: it too is updated in the table, slot by
 // slot, and never written back as a whole.
 //   Work is per key and per keyed window; a window without keys is read only
@@ -35,8 +35,9 @@
 // and the call takes its general path: more than LW_KEYS keys in a window,
 // a whole aligned group
 // of 64 keys without a head, fewer than LW_SPILL empty slots in a
-// window (clusters longer than a window), an overflow above LW_SPILL, too
-// few regions (lw_scan).  After such a batch the next 4, 8, ... 256 of its
+// window (clusters longer than a window), an overflow above LW_SPILL, a
+// region that reaches past the blocks held of the next window, too few regions
+// (lw_scan).  After such a batch the next 4, 8, ... 256 of its
 // kind on the stream go straight to the general path.
 #pragma once
 
@@ -74,15 +75,31 @@ static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8
 
 static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }
 
-// Scan state of a window: overflow map x -> max(x + a, b) (insert), 1 + the
-// last boundary slot (delete; 0: none), and the keys that start a region.
+// Scan state of a window: the map x -> max(x + a, b), lb, and the keys that
+// start a region.
+//   insert  the overflow map; lb = 1 + the largest overflow into the window
+//           whose region ends in the blocks held of it (lw_room).
+//   delete  a = -2, b = 1 where the last key's region reaches the window's end
+//           (else 0): of the windows before, the map at 0 is the last one's b;
+//           lb = 1 + the last boundary slot (0: none), with LW_FAR where the
+//           first one lies past the blocks held.
 struct LW {
   int32_t a, b;
   uint32_t lb, heads;
 };
+constexpr uint32_t LW_FAR = 0x80000000u;
 __host__ __device__ __forceinline__ LW lw_combine(LW x, LW y) {
   const int32_t b = x.b + y.a;
-  return LW{x.a + y.a, b > y.b ? b : y.b, x.lb > y.lb ? x.lb : y.lb, x.heads + y.heads};
+  const uint32_t xl = x.lb & ~LW_FAR, yl = y.lb & ~LW_FAR;
+  return LW{x.a + y.a, b > y.b ? b : y.b, xl > yl ? xl : yl, x.heads + y.heads};
+}
+// The region of an overflow x takes an empty slot for each of the x keys and
+// for each of the window's keys before the first with v = E_k - k >= x, which
+// starts the next region: the largest x for which these fit `held` slots is
+// the maximum of lw_fit over the window's keys and of held - nk (all of them).
+__host__ __device__ __forceinline__ int32_t lw_fit(int32_t v, int32_t held, int32_t k) { return v < held - k ? v : held - k; }
+__host__ __device__ __forceinline__ uint32_t lw_room(int32_t fit) {
+  return 1u + (uint32_t)(fit < 0 ? 0 : fit < LW_SPILL ? fit : LW_SPILL);
 }
 // b of a window that the localized form does not take: an overflow that no
 // window absorbs.
@@ -107,11 +124,11 @@ __device__ __forceinline__ LW lw_wave_excl(LW x, LW* total) {
               wave_read(inc.heads, 63)};
   return lw_dpp<DPP_WAVE_SHR1>(inc);
 }
-// Exclusive scan of the window states: pre[w] = {keys that overflow into
-// window w, 1 + the last boundary before it}.  More than LW_SPILL of the
-// former, or any past the last window (LW_BAD is both), raise the flag, in the
-// counters and in host memory (report); so do fewer regions than min_heads
-// (lw_min_heads).  Resets the counters before.  One workgroup and one launch
+// Exclusive scan of the window states: pre[w] = {insert: keys that overflow
+// into window w; 1 + the last boundary before it}.  More of the former than
+// there is room for, or any past the last window, a region that reaches a
+// boundary past the blocks held, and LW_BAD raise the flag, in the counters and
+// in host memory (report); so do fewer regions than min_heads (lw_min_heads).  Resets the counters before.  One workgroup and one launch
 // for up to LW_ONE windows a thread (5.2 us for 4097; a loop over more of them
 // took 34 us for 16385), two launches as rb_scan for more (7 us).
 constexpr uint32_t LW_ONE = 8;
@@ -120,18 +137,21 @@ __device__ __forceinline__ void lw_raise(uint32_t* ctr, uint32_t* report) {
   __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // Stores window w's prefix; whether it or (the last window) the end is bad.
+template <bool INS>
 __host__ __device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t W, uint2* __restrict__ pre,
                                                 uint32_t min_heads) {
   const int32_t o = p.a > p.b ? p.a : p.b;  // the map of the windows before, at 0
   pre[w] = make_uint2(o > 0 ? (uint32_t)o : 0u, p.lb);
-  if (w + 1 < W) return o > LW_SPILL;
+  // (windows that are not read have no overflow)
+  const bool bad = INS ? o > LW_SPILL || (o > 0 && (uint32_t)o >= x.lb) : o > 1 || (o > 0 && (x.lb & LW_FAR));
+  if (w + 1 < W) return bad;
   const LW all = lw_combine(p, x);
-  return o > LW_SPILL || (all.a > all.b ? all.a : all.b) > 0 || all.heads < min_heads;
+  return bad || (all.a > all.b ? all.a : all.b) > (INS ? 0 : 1) || all.heads < min_heads;
 }
-[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_one(const uint4* __restrict__ st, uint32_t W,
-                                                                         uint2* __restrict__ pre, uint32_t min_heads,
-                                                                         uint32_t* __restrict__ ctr,
-                                                                         uint32_t* __restrict__ report) {
+template <bool INS>
+__global__ __launch_bounds__(1024) void k_lw_one(const uint4* __restrict__ st, uint32_t W, uint2* __restrict__ pre,
+                                                 uint32_t min_heads, uint32_t* __restrict__ ctr,
+                                                 uint32_t* __restrict__ report) {
   __shared__ uint4 s_wave[16];
   __shared__ uint4 s_st[1024 * (LW_ONE + 1)];  // a thread's windows, one word of 16 bytes apart (banks)
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -165,7 +185,7 @@ __host__ __device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t
   bool bad = false;
 #pragma unroll
   for (uint32_t j = 0; j < LW_ONE; ++j) {
-    if (w0 + j < W) bad |= lw_put(p, lw_unpack(x[j]), w0 + j, W, pre, min_heads);
+    if (w0 + j < W) bad |= lw_put<INS>(p, lw_unpack(x[j]), w0 + j, W, pre, min_heads);
     p = lw_combine(p, lw_unpack(x[j]));
   }
   if (bad) lw_raise(ctr, report);
@@ -187,11 +207,10 @@ __host__ __device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t
   }
 }
 
-[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W,
-                                                                          const uint4* __restrict__ part,
-                                                                          uint2* __restrict__ pre, uint32_t min_heads,
-                                                                          uint32_t* __restrict__ ctr,
-                                                                          uint32_t* __restrict__ report) {
+template <bool INS>
+__global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, uint32_t W, const uint4* __restrict__ part,
+                                                  uint2* __restrict__ pre, uint32_t min_heads, uint32_t* __restrict__ ctr,
+                                                  uint32_t* __restrict__ report) {
   __shared__ uint4 s_wave[17];  // wave aggregates, then their prefixes; [16] = carry
   const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, i = blockIdx.x * RBS_PER + tid;
   const LW x = i < W ? lw_unpack(st[i]) : lw_none();
@@ -212,7 +231,7 @@ __host__ __device__ __forceinline__ bool lw_put(LW p, LW x, uint32_t w, uint32_t
   }
   __syncthreads();
   if (i >= W) return;
-  if (lw_put(lw_combine(lw_unpack(s_wave[wid]), ex), x, i, W, pre, min_heads)) lw_raise(ctr, report);
+  if (lw_put<INS>(lw_combine(lw_unpack(s_wave[wid]), ex), x, i, W, pre, min_heads)) lw_raise(ctr, report);
 }
 
 // The regions a batch must have, 24 (insert) or 25 (delete) per 32 keys
@@ -228,8 +247,9 @@ static inline uint32_t lw_min_heads(bool insert, uint32_t n, uint32_t W) {
 }
 
 static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
-static inline gqf_status lw_scan(hipStream_t s, DeviceState& ds, Arena& ar, const uint4* st, uint32_t W, uint2* pre,
-                                 uint32_t min_heads) {
+template <bool INS>
+static gqf_status lw_scan(hipStream_t s, DeviceState& ds, Arena& ar, const uint4* st, uint32_t W, uint2* pre,
+                          uint32_t min_heads) {
   const uint32_t P = (W + RBS_PER - 1) / RBS_PER;
   uint4* part = ar.take<uint4>(P ? P : 1);
   if (ar.used > ar.cap) {
@@ -238,11 +258,11 @@ static inline gqf_status lw_scan(hipStream_t s, DeviceState& ds, Arena& ar, cons
   }
   *reinterpret_cast<volatile uint32_t*>(ds.h_local) = 0u;
   if (W <= LW_ONE * 1024) {
-    GQF_LAUNCH(k_lw_one, dim3(1), dim3(1024), 0, s, st, W, pre, min_heads, ds.counters, ds.d_local);
+    GQF_LAUNCH(k_lw_one<INS>, dim3(1), dim3(1024), 0, s, st, W, pre, min_heads, ds.counters, ds.d_local);
     return GQF_OK;
   }
   GQF_LAUNCH(k_lw_reduce, dim3(P), dim3(RBS_PER), 0, s, st, W, part, ds.counters);
-  GQF_LAUNCH(k_lw_scan, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, min_heads, ds.counters, ds.d_local);
+  GQF_LAUNCH(k_lw_scan<INS>, dim3(P), dim3(RBS_PER), 0, s, st, W, part, pre, min_heads, ds.counters, ds.d_local);
   return GQF_OK;
 }
 // After the call's work: whether the localized form took the batch.
@@ -278,6 +298,10 @@ __global__ __launch_bounds__(256) void k_wm_bounds(const K* __restrict__ B, uint
   if (gt % WB_LANES == 0 && x <= W) bstart[x] = b;
 }
 
+// The largest value of the lanes of a wave.
+__device__ __forceinline__ int32_t lw_wave_max(int32_t x) {
+  return (int32_t)(wave_read(wave_incl_max((uint32_t)x ^ 0x80000000u), 63) ^ 0x80000000u);
+}
 // Heads among the 64 keys [k0, k0 + 64) of a window, one per lane, from
 // v = E_k - k (valid lanes only) and the running maximum M of the keys before
 // (initially the overflow into the window): bit of the calling lane.

@@ -26,15 +26,6 @@ constexpr uint32_t RL_HALO = 45;
 constexpr uint32_t RL_BLOCKS = 64 + RL_HALO;
 constexpr uint32_t RL_E_BITS = 13;  // a key's word: E_k or the head bit, D above
 
-// Whether a region that overflows into a window ends in the blocks held of it
-// (`room` empty slots there): it takes a slot for each of the at most LW_SPILL
-// keys of the windows before and for each of the window's keys that it takes
-// with it -- those before the first with E_k - k >= LW_SPILL, at most
-// (`chained`: the first with E_k - k >= the overflow starts a region).
-__host__ __device__ __forceinline__ bool rl_holds(uint32_t chained, uint32_t room) {
-  return (uint32_t)LW_SPILL + chained <= room;
-}
-
 __host__ __device__ __forceinline__ void rl_xor(unsigned long long* p, uint64_t d) {
 #ifdef __HIP_DEVICE_COMPILE__
   if (d) atomicXor(p, (unsigned long long)d);
@@ -341,7 +332,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
   if (blk >= nb) mask = 0;
   s_mask[lane] = mask;
   uint32_t e = 0, first = LW_SLOTS, last = 0;
-  uint32_t room = ~0u, chained = nk;  // insert: what a region that overflows into the window finds, and takes
+  int32_t held = 1 << 20;  // insert: empty slots of the blocks that the window before may hold (a short last window: all)
   bool bad = nk > LW_KEYS;
   if (INS) {
     if (blk < nb) empty[blk] = mask;
@@ -349,8 +340,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
     s_pre[lane] = inc - c;
     e = wave_read(inc, 63);
     if (w + 1 < W) bad = bad || e < (uint32_t)LW_SPILL;
-    // (a last window of fewer blocks is held whole)
-    if (after && nb > w * 64 + RL_HALO) room = wave_read(inc, RL_HALO - 1);
+    if (nb > w * 64 + RL_HALO) held = (int32_t)wave_read(inc, RL_HALO - 1);
   } else {
     const uint32_t own = mask ? 64 * lane + 64 - (uint32_t)__clzll(mask) : 0u;
     const uint32_t inc = wave_incl_max(own);
@@ -362,11 +352,11 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       const uint32_t lo = wave_read((uint32_t)mask, (int)fl), hi = wave_read((uint32_t)(mask >> 32), (int)fl);
       first = 64 * fl + (uint32_t)__builtin_ctzll(((uint64_t)hi << 32) | lo);
     }
-    bad = bad || first == LW_SLOTS || (after && first > 64 * RL_HALO);
+    bad = bad || first == LW_SLOTS;
   }
   __syncthreads();
-  int32_t M = 0;
-  uint32_t heads = 0;
+  int32_t M = 0, fit = held - (int32_t)nk;
+  uint32_t heads = 0, last_key = 0;  // delete: 1 + the window's last key (0: none)
   if (nk <= LW_KEYS) {
     uint32_t prev = 0;  // delete: 1 + the key before the group (0: none)
     const K kbase = (K)base << r;
@@ -382,16 +372,16 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       uint32_t info;
       if (INS) {
         info = s_pre[bk] + (uint32_t)__popcll(m & below);
-        const int32_t v = (int32_t)info - (int32_t)k;
+        const int32_t v = (int32_t)info - (int32_t)k, f = lw_fit(v, held, (int32_t)k);
+        if (on && f > fit) fit = f;
         head = lw_insert_head(v, on, M);
-        const uint64_t past = __ballot(on && v >= LW_SPILL);
-        if (past && chained == nk) chained = k0 + (uint32_t)__builtin_ctzll(past);
       } else {
         const uint64_t at = m & (below | (1ull << (rel & 63u)));
         const uint32_t lb = at ? 64 * bk + 64 - (uint32_t)__clzll(at) : s_pre[bk];
         uint32_t p = dpp_u32<DPP_WAVE_SHR1>(0u, rel + 1);
         if (lane == 0) p = prev;
         prev = wave_read(rel + 1, 63);
+        last_key = wave_read(rel + 1, (int)((nk - 1 - k0) & 63u));
         head = on && lb > p;
         info = head ? 1u : 0u;
       }
@@ -401,13 +391,15 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       if (k0 + 64 <= nk && hm == 0) bad = true;
     }
   }
-  bad = __any(bad || (INS && !rl_holds(chained, room)));
+  bad = __any(bad);
+  if (INS) fit = lw_wave_max(fit);
   if (lane == 0) {
-    const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
-    int32_t b = INS && nk ? M + a : 0;
+    const int32_t a = INS ? (int32_t)nk - (int32_t)e : -2;
+    int32_t b = INS ? (nk ? M + a : 0) : last <= last_key;
     if (b < 0) b = 0;
     if (bad) b = LW_BAD;
-    st[w] = lw_pack(LW{a, b, last ? base + last : 0u, heads});
+    const uint32_t lb = INS ? lw_room(fit) : (last ? base + last : 0u) | (first > 64 * RL_HALO ? LW_FAR : 0u);
+    st[w] = lw_pack(LW{a, b, lb, heads});
     if (!INS) fb[w] = (uint16_t)first;
   }
 }
@@ -492,7 +484,7 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
       for (; need > 1; --need) em &= em - 1ull;
       for (;;) {  // the empty slot that the region's last key takes
         while (em == 0 && c + 1 < nb && c + 1 < bw + RL_BLOCKS) em = empty[++c];
-        if (em == 0) break;  // not reached: the plan found room (rl_holds)
+        if (em == 0) break;  // not reached: the scan found room (lw_room)
         hi = 64 * (c - bw) + (uint32_t)__builtin_ctzll(em);
         em &= em - 1ull;
         if (k1 >= n || (uint32_t)(B[k1] >> rr) > base + hi) break;
@@ -500,8 +492,8 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
       }
     }
   } else {
-    if (w + 1 < W && fb[w + 1]) hi = LW_SLOTS + fb[w + 1] - 1;
     uint32_t hp = (uint32_t)(B[b1 - 1] >> rr);
+    if (w + 1 < W && fb[w + 1] && pre[w + 1].y <= hp + 1) hi = LW_SLOTS + fb[w + 1] - 1;  // no boundary after the last key
     while (k1 < n) {
       const uint32_t h = (uint32_t)(B[k1] >> rr), w2 = h / LW_SLOTS;
       if (h - w2 * LW_SLOTS >= fb[w2] || pre[w2].y > hp + 1) break;
@@ -510,7 +502,7 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
     }
   }
   uint32_t held = hi / 64 + 1;  // blocks held
-  if (held > RL_BLOCKS) held = RL_BLOCKS;  // not reached: the plan's bounds
+  if (held > RL_BLOCKS) held = RL_BLOCKS;  // not reached: the scan's bounds
   if (lane < held - 64) load(64 + lane);
   for (uint32_t i = 64 * rr + lane; i < held * rr; i += 64) {
     const uint64_t at = (uint64_t)bw * rr + i;

@@ -9,7 +9,8 @@
 namespace gqf {
 
 // ---------------------------------------------------------------- one key
-// Both work on any accessor a with a.get(slot) (elements at or past the last
+// An update on single elements: what SlPlanes does on bits, step by step, for
+// the checks of the region rules on the CPU.  Both work on any accessor a with a.get(slot) (elements at or past the last
 // slot S read as 0) and a.put(slot, element), on a canonical table.  Slots
 // before b, the last slot at or before fq that is empty or holds an entry at
 // its own quotient, belong to earlier quotients' runs and play no part.
@@ -103,6 +104,11 @@ __host__ __device__ __forceinline__ void sl_erase(A& a, uint32_t S, uint32_t fq,
   if (single) a.put(fq, a.get(fq) & ~4u);
 }
 
+// Blocks of the next window that a region may reach: 7.6 KB of LDS, 21 waves
+// per CU (16: 8.1 KB; 2^20-key steps 309 us, 11: 300).
+constexpr uint32_t SL_HALO = 11;
+constexpr uint32_t SL_BLOCKS = 64 + SL_HALO;
+
 // ---------------------------------------------------------------- plan
 // One wave per window.  Insert: el[i] = E_k within the window of batch key i,
 // the state (a, b).  Delete: el[i] = 1 iff a boundary of the window lies
@@ -141,10 +147,12 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
   const uint64_t mask = (INS ? ~(x.occ | x.cont | x.shf) : ~x.shf) & valid;
   s_mask[lane] = mask;
   uint32_t e = 0, first = LW_SLOTS, last = 0;
+  int32_t held = 1 << 20;  // empty slots of the blocks that the window before may hold (a short last window: all)
   if (INS) {
     const uint32_t c = (uint32_t)__popcll(mask), inc = wave_incl_add(c);
     s_pre[lane] = (uint16_t)(inc - c);
     e = wave_read(inc, 63);
+    if (base + 64 * SL_HALO < S) held = (int32_t)wave_read(inc, SL_HALO - 1);
   } else {
     // 1 + the last boundary before each 64-slot block
     const uint32_t own = mask ? 64 * lane + 64 - (uint32_t)__clzll(mask) : 0u;
@@ -160,8 +168,8 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
   }
   __syncthreads();
   bool bad = nk > LW_KEYS || (INS ? e < (uint32_t)LW_SPILL && w + 1 < W : first == LW_SLOTS);
-  int32_t M = 0;
-  uint32_t heads = 0;
+  int32_t M = 0, fit = held - (int32_t)nk;
+  uint32_t heads = 0, end = 0;  // delete: 1 + the window's last key (0: none)
   if (!bad) {
     uint32_t prev = 0;  // delete: 1 + the key before the group (0: none)
     for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
@@ -174,13 +182,16 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
       if (INS) {
         const uint32_t E = s_pre[blk] + (uint32_t)__popcll(m & ((1ull << (rel & 63u)) - 1ull));
         if (on) el[b0 + k] = (uint16_t)E;
-        head = lw_insert_head((int32_t)E - (int32_t)k, on, M);
+        const int32_t v = (int32_t)E - (int32_t)k, f = lw_fit(v, held, (int32_t)k);
+        if (on && f > fit) fit = f;
+        head = lw_insert_head(v, on, M);
       } else {
         const uint64_t at = m & ((2ull << (rel & 63u)) - 1ull);
         const uint32_t lb = at ? 64 * blk + 64 - (uint32_t)__clzll(at) : s_pre[blk];
         uint32_t p = dpp_u32<DPP_WAVE_SHR1>(0u, rel + 1);
         if (lane == 0) p = prev;
         prev = wave_read(rel + 1, 63);
+        end = wave_read(rel + 1, (int)((nk - 1 - k0) & 63u));
         head = on && lb > p;  // boundary lb - 1 after the key p - 1
         if (on) el[b0 + k] = head ? 1 : 0;
       }
@@ -189,12 +200,14 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
       if (k0 + 64 <= nk && hm == 0) bad = true;
     }
   }
+  if (INS) fit = lw_wave_max(fit);
   if (lane == 0) {
-    const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
-    int32_t b = INS && nk ? M + a : 0;
+    const int32_t a = INS ? (int32_t)nk - (int32_t)e : -2;
+    int32_t b = INS ? (nk ? M + a : 0) : last <= end;
     if (b < 0) b = 0;
     if (bad) b = LW_BAD;
-    st[w] = lw_pack(LW{a, b, last ? base + last : 0u, heads});
+    const uint32_t lb = INS ? lw_room(fit) : (last ? base + last : 0u) | (first > 64 * SL_HALO ? LW_FAR : 0u);
+    st[w] = lw_pack(LW{a, b, lb, heads});
     if (!INS) fb[w] = (uint16_t)first;
   }
 }
@@ -214,8 +227,6 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
 // written); the rebuild's decode, state and write passes take 250 us.  As
 // many deletes take 104 us, 160 when every run start that moves was paired
 // with its quotient one by one; decode, mark and rebuild take 290 us.
-constexpr uint32_t SL_HALO = 11;  // 7.6 KB of LDS, 21 waves per CU (16: 8.1 KB; 2^20-key steps 309 us, now 300)
-constexpr uint32_t SL_BLOCKS = 64 + SL_HALO;
 
 __host__ __device__ __forceinline__ void lds_xor(unsigned long long* p, uint64_t d) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -427,35 +438,6 @@ struct SlPlanes {
   }
 };
 
-// The same window as single elements, and the table outside it (sl_insert,
-// sl_erase): for a region that leaves the slots held.
-template <int BPE>
-struct SlAcc {
-  SlPlanes<BPE>& m;
-  uint8_t* t;
-  uint32_t S, base;
-  __device__ __forceinline__ uint32_t get(uint32_t i) const {
-    const uint32_t s = i - base;
-    if (s >= m.end) return sqf_get<BPE>(t, S, i);
-    return (m.get_rem(s) << 3) | (m.bit(m.occ, s) ? 4u : 0u) | (m.bit(m.cont, s) ? 2u : 0u) | (m.bit(m.shf, s) ? 1u : 0u);
-  }
-  __device__ __forceinline__ void put(uint32_t i, uint32_t e) {
-    const uint32_t s = i - base;
-    if (s < m.end) {
-      const uint64_t b = 1ull << (s & 63);
-      if (m.bit(m.occ, s) != ((e & 4u) != 0)) lds_xor(&m.occ[s >> 6], b);
-      if (m.bit(m.cont, s) != ((e & 2u) != 0)) lds_xor(&m.cont[s >> 6], b);
-      if (m.bit(m.shf, s) != ((e & 1u) != 0)) lds_xor(&m.shf[s >> 6], b);
-      m.put_rem(s, e >> 3);
-      m.mark(s >> 6, s >> 6);
-    } else if (i < S) {
-      uint8_t* p = t + (size_t)i * BPE;
-      if (BPE == 2) p[0] = (uint8_t)(e >> 8);
-      p[BPE - 1] = (uint8_t)e;
-    }
-  }
-};
-
 // Bit i of n (4 bits) to bit 0 of byte i: the product's terms do not overlap.
 __device__ __forceinline__ uint32_t nib_bytes(uint32_t n) { return __umul24(n, 0x204081u) & 0x01010101u; }
 
@@ -552,20 +534,21 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
     uint32_t need = w + 1 < W ? pre[w + 1].x : 0u;
     if (need) {
       uint32_t cs = base + LW_SLOTS;
-      auto empties = [&]() { return __ballot(cs + lane < S && (sqf_get<BPE>(t, S, cs + lane) & 7u) == 0); };
+      const uint32_t stop = base + 64 * SL_BLOCKS < S ? base + 64 * SL_BLOCKS : S;  // (the scan found room before it)
+      auto empties = [&]() { return __ballot(cs + lane < stop && (sqf_get<BPE>(t, S, cs + lane) & 7u) == 0); };
       uint64_t em = empties();
-      while ((uint32_t)__popcll(em) < need && cs + 64 < S) {
+      while ((uint32_t)__popcll(em) < need && cs + 64 < stop) {
         need -= (uint32_t)__popcll(em);
         cs += 64;
         em = empties();
       }
       for (; need > 1; --need) em &= em - 1ull;
       for (;;) {  // the empty slot that the region's last key takes at the latest
-        while (em == 0 && cs + 64 < S) {
+        while (em == 0 && cs + 64 < stop) {
           cs += 64;
           em = empties();
         }
-        if (em == 0) break;  // not reached: the scan found room
+        if (em == 0) break;  // not reached
         hi = cs + (uint32_t)__builtin_ctzll(em) - base;
         em &= em - 1ull;
         if (k1 >= n || (B[k1] >> r) > base + hi) break;
@@ -573,8 +556,8 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
       }
     }
   } else {
-    if (w + 1 < W && fb[w + 1]) hi = LW_SLOTS + fb[w + 1] - 1;
     uint32_t hp = B[b1 - 1] >> r;
+    if (w + 1 < W && fb[w + 1] && pre[w + 1].y <= hp + 1) hi = LW_SLOTS + fb[w + 1] - 1;  // no boundary after the last key
     while (k1 < n) {
       const uint32_t h = B[k1] >> r, w2 = h / LW_SLOTS;
       if (h - w2 * LW_SLOTS >= fb[w2] || pre[w2].y > hp + 1) break;
@@ -582,8 +565,8 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
       ++k1;
     }
   }
-  const bool held = hi < 64 * SL_BLOCKS;
-  const uint32_t nb = held ? hi / 64 + 1 : 64u;  // blocks held
+  if (hi >= 64 * SL_BLOCKS) hi = 64 * SL_BLOCKS - 1;  // not reached: the scan's bounds
+  const uint32_t nb = hi / 64 + 1;  // blocks held
   if (lane < nb - 64) load(64 + lane);
   __syncthreads();
   const uint32_t h0 = (B[b0 + s_head[0]] >> r) - base;
@@ -615,19 +598,10 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
   const uint32_t rmask = (1u << r) - 1u;
   for (uint32_t ri = lane; ri < nh; ri += 64) {
     const uint32_t ka = b0 + s_head[ri], kb = ri + 1 < nh ? b0 + s_head[ri + 1] : k1;
-    if (held || ri + 1 < nh) {
-      for (uint32_t k = ka; k < kb; ++k) {
-        const uint32_t fp = B[k];
-        if (INS) m.insert((fp >> r) - base, fp & rmask);
-        else m.erase((fp >> r) - base, fp & rmask);
-      }
-    } else {
-      SlAcc<BPE> acc{m, t, S, base};
-      for (uint32_t k = ka; k < kb; ++k) {
-        const uint32_t fp = B[k];
-        if (INS) sl_insert(acc, S, fp >> r, fp & rmask);
-        else sl_erase(acc, S, fp >> r, fp & rmask);
-      }
+    for (uint32_t k = ka; k < kb; ++k) {
+      const uint32_t fp = B[k];
+      if (INS) m.insert((fp >> r) - base, fp & rmask);
+      else m.erase((fp >> r) - base, fp & rmask);
     }
   }
 #pragma unroll
@@ -640,7 +614,7 @@ __global__ __launch_bounds__(64) void k_sl_apply(uint8_t* __restrict__ t, uint32
   // in which an earlier window's region may end (before the first region) and
   // the one in which the last region ends
   const uint32_t lo = (INS ? pw.x > 0 : fbw > 0) ? h0 : 0u;
-  const uint32_t last = held && base + hi < S ? hi : (S - base < 64 * nb ? S - base - 1 : 64 * nb - 1);
+  const uint32_t last = base + hi < S ? hi : S - base - 1;
   for (uint32_t s = 16 * lane; s < 64 * nb; s += 1024) {
     const uint32_t blk = s >> 6;
     if (!((s_dirty[blk >> 5] >> (blk & 31)) & 1u)) continue;

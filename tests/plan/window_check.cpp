@@ -98,20 +98,22 @@ static Plan plan(const Table& t, const std::vector<uint64_t>& B, uint32_t min_he
       continue;
     }
     const char* m = mask.data() + base;
-    uint32_t e = 0, room = 0, first = LW_SLOTS, last = 0;
+    uint32_t e = 0, first = LW_SLOTS, last = 0, end = 0;
+    int32_t held = 0;
     for (uint32_t s = 0; s < LW_SLOTS; ++s)
       if (m[s]) {
         ++e;
-        if (s < 64 * RL_HALO) ++room;
+        if (s < 64 * RL_HALO) ++held;
         if (first == LW_SLOTS) first = s;
         last = s + 1;
         if (INS) p.empty[(base + s) >> 6] |= 1ull << (s & 63);
       }
     bool bad = nk > LW_KEYS;
     if (INS) bad = bad || (w + 1 < W && e < (uint32_t)LW_SPILL);
-    else bad = bad || first == LW_SLOTS || (after && first > 64 * RL_HALO);
-    int32_t M = 0;
-    uint32_t heads = 0, chained = nk;
+    else bad = bad || first == LW_SLOTS;
+    if (nb <= 64 * w + RL_HALO) held = 1 << 20;
+    int32_t M = 0, fit = held - (int32_t)nk;
+    uint32_t heads = 0;
     for (uint32_t k0 = 0; !bad && k0 < nk; k0 += 64) {
       bool any = false;
       for (uint32_t k = k0; k < std::min(nk, k0 + 64); ++k) {
@@ -123,31 +125,31 @@ static Plan plan(const Table& t, const std::vector<uint64_t>& B, uint32_t min_he
           p.info[b0 + k] = (uint32_t)E;
           head = v >= M;
           M = std::max(M, v);
-          if (v >= LW_SPILL && chained == nk) chained = k;
+          fit = std::max(fit, lw_fit(v, held, (int32_t)k));
         } else {
           uint32_t lb = 0;
           for (uint32_t z = 0; z <= s; ++z)
             if (m[z]) lb = z + 1;
           head = lb > (k ? (uint32_t)(B[b0 + k - 1] >> r) - base + 1 : 0u);
           p.info[b0 + k] = head;
+          end = s + 1;
         }
         any |= head;
         heads += head;
       }
       if (k0 + 64 <= nk && !any) bad = true;
     }
-    if (INS && after && nb > 64 * w + RL_HALO) bad = bad || !rl_holds(chained, room);
-    const int32_t a = INS ? (int32_t)nk - (int32_t)e : 0;
-    int32_t b = INS && nk ? M + a : 0;
+    const int32_t a = INS ? (int32_t)nk - (int32_t)e : -2;
+    int32_t b = INS ? (nk ? M + a : 0) : last <= end;
     if (b < 0) b = 0;
     if (bad) b = LW_BAD;
-    p.st[w] = LW{a, b, last ? base + last : 0u, heads};
+    p.st[w] = LW{a, b, INS ? lw_room(fit) : (last ? base + last : 0u) | (first > 64 * RL_HALO ? LW_FAR : 0u), heads};
     p.fb[w] = first;
   }
   p.pre.resize(W);
   LW acc{0, 0, 0u, 0u};
   for (uint32_t w = 0; w < W; ++w) {
-    if (lw_put(acc, p.st[w], w, W, p.pre.data(), min_heads)) p.ok = false;
+    if (lw_put<INS>(acc, p.st[w], w, W, p.pre.data(), min_heads)) p.ok = false;
     acc = lw_combine(acc, p.st[w]);
   }
   return p;
@@ -198,8 +200,8 @@ static void apply(Table& t, const Plan& p, const std::vector<uint64_t>& B, uint3
       }
     }
   } else {
-    if (w + 1 < p.W && p.fb[w + 1]) hi = LW_SLOTS + p.fb[w + 1] - 1;
     uint32_t hp = (uint32_t)(B[b1 - 1] >> r);
+    if (w + 1 < p.W && p.fb[w + 1] && p.pre[w + 1].y <= hp + 1) hi = LW_SLOTS + p.fb[w + 1] - 1;
     while (k1 < n) {
       const uint32_t h = (uint32_t)(B[k1] >> r), w2 = h / LW_SLOTS;
       if (h - w2 * LW_SLOTS >= p.fb[w2] || p.pre[w2].y > hp + 1) break;
@@ -316,8 +318,9 @@ int main() {
         std::sort(B.begin(), B.end());
         const int before = accepted[0];
         both(base, B, nb, g, 1000 * x + c);
-        // (64 empty slots and `spare` more: x keys and those taken along fit)
-        if (x <= 64 && 64 + c <= 64 + spare && accepted[0] == before) fail("handed over", 1000 * x + c, spare);
+        // (64 empty slots and `spare` more: the x keys and those taken along)
+        const bool room = x <= 64 && (x + c <= 64 + spare || c == 0);
+        if (room != (accepted[0] > before)) fail(room ? "handed over" : "accepted", 1000 * x + c, spare);
       }
   for (uint32_t it = 0; it < 700; ++it) {
     const uint32_t q = 12 + u(4), nb = (1u << q) / 64 + 1, N = 1u << q;

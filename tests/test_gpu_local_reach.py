@@ -94,3 +94,41 @@ def test_sqf_insert_across_a_window(x, c):
     fps = np.unique(insert_set(np.unique(O.fingerprints(stored, Q, r)), O.fingerprints(batch, Q, r)))
     sqf_equal(f, sqf_table(fps, Q, r))
     st.destroy()
+
+
+@pytest.mark.parametrize("past,local", [(20, True), (690, True), (760, False), (1500, False)])
+@pytest.mark.parametrize("q,r", [(20, 5), (17, 13)])
+def test_sqf_clusters_past_a_window(q, r, past, local):
+    """A cluster of shifted entries from a window's end to `past` slots into the
+    next: updates in it are localized while the slots are held, handed over
+    beyond that; updates before it are localized in any case."""
+    say("sqf cluster past a window", q, r, past)
+    lo = W0 + 4096 - 20
+    pool = O.mt19937(11, 1 << 25)
+    fp = O.fingerprints(pool, q, r)
+    fq = (fp >> np.uint64(r)).astype(np.int64)
+    sel = np.flatnonzero((fq >= lo) & (fq < W0 + 4096 + past))
+    _, first = np.unique(fq[sel], return_index=True)
+    key = pool[sel[first]]
+    assert len(key) == 20 + past
+    own = pool[fq == lo]
+    own = own[np.unique(O.fingerprints(own, q, r), return_index=True)[1]][:4]  # shift the others by 3
+    alone = pool[np.flatnonzero(fq == W0 + 100)[:1]]
+    f = G.SQF(q, r)
+    f.bulk_build(dev(np.concatenate([own, key[1:], alone])))
+    fps = np.unique(O.fingerprints(np.concatenate([own, key[1:], alone]), q, r))
+    inside = pool[np.flatnonzero((fq == lo + 5) & ~np.isin(fp, fps))[:1]]
+    for batch, is_local in ((inside, local), (pool[np.flatnonzero(fq == W0 + 50)[:1]], True)):
+        st = G.Stream()  # a context of its own: no batch of it has been handed over yet
+        names = _kernels(lambda: f.insert(dev(batch), stream=st))
+        fps = np.unique(insert_set(fps, O.fingerprints(batch, q, r)))
+        sqf_equal(f, sqf_table(fps, q, r))
+        assert any("k_rb_write" in x for x in names) == (not is_local)
+        st.destroy()
+    for batch, is_local in ((key[6:7], local), (alone, True), (inside, local)):
+        st = G.Stream()
+        names = _kernels(lambda: f.delete(dev(batch), stream=st))
+        fps = fps[~np.isin(fps, O.fingerprints(batch, q, r))]
+        sqf_equal(f, sqf_table(fps, q, r))
+        assert any("k_rb_write" in x for x in names) == (not is_local)
+        st.destroy()
