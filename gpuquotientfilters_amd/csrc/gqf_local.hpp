@@ -36,7 +36,8 @@
 // a whole aligned group
 // of 64 keys without a head, fewer than LW_SPILL empty slots in a
 // window (clusters longer than a window), an overflow above LW_SPILL, a
-// region that reaches past the blocks held of the next window, too few regions
+// region that reaches past the blocks held of the next window, a region that
+// would take longer than the general path (lw_budget), too few regions
 // (lw_scan).  After such a batch the next 4, 8, ... 256 of its
 // kind on the stream go straight to the general path.
 #pragma once
@@ -245,6 +246,75 @@ __global__ __launch_bounds__(1024) void k_lw_scan(const uint4* __restrict__ st, 
 static inline uint32_t lw_min_heads(bool insert, uint32_t n, uint32_t W) {
   return n < W ? 0u : (uint32_t)((uint64_t)n * (insert ? 24 : 25) / 32);
 }
+
+// The longest region a batch may have, in quarters of a microsecond of its
+// lane: a region is updated key after key, and every key moves the entries from
+// its place to the cluster's end.  A key's time on MI355X, with the 64-slot
+// blocks from its quotient to that end (single regions of 1 .. 60 keys in
+// clusters of 1 .. 32 blocks): a + b per block, lw_key.  Past the budget the
+// general path is the faster one: it takes about 75 us (RSQF inserts 65) and
+// 4.5 or more per 2^20 slots, the call without its longest region about 40.
+// Without this rule, us a call, localized / general path:
+//   SQF   q=22 r=5 fill 0.9   30011 keys deleted 326 / 111
+//   RSQF  q=20 r=8 fill 0.9   64 copies of a key inserted 477 / 68, deleted 971 / 175
+//         q=24 r=8 fill 0.9   100003 keys inserted 264 / 161, deleted 498 / 204
+//         q=26 r=8 fill 0.95  1000 keys, 16 different ones, deleted 5197 / 645
+static inline uint32_t lw_budget(bool rsqf_insert, uint64_t slots) {
+  return (uint32_t)((rsqf_insert ? 96 : 128) + 18 * slots / (1u << 20));
+}
+struct LwKey {
+  uint32_t a, b;
+};
+// SQF slots of bpe bytes; RSQF remainders of r bits.
+template <bool INS>
+__host__ __device__ __forceinline__ LwKey lw_key_sqf(uint32_t bpe) {
+  return INS ? (bpe == 1 ? LwKey{5, 3} : LwKey{4, 5}) : (bpe == 1 ? LwKey{7, 5} : LwKey{8, 7});
+}
+template <bool INS>
+__host__ __device__ __forceinline__ LwKey lw_key_rsqf(uint32_t r) {
+  return INS ? LwKey{5, 1 + r * 5 / 16} : LwKey{10, 3 + r / 2};
+}
+// The longest region among a window's keys, 64 at a time -- in a loop of its
+// own, which few windows need (may): a key's cluster spans no more blocks than
+// lie without empty slots (boundaries) together, and the two beside them.
+template <bool INS>
+struct LwChain {
+  LwKey key;
+  uint64_t nz;      // blocks with empty slots (insert) or boundaries (delete)
+  uint32_t spread;  // insert: sixteenths of a block to the next empty slot
+  uint32_t carry = 0, keys = 0, longest = 0;
+  __device__ __forceinline__ LwChain(LwKey k, uint64_t nz_, uint32_t empties)
+      : key(k), nz(nz_), spread(INS ? 1024u / (empties ? empties : 1u) : 0u) {}
+  // Whether the longest region of nk keys with so many heads may be past the
+  // budget.
+  __device__ __forceinline__ bool may(uint32_t nk, uint32_t heads, uint32_t budget) const {
+    const uint32_t most = nk - heads + 1u;
+    uint32_t gap = 2;
+    for (uint64_t z = ~nz; z; z &= z << 1) ++gap;
+    return most * (key.a + key.b * (gap + (most * spread >> 4))) > budget;
+  }
+  // A key of block blk and its slot s there, whose word of the plane is mask;
+  // the heads of the 64 keys: heads.
+  __device__ __forceinline__ void add(bool on, uint64_t mask, uint32_t s, uint32_t blk, bool head, uint64_t heads) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t n = 1;  // blocks to the cluster's end
+    if (!(mask & (INS ? ~0ull << s : ~((2ull << s) - 1ull)))) {
+      const uint64_t later = nz & ~((2ull << blk) - 1ull);
+      n += (later ? (uint32_t)__builtin_ctzll(later) : 64u) - blk;
+    }
+    if (INS) {  // the empty slots that the region's keys before it have taken
+      const uint64_t h = heads & ((2ull << lane) - 1ull);
+      const uint32_t before = h ? lane - 63u + (uint32_t)__clzll(h) : lane + keys;
+      n += before * spread >> 4;
+      keys = heads ? (uint32_t)__clzll(heads) + 1u : keys + 64u;
+    }
+    const uint32_t cost = on ? key.a + key.b * n : 0u, sum = wave_incl_add(cost);
+    const uint32_t from = wave_incl_max(head ? sum - cost + 1 : 0u);  // 1 + the costs before the last head
+    const uint32_t since = from ? sum + 1 - from : sum + carry;
+    carry = wave_read(since, 63);
+    longest = since > longest ? since : longest;
+  }
+};
 
 static inline size_t lw_scan_bytes(uint32_t W) { return aligned_bytes((size_t)((W + RBS_PER - 1) / RBS_PER) * 16); }
 template <bool INS>

@@ -1798,7 +1798,7 @@ static gqf_status rsqf_local(hipStream_t s, DeviceState& ds, Arena& ar, const gq
   const double mb = (double)g.nb * 16;  // occupieds + run ends
   GQF_LAUNCH_B(mb, k_rl_pop<K>, dim3((W + 63) / 64), dim3(1024), 0, s, d.meta, g.nb, W, B, n, g.r, bstart, dw, gs);
   GQF_LAUNCH_B(mb + (double)n * (sizeof(K) + 4), (k_rl_plan<K, INS>), dim3(W), dim3(64), 0, s, d.meta, g.nb, g.r, dw, gs, B,
-               bstart, W, key, empty, fb, st);
+               bstart, W, key, empty, fb, st, lw_budget(INS, g.cap));
   GQF_TRY((lw_scan<INS>(s, ds, ar, st, W, pre, lw_min_heads(INS, n, W))));
   uint64_t* meta = reinterpret_cast<uint64_t*>(f.blocks);
   uint64_t* remg = reinterpret_cast<uint64_t*>(reinterpret_cast<uint8_t*>(f.blocks) + rsqf_meta_bytes(g.nb));

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
                                                 const uint32_t* __restrict__ dw, const uint32_t* __restrict__ gs,
                                                 const K* __restrict__ B, const uint32_t* __restrict__ bstart, uint32_t W,
                                                 uint32_t* __restrict__ key, uint64_t* __restrict__ empty,
-                                                uint16_t* __restrict__ fb, uint4* __restrict__ st) {
+                                                uint16_t* __restrict__ fb, uint4* __restrict__ st, uint32_t budget) {
   __shared__ uint64_t s_mask[64], s_occ[64], s_end[64];
   __shared__ uint32_t s_pre[64];
   __shared__ int32_t s_D[64];
@@ -331,6 +331,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
   }
   if (blk >= nb) mask = 0;
   s_mask[lane] = mask;
+  const uint64_t nz = __ballot(mask != 0);
   uint32_t e = 0, first = LW_SLOTS, last = 0;
   int32_t held = 1 << 20;  // insert: empty slots of the blocks that the window before may hold (a short last window: all)
   bool bad = nk > LW_KEYS;
@@ -346,9 +347,8 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
     const uint32_t inc = wave_incl_max(own);
     s_pre[lane] = dpp_u32<DPP_WAVE_SHR1>(0u, inc);
     last = wave_read(inc, 63);
-    const uint64_t any = __ballot(mask != 0);
-    if (any) {
-      const uint32_t fl = (uint32_t)__builtin_ctzll(any);
+    if (nz) {
+      const uint32_t fl = (uint32_t)__builtin_ctzll(nz);
       const uint32_t lo = wave_read((uint32_t)mask, (int)fl), hi = wave_read((uint32_t)(mask >> 32), (int)fl);
       first = 64 * fl + (uint32_t)__builtin_ctzll(((uint64_t)hi << 32) | lo);
     }
@@ -357,6 +357,7 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
   __syncthreads();
   int32_t M = 0, fit = held - (int32_t)nk;
   uint32_t heads = 0, last_key = 0;  // delete: 1 + the window's last key (0: none)
+  LwChain<INS> chain(lw_key_rsqf<INS>(r), nz, e);
   if (nk <= LW_KEYS) {
     uint32_t prev = 0;  // delete: 1 + the key before the group (0: none)
     const K kbase = (K)base << r;
@@ -390,8 +391,19 @@ __global__ __launch_bounds__(64) void k_rl_plan(const uint64_t* __restrict__ met
       heads += (uint32_t)__popcll(hm);
       if (k0 + 64 <= nk && hm == 0) bad = true;
     }
+    if (nk && chain.may(nk, heads, budget)) {
+      int32_t M2 = 0;
+      for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
+        const uint32_t k = k0 + lane;
+        const bool on = k < nk;
+        const uint32_t rel = on ? (uint32_t)((B[b0 + k] - kbase) >> r) & (LW_SLOTS - 1) : 0u;
+        const uint32_t x = on ? key[b0 + k] & ((1u << RL_E_BITS) - 1u) : 0u;
+        const bool head = INS ? lw_insert_head((int32_t)x - (int32_t)k, on, M2) : on && x != 0;
+        chain.add(on, s_mask[rel >> 6], rel & 63u, rel >> 6, head, __ballot(head));
+      }
+    }
   }
-  bad = __any(bad);
+  bad = __any(bad || chain.longest > budget);
   if (INS) fit = lw_wave_max(fit);
   if (lane == 0) {
     const int32_t a = INS ? (int32_t)nk - (int32_t)e : -2;

@@ -333,7 +333,7 @@ static gqf_status sqf_local_t(hipStream_t s, DeviceState& ds, Arena& ar, const g
     return GQF_ERR_INVALID;
   }
   GQF_LAUNCH_B((double)g.bytes + (double)n * 6, (k_sl_plan<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S, g.r, B, n,
-               bstart, W, el, fb, st);
+               bstart, W, el, fb, st, lw_budget(false, g.S));
   GQF_TRY((lw_scan<INS>(s, ds, ar, st, W, pre, lw_min_heads(INS, n, W))));
   GQF_LAUNCH_B(2.0 * (double)g.bytes + (double)n * 6, (k_sl_apply<BPE, INS>), dim3(W), dim3(64), 0, s, wq.table, g.S,
                g.r, B, n, bstart, W, pre, el, fb, ds.counters);

@@ -10,10 +10,11 @@ namespace gqf {
 
 // ---------------------------------------------------------------- one key
 // An update on single elements: what SlPlanes does on bits, step by step, for
-// the checks of the region rules on the CPU.  Both work on any accessor a with a.get(slot) (elements at or past the last
-// slot S read as 0) and a.put(slot, element), on a canonical table.  Slots
-// before b, the last slot at or before fq that is empty or holds an entry at
-// its own quotient, belong to earlier quotients' runs and play no part.
+// the checks of the region rules on the CPU.  Both work on any accessor a with
+// a.get(slot) (elements at or past the last slot S read as 0) and a.put(slot,
+// element), on a canonical table.  Slots before b, the last slot at or before
+// fq that is empty or holds an entry at its own quotient, belong to earlier
+// quotients' runs and play no part.
 
 // The start of fq's run, or where it would start, given a non-empty slot fq.
 template <class A>
@@ -119,7 +120,7 @@ template <int BPE, bool INS>
 __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, uint32_t S, uint32_t r,
                                                 const uint32_t* __restrict__ B, uint32_t n,
                                                 uint32_t* __restrict__ bstart, uint32_t W, uint16_t* __restrict__ el,
-                                                uint16_t* __restrict__ fb, uint4* __restrict__ st) {
+                                                uint16_t* __restrict__ fb, uint4* __restrict__ st, uint32_t budget) {
   __shared__ uint64_t s_mask[64];
   __shared__ uint16_t s_pre[64];
   const uint32_t w = blockIdx.x, lane = threadIdx.x;
@@ -146,6 +147,7 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
   const uint64_t valid = s0 + 64 <= S ? ~0ull : (s0 < S ? (1ull << (S - s0)) - 1ull : 0ull);
   const uint64_t mask = (INS ? ~(x.occ | x.cont | x.shf) : ~x.shf) & valid;
   s_mask[lane] = mask;
+  const uint64_t nz = __ballot(mask != 0);
   uint32_t e = 0, first = LW_SLOTS, last = 0;
   int32_t held = 1 << 20;  // empty slots of the blocks that the window before may hold (a short last window: all)
   if (INS) {
@@ -159,9 +161,8 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
     const uint32_t inc = wave_incl_max(own);
     s_pre[lane] = (uint16_t)dpp_u32<DPP_WAVE_SHR1>(0u, inc);
     last = wave_read(inc, 63);
-    const uint64_t any = __ballot(mask != 0);
-    if (any) {
-      const uint32_t fl = (uint32_t)__builtin_ctzll(any);
+    if (nz) {
+      const uint32_t fl = (uint32_t)__builtin_ctzll(nz);
       const uint32_t lo = wave_read((uint32_t)mask, (int)fl), hi = wave_read((uint32_t)(mask >> 32), (int)fl);
       first = 64 * fl + (uint32_t)__builtin_ctzll(((uint64_t)hi << 32) | lo);
     }
@@ -170,6 +171,7 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
   bool bad = nk > LW_KEYS || (INS ? e < (uint32_t)LW_SPILL && w + 1 < W : first == LW_SLOTS);
   int32_t M = 0, fit = held - (int32_t)nk;
   uint32_t heads = 0, end = 0;  // delete: 1 + the window's last key (0: none)
+  LwChain<INS> chain(lw_key_sqf<INS>(BPE), nz, e);
   if (!bad) {
     uint32_t prev = 0;  // delete: 1 + the key before the group (0: none)
     for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
@@ -198,6 +200,17 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
       const uint64_t hm = __ballot(head);
       heads += (uint32_t)__popcll(hm);
       if (k0 + 64 <= nk && hm == 0) bad = true;
+    }
+    if (nk && chain.may(nk, heads, budget)) {
+      int32_t M2 = 0;
+      for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
+        const uint32_t k = k0 + lane;
+        const bool on = k < nk;
+        const uint32_t rel = on ? (B[b0 + k] >> r) - base : 0u, x = on ? el[b0 + k] : 0u;
+        const bool head = INS ? lw_insert_head((int32_t)x - (int32_t)k, on, M2) : on && x != 0;
+        chain.add(on, s_mask[(rel >> 6) & 63u], rel & 63u, (rel >> 6) & 63u, head, __ballot(head));
+      }
+      if (__any(chain.longest > budget)) bad = true;
     }
   }
   if (INS) fit = lw_wave_max(fit);

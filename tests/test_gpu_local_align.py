@@ -36,7 +36,7 @@ def test_tables_off_a_16_byte_boundary(q, r, off):
         fps = np.unique(O.fingerprints(keys, q, r))
         S = G.SQF.num_slots(q)
         new = O.mt19937(501 + q, S)
-        for n in (1, 65, S // 82):
+        for n in (1, 65, S // 200):
             names = _kernels(lambda: f.insert(dev(new[:n]), stream=st))
             assert any("k_sl_apply" in x for x in names) and not any("k_rb_write" in x for x in names)
             fps = np.unique(insert_set(fps, O.fingerprints(new[:n], q, r)))
