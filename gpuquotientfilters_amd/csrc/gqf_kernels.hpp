@@ -1220,6 +1220,10 @@ __global__ __launch_bounds__(SEG_THREADS) void k_rs_seg_slow(K* __restrict__ key
 constexpr int ONE_THREADS = 1024;
 constexpr uint32_t ONE_TILE = ONE_THREADS * SORT_ITEMS;  // 16384 keys
 constexpr uint32_t ONE_BB = 14;
+// Crowded buckets (many copies of a few keys) of so few keys take Batcher's
+// bitonic network: the counting passes take 30 us for any number of keys, this
+// 10 (64 keys), 15 (512), 19 (1000) and 25 (2000); at 4000 it would take 40.
+constexpr uint32_t ONE_BITONIC = 2048;
 template <typename K>
 __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restrict__ in, K* __restrict__ out, uint32_t n,
                                                         uint32_t fp_bits, uint32_t nbits) {
@@ -1282,7 +1286,29 @@ __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restri
 #pragma unroll
       for (int i = 0; i < SORT_ITEMS; ++i) {
         const uint32_t at = 4 * T * (i / 4) + 4 * tid + (i & 3);
-        if (at < n) out[at] = (K)k[i];
+        if (at < n) {
+          if (n <= ONE_BITONIC) s_keys[at] = k[i];
+          else out[at] = (K)k[i];
+        }
+      }
+      if (n <= ONE_BITONIC) {
+        uint32_t N = 2;
+        while (N < n) N *= 2;
+        for (uint32_t p = n + tid; p < N; p += T) s_keys[p] = ~0u;
+        __syncthreads();
+        for (uint32_t run = 2; run <= N; run *= 2)
+          for (uint32_t j = run / 2; j; j /= 2) {
+            for (uint32_t p = tid; p < N / 2; p += T) {
+              const uint32_t lo = 2 * p - (p & (j - 1)), a = s_keys[lo], b = s_keys[lo + j];
+              if ((a > b) == ((lo & run) == 0)) {
+                s_keys[lo] = b;
+                s_keys[lo + j] = a;
+              }
+            }
+            __syncthreads();
+          }
+        for (uint32_t p = tid; p < n; p += T) out[p] = (K)s_keys[p];
+        return;
       }
       __syncthreads();
       seg_counting_sort<K, T>(out, n, nbits, s_keys, reinterpret_cast<uint16_t*>(s_c), s_tmp);
