@@ -34,6 +34,19 @@ constexpr int PL_THREADS = 512;
 // 216 : 225.
 constexpr uint64_t PL_MIN = 7u << 19;
 constexpr uint32_t PL_QMIN_SQF = 20, PL_QMIN_RSQF = 24;
+// SQF walks through long clusters: the group's walk takes as many steps as the
+// direct one, with a workgroup per group (256 up to q = 23) and the way there
+// and back on top.  64ths of a step of 32 slots per key (0.3 steps at fill
+// 0.85, 0.85 at 0.9, 3.7 at 0.95, 8 at 0.97, 71 when full) up to which the
+// groups stay ahead.  us, direct : by groups, for 2^22 and 2^24 keys: q = 20 at
+// 0.85 158 : 147, 553 : 458, at 0.9 240 : 317, 863 : 1032; q = 23 at 0.85
+// 154 : 145, 544 : 406, at 0.9 242 : 264, 862 : 816; q = 24 at 0.95
+// 554 : 503, 2026 : 1801, at 0.98 1590 : 1672, 5833 : 5694, full 7685 : 13122,
+// 28264 : 45663; q = 26 at 0.98 889 : 698, 3274 : 2081.
+// Counted in PL_SAMPLE of the groups (by all of them, one counter for the waves
+// takes 125 us at q = 26; a sum in the gather, 5 to 8).
+constexpr uint32_t PL_SAMPLE = 64, PL_SAMPLE_WAVES = PL_SAMPLE * (PL_THREADS / 64);
+inline uint32_t pl_steps_max(uint32_t q) { return q <= 23 ? 40 : q == 24 ? 400 : 1280; }
 
 struct PlPlan {
   PsPlan p;
@@ -60,7 +73,7 @@ inline bool pl_plan(uint64_t n, uint32_t q, uint32_t r, uint32_t qmin, PlPlan* o
 }
 static inline size_t pl_bytes(const PlPlan& o, uint64_t n) {
   const size_t nd = o.p.ngroups;
-  return aligned_bytes(nd * o.p.cap * 4) + aligned_bytes(nd * 4) + aligned_bytes(n * 2) +
+  return aligned_bytes(nd * o.p.cap * 4) + aligned_bytes((nd + 2) * 4) + aligned_bytes(n * 2) +
          aligned_bytes(o.tiles * nd * 4) + aligned_bytes(o.tiles * nd * 2) + 4096;
 }
 
@@ -89,10 +102,11 @@ __device__ __forceinline__ uint32_t pl_select(uint32_t x, uint32_t k) {
 
 // sqf_lookup_win's walk for the quotient at `at` in the loaded slots (end of
 // them, at least 32 before `at`): the slot, SQF_NOT_FOUND or PL_PENDING.  In
-// 32-bit steps from where the walk stands, not words of the table: 64-bit
+// 32-bit steps from where the walk stands (counted), not words of the table: 64-bit
 // shifts and counts of whole words took 142 us at 2^24 keys.
 __device__ __forceinline__ uint32_t pl_sqf_walk(const uint32_t* s_raw, const uint32_t* s_occ, const uint32_t* s_cont,
-                                                const uint32_t* s_shf, uint32_t end, uint32_t at, uint32_t fr) {
+                                                const uint32_t* s_shf, uint32_t end, uint32_t at, uint32_t fr,
+                                                uint32_t& steps) {
   uint32_t s = at - 31, occ = pl_bits(s_occ, s);  // (bit 31: the quotient's)
   if (!(occ >> 31)) return SQF_NOT_FOUND;
   // the cluster's start, and the run starts to skip after it
@@ -100,6 +114,7 @@ __device__ __forceinline__ uint32_t pl_sqf_walk(const uint32_t* s_raw, const uin
   while (ns == 0) {
     k += (uint32_t)__popc(occ);
     if (s < 32) return PL_PENDING;
+    ++steps;
     s -= 32;
     ns = ~pl_bits(s_shf, s);
     occ = pl_bits(s_occ, s);
@@ -113,6 +128,7 @@ __device__ __forceinline__ uint32_t pl_sqf_walk(const uint32_t* s_raw, const uin
     while ((c = (uint32_t)__popc(rs)) < k) {
       k -= c;
       s += 32;
+      ++steps;
       if (s + 32 > end) return PL_PENDING;
       rs = ~pl_bits(s_cont, s);
     }
@@ -157,14 +173,29 @@ __device__ __forceinline__ void pl_each(uint32_t* p, uint32_t m, F walk) {
   }
 }
 
+// The sampled waves' steps and how many of the waves are done, in one word; the
+// last wave compares.  *crowded: raised for more than 64 steps_max steps.
+__device__ __forceinline__ void pl_count(unsigned long long* steps, uint32_t took, uint32_t steps_max,
+                                         uint32_t* crowded) {
+  for (int x = 32; x; x >>= 1) took += (uint32_t)__shfl_xor((int)took, x);
+  if (threadIdx.x & 63u) return;
+  const uint32_t sum = took >> 6;
+  const unsigned long long old = atomicAdd(steps, ((unsigned long long)sum << 16) + 1ull);
+  if ((uint32_t)(old & 0xFFFFu) == PL_SAMPLE_WAVES - 1 && (old >> 16) + sum > steps_max) *crowded = 1u;
+}
+
 // Group blockIdx.x of a table of 1-byte slots (16-byte aligned, S slots).
 [[maybe_unused]] static __global__ __launch_bounds__(PL_THREADS) void k_pl_sqf(
     const uint8_t* __restrict__ t, uint32_t S, uint32_t qb, uint32_t r, const uint32_t* __restrict__ gsize, uint32_t cap,
-    uint32_t* __restrict__ io) {
+    uint32_t* __restrict__ io, unsigned long long* __restrict__ steps, uint32_t steps_max, uint32_t* __restrict__ crowded) {
   __shared__ __align__(16) uint32_t s_raw[PL_SLOTS / 4];
   __shared__ uint32_t s_occ[PL_WORDS], s_cont[PL_WORDS], s_shf[PL_WORDS];
   const uint32_t g = blockIdx.x, q0 = g << qb, m = gsize[g] < cap ? gsize[g] : cap;
-  if (m == 0) return;
+  const bool sampled = g % (gridDim.x / PL_SAMPLE) == 0;
+  if (m == 0) {
+    if (sampled) pl_count(steps, 0u, steps_max, crowded);
+    return;
+  }
   // (group 0: PL_BACK slots that read as empty stand before slot 0, a cluster
   // start to the walk as slot 0 itself is)
   const uint32_t lo = q0 - PL_BACK, end = (1u << qb) + PL_BACK + PL_FWD;
@@ -193,10 +224,12 @@ __device__ __forceinline__ void pl_each(uint32_t* p, uint32_t m, F walk) {
   __syncthreads();
   uint32_t* p = io + (uint64_t)g * cap;
   const uint32_t qmask = (1u << qb) - 1u, rmask = (1u << r) - 1u;
+  uint32_t took = 0;
   pl_each(p, m, [&](uint32_t key) {
-    const uint32_t a = pl_sqf_walk(s_raw, s_occ, s_cont, s_shf, end, ((key >> r) & qmask) + PL_BACK, key & rmask);
+    const uint32_t a = pl_sqf_walk(s_raw, s_occ, s_cont, s_shf, end, ((key >> r) & qmask) + PL_BACK, key & rmask, took);
     return a >= PL_PENDING ? a : a + lo;
   });
+  if (sampled) pl_count(steps, took, steps_max, crowded);
 }
 
 // The direct walk, for k_pl_gather.
@@ -211,7 +244,8 @@ struct SqfWalk {
 
 // ---------------------------------------------------------------- answers
 // Tile blockIdx.x: the answers of its keys from the groups' regions, in the
-// order of the keys; direct(key): the walk in the table.
+// order of the keys; direct(key): the walk in the table.  *crowded is raised
+// for keys without a place in their region.
 template <typename Walk>
 __global__ __launch_bounds__(PS_THREADS) void k_pl_gather(Walk direct, const uint32_t* __restrict__ keys, uint32_t n,
                                                           uint32_t nd, uint32_t tile, uint32_t cap, uint32_t lanes,
@@ -300,12 +334,13 @@ __global__ __launch_bounds__(PS_THREADS) void k_pl_gather(Walk direct, const uin
 }
 
 // ---------------------------------------------------------------- host
-// After the call: a stream whose keys crowd into few groups takes the direct
-// walk for its next calls.
+// After the call: a stream whose keys crowd into few groups, or whose walks
+// are long, takes the direct walk for its next calls.
 static inline void pl_report(DeviceState& ds, LocalKind k) {
   lw_report(ds, k, *static_cast<volatile uint32_t*>(ds.h_local) == 0);
 }
-// walks(gsize, cap, io) launches the walks of all groups.  No host wait.
+// walks(gsize, cap, io, steps) launches the walks of all groups; steps: a
+// cleared word of 64 bits.  No host wait.
 template <bool WIDE, typename Walk, typename F>
 static gqf_status pl_lookup(hipStream_t s, DeviceState& ds, const PlPlan& o, const uint32_t* keys, uint32_t fp_bits,
                             uint32_t n, uint32_t* out, const Walk& direct, F walks) {
@@ -313,7 +348,7 @@ static gqf_status pl_lookup(hipStream_t s, DeviceState& ds, const PlPlan& o, con
   const uint32_t nd = p.ngroups, bits = p.shift + p.gb, hbits = bits > 32 ? bits - 32 : 0u;
   Arena ar(ds.ws, ds.ws_cap);
   uint32_t* mid = ar.take<uint32_t>((size_t)nd * p.cap);
-  uint32_t* gsize = ar.take<uint32_t>(nd);
+  uint32_t* gsize = ar.take<uint32_t>(nd + 2);
   uint16_t* place = ar.take<uint16_t>((size_t)n + 4);
   uint32_t* tbase = ar.take<uint32_t>((size_t)o.tiles * nd);
   uint16_t* tfirst = ar.take<uint16_t>((size_t)o.tiles * nd);
@@ -322,10 +357,10 @@ static gqf_status pl_lookup(hipStream_t s, DeviceState& ds, const PlPlan& o, con
     return GQF_ERR_INVALID;
   }
   *ds.h_local = 0;
-  GQF_LAUNCH(k_ps_reset, dim3(1), dim3(PS_THREADS), 0, s, gsize, nd, ds.counters);
+  GQF_LAUNCH(k_ps_reset, dim3(1), dim3(PS_THREADS), 0, s, gsize, nd + 2, ds.counters);
   GQF_LAUNCH_B((double)n * 10.0, (k_ps_scatter<WIDE, true>), dim3(p.wgs), dim3(PS_THREADS), 0, s, keys, n, fp_bits,
                p.shift, nd, hbits, p.tile, p.cap, gsize, mid, ds.counters, PsBack{place, tbase, tfirst});
-  walks(gsize, p.cap, mid);
+  walks(gsize, p.cap, mid, reinterpret_cast<unsigned long long*>(gsize + nd));
   GQF_LAUNCH_B((double)n * 10.0, (k_pl_gather<Walk>), dim3(o.tiles), dim3(PS_THREADS), 0, s, direct, keys, n, nd, p.tile,
                p.cap, o.lanes, tbase, tfirst, place, mid, out, ds.d_local);
   return GQF_OK;

@@ -2019,10 +2019,11 @@ static gqf_status rsqf_pl_lookup(hipStream_t s, DeviceState& ds, const gqf_rsqf&
   const RsqfDev d = rdev(f);
   const uint32_t bits = f.qbits + f.rbits;
   const double b = (double)d.nb * (32 + 8 * f.rbits) + (double)n * 8.0;
-  auto walks = [&](const uint32_t* gsize, uint32_t cap, uint32_t* io) {
+  auto walks = [&](const uint32_t* gsize, uint32_t cap, uint32_t* io, unsigned long long*) {
     if (f.rbits == 8) GQF_LAUNCH_B(b, k_pl_rsqf<8>, dim3(pl.p.ngroups), dim3(PL_THREADS), 0, s, d, pl.p.qb, gsize, cap, io);
     else GQF_LAUNCH_B(b, k_pl_rsqf<0>, dim3(pl.p.ngroups), dim3(PL_THREADS), 0, s, d, pl.p.qb, gsize, cap, io);
   };
+  // (offsets bound the walks: their steps are not counted)
   if (bits > 32) return pl_lookup<true>(s, ds, pl, keys, bits, n, out, RsqfWalk{d, f.qbits}, walks);
   return pl_lookup<false>(s, ds, pl, keys, bits, n, out, RsqfWalk{d, f.qbits}, walks);
 }

@@ -564,11 +564,14 @@ gqf_status gqf_sqf_lookup(gqf_sqf qf, int sorted, int n, const uint32_t* d_keys,
     PlPlan pl;
     if (g.bpe == 1 && !g.packed && win && pl_plan(un, g.q, g.r, PL_QMIN_SQF, &pl) && lw_try(*cs.ds, LOCAL_SQF_LOOKUP) &&
         (pl_bytes(pl, un) <= cs.ds->ws_cap || ws_try_reserve(*cs.ds, pl_bytes(pl, un)))) {
+      const uint32_t steps_max = (uint32_t)((uint64_t)un * PL_SAMPLE / pl.p.ngroups * pl_steps_max(g.q) >> 12);
+      uint32_t* const slow = cs.ds->d_local;
       GQF_TRY(pl_lookup<false>(cs.stream, *cs.ds, pl, d_keys, (g.q + g.r) | sqf_hash_flag(), un, d_out,
                                SqfWalk{qf.table, g.S, g.q, g.r, sqf_hash_flag()},
-                               [&](const uint32_t* gsize, uint32_t cap, uint32_t* io) {
+                               [&](const uint32_t* gsize, uint32_t cap, uint32_t* io, unsigned long long* steps) {
                                  GQF_LAUNCH_B((double)g.bytes + (double)un * 8.0, k_pl_sqf, dim3(pl.p.ngroups),
-                                              dim3(PL_THREADS), 0, cs.stream, qf.table, g.S, pl.p.qb, g.r, gsize, cap, io);
+                                              dim3(PL_THREADS), 0, cs.stream, qf.table, g.S, pl.p.qb, g.r, gsize, cap, io,
+                                              steps, steps_max, slow);
                                }));
       GQF_TRY(cs.end(ms, false));
       pl_report(*cs.ds, LOCAL_SQF_LOOKUP);
