@@ -43,6 +43,20 @@ struct PsPlan {
   uint32_t gb, shift, ngroups, qb;  // digit bits, bits below them, 1 << gb, log2 of a group's quotients
   uint32_t tile, wgs, cap;          // keys per tile, workgroups of the partition, keys a group has room for
 };
+// The partition of n keys of a table of 2^q quotients: digits and tiles.  A
+// workgroup takes a CU's LDS: 256 of them, the same number of tiles each.
+// Returns the tiles.
+inline uint32_t ps_tiles(uint64_t n, uint32_t q, uint32_t r, PsPlan* p) {
+  p->gb = q > DB_QB + PS_GB_MIN ? q - DB_QB : PS_GB_MIN;
+  p->qb = q - p->gb;
+  p->shift = p->qb + r;
+  p->ngroups = 1u << p->gb;
+  const uint64_t rounds = (n + 256ull * PS_TILE - 1) / (256ull * PS_TILE);
+  p->tile = (uint32_t)(((n + 256 * rounds - 1) / (256 * rounds) + 3) & ~3ull);
+  const uint32_t tiles = (uint32_t)((n + p->tile - 1) / p->tile);
+  p->wgs = tiles < 256 ? tiles : 256;
+  return tiles;
+}
 // The plan of n keys into a table of 2^q quotients; false where the sort
 // applies: few keys (their launches count, not their moves), tables of more
 // than 2^26 quotients (more digits than runs of stores allow), remainders
@@ -55,15 +69,7 @@ struct PsPlan {
 constexpr uint32_t PS_MEAN_MAX = PS_TILE - 640, DB_LOAD_MAX = 208;
 inline bool ps_plan(uint64_t n, uint32_t q, uint32_t r, uint32_t sparse, PsPlan* p) {
   if (n <= 256ull * 7600 || n * sparse < (1ull << q) || q < 20 || q > DB_QB + PS_GB_MAX || r > 8 || n >= (1ull << 30)) return false;
-  p->gb = q > DB_QB + PS_GB_MIN ? q - DB_QB : PS_GB_MIN;
-  p->qb = q - p->gb;
-  p->shift = p->qb + r;
-  p->ngroups = 1u << p->gb;
-  // a workgroup takes a CU's LDS: 256 of them, the same number of tiles each
-  const uint64_t rounds = (n + 256ull * PS_TILE - 1) / (256ull * PS_TILE);
-  p->tile = (uint32_t)(((n + 256 * rounds - 1) / (256 * rounds) + 3) & ~3ull);
-  const uint64_t tiles = (n + p->tile - 1) / p->tile;
-  p->wgs = (uint32_t)(tiles < 256 ? tiles : 256);
+  (void)ps_tiles(n, q, r, p);
   const uint64_t mean = n >> p->gb, cap = (2 * mean + 2048 + 63) & ~63ull;
   if (mean > PS_MEAN_MAX || 32 * n > ((uint64_t)DB_LOAD_MAX << q)) return false;
   p->cap = (uint32_t)(cap < PS_TILE ? cap : PS_TILE);
@@ -238,7 +244,6 @@ __global__ __launch_bounds__(PS_THREADS) void k_ps_scatter(const uint32_t* __res
 // ---------------------------------------------------------------- runs
 // Group g: gsize[g] keys from g cap on, as many remainder bytes at most from
 // byte g cap on (cap: a multiple of 64).
-static_assert(DB_Q == 32, "a thread's occupied bits are one word");
 
 // LDS writes of the wave's lanes before, reads after.
 __device__ __forceinline__ void db_wave_sync() {

@@ -1224,9 +1224,9 @@ constexpr uint32_t ONE_BB = 14;
 // bitonic network: the counting passes take 30 us for any number of keys, this
 // 10 (64 keys), 15 (512), 19 (1000) and 25 (2000); at 4000 it would take 40.
 constexpr uint32_t ONE_BITONIC = 2048;
-template <typename K>
-__global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restrict__ in, K* __restrict__ out, uint32_t n,
-                                                        uint32_t fp_bits, uint32_t nbits) {
+[[maybe_unused]] static __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restrict__ in,
+                                                                                uint32_t* __restrict__ out, uint32_t n,
+                                                                                uint32_t fp_bits, uint32_t nbits) {
   constexpr int T = ONE_THREADS, W = T / 64;
   __shared__ __align__(16) uint32_t s_keys[ONE_TILE];
   __shared__ __align__(16) uint32_t s_c[(1u << ONE_BB) / 2];  // bucket counters / cursors; the counting passes' table
@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restri
 #pragma unroll
   for (int i = 0; i < SORT_ITEMS; ++i) {
     const uint32_t at = 4 * T * (i / 4) + 4 * tid + (i & 3);
-    k[i] = at < n ? (uint32_t)sort_load_key<K, true>(in, at, fp_bits) : 0u;
+    k[i] = at < n ? sort_load_key<uint32_t, true>(in, at, fp_bits) : 0u;
   }
   auto each = [&](auto f) {
 #pragma unroll
@@ -1288,7 +1288,7 @@ __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restri
         const uint32_t at = 4 * T * (i / 4) + 4 * tid + (i & 3);
         if (at < n) {
           if (n <= ONE_BITONIC) s_keys[at] = k[i];
-          else out[at] = (K)k[i];
+          else out[at] = k[i];
         }
       }
       if (n <= ONE_BITONIC) {
@@ -1307,11 +1307,11 @@ __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restri
             }
             __syncthreads();
           }
-        for (uint32_t p = tid; p < n; p += T) out[p] = (K)s_keys[p];
+        for (uint32_t p = tid; p < n; p += T) out[p] = s_keys[p];
         return;
       }
       __syncthreads();
-      seg_counting_sort<K, T>(out, n, nbits, s_keys, reinterpret_cast<uint16_t*>(s_c), s_tmp);
+      seg_counting_sort<uint32_t, T>(out, n, nbits, s_keys, reinterpret_cast<uint16_t*>(s_c), s_tmp);
       return;
     }
   }
@@ -1330,7 +1330,7 @@ __global__ __launch_bounds__(ONE_THREADS) void k_rs_one(const uint32_t* __restri
       const uint32_t y = s_keys[j];
       rank += (y < x || (y == x && j < p)) ? 1u : 0u;
     }
-    out[rank] = (K)x;
+    out[rank] = x;
   }
 }
 
@@ -1441,11 +1441,13 @@ gqf_status radix_sort(hipStream_t s, Arena& ar, const void* in, bool hash, uint3
     if (vals_out) *vals_out = vb[0];
     return GQF_OK;
   }
-  if (hash && !with_vals && lo_bit == 0 && hi_bit <= 32 && n <= ONE_TILE) {
-    GQF_LAUNCH_B((double)n * (4.0 + sizeof(K)), k_rs_one<K>, dim3(1), dim3(ONE_THREADS), 0, s,
-                 reinterpret_cast<const uint32_t*>(in), kb[0], n, fp_bits, hi_bit);
-    *keys_out = kb[0];
-    return GQF_OK;
+  if constexpr (sizeof(K) == 4) {
+    if (hash && !with_vals && lo_bit == 0 && hi_bit <= 32 && n <= ONE_TILE) {
+      GQF_LAUNCH_B((double)n * 8.0, k_rs_one, dim3(1), dim3(ONE_THREADS), 0, s, reinterpret_cast<const uint32_t*>(in),
+                   kb[0], n, fp_bits, hi_bit);
+      *keys_out = kb[0];
+      return GQF_OK;
+    }
   }
   if (n <= (uint32_t)SORT_TILE) {
     // one workgroup, every pass in LDS, one launch

@@ -76,6 +76,15 @@ static inline bool lw_auto(uint64_t n, uint64_t slots) { return n * (slots >= (8
 
 static inline uint32_t lw_windows(uint64_t slots) { return (uint32_t)((slots + LW_SLOTS - 1) / LW_SLOTS); }
 
+// Bits of a word that regions share: only a region's own change.
+__host__ __device__ __forceinline__ void lw_xor(unsigned long long* p, uint64_t d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (d) atomicXor(p, (unsigned long long)d);
+#else
+  *p ^= d;
+#endif
+}
+
 // Scan state of a window: the map x -> max(x + a, b), lb, and the keys that
 // start a region.
 //   insert  the overflow map; lb = 1 + the largest overflow into the window

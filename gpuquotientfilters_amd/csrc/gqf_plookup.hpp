@@ -57,14 +57,7 @@ struct PlPlan {
 inline bool pl_plan(uint64_t n, uint32_t q, uint32_t r, uint32_t qmin, PlPlan* o) {
   if (n < PL_MIN || q < qmin || q > DB_QB + PS_GB_MAX || r > 8 || n >= (1ull << 30)) return false;
   PsPlan& p = o->p;
-  p.gb = q > DB_QB + PS_GB_MIN ? q - DB_QB : PS_GB_MIN;
-  p.qb = q - p.gb;
-  p.shift = p.qb + r;
-  p.ngroups = 1u << p.gb;
-  const uint64_t rounds = (n + 256ull * PS_TILE - 1) / (256ull * PS_TILE);
-  p.tile = (uint32_t)(((n + 256 * rounds - 1) / (256 * rounds) + 3) & ~3ull);
-  o->tiles = (uint32_t)((n + p.tile - 1) / p.tile);
-  p.wgs = o->tiles < 256 ? o->tiles : 256;
+  o->tiles = ps_tiles(n, q, r, &p);
   const uint64_t mean = n >> p.gb;
   p.cap = (uint32_t)((mean + mean / 4 + 1024 + 63) & ~63ull);
   o->lanes = 3;

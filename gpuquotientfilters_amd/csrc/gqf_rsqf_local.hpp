@@ -26,14 +26,6 @@ constexpr uint32_t RL_HALO = 45;
 constexpr uint32_t RL_BLOCKS = 64 + RL_HALO;
 constexpr uint32_t RL_E_BITS = 13;  // a key's word: E_k or the head bit, D above
 
-__host__ __device__ __forceinline__ void rl_xor(unsigned long long* p, uint64_t d) {
-#ifdef __HIP_DEVICE_COMPILE__
-  if (d) atomicXor(p, (unsigned long long)d);
-#else
-  *p ^= d;
-#endif
-}
-
 // ---------------------------------------------------------------- one key
 // A window and the blocks after it that its last region reaches: occupied
 // and run-end bits and the remainder bit string (slot s at bits [s r, s r +
@@ -123,7 +115,7 @@ struct RlPlanes {
       }
     }
     if (p > e || y > e || e >= end) return;  // not reached: the region is held
-    if (!stored) rl_xor(&occ[fw], 1ull << (fq & 63));
+    if (!stored) lw_xor(&occ[fw], 1ull << (fq & 63));
     // run ends of [y, e]: those of [y, e) move up by one; slot y ends a run
     // iff the quotient is new
     uint64_t top = 0;
@@ -137,7 +129,7 @@ struct RlPlanes {
         v = (v & ~(1ull << (y & 63))) | ((stored ? 0ull : 1ull) << (y & 63));
       }
       if (w == ew) reg &= upto(e & 63);
-      rl_xor(&ends[w], (old ^ v) & reg);
+      lw_xor(&ends[w], (old ^ v) & reg);
     }
     // remainders of [p, e]
     const uint32_t b0 = p * rb(), b1 = (e + 1) * rb() - 1, i0 = b0 >> 6, i1 = b1 >> 6, o = b0 & 63;
@@ -155,7 +147,7 @@ struct RlPlanes {
       }
       if (i == i1) mask &= upto(b1 & 63);
       if (mask == ~0ull) rem[i] = v;
-      else rl_xor(&rem[i], (old ^ v) & mask);
+      else lw_xor(&rem[i], (old ^ v) & mask);
     }
     // entries of quotients below their first slots: one more in these blocks
     for (uint32_t j = fw + 1; j <= ew; ++j) off[j] += 1;
@@ -211,9 +203,9 @@ struct RlPlanes {
         v &= ~(1ull << (l & 63));
         reg &= upto(l & 63);
       }
-      rl_xor(&ends[w], (old ^ v) & reg);
+      lw_xor(&ends[w], (old ^ v) & reg);
     }
-    if (start == x) rl_xor(&occ[fw], 1ull << (fq & 63));
+    if (start == x) lw_xor(&occ[fw], 1ull << (fq & 63));
     // remainders of [p, l]; slot l's becomes 0
     const uint32_t b0 = p * rb(), bl = l * rb(), b1 = bl + rb() - 1, i0 = b0 >> 6, i1 = b1 >> 6;
     for (uint32_t i = i0; i <= i1; ++i) {
@@ -223,7 +215,7 @@ struct RlPlanes {
       if (i == i1) mask &= upto(b1 & 63);
       if (64 * i + 63 >= bl) v = 64 * i >= bl ? 0ull : v & ~from(bl & 63);
       if (mask == ~0ull) rem[i] = v;
-      else rl_xor(&rem[i], (old ^ v) & mask);
+      else lw_xor(&rem[i], (old ^ v) & mask);
     }
     for (uint32_t j = fw + 1; j <= lw; ++j) off[j] -= 1;
     mark(fw, lw);
@@ -574,8 +566,8 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
       *reinterpret_cast<uint4*>(rec) = make_uint4((uint32_t)s_occ[i], (uint32_t)(s_occ[i] >> 32), (uint32_t)s_end[i],
                                                   (uint32_t)(s_end[i] >> 32));
     } else {
-      rl_xor(reinterpret_cast<U*>(rec), (rec[0] ^ s_occ[i]) & x);
-      rl_xor(reinterpret_cast<U*>(rec) + 1, (rec[1] ^ s_end[i]) & x);
+      lw_xor(reinterpret_cast<U*>(rec), (rec[0] ^ s_occ[i]) & x);
+      lw_xor(reinterpret_cast<U*>(rec) + 1, (rec[1] ^ s_end[i]) & x);
     }
     if (s_off[i]) rec[2] = (rec[2] + (uint64_t)(int64_t)s_off[i]) & 0xFFull;
   }
@@ -593,7 +585,7 @@ __global__ __launch_bounds__(64) void k_rl_apply(uint64_t* __restrict__ meta, ui
       x &= 64 * i >= bit ? 0ull : (64 * i + 64 <= bit ? ~0ull : ~m.from(bit & 63));
     }
     if (x == ~0ull) *g = s_rem[i];
-    else if (x) rl_xor(reinterpret_cast<U*>(g), (*g ^ s_rem[i]) & x);
+    else if (x) lw_xor(reinterpret_cast<U*>(g), (*g ^ s_rem[i]) & x);
   }
 }
 

@@ -241,14 +241,6 @@ __global__ __launch_bounds__(64) void k_sl_plan(const uint8_t* __restrict__ t, u
 // many deletes take 104 us, 160 when every run start that moves was paired
 // with its quotient one by one; decode, mark and rebuild take 290 us.
 
-__host__ __device__ __forceinline__ void lds_xor(unsigned long long* p, uint64_t d) {
-#ifdef __HIP_DEVICE_COMPILE__
-  if (d) atomicXor(p, (unsigned long long)d);
-#else
-  *p ^= d;
-#endif
-}
-
 template <int BPE>
 struct SlPlanes {
   using E = typename std::conditional<BPE == 1, uint8_t, uint16_t>::type;
@@ -339,7 +331,7 @@ struct SlPlanes {
     const uint64_t fbit = 1ull << (fq & 63);
     const bool stored = (occ[fw] & fbit) != 0;
     if (((occ[fw] | cont[fw] | shf[fw]) & fbit) == 0) {
-      lds_xor(&occ[fw], fbit);
+      lw_xor(&occ[fw], fbit);
       put_rem(fq, fr);
       mark(fw, fw);
       return;
@@ -349,7 +341,7 @@ struct SlPlanes {
     if (s >= end || (stored && find(s, fr, &p))) return;
     const uint32_t e = next(p, [&](uint32_t w) { return ~(uint64_t)(occ[w] | cont[w] | shf[w]); });
     if (e >= end) return;  // not reached: the region is held
-    if (!stored) lds_xor(&occ[fw], fbit);
+    if (!stored) lw_xor(&occ[fw], fbit);
     // flags of [p, e]: the entries after p moved up by one, away from their
     // quotients; a run's old first entry continues it
     const bool first = p == s;
@@ -366,8 +358,8 @@ struct SlPlanes {
         if (p == fq) z = ~pb;
       }
       if (stored && first && (p + 1) >> 6 == w) c |= 1ull << ((p + 1) & 63);
-      lds_xor(&cont[w], (old ^ c) & reg);
-      lds_xor(&shf[w], ((uint64_t)shf[w] ^ z) & reg);
+      lw_xor(&cont[w], (old ^ c) & reg);
+      lw_xor(&shf[w], ((uint64_t)shf[w] ^ z) & reg);
     }
     uint64_t in = fr;
     const uint32_t i0 = p / PW, i1 = e / PW;
@@ -379,7 +371,7 @@ struct SlPlanes {
       const uint64_t mask = i == i1 ? up & (~0ull >> (64 - RB * (e % PW + 1))) : up;
       in = old >> (64 - RB);
       if (mask == ~0ull) rem[i] = v;
-      else lds_xor(&rem[i], (old ^ v) & mask);
+      else lw_xor(&rem[i], (old ^ v) & mask);
     }
     mark(fw, ew);
   }
@@ -429,10 +421,10 @@ struct SlPlanes {
         c &= ~pb;
         if (p == fq) z &= ~pb;
       }
-      lds_xor(&cont[w], (old ^ c) & reg);
-      lds_xor(&shf[w], ((uint64_t)shf[w] ^ z) & reg);
+      lw_xor(&cont[w], (old ^ c) & reg);
+      lw_xor(&shf[w], ((uint64_t)shf[w] ^ z) & reg);
     }
-    if (first && !more) lds_xor(&occ[fw], 1ull << (fq & 63));
+    if (first && !more) lw_xor(&occ[fw], 1ull << (fq & 63));
     const uint32_t i0 = p / PW, i1 = l / PW;
     for (uint32_t i = i0; i <= i1; ++i) {
       const uint64_t old = rem[i];
@@ -445,7 +437,7 @@ struct SlPlanes {
         mask &= ~0ull >> (64 - RB - at);
       }
       if (mask == ~0ull) rem[i] = v;
-      else lds_xor(&rem[i], (old ^ v) & mask);
+      else lw_xor(&rem[i], (old ^ v) & mask);
     }
     mark(fw, lw);
   }
