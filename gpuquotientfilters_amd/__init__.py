@@ -256,8 +256,9 @@ def sqf_insert_path():
 
 
 def set_rsqf_insert_path(path):
-    """How this thread's RSQF inserts update the table: INSERT_AUTO (default)
-    or INSERT_LOCAL (in place, window by window, falling back to the rebuild
+    """How this thread's RSQF inserts update the table: INSERT_AUTO (default:
+    small batches update only the slots they change, others as INSERT_LOCAL),
+    INSERT_LOCAL (in place, window by window, falling back to the rebuild
     where a window cannot be rewritten alone), INSERT_REBUILD (decode and
     rebuild every slot).  The resulting tables are the same."""
     check(lib().gqf_rsqf_set_insert_path(int(path)))

@@ -65,7 +65,9 @@ struct BTile {
 // crowded ones (many copies of a few).  A group of more keys than LDS holds
 // raises BS_HANDED before any key has moved: the kernels that follow leave
 // every table alone and the call launches the 8-bit passes (as do the batch's
-// next builds, for a while).
+// next builds, for a while).  The same 48 filters with half of the keys one
+// key: 0.26 ms a build by the passes, 0.36 when handed over; a workgroup for
+// each large group took 3.1.
 constexpr uint32_t BS_TOP = 0xFFFFFFFFu;
 constexpr uint32_t BS_HANDED = 0x80000000u;  // in `left`, and then every filter's error word
 __device__ __forceinline__ uint32_t bs_shift(uint32_t shift, uint32_t bits) {

@@ -32,14 +32,13 @@
 //   Work is per key and per keyed window; a window without keys is read only
 // when its predecessor has some (it must absorb what overflows).  Batches
 // that do not fit this form raise ctr[CTR_MISC] before anything is written
-// and the call takes its general path: more than LW_KEYS keys in a window,
-// a whole aligned group
-// of 64 keys without a head, fewer than LW_SPILL empty slots in a
-// window (clusters longer than a window), an overflow above LW_SPILL, a
-// region that reaches past the blocks held of the next window, a region that
-// would take longer than the general path (lw_budget), too few regions
-// (lw_scan).  After such a batch the next 4, 8, ... 256 of its
-// kind on the stream go straight to the general path.
+// and the call takes its general path: more than LW_KEYS keys in a window, a
+// whole aligned group of 64 keys without a head, fewer than LW_SPILL empty
+// slots in a window (clusters longer than a window), an overflow above
+// LW_SPILL, a region that reaches past the blocks held of the next window, a
+// region that would take longer than the general path (lw_budget), too few
+// regions (lw_scan).  After such a batch the next 4, 8, ... 256 of its kind on
+// the stream go straight to the general path.
 #pragma once
 
 #include "gqf_rebuild.hpp"
